@@ -21,12 +21,14 @@
 //     the cell counts writes par_entry into the stream; a pack kernel moves
 //     the cells and a one-workgroup kernel writes the header: no host prefix
 //     sum, no host sync (reference phases 1-4 + two syncs).
-//   decode: one wave per partition: 64 lanes decode equal spans of its bits
-//     speculatively and settle the span starts in rounds (a prefix code
-//     resynchronises within a few codewords), a 4096-entry prefix table
-//     yields the symbol of any code of up to 12 bits in one LDS probe and
-//     longer codes' lengths come from per-length limit compares; symbols are
-//     staged in LDS and leave in 16-byte stores.
+//   decode: a 2048-entry prefix table in LDS yields the symbol of any code
+//     of up to 11 bits in one probe, chained tables those of longer ones.
+//     Short streams: one wave per partition, 64 lanes decode equal spans of
+//     its bits speculatively and settle the span starts in rounds (a prefix
+//     code resynchronises within a few codewords); symbols are staged in LDS
+//     and leave in 16-byte stores.  Long streams: one lane per partition.
+#include <type_traits>
+
 #include "fzh_scan.h"
 
 namespace fzh {
@@ -279,33 +281,41 @@ huf_header_kernel(uint8_t* __restrict__ out, uint64_t n, uint32_t bklen, uint32_
 // gives each lane its output offset; a last decode of each span writes its
 // symbols to LDS and the wave stores the partition with 16-byte stores.
 //
-// Per codeword: a probe of a 2^12-entry table (length and symbol -- the
-// symbol itself for 1- and 2-byte keys -- of every code of up to 12 bits);
-// the 12-bit prefixes of longer codes point into a second table indexed by
-// the next B2 bits (B2 chosen so the table fits; all long codes of typical
-// books); codes longer still take the canonical comparison against the
-// per-length limits first[l] << (32 - l), which do not increase with l
-// (first[l] = round((first[l+1] + numl[l+1]) / 2)), so the length is one
-// more than the number of limits above the window (the bit loop of
-// hf_kernels.cu:258-312 in a few compares).  A window with no code of the
-// book decodes as a 31-bit code with a flag that fails the partition, so
-// the loops never branch on it.  Bits come from a 64-bit register buffer
-// refilled from the partition's cells in LDS.
+// Per codeword: a probe of a 2^11-entry table (length and symbol -- the
+// symbol itself for 1- and 2-byte keys -- of every code of up to 11 bits);
+// the prefixes of longer codes point into a second table indexed by as many
+// more bits as fit, its long prefixes into a third, and so on (all codes
+// that occur in typical books); codes longer still take the canonical
+// comparison against the per-length limits first[l] << (32 - l), which do
+// not increase with l (first[l] = round((first[l+1] + numl[l+1]) / 2)), so
+// the length is one more than the number of limits above the window (the
+// bit loop of hf_kernels.cu:258-312 in a few compares).  A window with no
+// code of the book decodes as a 31-bit code with a flag that fails the
+// partition, so the loops never branch on it.  Bits come from a 64-bit
+// register buffer refilled from the partition's cells in LDS.
 //
 // A partition's cells are staged in LDS when they fit (DEC_CELLS cells and
 // partitions of at most DEC_SUBLEN_MAX symbols, which covers the coarse 768
 // and fine 1024 layouts); any other partition is decoded by the same steps
 // reading its cells from memory and writing its symbols there.
-constexpr int DEC_LUT_BITS = 12;
-constexpr uint32_t DEC_LUT2 = 1024;  // second-level entries
+constexpr int DEC_LUT_BITS = 11;
+constexpr uint32_t DEC_LUT2 = 2048;     // entries of the second level, at most
+constexpr uint32_t DEC_POOL = 3072;     // entries of the levels after the first
+constexpr int DEC_LEVELS = 4;           // levels after the first
 constexpr uint32_t DEC_CELLS = 448;
 constexpr uint32_t DEC_SUBLEN_MAX = 1024;
 constexpr uint32_t DEC_INVALID = 0xFFFFFFFFu;
-// table entry: value (symbol, or key index with DEC_KEY) in bits 0-23,
-// code length in bits 24-28
+// Table entry: value (symbol, or key index with DEC_KEY) in bits 0-23, code
+// length in bits 24-28.  An entry with DEC_LONG is the prefix of longer
+// codes and says where the next level's probe goes on: the window shifted
+// left by bits 0-4, right by bits 5-9, plus the row's word offset in bits
+// 10-23; DEC_DEEP where no level follows.
 constexpr uint32_t DEC_KEY = 1u << 29;
 constexpr uint32_t DEC_BAD = (1u << 30) | (31u << 24);  // no code: skip 31 bits, fail
-constexpr uint32_t DEC_LONG = 1u << 31;                 // first level: prefix of a longer code
+constexpr uint32_t DEC_LONG = 1u << 31;
+constexpr uint32_t DEC_DEEP = DEC_LONG | DEC_KEY;
+constexpr uint32_t dec_probe(uint32_t row, uint32_t shl, uint32_t bits) { return (row << 10) | ((32 - bits) << 5) | shl; }
+constexpr uint32_t DEC_LEVEL1 = dec_probe(0, 0, DEC_LUT_BITS);
 
 // waves per workgroup: the tables are built once per workgroup, so
 // workgroups are large; 4-byte keys halve it to keep the LDS under 64 KiB
@@ -313,25 +323,38 @@ template <typename T>
 constexpr int dec_waves() { return sizeof(T) == 4 ? 4 : 8; }
 
 struct DecTables {
-    const uint32_t* lut;   // DEC_LUT_BITS-bit prefix -> entry, or DEC_LONG | prefix
-    const uint32_t* lut2;  // long prefix, next b2 bits -> entry; 0 = longer code or none
+    const uint32_t* lut;   // the levels one after another
     const uint64_t* lim;   // first[l] << (32 - l)
     const int32_t* diff;   // entry[l] - first[l]
-    uint32_t maxl, nkeys, b2;
+    uint32_t maxl, nkeys;
 };
 
-// Entry of a code longer than DEC_LUT_BITS bits at the head of W, given its
-// first-level entry e.
-__device__ __forceinline__ uint32_t dec_long(const DecTables& t, uint32_t W, uint32_t e) {
-    if (t.b2) {
-        const uint32_t e2 = t.lut2[((e & 0xFFFFu) << t.b2) | ((W << DEC_LUT_BITS) >> (32 - t.b2))];
-        if (e2) return e2;
-    }
+// The entry that the probe st (DEC_LEVEL1 or a DEC_LONG entry) finds at W.
+__device__ __forceinline__ uint32_t dec_lookup(const DecTables& t, uint32_t W, uint32_t st) {
+    return t.lut[((st >> 10) & 0x3FFFu) + ((W << (st & 31u)) >> ((st >> 5) & 31u))];
+}
+
+// Entry of the code at the head of W, longer than every table level holds.
+__device__ __forceinline__ uint32_t dec_deep(const DecTables& t, uint32_t W) {
     uint32_t lv = DEC_LUT_BITS + 1;
     for (uint32_t l = DEC_LUT_BITS + 1; l < t.maxl; l++) lv += (uint64_t)W < t.lim[l] ? 1u : 0u;
     const uint32_t k = (W >> (32 - lv)) + (uint32_t)t.diff[lv];
     if (lv > t.maxl || (uint64_t)W < t.lim[lv] || k >= t.nkeys) return DEC_BAD;
     return (lv << 24) | DEC_KEY | k;
+}
+
+// Entry of a code longer than DEC_LUT_BITS bits at the head of W, given its
+// first-level entry e.
+__device__ __forceinline__ uint32_t dec_long(const DecTables& t, uint32_t W, uint32_t e) {
+    if (e < DEC_DEEP) {
+        e = dec_lookup(t, W, e);
+        if ((int32_t)e >= 0) return e;
+        while (e < DEC_DEEP) {  // rows name later levels only
+            e = dec_lookup(t, W, e);
+            if ((int32_t)e >= 0) return e;
+        }
+    }
+    return dec_deep(t, W);
 }
 
 __device__ __forceinline__ uint32_t dec_entry(const DecTables& t, uint32_t W) {
@@ -487,108 +510,183 @@ __device__ __forceinline__ bool dec_partition(const uint32_t* cells, uint32_t nc
     return true;
 }
 
+// The stream's header fields, checked against n and the buffer size.
+constexpr int cdiv_c(int a, int b) { return (a + b - 1) / b; }
+
+struct DecHead {
+    uint32_t sublen, pardeg, e1, nkeys, ncells;
+    const uint32_t* par_nbit;
+    const uint32_t* par_entry;
+    const uint32_t* cells;
+};
+
 template <typename T>
-__global__ void __launch_bounds__(64 * dec_waves<T>())
-huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
-               int* __restrict__ d_status) {
-    constexpr bool FOLD = sizeof(T) <= 2;
-    constexpr int DEC_WAVES = dec_waves<T>();
-    __shared__ uint32_t s_first[32], s_entry[32];
-    __shared__ uint64_t s_lim[32];
-    __shared__ int32_t s_diff[32];
-    __shared__ uint32_t s_lut[1 << DEC_LUT_BITS];
-    __shared__ uint32_t s_lut2[DEC_LUT2];
-    __shared__ uint32_t s_cells[DEC_WAVES][DEC_CELLS + 4];
-    __shared__ uint4 s_out[DEC_WAVES][DEC_SUBLEN_MAX * sizeof(T) / 16];
-    if (in_bytes < HDR_BYTES) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *d_status = 1;
-        return;
-    }
+__device__ __forceinline__ bool dec_head(const uint8_t* __restrict__ in, uint64_t in_bytes, uint64_t n, DecHead& h) {
+    if (in_bytes < HDR_BYTES) return false;
     const int32_t sublen = *reinterpret_cast<const int32_t*>(in + 4);
     const int32_t pardeg = *reinterpret_cast<const int32_t*>(in + 8);
     const uint32_t* ent = reinterpret_cast<const uint32_t*>(in + 40);
     const uint32_t e1 = ent[1], e2 = ent[2], e3 = ent[3], e4 = ent[4], e5 = ent[5];
-    const bool hdr_ok = sublen > 0 && pardeg >= 0 && (uint64_t)pardeg == (n + sublen - 1) / sublen &&
-                        e1 <= e2 && e2 - e1 >= 256 && (e2 - e1 - 256) / sizeof(T) <= 65536 && e2 <= e3 &&
-                        e3 <= e4 && e4 <= e5 && e5 <= in_bytes && e3 - e2 == 4ull * pardeg &&
-                        e4 - e3 == 4ull * pardeg && (e4 % 4) == 0 && (e1 % 4) == 0;
-    if (!hdr_ok) {
+    if (!(sublen > 0 && pardeg >= 0 && (uint64_t)pardeg == (n + sublen - 1) / sublen && e1 <= e2 && e2 - e1 >= 256 &&
+          (e2 - e1 - 256) / sizeof(T) <= 65536 && e2 <= e3 && e3 <= e4 && e4 <= e5 && e5 <= in_bytes &&
+          e3 - e2 == 4ull * pardeg && e4 - e3 == 4ull * pardeg && (e4 % 4) == 0 && (e1 % 4) == 0))
+        return false;
+    h.sublen = (uint32_t)sublen;
+    h.pardeg = (uint32_t)pardeg;
+    h.e1 = e1;
+    h.nkeys = (e2 - e1 - 256) / sizeof(T);
+    h.ncells = (e5 - e4) / 4;
+    h.par_nbit = reinterpret_cast<const uint32_t*>(in + e2);
+    h.par_entry = reinterpret_cast<const uint32_t*>(in + e3);
+    h.cells = reinterpret_cast<const uint32_t*>(in + e4);
+    return true;
+}
+
+struct DecLds {
+    uint32_t lut[(1 << DEC_LUT_BITS) + DEC_POOL];
+    uint64_t lim[32];
+    int32_t diff[32];
+};
+
+// One table level: entry i (of `count`) stands for the window whose top
+// bits are i in L0 + b bits; codes of (L0, L0 + b] bits get their entry,
+// longer ones longer(i).  A code's length is the first l at which its top
+// l bits reach first[l] (the bit loop of hf_kernels.cu:258-312); fv holds
+// first[l] in lane l, so the compares are independent and their operands
+// scalar, and a thread's keys are loaded together.
+template <typename T, int BLOCK, int PER, typename F>
+__device__ __forceinline__ void dec_level(uint32_t* tab, uint32_t count, uint32_t l0, uint32_t b, uint32_t fv,
+                                          const int32_t* diff, const T* __restrict__ keys, uint32_t nkeys, F&& longer) {
+    constexpr bool FOLD = sizeof(T) <= 2;
+    for (uint32_t i0 = threadIdx.x; i0 < count; i0 += BLOCK * PER) {
+        uint32_t W[PER], lv[PER], k[PER], key[PER];
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            W[i] = (i0 + i * BLOCK) << (32 - l0 - b);
+            lv[i] = 0;
+        }
+        for (uint32_t l = l0 + b; l > l0; l--) {
+            const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)fv, (int)l);
+#pragma unroll
+            for (int i = 0; i < PER; i++)
+                if ((W[i] >> (32 - l)) >= f) lv[i] = l;
+        }
+#pragma unroll
+        for (int i = 0; i < PER; i++) k[i] = lv[i] ? (W[i] >> (32 - lv[i])) + (uint32_t)diff[lv[i]] : 0u;
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            key[i] = FOLD && lv[i] && k[i] < nkeys ? (uint32_t)keys[k[i]] : (DEC_KEY | k[i]);
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            if (i0 + i * BLOCK < count)
+                tab[i0 + i * BLOCK] =
+                    lv[i] == 0 ? longer(i0 + i * BLOCK) : (k[i] >= nkeys ? DEC_BAD : (lv[i] << 24) | key[i]);
+    }
+}
+
+// Builds the tables of the stream's book (all BLOCK threads; ends with a
+// barrier).
+template <typename T, int BLOCK>
+__device__ __forceinline__ DecTables dec_build(const uint8_t* __restrict__ in, const DecHead& h, DecLds& t,
+                                               bool& zero_len) {
+    const uint32_t* fb = reinterpret_cast<const uint32_t*>(in + h.e1);
+    const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
+    const uint32_t nkeys = h.nkeys;
+    // lane l < 32 of every wave: first[l], entry[l]; is l a code length of the book?
+    const uint32_t l32 = (uint32_t)lane_id() & 31u;
+    const uint32_t fv = fb[l32], en = fb[32 + l32], en1 = l32 < 31 ? fb[33 + l32] : nkeys;
+    const uint32_t used = (uint32_t)__ballot(l32 > 0 && en1 > en);
+    // the longest length a window can have: the last with a code, or the
+    // first at which every value is one (first[l] = 0)
+    const uint32_t all = (uint32_t)__ballot(l32 > 0 && fv == 0);
+    uint32_t maxl = used ? 31u - (uint32_t)__builtin_clz(used) : 1u;
+    if (all) maxl = min(maxl, (uint32_t)__builtin_ctz(all));
+    zero_len = (uint32_t)__builtin_amdgcn_readlane((int)en, 1) == 1;
+    if (threadIdx.x < 32) {
+        t.lim[threadIdx.x] = threadIdx.x ? (uint64_t)fv << (32 - threadIdx.x) : ~0ull;
+        t.diff[threadIdx.x] = (int32_t)(en - fv);
+    }
+    __syncthreads();
+    // The long codes' prefixes are [0, first[l]) at every length l (the
+    // smallest values of their lengths), so a level is indexed by the prefix
+    // that is still long and as many more bits as fit its part of the pool.
+    uint32_t lev_l[DEC_LEVELS], lev_b[DEC_LEVELS], lev_n[DEC_LEVELS], lev_o[DEC_LEVELS];
+    uint32_t at = DEC_LUT_BITS, off = 1u << DEC_LUT_BITS;
+#pragma unroll
+    for (int j = 0; j < DEC_LEVELS; j++) {
+        const uint32_t room = (1u << DEC_LUT_BITS) + DEC_POOL - off;
+        const uint32_t cap = j == 0 ? DEC_LUT2 : room - room / 4;
+        const uint32_t c = maxl > at ? (uint32_t)__builtin_amdgcn_readlane((int)fv, (int)at) : 0u;
+        uint32_t b = 0;
+        if (c > 0)
+            while (b < maxl - at && ((uint64_t)c << (b + 1)) <= cap) b++;
+        lev_l[j] = at;
+        lev_b[j] = b;
+        lev_n[j] = b ? c << b : 0u;
+        lev_o[j] = off;
+        off += lev_n[j];
+        at += b;
+    }
+    const auto next = [&](int j, uint32_t i) {  // entry of a code longer than the level before level j
+        return j < DEC_LEVELS && lev_b[j] ? DEC_LONG | dec_probe(lev_o[j] + (i << lev_b[j]), lev_l[j], lev_b[j])
+                                          : DEC_DEEP;
+    };
+    dec_level<T, BLOCK, cdiv_c(1 << DEC_LUT_BITS, BLOCK)>(t.lut, 1u << DEC_LUT_BITS, 0, DEC_LUT_BITS, fv, t.diff, keys,
+                                                          nkeys, [&](uint32_t i) { return next(0, i); });
+#pragma unroll
+    for (int j = 0; j < DEC_LEVELS; j++)
+        if (lev_n[j])
+            dec_level<T, BLOCK, 4>(t.lut + lev_o[j], lev_n[j], lev_l[j], lev_b[j], fv, t.diff, keys, nkeys,
+                                   [&](uint32_t i) { return next(j + 1, i); });
+    __syncthreads();
+    return DecTables{t.lut, t.lim, t.diff, maxl, nkeys};
+}
+
+// A partition whose book has one symbol with a zero-length code.
+template <typename T>
+__device__ __forceinline__ void dec_constant(T* __restrict__ dst, uint32_t cnt, T v) {
+    for (uint32_t j = (uint32_t)lane_id(); j < cnt; j += 64) dst[j] = v;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64 * dec_waves<T>())
+huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
+               int* __restrict__ d_status) {
+    constexpr int DEC_WAVES = dec_waves<T>();
+    __shared__ DecLds s_tab;
+    __shared__ uint32_t s_cells[DEC_WAVES][DEC_CELLS + 4];
+    __shared__ uint4 s_out[DEC_WAVES][DEC_SUBLEN_MAX * sizeof(T) / 16];
+    DecHead h;
+    if (!dec_head<T>(in, in_bytes, n, h)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) *d_status = 1;
         return;
     }
-    const uint32_t nkeys = (e2 - e1 - 256) / sizeof(T);
-    const T* keys = reinterpret_cast<const T*>(in + e1 + 256);
-    if (threadIdx.x < 32) {
-        const uint32_t f = reinterpret_cast<const uint32_t*>(in + e1)[threadIdx.x];
-        const uint32_t en = reinterpret_cast<const uint32_t*>(in + e1 + 128)[threadIdx.x];
-        s_first[threadIdx.x] = f;
-        s_entry[threadIdx.x] = en;
-        s_lim[threadIdx.x] = threadIdx.x ? (uint64_t)f << (32 - threadIdx.x) : ~0ull;
-        s_diff[threadIdx.x] = (int32_t)(en - f);
-    }
-    __syncthreads();
-    // longest code of the book: the last length with a symbol (entry[l+1] > entry[l])
-    uint32_t maxl = 1;
-    for (uint32_t l = 1; l < 31; l++)
-        if (s_entry[l + 1] > s_entry[l]) maxl = l;
-    if (s_entry[31] < nkeys) maxl = 31;
-    // The canonical loop on the window W from length l0 up to length lmax:
-    // the entry of the code, DEC_BAD when the window starts no code of the
-    // book, or (first level) DEC_LONG | (W's 12-bit prefix) for a code longer
-    // than 12 bits; 0 (second level) for a code longer than lmax.
-    auto canon = [&](uint32_t W, uint32_t l0, uint32_t lmax, bool first_level) -> uint32_t {
-        for (uint32_t lv = l0; lv <= lmax; lv++) {
-            const uint32_t v = W >> (32 - lv);
-            if (!(v < s_first[lv])) {
-                const uint32_t k = s_entry[lv] + v - s_first[lv];
-                if (k >= nkeys) return DEC_BAD;
-                return (lv << 24) | (FOLD ? (uint32_t)keys[k] : (DEC_KEY | k));
-            }
-        }
-        return first_level ? (DEC_LONG | (W >> (32 - DEC_LUT_BITS))) : 0u;
-    };
-    for (uint32_t pat = threadIdx.x; pat < (1u << DEC_LUT_BITS); pat += blockDim.x)
-        s_lut[pat] = canon(pat << (32 - DEC_LUT_BITS), 1, DEC_LUT_BITS, true);
-    // second level: the long codes' 12-bit prefixes are [0, first[12]) (the
-    // smallest values of their lengths); B2 more bits index it
-    const uint32_t n_long = maxl > (uint32_t)DEC_LUT_BITS ? s_first[DEC_LUT_BITS] : 0u;
-    uint32_t b2 = 0;
-    if (n_long > 0)
-        while (b2 < maxl - DEC_LUT_BITS && (n_long << (b2 + 1)) <= DEC_LUT2) b2++;
-    for (uint32_t i = threadIdx.x; i < (b2 ? n_long << b2 : 0u); i += blockDim.x) {
-        const uint32_t W = ((i >> b2) << (32 - DEC_LUT_BITS)) | ((i & ((1u << b2) - 1u)) << (32 - DEC_LUT_BITS - b2));
-        s_lut2[i] = canon(W, DEC_LUT_BITS + 1, DEC_LUT_BITS + b2, false);
-    }
-    __syncthreads();
-    const DecTables tb{s_lut, s_lut2, s_lim, s_diff, maxl, nkeys, b2};
+    const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
+    bool zero_len;
+    const DecTables tb = dec_build<T, 64 * DEC_WAVES>(in, h, s_tab, zero_len);
     const uint32_t w = wave_in_wg();
     const uint32_t l = (uint32_t)lane_id();
-    const uint32_t ncells_total = (e5 - e4) / 4;
-    const uint32_t* par_nbit = reinterpret_cast<const uint32_t*>(in + e2);
-    const uint32_t* par_entry = reinterpret_cast<const uint32_t*>(in + e3);
-    const uint32_t* cells = reinterpret_cast<const uint32_t*>(in + e4);
     uint32_t* cst = s_cells[w];
     T* ost = reinterpret_cast<T*>(s_out[w]);
-    for (uint32_t p = blockIdx.x * DEC_WAVES + w; p < (uint32_t)pardeg; p += gridDim.x * DEC_WAVES) {
-        const uint32_t nbit = par_nbit[p];
-        const uint32_t pe = par_entry[p];
+    for (uint32_t p = blockIdx.x * DEC_WAVES + w; p < h.pardeg; p += gridDim.x * DEC_WAVES) {
+        const uint32_t nbit = h.par_nbit[p];
+        const uint32_t pe = h.par_entry[p];
         const uint32_t ncell = (uint32_t)(((uint64_t)nbit + 31) / 32);
-        const uint64_t o0 = (uint64_t)p * (uint32_t)sublen;
-        const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)sublen ? (n - o0) : (uint64_t)sublen);
+        const uint64_t o0 = (uint64_t)p * h.sublen;
+        const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
         T* dst = out + o0;
-        if ((uint64_t)pe + ncell > ncells_total) {
+        if ((uint64_t)pe + ncell > h.ncells) {
             if (l == 0) *d_status = 1;
             continue;
         }
-        if (s_entry[1] == 1 && nbit == 0) {  // one symbol with a zero-length code
-            const T k0 = nkeys ? keys[0] : (T)0;
-            for (uint32_t j = l; j < cnt; j += 64) dst[j] = k0;
+        if (zero_len && nbit == 0) {
+            dec_constant(dst, cnt, h.nkeys ? keys[0] : (T)0);
             continue;
         }
         bool ok;
-        if (ncell <= DEC_CELLS && (uint32_t)sublen <= DEC_SUBLEN_MAX) {
+        if (ncell <= DEC_CELLS && h.sublen <= DEC_SUBLEN_MAX) {
             wave_lds_sync();  // the previous partition's staging reads are done
-            for (uint32_t i = l; i < ncell + 4; i += 64) cst[i] = i < ncell ? cells[pe + i] : 0u;
+            for (uint32_t i = l; i < ncell + 4; i += 64) cst[i] = i < ncell ? h.cells[pe + i] : 0u;
             wave_lds_sync();
             ok = dec_partition<T, true>(cst, ncell, tb, nbit, cnt, keys, ost, dst);
             wave_lds_sync();
@@ -603,9 +701,225 @@ huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict_
                 for (uint32_t i = done + l; i < cnt; i += 64) dst[i] = ost[i];
             }
         } else {
-            ok = dec_partition<T, false>(cells + pe, ncell, tb, nbit, cnt, keys, ost, dst);
+            ok = dec_partition<T, false>(h.cells + pe, ncell, tb, nbit, cnt, keys, ost, dst);
         }
         if (!ok && l == 0) *d_status = 1;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Decode, one lane per partition (long streams)
+// ---------------------------------------------------------------------------
+// A lane that owns a partition decodes it from its first bit: every codeword
+// once, where the wave-per-partition kernel decodes each two to three times
+// (speculative spans, corrections, the writing pass) and waits for the
+// slowest of 64 lanes in each.  Every step is one table probe for all 64
+// lanes; a lane whose probe names a longer code goes on in the next level
+// with its next step instead of in a branch (2% of the codewords of a
+// spiky field are long, which is some lane of the wave in 3 steps of 4: the
+// branch took 160 instead of 113 us on a lone wave, and 670 where whole
+// partitions hold the longest codes).  Lanes drift apart by their long codes
+// and each writes its own place of the output.
+//   bits in: the lane's next 8 cells are always in flight or held in
+//     registers (two 16-byte loads) and go into its 16-cell LDS ring when 8
+//     cells are free, which is checked once per 8 steps (they use at most 8
+//     cells); the ring's 16-byte pieces are rotated by lane, so lanes at
+//     equal positions use different banks.
+//   symbols out: a strip of two 16-symbol segments per lane in LDS; every 16
+//     steps the wave stores the segments that are full, 32 bytes of each of
+//     its 64 partitions (2-byte symbols).
+// Serial over a partition (about 113 us for 768 symbols on any stream), and
+// bound by VALU issue (33 instructions a step) beside the LDS probe latency
+// once three waves share a SIMD.  One wave per partition against one lane
+// per partition, 768 symbols each, spiky / smooth field: 2^24 symbols 95 /
+// 70 against 121 / 127 us, 20 Mi 115 / 95 against 120 / 131, 2^25 185 / 141
+// against 121 / 128, 2^26 340 / 257 against 161 / 171, 2^27 595 / 490
+// against 244 / 246.
+constexpr size_t DECL_MIN_PARTS = 32768;
+constexpr int DECL_WAVES = 4;  // with 52.6 KiB of LDS three workgroups fit a CU: three waves per SIMD
+
+typedef uint32_t huf_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <typename T>
+struct LaneDec {
+    uint32_t* ring;  // this lane's 16 cells, pieces rotated by rot
+    uint32_t rot;    // 4 * (lane / 4 % 4)
+    uint32_t base;   // the partition's first cell
+    uint32_t left;   // cells from there to the end of the stream
+    uint32_t F;      // cells [F, F + 8) are in q, [.., F) in the ring
+    uint32_t rp;     // next cell to read from the ring
+    uint4 q0, q1;
+    uint32_t w0, w1, s;  // window = {w0, w1} >> s, s < 32; w1 = cell rp - 1
+
+    __device__ __forceinline__ void fetch(const DecHead& h) {
+        // the stream is below 4 GiB: 32-bit byte offsets
+        const char* c = reinterpret_cast<const char*>(h.cells);
+        const uint32_t o = 4 * (base + F);
+        if (F + 8 <= left) {
+            const huf_u32x4_a4 x = *reinterpret_cast<const huf_u32x4_a4*>(c + o);
+            const huf_u32x4_a4 y = *reinterpret_cast<const huf_u32x4_a4*>(c + o + 16);
+            q0 = make_uint4(x.x, x.y, x.z, x.w);
+            q1 = make_uint4(y.x, y.y, y.z, y.w);
+        } else {
+            auto at = [&](uint32_t i) { return F + i < left ? *reinterpret_cast<const uint32_t*>(c + o + 4 * i) : 0u; };
+            q0 = make_uint4(at(0), at(1), at(2), at(3));
+            q1 = make_uint4(at(4), at(5), at(6), at(7));
+        }
+    }
+    __device__ __forceinline__ void commit() {
+        *reinterpret_cast<uint4*>(ring + ((F + rot) & 15u)) = q0;
+        *reinterpret_cast<uint4*>(ring + ((F + 4 + rot) & 15u)) = q1;
+        F += 8;
+    }
+    // keeps at least 9 unread cells in the ring (a block reads at most 8)
+    __device__ __forceinline__ void refill(const DecHead& h) {
+        if (F - rp <= 8) {
+            commit();
+            fetch(h);
+        }
+    }
+    __device__ __forceinline__ uint32_t peek() const { return ring[(rp + rot) & 15u]; }
+    __device__ __forceinline__ void start(const DecHead& h, uint32_t pe) {
+        base = pe;
+        left = h.ncells - pe;  // pe <= ncells: checked by the caller
+        F = rp = 0;
+        fetch(h);
+        commit();
+        fetch(h);
+        commit();
+        fetch(h);
+        w0 = 0;
+        w1 = peek();
+        rp = 1;
+        s = 0;
+    }
+    __device__ __forceinline__ uint32_t window() const { return __builtin_amdgcn_alignbit(w0, w1, s); }
+    // L < 32 bits on; nx = peek() from before the entry was known, so its
+    // LDS read runs beside the table's (reading only in the lanes that need
+    // it, after the table's, was 138 instead of 113 us on a lone wave)
+    __device__ __forceinline__ void consume(uint32_t L, uint32_t nx) {
+        const bool c = s < L;
+        w0 = c ? w1 : w0;
+        w1 = c ? nx : w1;
+        rp += c ? 1u : 0u;
+        s = (s - L) & 31u;
+    }
+    __device__ __forceinline__ uint32_t bitpos() const { return 32 * (rp - 1) - s; }
+};
+
+// The wave's 64 partitions from p0 (lanes past the last have no symbols).
+template <typename T>
+__device__ __forceinline__ void dec_lanes(const DecHead& h, const DecTables& t, const T* __restrict__ keys,
+                                          uint32_t p0, uint64_t n, T* __restrict__ out, uint32_t* ring,
+                                          uint32_t* strip, int* __restrict__ d_status) {
+    constexpr uint32_t SEG = 16;                            // symbols per stored segment
+    constexpr uint32_t SW = 2 * SEG * sizeof(T) / 4;        // words of a lane's strip (two segments)
+    constexpr uint32_t PIECES = SEG * sizeof(T) / 16;       // 16-byte pieces of a segment
+    const uint32_t l = (uint32_t)lane_id();
+    const uint32_t p = p0 + l;
+    const bool on = p < h.pardeg;
+    const uint64_t o0 = (uint64_t)p * h.sublen;
+    const uint32_t cnt = !on ? 0u : (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
+    const uint32_t nbit = on ? h.par_nbit[p] : 0u;
+    LaneDec<T> d;
+    d.ring = ring + 16 * l;
+    d.rot = l & 12u;
+    d.start(h, on ? h.par_entry[p] : 0u);
+    // symbol k of the lane at byte (k sizeof(T) + 4 (l / 4)) mod strip size
+    T* my = reinterpret_cast<T*>(strip + SW * l);
+    constexpr uint32_t MASK = 2 * SEG - 1;
+    const uint32_t turn = (l >> 2) * (4 / (uint32_t)sizeof(T));
+    const uint32_t end = turn + cnt;
+    uint32_t k = turn, flushed = 0;  // turn + symbols decoded, segments stored
+    uint32_t st = DEC_LEVEL1, acc = 0;
+    while (__ballot(k < end)) {
+        for (int blk = 0; blk < 2; blk++) {
+            d.refill(h);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t nx = d.peek();
+                const uint32_t W = d.window();
+                uint32_t e = dec_lookup(t, W, st);
+                if (e >= DEC_DEEP) {
+                    e = dec_deep(t, W);
+                    if (e & DEC_KEY) e = (e & (31u << 24)) | (uint32_t)keys[e & 0xFFFFFFu];
+                }
+                const bool more = (int32_t)e < 0;
+                my[k & MASK] = (T)e;  // past the lane's last symbol: a free slot
+                const bool emit = !more && k < end;
+                const uint32_t em = emit ? e : 0u;
+                acc |= em;
+                k += emit ? 1u : 0u;
+                st = more ? e : DEC_LEVEL1;
+                d.consume((em >> 24) & 31u, nx);
+            }
+        }
+        // 16 probes decode at most 16 symbols, so after this at most 15 wait
+        wave_lds_sync();
+        const uint32_t mine = (flushed << 1) | (k - turn >= SEG * (flushed + 1) ? 1u : 0u);
+#pragma unroll
+        for (uint32_t i = 0; i < PIECES; i++) {
+            const uint32_t r = (64 / PIECES) * i + l / PIECES, c = l % PIECES;
+            const uint32_t v = (uint32_t)__shfl((int)mine, (int)r, 64);
+            const uint32_t f = v >> 1;
+            const uint32_t* row = strip + SW * r;
+            const uint32_t w0 = (f & 1u) * (SW / 2) + 4 * c + (r >> 2);
+            const uint4 x = make_uint4(row[w0 & (SW - 1)], row[(w0 + 1) & (SW - 1)], row[(w0 + 2) & (SW - 1)],
+                                       row[(w0 + 3) & (SW - 1)]);
+            if (v & 1u) gst_u4(out + (uint64_t)(p0 + r) * h.sublen + f * SEG + c * (16 / (uint32_t)sizeof(T)), x);
+        }
+        flushed += mine & 1u;
+        wave_lds_sync();
+    }
+    for (uint32_t j = SEG * flushed; j < k - turn; j++) out[o0 + j] = my[(j + turn) & MASK];  // the last partition's remainder
+    if (on && ((acc & (1u << 30)) || d.bitpos() != nbit)) *d_status = 1;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64 * DECL_WAVES)
+huf_dec_lane_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
+                    int* __restrict__ d_status) {
+    static_assert(sizeof(T) <= 2, "the tables hold the symbols of 1- and 2-byte keys");
+    __shared__ DecLds s_tab;
+    __shared__ uint4 s_ring[DECL_WAVES][64 * 4];
+    __shared__ uint32_t s_strip[DECL_WAVES][64 * 8 * sizeof(T)];
+    DecHead h;
+    if (!dec_head<T>(in, in_bytes, n, h)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *d_status = 1;
+        return;
+    }
+    const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
+    bool zero_len;
+    const DecTables tb = dec_build<T, 64 * DECL_WAVES>(in, h, s_tab, zero_len);
+    const uint32_t w = wave_in_wg();
+    const uint32_t l = (uint32_t)lane_id();
+    const bool whole = h.sublen % 16 == 0;  // segments of 16 symbols, 16-byte aligned
+    for (uint32_t p0 = (blockIdx.x * DECL_WAVES + w) * 64; p0 < h.pardeg; p0 += gridDim.x * DECL_WAVES * 64) {
+        const uint32_t p = p0 + l;
+        bool odd = false;
+        if (p < h.pardeg) {
+            const uint32_t nbit = h.par_nbit[p];
+            odd = (uint64_t)h.par_entry[p] + ((uint64_t)nbit + 31) / 32 > h.ncells || (zero_len && nbit == 0);
+        }
+        if (whole && !__ballot(odd)) {
+            dec_lanes<T>(h, tb, keys, p0, n, out, reinterpret_cast<uint32_t*>(s_ring[w]), s_strip[w], d_status);
+            continue;
+        }
+        // other layouts, constant and malformed partitions: the wave takes them in turn
+        for (uint32_t r = 0; r < 64 && p0 + r < h.pardeg; r++) {
+            const uint32_t nbit = h.par_nbit[p0 + r], pe = h.par_entry[p0 + r];
+            const uint32_t ncell = (uint32_t)(((uint64_t)nbit + 31) / 32);
+            const uint64_t o0 = (uint64_t)(p0 + r) * h.sublen;
+            const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
+            bool ok = (uint64_t)pe + ncell <= h.ncells;
+            if (ok) {
+                if (zero_len && nbit == 0)
+                    dec_constant(out + o0, cnt, h.nkeys ? keys[0] : (T)0);
+                else
+                    ok = dec_partition<T, false>(h.cells + pe, ncell, tb, nbit, cnt, keys, nullptr, out + o0);
+            }
+            if (!ok && l == 0) *d_status = 1;
+        }
     }
 }
 
@@ -738,13 +1052,17 @@ int fzh_huffman_decode(void* stream, const void* d_in, size_t in_bytes, int elem
     if (n == 0) return FZH_OK;
     if (!d_status) return fail(FZH_E_INVALID, "huffman dec: null status");
     if ((uintptr_t)d_in % 4 || (uintptr_t)d_out % 16) return fail(FZH_E_INVALID, "huffman dec: input 4-byte, output 16-byte alignment required");
-    // persistent workgroups: each builds the decode tables once and then
-    // takes partitions in turn (the partition count is in the stream; the
-    // coarse 768-symbol partitions bound it)
+    // the partition count is in the stream; the coarse 768-symbol partitions
+    // bound it
     const size_t pardeg = cdiv(n, SUBLEN);
     hipStream_t s = S(stream);
 #define FZH_HUF_DEC(T)                                                                                         \
-    {                                                                                                          \
+    if (sizeof(T) <= 2 && pardeg >= DECL_MIN_PARTS) {                                                        \
+        using U = std::conditional_t<sizeof(T) <= 2, T, uint16_t>;                                             \
+        const unsigned blocks = (unsigned)std::min<size_t>(cdiv(pardeg, 64 * DECL_WAVES), 65536);              \
+        launch_k("huf_dec_lane_kernel", huf_dec_lane_kernel<U>, dim3(blocks), dim3(64 * DECL_WAVES), 0, s,     \
+                 (const uint8_t*)d_in, in_bytes, (U*)d_out, n, d_status);                                      \
+    } else {                                                                                                   \
         const unsigned blocks = (unsigned)std::min<size_t>(cdiv(pardeg, dec_waves<T>()), 768);                \
         launch_k("huf_dec_kernel", huf_dec_kernel<T>, dim3(blocks), dim3(64 * dec_waves<T>()), 0, s,          \
                  (const uint8_t*)d_in, in_bytes, (T*)d_out, n, d_status);                                      \
