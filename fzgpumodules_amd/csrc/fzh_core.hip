@@ -110,8 +110,11 @@ int zero_bytes(hipStream_t s, void* p, size_t n) {
     return FZH_OK;
 }
 
-// One workgroup per segment, 16-byte copies when both ends are aligned
-// (src/pipeline/concat_kernel.cu:27-61 semantics).
+// gridDim.y workgroups share each segment, 16-byte copies when both ends are
+// aligned (src/pipeline/concat_kernel.cu:27-61 semantics).  Bound by memory,
+// so a segment needs many workgroups and several loads in flight per thread:
+// 60 segments of 90 MiB in all took 651 us with one workgroup each, 33
+// us shared.
 __global__ void __launch_bounds__(256) gather_kernel(const fzh_copy_desc* __restrict__ d, int n) {
     const int seg = blockIdx.x;
     if (seg >= n) return;
@@ -119,12 +122,21 @@ __global__ void __launch_bounds__(256) gather_kernel(const fzh_copy_desc* __rest
     uint8_t* dst = (uint8_t*)d[seg].dst;
     const size_t bytes = d[seg].bytes;
     if (!src || !dst || !bytes) return;
+    const size_t G = (size_t)gridDim.y * 256, g = (size_t)blockIdx.y * 256 + threadIdx.x;
     if (((uintptr_t)src | (uintptr_t)dst) % 16 == 0) {
         const size_t nw = bytes / 16;
-        for (size_t i = threadIdx.x; i < nw; i += blockDim.x) gst_u4(dst + 16 * i, gld_u4(src + 16 * i));
-        for (size_t i = nw * 16 + threadIdx.x; i < bytes; i += blockDim.x) gp(dst)[i] = gp(src)[i];
+        size_t i = g;
+        for (; i + 3 * G < nw; i += 4 * G) {
+            uint4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = gld_u4(src + 16 * (i + u * G));
+#pragma unroll
+            for (int u = 0; u < 4; u++) gst_u4(dst + 16 * (i + u * G), v[u]);
+        }
+        for (; i < nw; i += G) gst_u4(dst + 16 * i, gld_u4(src + 16 * i));
+        for (i = nw * 16 + g; i < bytes; i += G) gp(dst)[i] = gp(src)[i];
     } else {
-        for (size_t i = threadIdx.x; i < bytes; i += blockDim.x) gp(dst)[i] = gp(src)[i];
+        for (size_t i = g; i < bytes; i += G) gp(dst)[i] = gp(src)[i];
     }
 }
 
@@ -258,7 +270,9 @@ int fzh_workspace_init(void* stream, void* d_ws, size_t ws_bytes) {
 
 int fzh_gather(void* stream, const fzh_copy_desc* d_descs, int n_segs) {
     if (n_segs <= 0) return FZH_OK;
-    gather_kernel<<<n_segs, 256, 0, S(stream)>>>(d_descs, n_segs);
+    // the sizes are device data: about 4096 workgroups in all, up to 64 a segment
+    const unsigned per = (unsigned)std::min(std::max(4096 / n_segs, 1), 64);
+    gather_kernel<<<dim3((unsigned)n_segs, per), 256, 0, S(stream)>>>(d_descs, n_segs);
     FZH_CHECK_LAUNCH("gather_kernel");
     return FZH_OK;
 }
