@@ -267,32 +267,103 @@ scatter_assign_kernel(const float* __restrict__ val, const uint32_t* __restrict_
 template <typename T>
 __device__ __forceinline__ uint32_t ldv(const T* p, uint64_t i) { return (uint32_t)p[i]; }
 
-// one thread per output byte (sub-byte), per element (>= 8 bits)
+// Bound by memory: a thread takes 16 elements, which are whole 16-byte words
+// of the elements and 2 * NB bytes of the packed array, so both sides move in
+// wide accesses and the packing is constant shifts (6 Mi 16-bit codes at 16
+// bits: 6.9 us; 10.5 with one byte store per output byte).  The last n % 16
+// elements, at most 60 packed bytes, take a thread per byte.
+template <int NB, typename F>
+__device__ __forceinline__ void pack_tail(uint64_t n, uint8_t* __restrict__ out, uint64_t b0, uint64_t nout,
+                                          uint32_t t, F&& element) {
+    const uint64_t b = b0 + t;
+    if (b >= nout) return;
+    uint32_t v = 0;
+    if constexpr (NB < 8) {
+#pragma unroll
+        for (int k = 0; k < 8 / NB; k++) {
+            const uint64_t e = b * (8 / NB) + k;
+            if (e < n) v |= (element(e) & ((1u << NB) - 1u)) << (k * NB);
+        }
+    } else {
+        v = element(b / (NB / 8)) >> (8 * (b % (NB / 8)));
+    }
+    out[b] = (uint8_t)v;
+}
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(256)
+bitpack_enc_vec_kernel(const T* __restrict__ in, uint64_t n, uint8_t* __restrict__ out) {
+    constexpr uint32_t MASK = NB >= 32 ? 0xFFFFFFFFu : ((1u << (NB & 31)) - 1u);
+    const uint64_t n16 = n / 16, stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n16; g += stride) {
+        T v[16];
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(T); i++)
+            reinterpret_cast<uint4*>(v)[i] = reinterpret_cast<const uint4*>(in)[g * sizeof(T) + i];
+        uint32_t o[(16 * NB + 31) / 32] = {};
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[e * NB / 32] |= ((uint32_t)v[e] & MASK) << (e * NB % 32);
+        uint8_t* d = out + g * 2 * NB;
+        if constexpr (NB == 1) *reinterpret_cast<uint16_t*>(d) = (uint16_t)o[0];
+        else if constexpr (NB == 2) *reinterpret_cast<uint32_t*>(d) = o[0];
+        else if constexpr (NB == 4) *reinterpret_cast<uint2*>(d) = make_uint2(o[0], o[1]);
+        else
+#pragma unroll
+            for (int i = 0; i < NB / 8; i++)
+                reinterpret_cast<uint4*>(d)[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+    }
+    if (blockIdx.x == 0)
+        pack_tail<NB>(n, out, n16 * 2 * NB, (n * NB + 7) / 8, threadIdx.x, [&](uint64_t e) { return (uint32_t)in[e]; });
+}
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(256)
+bitpack_dec_vec_kernel(const uint8_t* __restrict__ in, uint64_t n, T* __restrict__ out) {
+    constexpr uint32_t MASK = NB >= 32 ? 0xFFFFFFFFu : ((1u << (NB & 31)) - 1u);
+    const uint64_t n16 = n / 16, stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n16; g += stride) {
+        const uint8_t* d = in + g * 2 * NB;
+        uint32_t o[NB < 8 ? 2 : NB / 2];
+        if constexpr (NB == 1) o[0] = *reinterpret_cast<const uint16_t*>(d);
+        else if constexpr (NB == 2) o[0] = *reinterpret_cast<const uint32_t*>(d);
+        else if constexpr (NB == 4) *reinterpret_cast<uint2*>(o) = *reinterpret_cast<const uint2*>(d);
+        else
+#pragma unroll
+            for (int i = 0; i < NB / 8; i++) reinterpret_cast<uint4*>(o)[i] = reinterpret_cast<const uint4*>(d)[i];
+        T v[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) v[e] = (T)((o[e * NB / 32] >> (e * NB % 32)) & MASK);
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(T); i++)
+            reinterpret_cast<uint4*>(out)[g * sizeof(T) + i] = reinterpret_cast<const uint4*>(v)[i];
+    }
+    const uint64_t e = n16 * 16 + threadIdx.x;
+    if (blockIdx.x == 0 && e < n) {
+        uint32_t v = 0;
+        if constexpr (NB < 8) v = (in[e / (8 / NB)] >> ((e % (8 / NB)) * NB)) & MASK;
+        else
+#pragma unroll
+            for (int b = 0; b < NB / 8; b++) v |= (uint32_t)in[e * (NB / 8) + b] << (8 * b);
+        out[e] = (T)v;
+    }
+}
+
+// Arrays that are not 16-byte aligned: one thread per packed byte (packing)
+// or element (unpacking).
 template <typename T>
 __global__ void __launch_bounds__(256)
 bitpack_enc_kernel(const T* __restrict__ in, uint64_t n, int nbits, uint8_t* __restrict__ out) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    if (nbits < 8) {
-        const int epb = 8 / nbits;
-        const uint32_t mask = (1u << nbits) - 1u;
-        const uint64_t nout = (n * nbits + 7) / 8;
-        for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < nout; b += stride) {
-            uint32_t packed = 0;
-            for (int k = 0; k < epb; k++) {
-                const uint64_t e = b * epb + k;
-                if (e < n) packed |= (ldv(in, e) & mask) << (k * nbits);
-            }
-            out[b] = (uint8_t)packed;
-        }
-    } else {
-        const int bytes = nbits / 8;
-        const uint32_t mask = nbits >= 32 ? 0xFFFFFFFFu : ((1u << nbits) - 1u);
-        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-            uint32_t v = ldv(in, i) & mask;
-            for (int b = 0; b < bytes; b++) {
-                out[i * bytes + b] = (uint8_t)(v & 0xFFu);
-                v >>= 8;
-            }
+    const uint64_t nout = (n * nbits + 7) / 8;
+    const auto element = [&](uint64_t e) { return (uint32_t)in[e]; };
+    for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < nout; b += stride) {
+        switch (nbits) {
+        case 1: pack_tail<1>(n, out, b, nout, 0, element); break;
+        case 2: pack_tail<2>(n, out, b, nout, 0, element); break;
+        case 4: pack_tail<4>(n, out, b, nout, 0, element); break;
+        case 8: pack_tail<8>(n, out, b, nout, 0, element); break;
+        case 16: pack_tail<16>(n, out, b, nout, 0, element); break;
+        default: pack_tail<32>(n, out, b, nout, 0, element); break;
         }
     }
 }
@@ -315,35 +386,77 @@ bitpack_dec_kernel(const uint8_t* __restrict__ in, uint64_t n, int nbits, T* __r
     }
 }
 
+template <typename T, int NB>
+void launch_bitpack_vec(hipStream_t s, bool enc, const void* in, size_t n, void* out) {
+    if constexpr (NB <= 8 * (int)sizeof(T)) {
+        const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(n / 16, 256), 8192));
+        if (enc)
+            bitpack_enc_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const T*)in, n, (uint8_t*)out);
+        else
+            bitpack_dec_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const uint8_t*)in, n, (T*)out);
+    }
+}
+
+template <typename T>
+void launch_bitpack(hipStream_t s, bool enc, const void* in, size_t n, int nbits, void* out) {
+    if (((uintptr_t)in | (uintptr_t)out) % 16 == 0) {
+        switch (nbits) {
+        case 1: return launch_bitpack_vec<T, 1>(s, enc, in, n, out);
+        case 2: return launch_bitpack_vec<T, 2>(s, enc, in, n, out);
+        case 4: return launch_bitpack_vec<T, 4>(s, enc, in, n, out);
+        case 8: return launch_bitpack_vec<T, 8>(s, enc, in, n, out);
+        case 16: return launch_bitpack_vec<T, 16>(s, enc, in, n, out);
+        default: return launch_bitpack_vec<T, 32>(s, enc, in, n, out);
+        }
+    }
+    const size_t work = enc ? (n * nbits + 7) / 8 : n;
+    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(work, 256), 4096));
+    if (enc)
+        bitpack_enc_kernel<T><<<blocks, 256, 0, s>>>((const T*)in, n, nbits, (uint8_t*)out);
+    else
+        bitpack_dec_kernel<T><<<blocks, 256, 0, s>>>((const uint8_t*)in, n, nbits, (T*)out);
+}
+
+// Maximum in two launches: 16-byte loads, four in flight per thread, one
+// partial maximum per workgroup, then one workgroup over the partials.  (One
+// launch whose last workgroup finishes the reduction needs a device fence in
+// every workgroup, which writes back the codes its XCD's L2 still holds: 26
+// us for 6 Mi 2-byte codes, 131 with a single thread reading the partials;
+// 5.9 us for the two launches.)
 template <typename T>
 __global__ void __launch_bounds__(256)
-max_kernel(const T* __restrict__ in, uint64_t n, uint32_t* __restrict__ partial, uint32_t* __restrict__ counter,
-           uint32_t* __restrict__ result) {
+max_partial_kernel(const T* __restrict__ in, uint64_t n, uint32_t* __restrict__ partial) {
     __shared__ uint32_t sm[4];
+    constexpr int E = 16 / sizeof(T);
+    const uint64_t nv = (uintptr_t)in % 16 == 0 ? n / E : 0, stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t m = 0;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t v = (uint32_t)in[i];
-        m = v > m ? v : m;
+    for (uint64_t v0 = t; v0 < nv; v0 += 4 * stride) {
+        uint4 w[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            w[u] = v0 + u * stride < nv ? reinterpret_cast<const uint4*>(in)[v0 + u * stride] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int k = 0; k < E; k++) m = max(m, (uint32_t) reinterpret_cast<const T*>(&w[u])[k]);
     }
+    for (uint64_t i = nv * E + t; i < n; i += stride) m = max(m, (uint32_t)in[i]);
     m = wave_max(m);
     if (lane_id() == 0) sm[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < 4; i++) m = sm[i] > m ? sm[i] : m;
-        m = sm[0] > m ? sm[0] : m;
-        partial[blockIdx.x] = m;
-        __threadfence();
-        if (atomicAdd(counter, 1u) == gridDim.x - 1) {
-            __threadfence();
-            uint32_t g = 0;
-            for (uint32_t b = 0; b < gridDim.x; b++) {
-                const uint32_t v = __hip_atomic_load(&partial[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                g = v > g ? v : g;
-            }
-            *result = g;
-            *counter = 0u;
-        }
-    }
+    if (threadIdx.x == 0) partial[blockIdx.x] = max(max(sm[0], sm[1]), max(sm[2], sm[3]));
+}
+
+__global__ void __launch_bounds__(256)
+max_final_kernel(const uint32_t* __restrict__ partial, uint32_t np, uint32_t* __restrict__ result) {
+    __shared__ uint32_t sm[4];
+    uint32_t m = 0;
+    for (uint32_t b = threadIdx.x; b < np; b += 256) m = max(m, partial[b]);
+    m = wave_max(m);
+    if (lane_id() == 0) sm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) *result = max(max(sm[0], sm[1]), max(sm[2], sm[3]));
 }
 
 }  // namespace
@@ -524,16 +637,16 @@ size_t fzh_max_u32_ws_bytes(void) { return 256 + 4 * 1024; }
 int fzh_max_u32(void* stream, const void* d_in, size_t n, int elem_bytes, uint32_t* d_max, void* d_ws,
                    size_t ws_bytes) {
     if (ws_bytes < fzh_max_u32_ws_bytes()) return fail(FZH_E_CAPACITY, "max: workspace too small");
-    uint32_t* counter = (uint32_t*)d_ws;
     uint32_t* partial = (uint32_t*)((uint8_t*)d_ws + 256);
-    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(std::max<size_t>(n, 1), 256 * 8), 1024));
+    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(std::max<size_t>(n, 1), 256 * 32), 1024));
     hipStream_t s = S(stream);
     switch (elem_bytes) {
-    case 1: max_kernel<uint8_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, partial, counter, d_max); break;
-    case 2: max_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint16_t*)d_in, n, partial, counter, d_max); break;
-    case 4: max_kernel<uint32_t><<<blocks, 256, 0, s>>>((const uint32_t*)d_in, n, partial, counter, d_max); break;
+    case 1: max_partial_kernel<uint8_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, partial); break;
+    case 2: max_partial_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint16_t*)d_in, n, partial); break;
+    case 4: max_partial_kernel<uint32_t><<<blocks, 256, 0, s>>>((const uint32_t*)d_in, n, partial); break;
     default: return fail(FZH_E_INVALID, "max: elem_bytes must be 1, 2 or 4");
     }
+    max_final_kernel<<<1, 256, 0, s>>>(partial, blocks, d_max);
     FZH_CHECK_LAUNCH("max_kernel");
     return FZH_OK;
 }
@@ -542,13 +655,11 @@ int fzh_bitpack_enc(void* stream, const void* d_in, size_t n, int elem_bytes, in
     if (nbits <= 0 || nbits > 8 * elem_bytes || (nbits & (nbits - 1)) != 0)
         return fail(FZH_E_INVALID, "bitpack: nbits must be a power of two <= 8*sizeof(T)");
     if (n == 0) return FZH_OK;
-    const size_t work = nbits < 8 ? (n * nbits + 7) / 8 : n;
-    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(work, 256), 4096));
     hipStream_t s = S(stream);
     switch (elem_bytes) {
-    case 1: bitpack_enc_kernel<uint8_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, nbits, (uint8_t*)d_out); break;
-    case 2: bitpack_enc_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint16_t*)d_in, n, nbits, (uint8_t*)d_out); break;
-    case 4: bitpack_enc_kernel<uint32_t><<<blocks, 256, 0, s>>>((const uint32_t*)d_in, n, nbits, (uint8_t*)d_out); break;
+    case 1: launch_bitpack<uint8_t>(s, true, d_in, n, nbits, d_out); break;
+    case 2: launch_bitpack<uint16_t>(s, true, d_in, n, nbits, d_out); break;
+    case 4: launch_bitpack<uint32_t>(s, true, d_in, n, nbits, d_out); break;
     default: return fail(FZH_E_INVALID, "bitpack: elem_bytes must be 1, 2 or 4");
     }
     FZH_CHECK_LAUNCH("bitpack_enc_kernel");
@@ -559,12 +670,11 @@ int fzh_bitpack_dec(void* stream, const void* d_in, size_t n, int elem_bytes, in
     if (nbits <= 0 || nbits > 8 * elem_bytes || (nbits & (nbits - 1)) != 0)
         return fail(FZH_E_INVALID, "bitpack: nbits must be a power of two <= 8*sizeof(T)");
     if (n == 0) return FZH_OK;
-    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(n, 256), 4096));
     hipStream_t s = S(stream);
     switch (elem_bytes) {
-    case 1: bitpack_dec_kernel<uint8_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, nbits, (uint8_t*)d_out); break;
-    case 2: bitpack_dec_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, nbits, (uint16_t*)d_out); break;
-    case 4: bitpack_dec_kernel<uint32_t><<<blocks, 256, 0, s>>>((const uint8_t*)d_in, n, nbits, (uint32_t*)d_out); break;
+    case 1: launch_bitpack<uint8_t>(s, false, d_in, n, nbits, d_out); break;
+    case 2: launch_bitpack<uint16_t>(s, false, d_in, n, nbits, d_out); break;
+    case 4: launch_bitpack<uint32_t>(s, false, d_in, n, nbits, d_out); break;
     default: return fail(FZH_E_INVALID, "bitpack: elem_bytes must be 1, 2 or 4");
     }
     FZH_CHECK_LAUNCH("bitpack_dec_kernel");
