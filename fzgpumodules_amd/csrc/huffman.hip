@@ -15,9 +15,10 @@
 //   histogram: privatized per-wave LDS histograms, consecutive equal symbols
 //     merged in-lane before the LDS atomic (the dominant code otherwise
 //     serialises a 64-lane conflict).
-//   encode: one wave per partition packs its codewords in parallel (bit
-//     offsets from a wave prefix sum, LDS OR into cells) and writes them to
-//     the partition's scratch slot plus par_nbit; a segmented device scan of
+//   encode: one wave per partition packs its codewords in parallel (a run of
+//     symbols per lane, bit offsets from one wave prefix sum, whole cells
+//     ORed into LDS) and writes them to the partition's scratch slot plus
+//     par_nbit; a segmented device scan of
 //     the cell counts writes par_entry into the stream; a pack kernel moves
 //     the cells and a one-workgroup kernel writes the header: no host prefix
 //     sum, no host sync (reference phases 1-4 + two syncs).
@@ -113,7 +114,17 @@ hist_global_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, uint32_
 // ---------------------------------------------------------------------------
 // cells per partition slot (every codeword is at most 28 bits)
 constexpr int cells_of(int sl) { return (sl * 28 + 31) / 32 + 2; }
+constexpr unsigned ENC_BLOCKS = 4096;  // encode workgroups, at most
 
+// A lane takes SL / 64 consecutive symbols: their lengths add up in the lane,
+// so one wave scan places all of them, and their codes are shifted together
+// in a register that goes to LDS a whole cell at a time (about two OR
+// operations per lane and 12 symbols of 6.5 bits).  With symbols strided by
+// 64 over the lanes every symbol took a wave scan and one or two LDS ORs that
+// collide with its neighbours' in the same cell: 2^27 symbols 234 us, now 96.
+// Each workgroup stages the codebook once and takes several partitions; more
+// workgroups (one partition a wave: 117 us) stage it more often, fewer (2048:
+// 103) leave too few waves to cover the loads.
 // BOOK_LDS: the codebook is staged in LDS (bklen <= 8192), else read from
 // global memory.  (A template parameter, not a pointer chosen at run time:
 // a pointer that may be either LDS or global makes every lookup a FLAT
@@ -134,55 +145,72 @@ huf_enc_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, const uint3
         __syncthreads();
     }
     const uint32_t ent1 = HDR_BYTES, ent2 = ent1 + rev_bytes;
-    const uint32_t p = blockIdx.x * 4 + wv;
     const int l = lane_id();
-    if (p >= pardeg) return;
-    const uint64_t s0 = (uint64_t)p * SL;
-    const uint32_t cnt = (uint32_t)((n - s0) < (uint64_t)SL ? (n - s0) : SL);
-    for (int i = l; i < CELLS; i += 64) cells[i] = 0u;
-    // symbol s0 + l + 64k, bit offsets in (k, lane) order = symbol order
-    uint32_t code[K], len[K];
+    constexpr int B = K * (int)sizeof(T);
+    constexpr int V = B % 16 == 0 ? 16 : (B % 8 == 0 ? 8 : 4);  // bytes per load
+    const bool wide = (uintptr_t)in % V == 0;
+    for (uint32_t p = blockIdx.x * 4 + wv; p < pardeg; p += gridDim.x * 4) {
+        const uint64_t s0 = (uint64_t)p * SL;
+        const uint32_t cnt = (uint32_t)((n - s0) < (uint64_t)SL ? (n - s0) : SL);
+        // lane l: symbols K l .. K l + K - 1 of the partition
+        T sym[K];
+        if (cnt == SL && wide) {
+            const T* src = in + s0 + K * l;
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const uint32_t j = l + 64 * k;
-        uint32_t w = 0;
-        if (j < cnt) {
-            const uint32_t sym = ld_sym(in, s0 + j);
-            if (sym < bklen) w = BOOK_LDS ? s_bk[sym] : bk4[sym];  // an out-of-range symbol (reported by its caller) gets no code
-        }
-        len[k] = j < cnt ? (w >> 27) : 0u;
-        code[k] = w & 0x07FFFFFFu;
-    }
-    wave_lds_sync();
-    uint32_t run = 0;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const uint32_t incl = wave_incl_scan(len[k]);
-        const uint32_t b = run + incl - len[k];
-        const uint32_t L = len[k];
-        if (L) {
-            const uint32_t c = b >> 5, sh = b & 31u;
-            if (sh + L <= 32) {
-                atomicOr(&cells[c], code[k] << (32 - sh - L));
-            } else {
-                atomicOr(&cells[c], code[k] >> (sh + L - 32));
-                atomicOr(&cells[c + 1], code[k] << (64 - sh - L));
+            for (int i = 0; i < B / V; i++) {
+                if constexpr (V == 16)
+                    reinterpret_cast<uint4*>(sym)[i] = reinterpret_cast<const uint4*>(src)[i];
+                else if constexpr (V == 8)
+                    reinterpret_cast<uint2*>(sym)[i] = reinterpret_cast<const uint2*>(src)[i];
+                else
+                    reinterpret_cast<uint32_t*>(sym)[i] = reinterpret_cast<const uint32_t*>(src)[i];
             }
+        } else {
+#pragma unroll
+            for (int k = 0; k < K; k++) sym[k] = K * l + k < (int)cnt ? in[s0 + K * l + k] : (T)0;
         }
-        run += lane63(incl);
-    }
-    const uint32_t nbit = run;
-    const uint32_t ncell = (nbit + 31) / 32;
-    wave_lds_sync();
-    uint32_t* dst = scells + (uint64_t)p * CELLS;
-    for (uint32_t i = l; i < ncell; i += 64) dst[i] = cells[i];
-    if (l == 0) {
-        reinterpret_cast<uint32_t*>(out + ent2)[p] = nbit;
-        ncell_out[p] = ncell;
-    }
-    if (p == 0) {
-        for (uint32_t i = l; i < rev_bytes; i += 64) out[ent1 + i] = revbook[i];
-        for (uint32_t i = 64 + l; i < HDR_BYTES; i += 64) out[i] = 0;
+        uint32_t word[K], bits = 0;  // length << 27 | code
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const uint32_t x = (uint32_t)sym[k];
+            // a symbol past the partition's end or out of range (reported by the caller) gets no code
+            const bool ok = x < bklen && (cnt == SL || K * l + k < (int)cnt);
+            word[k] = ok ? (BOOK_LDS ? s_bk[x] : bk4[x]) : 0u;
+            bits += word[k] >> 27;
+        }
+        const uint32_t incl = wave_incl_scan(bits);
+        const uint32_t nbit = lane63(incl);
+        const uint32_t ncell = (nbit + 31) / 32;
+        for (uint32_t i = l; i <= ncell; i += 64) cells[i] = 0u;
+        wave_lds_sync();
+        // the lane's codes shifted into place; a cell leaves the register when it
+        // is full, and what lanes share of a cell is ORed together in LDS
+        uint32_t at = (incl - bits) >> 5, fill = (incl - bits) & 31u, hi = 0;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const uint32_t c = word[k] & 0x07FFFFFFu;
+            const uint32_t to = fill + (word[k] >> 27);  // 0 .. 62
+            const uint32_t x = __builtin_amdgcn_alignbit(c, 0u, to);  // c << (32 - to % 32), 0 if that is 32
+            if (to >= 32) {
+                atomicOr(&cells[at], hi | (c >> (to & 31u)));
+                at++;
+            }
+            hi = to >= 32 ? x : hi | x;
+            fill = to & 31u;
+        }
+        if (fill) atomicOr(&cells[at], hi);
+        wave_lds_sync();
+        uint32_t* dst = scells + (uint64_t)p * CELLS;
+        for (uint32_t i = l; i < ncell; i += 64) dst[i] = cells[i];
+        if (l == 0) {
+            reinterpret_cast<uint32_t*>(out + ent2)[p] = nbit;
+            ncell_out[p] = ncell;
+        }
+        if (p == 0) {
+            for (uint32_t i = l; i < rev_bytes; i += 64) out[ent1 + i] = revbook[i];
+            for (uint32_t i = 64 + l; i < HDR_BYTES; i += 64) out[i] = 0;
+        }
+        wave_lds_sync();
     }
 }
 
@@ -961,11 +989,12 @@ int enc_impl(hipStream_t s, const void* in, size_t n, uint32_t bklen, const uint
     const bool book_in_lds = bklen <= 8192;
     const size_t lds = (size_t)4 * CELLS * 4 + (book_in_lds ? 4 * (size_t)bklen : 0);
     const unsigned blocks = (unsigned)cdiv(pardeg, 4);
+    const unsigned eb = std::min(blocks, ENC_BLOCKS);
     if (book_in_lds)
-        launch_k("huf_enc_kernel", huf_enc_kernel<T, SL, true>, dim3(blocks), dim3(256), (uint32_t)lds, s, (const T*)in, n,
+        launch_k("huf_enc_kernel", huf_enc_kernel<T, SL, true>, dim3(eb), dim3(256), (uint32_t)lds, s, (const T*)in, n,
                  bklen, bk4, rev, rev_bytes, o8, scells, ncell, pardeg);
     else
-        launch_k("huf_enc_kernel", huf_enc_kernel<T, SL, false>, dim3(blocks), dim3(256), (uint32_t)lds, s, (const T*)in,
+        launch_k("huf_enc_kernel", huf_enc_kernel<T, SL, false>, dim3(eb), dim3(256), (uint32_t)lds, s, (const T*)in,
                  n, bklen, bk4, rev, rev_bytes, o8, scells, ncell, pardeg);
     if (int rc = scan_u32(s, ncell, reinterpret_cast<uint32_t*>(o8 + ent3), pardeg, nullptr, tot, w + L.o_scan))
         return rc;
