@@ -40,10 +40,13 @@ struct SizeOverride {
 // the total and then serves the readback entries, taking any word that lies
 // in the header or the total from the values it just computed (so the
 // readback never depends on another workgroup's stores).
+// With `copy` (16-byte aligned, as large as the concat can get) the whole
+// result goes there too, each word stored twice; slot 0 of a fused RZE
+// launch is copied by the workgroups that place its chunks.
 __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n, uint8_t* __restrict__ out,
-                                                    uint64_t* __restrict__ total, const ReadbackArgs& r, int nr,
-                                                    uint8_t* __restrict__ mapped, uint32_t blk, uint32_t nblk,
-                                                    const SizeOverride& ov) {
+                                                    uint8_t* __restrict__ copy, uint64_t* __restrict__ total,
+                                                    const ReadbackArgs& r, int nr, uint8_t* __restrict__ mapped,
+                                                    uint32_t blk, uint32_t nblk, const SizeOverride& ov) {
     __shared__ uint64_t s_off[FZH_CONCAT_MAX_SLOTS], s_sz[FZH_CONCAT_MAX_SLOTS];
     __shared__ uint64_t s_total;
     const int t = threadIdx.x;
@@ -69,29 +72,40 @@ __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n,
         const uint64_t sz = s_sz[si], nw = (sz + 15) / 16;
         const uint8_t* src = reinterpret_cast<const uint8_t*>(a.slot[si].src);
         uint8_t* d8 = out + s_off[si];
-        if (reinterpret_cast<const void*>(d8) == reinterpret_cast<const void*>(src)) {
-            if (g < nw * 16 - sz) d8[sz + g] = 0;  // produced in place: the pad only
+        uint8_t* c8 = copy ? copy + s_off[si] : nullptr;
+        const bool placed = reinterpret_cast<const void*>(d8) == reinterpret_cast<const void*>(src);
+        if (placed && (!c8 || ov.has_size0)) {  // produced in place: the pad only
+            if (g < nw * 16 - sz) {
+                d8[sz + g] = 0;
+                if (c8) c8[sz + g] = 0;
+            }
             continue;
         }
-        uint4* dst = reinterpret_cast<uint4*>(d8);
+        if (placed && g < nw * 16 - sz) d8[sz + g] = 0;
+        uint4* dst = placed ? nullptr : reinterpret_cast<uint4*>(d8);
+        uint4* cpy = reinterpret_cast<uint4*>(c8);
+        const auto put = [&](uint64_t w, uint4 v) {
+            if (dst) dst[w] = v;
+            if (cpy) cpy[w] = v;
+        };
         const uint4* src4 = reinterpret_cast<const uint4*>(src);
         const uint64_t full = sz / 16;
         uint64_t w = g;
         // four words per step, loads issued before the stores
         for (; w + 3 * G < full; w += 4 * G) {
             const uint4 v0 = src4[w], v1 = src4[w + G], v2 = src4[w + 2 * G], v3 = src4[w + 3 * G];
-            dst[w] = v0;
-            dst[w + G] = v1;
-            dst[w + 2 * G] = v2;
-            dst[w + 3 * G] = v3;
+            put(w, v0);
+            put(w + G, v1);
+            put(w + 2 * G, v2);
+            put(w + 3 * G, v3);
         }
         for (; w < nw; w += G) {
             if (w < full) {
-                dst[w] = src4[w];
+                put(w, src4[w]);
             } else {
                 uint32_t v[4] = {0, 0, 0, 0};
                 for (uint64_t b = 16 * w; b < sz; b++) v[(b & 15) >> 2] |= (uint32_t)src[b] << (8 * (b & 3));
-                dst[w] = make_uint4(v[0], v[1], v[2], v[3]);
+                put(w, make_uint4(v[0], v[1], v[2], v[3]));
             }
         }
     }
@@ -103,7 +117,10 @@ __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n,
         if (j >= (uint64_t)n) return 0u;
         return (k & 1) ? (uint32_t)s_sz[j] : (uint32_t)(s_sz[j] >> 32);
     };
-    for (uint64_t k = t; k < hdr / 4; k += 256) reinterpret_cast<uint32_t*>(out)[k] = hword(k);
+    for (uint64_t k = t; k < hdr / 4; k += 256) {
+        reinterpret_cast<uint32_t*>(out)[k] = hword(k);
+        if (copy) reinterpret_cast<uint32_t*>(copy)[k] = hword(k);
+    }
     if (t == 0) *total = s_total;
     // the entries' words flattened over the workgroup's threads: one load
     // round trip for all of them instead of one per entry
@@ -128,14 +145,17 @@ __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n,
 
 
 // Validates and packs the concat slots and readback entries for a launch;
-// grid: workgroups for the slots' copies.
-inline int build_concat_args(const fzh_concat_slot* slots, int n, void* d_out, uint64_t out_cap, uint64_t* d_total,
-                             const fzh_readback_entry* entries, int n_entries, void* d_mapped_dst, ConcatArgs& a,
-                             ReadbackArgs& r, unsigned& grid) {
+// grid: workgroups for the slots' copies.  d_copy: a second destination of
+// the whole result, or null; copy_first: slot 0 goes there by those
+// workgroups too although it is produced in place.
+inline int build_concat_args(const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, bool copy_first,
+                             uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries, int n_entries,
+                             void* d_mapped_dst, ConcatArgs& a, ReadbackArgs& r, unsigned& grid) {
     if (n < 0 || n > FZH_CONCAT_MAX_SLOTS) return fail(FZH_E_INVALID, "concat: 0..32 slots");
     if (n_entries < 0 || n_entries > FZH_READBACK_MAX) return fail(FZH_E_INVALID, "readback: at most 32 entries");
     if (!d_out || !d_total) return fail(FZH_E_INVALID, "concat: null pointer");
-    if (reinterpret_cast<uintptr_t>(d_out) % 16 != 0 || reinterpret_cast<uintptr_t>(d_total) % 8 != 0)
+    if (reinterpret_cast<uintptr_t>(d_out) % 16 != 0 || reinterpret_cast<uintptr_t>(d_copy) % 16 != 0 ||
+        reinterpret_cast<uintptr_t>(d_total) % 8 != 0)
         return fail(FZH_E_INVALID, "concat: output must be 16-byte and the total 8-byte aligned");
     if (n_entries > 0 && (!d_mapped_dst || reinterpret_cast<uintptr_t>(d_mapped_dst) % 4 != 0))
         return fail(FZH_E_INVALID, "readback: destination must be 4-byte aligned");
@@ -152,7 +172,7 @@ inline int build_concat_args(const fzh_concat_slot* slots, int n, void* d_out, u
         a.slot[i] = s;
         bound += (s.cap + 15) & ~uint64_t(15);
         const bool first_in_place = i == 0 && s.src == static_cast<const uint8_t*>(d_out) + hdr;
-        if (!first_in_place) copy_words += (s.cap + 15) / 16;
+        if (!first_in_place || (d_copy && copy_first)) copy_words += (s.cap + 15) / 16;
     }
     if (bound > out_cap) return fail(FZH_E_CAPACITY, "concat: output buffer too small");
     std::memset(&r, 0, sizeof(r));
@@ -162,7 +182,8 @@ inline int build_concat_args(const fzh_concat_slot* slots, int n, void* d_out, u
             return fail(FZH_E_INVALID, "readback: entries must be non-null 4-byte multiples");
         r.e[i] = e;
     }
-    grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>(cdiv(copy_words, 1024), 1), 256);
+    // (a second destination moves the primary output as well: more bytes, more workgroups)
+    grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>(cdiv(copy_words, 1024), 1), d_copy && copy_first ? 1024 : 256);
     return FZH_OK;
 }
 

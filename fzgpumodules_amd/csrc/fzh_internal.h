@@ -46,8 +46,13 @@ struct RzePackDesc {
 int rze_enc_prepare(hipStream_t s, const void* d_in, size_t nbytes, int sew, void* d_out, size_t out_cap,
                     uint64_t* d_out_size, void* d_ws, size_t ws_bytes, RzePackDesc* desc);
 int rze_pack_concat_readback(hipStream_t s, const RzePackDesc& d, const fzh_concat_slot* slots, int n, void* d_out,
-                             uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries, int n_entries,
-                             void* d_mapped_dst);
+                             void* d_copy, uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries,
+                             int n_entries, void* d_mapped_dst);
+
+// fzh_concat_readback with a second destination of the whole result (both
+// launches: d_copy null, or 16-byte aligned and out_cap bytes).
+int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, uint64_t out_cap,
+                    uint64_t* d_total, const fzh_readback_entry* entries, int n_entries, void* d_mapped_dst);
 
 // Optional per-kernel device timing.  launch_k launches like
 // kernel<<<grid, block, shm, s>>>(args...); while timing is on

@@ -26,6 +26,17 @@ constexpr size_t kConcatWsBytes = 1024;  // [0, 512): offsets/sizes table; [512]
 
 size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// p is device memory of the current GPU (a kernel may store there).
+bool isDeviceMemory(const void* p) {
+    hipPointerAttribute_t a;
+    int dev = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that HIP does not know: not an error of this call
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
+}
+
 struct Timer {
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
     float ms() const {
@@ -377,14 +388,14 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
         if (defer_rze) defer_rze->setDeferPack(false);
         if (pd)
             throwIfFzh(fzh::rze_pack_concat_readback(stream, *static_cast<const fzh::RzePackDesc*>(pd), slots.data(),
-                                                     (int)slots.size(), concat_buf_, concat_cap_,
+                                                     (int)slots.size(), concat_buf_, copy_to_, concat_cap_,
                                                      (uint64_t*)((uint8_t*)concat_ws_ + 512), rb.data(),
                                                      (int)rb.size(), rb_dev_),
                        "Pipeline concat");
         else
-            throwIfFzh(fzh_concat_readback(stream, slots.data(), (int)slots.size(), concat_buf_, concat_cap_,
-                                           (uint64_t*)((uint8_t*)concat_ws_ + 512), rb.data(), (int)rb.size(),
-                                           rb_dev_),
+            throwIfFzh(fzh::concat_readback(stream, slots.data(), (int)slots.size(), concat_buf_, copy_to_, concat_cap_,
+                                            (uint64_t*)((uint8_t*)concat_ws_ + 512), rb.data(), (int)rb.size(),
+                                            rb_dev_),
                        "Pipeline concat");
         return;
     }
@@ -535,12 +546,35 @@ void Pipeline::compress(const void* d_input, size_t input_size, void* d_output_b
     if (!d_output_buf || !actual_output_size) throw std::invalid_argument("compress(): null output argument");
     void* out = nullptr;
     size_t sz = 0;
-    compress(d_input, input_size, &out, &sz, stream);
+    // The concat launch writes the caller's buffer along with the pool's (which
+    // writeToFile reads) where that is safe: a result of any size fits, the
+    // buffer is this GPU's memory, aligned, and not part of the pool's.  A copy
+    // of its own behind the host's wait for the size took a launch and a second
+    // wait (10 us of a 73 us compress of 1800 x 3600 values).
+    const uint8_t* lo = (const uint8_t*)d_output_buf;
+    const bool direct = finalized_ && outputs_.size() > 1 && !graph_mode_ &&
+                        reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0 &&
+                        output_buf_capacity >= getMaxCompressedSize(input_size) && isDeviceMemory(d_output_buf);
+    if (direct) {
+        ensureBuffers(round_up(input_size, input_alignment_));
+        const uint8_t* c = (const uint8_t*)concat_buf_;
+        if (lo + output_buf_capacity <= c || c + concat_cap_ <= lo) copy_to_ = d_output_buf;
+    }
+    const bool copied = copy_to_ != nullptr;
+    try {
+        compress(d_input, input_size, &out, &sz, stream);
+    } catch (...) {
+        copy_to_ = nullptr;
+        throw;
+    }
+    copy_to_ = nullptr;
     if (sz > output_buf_capacity)
         throw std::runtime_error("compress(): output buffer too small (" + std::to_string(output_buf_capacity) +
                                  " bytes, need " + std::to_string(sz) + ")");
-    hipck(hipMemcpyAsync(d_output_buf, out, sz, hipMemcpyDeviceToDevice, stream), "hipMemcpyAsync");
-    hipck(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    if (!copied) {
+        hipck(hipMemcpyAsync(d_output_buf, out, sz, hipMemcpyDeviceToDevice, stream), "hipMemcpyAsync");
+        hipck(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    }
     *actual_output_size = sz;
 }
 
@@ -610,7 +644,7 @@ std::vector<std::pair<const void*, size_t>> Pipeline::parseConcat(const void* d_
 }
 
 void Pipeline::runInverse(const std::vector<std::pair<const void*, size_t>>& slots, hipStream_t stream,
-                          void* d_final, size_t final_cap, void** d_result, size_t* result_size) {
+                          void* d_final, size_t final_cap, size_t final_want, void** d_result, size_t* result_size) {
     if (inv_buf_.size() != buffers_.size()) {
         inv_buf_.resize(buffers_.size(), nullptr);
         inv_cap_.resize(buffers_.size(), 0);
@@ -643,7 +677,8 @@ void Pipeline::runInverse(const std::vector<std::pair<const void*, size_t>>& slo
             }
             const size_t need = n.stage->estimateOutputSizes(sizes).at(0);
             void* out;
-            if (tgt_node == 0 && d_final && final_cap >= need) {
+            if (tgt_node == 0 && d_final &&
+                (final_cap >= need || (final_want > 0 && n.stage->limitInverseOutput(final_want)))) {
                 out = d_final;
             } else {
                 const int b = tgt_buf;
@@ -727,12 +762,12 @@ void Pipeline::decompress(const void* d_input, size_t input_size, void** d_outpu
             if (!decomp_out_) throw std::runtime_error("decompress(): allocation failed");
             decomp_cap_ = round_up(input_size_, 256);
         }
-        runInverse(slots, stream, decomp_out_, decomp_cap_, &res, &rs);
+        runInverse(slots, stream, decomp_out_, decomp_cap_, 0, &res, &rs);
     } else {
         void* d = nullptr;
         hipck(hipMalloc(&d, std::max<size_t>(input_size_, 16)), "hipMalloc");
         try {
-            runInverse(slots, stream, d, input_size_, &res, &rs);
+            runInverse(slots, stream, d, input_size_, 0, &res, &rs);
         } catch (...) {
             (void)hipFree(d);
             throw;
@@ -773,7 +808,11 @@ void Pipeline::decompress(const void* d_input, size_t input_size, void* d_output
     void* res = nullptr;
     size_t rs = 0;
     const bool direct = reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0;
-    runInverse(slots, stream, direct ? d_output_buf : nullptr, direct ? output_buf_capacity : 0, &res, &rs);
+    // a buffer of the original size: the source stage leaves out the padding
+    // (a padded result of its own, a copy and a second wait were 20 of 75 us
+    // for 1800 x 3600 values)
+    const size_t limit = direct && want < input_size_ && isDeviceMemory(d_output_buf) ? want : 0;
+    runInverse(slots, stream, direct ? d_output_buf : nullptr, direct ? output_buf_capacity : 0, limit, &res, &rs);
     const size_t n = std::min(rs, want);
     if (res != d_output_buf) {
         hipck(hipMemcpyAsync(d_output_buf, res, n, hipMemcpyDeviceToDevice, stream), "hipMemcpyAsync");

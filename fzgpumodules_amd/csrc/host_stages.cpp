@@ -96,7 +96,8 @@ void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, co
         if (inputs.size() < numPorts() || outputs.empty() || sizes.size() < numPorts())
             throw std::runtime_error("LorenzoQuantStage (inverse): Requires " + std::to_string(numPorts()) +
                                      " inputs and 1 output");
-        const size_t n = sizes[0] / sizeof(TC);
+        const size_t nc = sizes[0] / sizeof(TC), n = inv_limit_ ? std::min(nc, inv_limit_) : nc;
+        inv_limit_ = 0;
         actual_output_sizes_.assign(1, n * sizeof(TI));
         if (n == 0) return;
         size_t nx, ny, nz;

@@ -74,7 +74,8 @@ rze_enc_kernel(const uint8_t* __restrict__ in, uint64_t nbytes, uint8_t* __restr
 // sizes before its chunk itself).  Raw chunks below `nshuf` (bit-shuffled
 // blocks) come from the scratch slot, other raw chunks straight from the
 // input.
-__device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c, uint32_t* s_sum) {
+__device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c, uint32_t* s_sum,
+                                               uint8_t* __restrict__ copy) {
     const uint8_t* __restrict__ in = d.in;
     const uint64_t nbytes = d.nbytes;
     const uint8_t* __restrict__ scratch = d.scratch;
@@ -97,16 +98,30 @@ __device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c,
     const uint32_t clean = size & 0x7FFFFFFFu;
     const bool raw = (size & 0x80000000u) != 0u;
     const uint64_t dst = hdr + off;
+    const uint8_t* from = scratch + (uint64_t)c * CS;
+    uint64_t limit = CS;
     if (raw && c >= nshuf) {
-        const uint64_t src = (uint64_t)c * CS;
-        copy_to_unaligned16<256>(in + src, nbytes - src, out + dst, clean);
-    } else {
-        copy_to_unaligned16<256>(scratch + (uint64_t)c * CS, CS, out + dst, clean);
+        from = in + (uint64_t)c * CS;
+        limit = nbytes - (uint64_t)c * CS;
+    }
+    copy_to_unaligned16<256>(from, limit, out + dst, clean);
+    if (copy) {  // the stream's second place: what the encoder wrote of the header, too
+        copy_to_unaligned16<256>(from, limit, copy + dst, clean);
+        if (threadIdx.x == 0) {
+            reinterpret_cast<uint32_t*>(copy + 8)[c] = size;
+            if (c == 0) {
+                reinterpret_cast<uint32_t*>(copy)[0] = (uint32_t)nbytes;
+                reinterpret_cast<uint32_t*>(copy)[1] = nc;
+            }
+        }
     }
     if (c == nc - 1) {
         const uint64_t end = hdr + (uint32_t)(off + clean);
         const uint64_t padded = (end + 3) & ~3ull;
-        if ((uint64_t)threadIdx.x < padded - end) out[end + threadIdx.x] = 0;
+        if ((uint64_t)threadIdx.x < padded - end) {
+            out[end + threadIdx.x] = 0;
+            if (copy) copy[end + threadIdx.x] = 0;
+        }
         if (threadIdx.x == 0) *d.out_size = padded;
     }
 }
@@ -115,7 +130,7 @@ __global__ void __launch_bounds__(256) rze_pack_kernel(RzePackDesc d) {
     __shared__ uint32_t s_sum[4];
     const uint32_t c = xcd_swizzle(blockIdx.x, gridDim.x);
     if (c >= d.nc) return;  // uniform over the workgroup
-    rze_pack_chunk(d, c, s_sum);
+    rze_pack_chunk(d, c, s_sum, nullptr);
 }
 
 // The pack step and the pipeline's concat + readback in one launch:
@@ -124,12 +139,12 @@ __global__ void __launch_bounds__(256) rze_pack_kernel(RzePackDesc d) {
 // RZE stream's size summed from the clean sizes rather than read from the
 // size word the pack workgroups are still writing.
 __global__ void __launch_bounds__(256)
-rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__ out, uint64_t* __restrict__ total,
-                       ReadbackArgs r, int nr, uint8_t* __restrict__ mapped) {
+rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__ out, uint8_t* __restrict__ copy,
+                       uint64_t* __restrict__ total, ReadbackArgs r, int nr, uint8_t* __restrict__ mapped) {
     __shared__ uint32_t s_sum[4];
     const uint32_t b = blockIdx.x;
     if (b < d.nc) {
-        rze_pack_chunk(d, b, s_sum);
+        rze_pack_chunk(d, b, s_sum, copy ? copy + (d.out - out) : nullptr);
         return;
     }
     uint32_t sum;
@@ -142,7 +157,7 @@ rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__
     }
     const uint64_t end = 8ull + 4ull * d.nc + sum;
     const uint64_t size0 = (end + 3) & ~3ull;
-    concat_readback_body(a, n, out, total, r, nr, mapped, b - d.nc, gridDim.x - d.nc,
+    concat_readback_body(a, n, out, copy, total, r, nr, mapped, b - d.nc, gridDim.x - d.nc,
                          SizeOverride{true, size0, reinterpret_cast<uintptr_t>(d.out_size), size0});
 }
 
@@ -498,17 +513,18 @@ int rze_enc_prepare(hipStream_t s, const void* d_in, size_t nbytes, int sew, voi
 }
 
 int rze_pack_concat_readback(hipStream_t s, const RzePackDesc& d, const fzh_concat_slot* slots, int n, void* d_out,
-                             uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries, int n_entries,
-                             void* d_mapped_dst) {
+                             void* d_copy, uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries,
+                             int n_entries, void* d_mapped_dst) {
     ConcatArgs a;
     ReadbackArgs r;
     unsigned grid = 1;
-    if (int rc = build_concat_args(slots, n, d_out, out_cap, d_total, entries, n_entries, d_mapped_dst, a, r, grid))
+    if (int rc = build_concat_args(slots, n, d_out, d_copy, false, out_cap, d_total, entries, n_entries, d_mapped_dst,
+                                   a, r, grid))
         return rc;
     if (n < 1 || slots[0].src != d.out)
         return fail(FZH_E_INVALID, "RZE pack + concat: slot 0 must be the RZE stream");
     launch_k("rze_pack_concat_kernel", rze_pack_concat_kernel, dim3(d.nc + grid), dim3(256), 0, s, d, a, n,
-             (uint8_t*)d_out, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
+             (uint8_t*)d_out, (uint8_t*)d_copy, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
     FZH_CHECK_LAUNCH("rze_pack_concat_kernel");
     return FZH_OK;
 }

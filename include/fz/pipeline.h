@@ -178,8 +178,10 @@ class Pipeline {
     void ensureBuffers(size_t padded_input);
     void launchForward(const void* d_in, size_t padded, bool zero_view, hipStream_t stream);
     void finishCompress(hipStream_t stream, void** d_output, size_t* output_size);
+    // final_want: the bytes the caller asked for, where its buffer holds no
+    // more than those (0: the buffer takes the padded result or none).
     void runInverse(const std::vector<std::pair<const void*, size_t>>& outputs, hipStream_t stream,
-                    void* d_final, size_t final_cap, void** d_result, size_t* result_size);
+                    void* d_final, size_t final_cap, size_t final_want, void** d_result, size_t* result_size);
     std::vector<std::pair<const void*, size_t>> parseConcat(const void* d_input, size_t input_size,
                                                             hipStream_t stream);
     void collectReadbacks();
@@ -193,6 +195,7 @@ class Pipeline {
     std::vector<std::unique_ptr<Stage>> stages_;
     struct Edge { Stage* dep; Stage* prod; std::string name; };
     std::vector<Edge> edges_;
+    void* copy_to_ = nullptr;       // the running compress() call's own buffer, written with the concat
     std::vector<Node> nodes_;       // topological order
     std::vector<Buffer> buffers_;   // 0 = pipeline input
     std::vector<int> outputs_;      // buffer ids of pipeline outputs, in order

@@ -122,6 +122,11 @@ class Stage {
     // passes the caller's buffer instead of a padded copy.
     virtual bool acceptZeroPaddedInput(size_t valid_bytes) { (void)valid_bytes; return false; }
 
+    // Asks the next inverse execute() to reconstruct only the first `bytes`
+    // bytes of the (padded) input and store nothing past them.  False if the
+    // stage cannot: it then stores all of it.
+    virtual bool limitInverseOutput(size_t bytes) { (void)bytes; return false; }
+
     virtual DeviceSize getDeviceOutputSize(int index) const { (void)index; return {}; }
 
     // Device values postStreamSync() needs, registered by execute().  A

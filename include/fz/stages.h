@@ -166,6 +166,15 @@ class LorenzoQuantStage : public Stage {
         valid_elems_ = valid_bytes / sizeof(TInput);
         return !is_inverse_ && valid_bytes % sizeof(TInput) == 0;
     }
+    // The tiles of the given dims (all elements in 1D) hold every value that
+    // the inverse stores but patches, whose indices the kernels check.
+    bool limitInverseOutput(size_t bytes) override {
+        const size_t n = bytes / sizeof(TInput);
+        if (!is_inverse_ || bytes == 0 || bytes % sizeof(TInput) != 0) return false;
+        if (ndim() > 1 && (config_.dims[0] == 0 || config_.dims[0] * config_.dims[1] * config_.dims[2] > n)) return false;
+        inv_limit_ = n;
+        return true;
+    }
     DeviceSize getDeviceOutputSize(int index) const override {
         if (is_inverse_) return {};
         if (index == 1 && d_count_ptr_) return {d_count_ptr_, 2, (uint32_t)sizeof(TInput)};
@@ -204,6 +213,7 @@ class LorenzoQuantStage : public Stage {
 
     Config config_;
     bool is_inverse_ = false;
+    size_t inv_limit_ = 0;  // elements of the next inverse execute() (0: all)
     std::vector<size_t> actual_output_sizes_ = std::vector<size_t>(4, 0), saved_output_sizes_;
     size_t num_elements_ = 0;
     uint32_t actual_outlier_count_ = 0;
