@@ -13,7 +13,8 @@
 //   lorenzo     codes + per-tile lists (kListSlots entries) + per-tile counts,
 //               one launch per tile shape (3D, 2D, 1D fields)
 //   rze         fused Bitshuffle+RZE, one workgroup per chunk, into a chunk
-//               scratch slot
+//               scratch slot; or, with a Huffman coder, one histogram and one
+//               codebook per field and one wave per 768-code partition
 //   scan        one exclusive scan (mod 2^32) over [tile outliers | tile
 //               patches | chunk bytes]; per-field offsets are differences
 //   finalize    one thread per field: result layout, concat header, pads
@@ -21,6 +22,7 @@
 //   scatter     tile lists to their place in the field's outlier / patch
 //               arrays; a tile whose list outgrew kListSlots is recomputed
 #include "fzh_batch.h"
+#include "fzh_huffman_enc.h"
 #include "fzh_lorenzo_tile.h"
 #include "fzh_rze_chunk.h"
 #include "fzh_scan.h"
@@ -319,6 +321,88 @@ __global__ void __launch_bounds__(256) rze_batch_kernel(const Plan* __restrict__
 }
 
 // ---------------------------------------------------------------------------
+// Huffman coder: histogram and codebook per field, one wave per partition.
+// A 256 KiB field alone pays a dozen launches and two host waits for its
+// 65536 codes (43 us a field with eight host threads); here every stage is
+// one launch for all fields, the codebooks' serial merges side by side.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) hist_batch_kernel(const Plan* __restrict__ pp) {
+    const Plan& p = *pp;
+    extern __shared__ uint32_t sh[];
+    const uint32_t bklen = p.huf.bklen, rs = bklen + 1;  // eight replicas: two per wave, by lane parity
+    for (uint32_t i = threadIdx.x; i < 8 * rs; i += 256) sh[i] = 0;
+    __syncthreads();
+    uint32_t* h = sh + (size_t)(2 * (threadIdx.x >> 6) + (threadIdx.x & 1)) * rs;
+    const uint32_t f = rfl(gp(p.ufield)[blockIdx.x]);
+    const Field fd = uniform_field(p.fields + f);
+    const uint64_t b = (uint64_t)(blockIdx.x - fd.unit0) * kVbUnit, e = min(fd.n, b + kVbUnit);
+    const uint16_t* c = p.codes + fd.codes_off;  // codes_off and b are multiples of 8
+    const uint64_t e8 = b + ((e - b) & ~7ull);
+    for (uint64_t i = b + 8 * (uint64_t)threadIdx.x; i < e8; i += 2048) {
+        const uint4 w = gld_u4(c + i);
+        const uint16_t* v = reinterpret_cast<const uint16_t*>(&w);
+        uint32_t cur = v[0], cnt = 1;
+#pragma unroll
+        for (int k = 1; k < 8; k++) {
+            if (v[k] == cur) {
+                cnt++;
+            } else {
+                if (cur < bklen) atomicAdd(&h[cur], cnt);
+                cur = v[k];
+                cnt = 1;
+            }
+        }
+        if (cur < bklen) atomicAdd(&h[cur], cnt);
+    }
+    if (e8 + threadIdx.x < e) {
+        const uint32_t v = gp(c)[e8 + threadIdx.x];
+        if (v < bklen) atomicAdd(&h[v], 1u);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < bklen; i += 256) {
+        uint32_t t = 0;
+        for (uint32_t r = 0; r < 8; r++) t += sh[r * rs + i];
+        if (t) atomicAdd(&p.huf.freq[(size_t)f * bklen + i], t);
+    }
+}
+
+__global__ void __launch_bounds__(256) huf_enc_batch_kernel(const Plan* __restrict__ pp) {
+    const Plan& p = *pp;
+    extern __shared__ uint32_t sh[];
+    const uint32_t w = wave_in_wg();
+    const int l = lane_id();
+    uint32_t* cells = sh + w * kHufCells;
+    uint32_t* s_bk = sh + 4 * kHufCells;
+    const uint32_t f = rfl(gp(p.huf.wg_field)[blockIdx.x]), p0 = rfl(gp(p.huf.wg_part)[blockIdx.x]);
+    const Field fd = uniform_field(p.fields + f);
+    const uint32_t bklen = p.huf.bklen;
+    for (uint32_t i = threadIdx.x; i < bklen; i += 256) s_bk[i] = gp(p.huf.bk4)[(size_t)f * bklen + i];
+    __syncthreads();
+    const uint32_t cbase = p.T * (p.strict ? 2u : 1u);
+    uint8_t* st = p.out + fd.out_off + p.hdr;  // the field's stream
+    if (p0 == 0) {
+        for (uint32_t i = threadIdx.x; i < p.huf.rev_bytes; i += 256)
+            gp(st)[HDR_BYTES + i] = gp(p.huf.rev)[(size_t)f * p.huf.rev_stride + i];
+        if (threadIdx.x < HDR_BYTES - 64) gp(st)[64 + threadIdx.x] = 0;
+    }
+    const uint32_t p1 = min(p0 + kHufUnit, fd.nchunks);
+    for (uint32_t lp = p0 + w; lp < p1; lp += 4) {
+        const uint64_t s0 = (uint64_t)lp * kHufPart;
+        const uint32_t cnt = (uint32_t)min((uint64_t)kHufPart, fd.n - s0);
+        const uint32_t nbit = huf_encode_partition<uint16_t, (int)kHufPart, true>(p.codes + fd.codes_off + s0, cnt, true,
+                                                                                  s_bk, nullptr, bklen, cells);
+        const uint32_t ncell = (nbit + 31) / 32;
+        uint32_t* dst = p.huf.cells + (uint64_t)(fd.chunk0 + lp) * kHufCells;
+        for (uint32_t i = l; i < ncell; i += 64) gp(dst)[i] = cells[i];
+        if (l == 0) {
+            gp(reinterpret_cast<uint32_t*>(st + HDR_BYTES + p.huf.rev_bytes))[lp] = nbit;
+            gp(p.counts)[cbase + fd.chunk0 + lp] = ncell;
+        }
+        wave_lds_sync();
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Per-field layout of the result (fz::Pipeline's concat, fzh_core.hip)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint64_t pad16(uint64_t v) { return (v + 15) & ~15ull; }
@@ -327,12 +411,10 @@ __device__ __forceinline__ void zero_range(uint8_t* b, uint64_t from, uint64_t t
     for (uint64_t i = from; i < to; i++) b[i] = 0;
 }
 
-__global__ void __launch_bounds__(256) finalize_kernel(const Plan* __restrict__ pp) {
-    const Plan& p = *pp;
-    const uint32_t f = blockIdx.x * 256 + threadIdx.x;
-    if (f >= p.F) return;
-    const Field& fd = p.fields[f];
-    const uint32_t cbase = p.T * (p.strict ? 2u : 1u);
+// Field f's result around a coder stream of `len` bytes, stored as `bytes`
+// (one thread).  False if it does not fit the field's region.
+__device__ __forceinline__ bool finalize_field(const Plan& p, uint32_t f, const Field& fd, uint64_t len, uint64_t bytes,
+                                               uint32_t ex_c, uint32_t flags) {
     const uint32_t ex_t = p.excl[fd.tile0];
     const uint32_t k = p.excl[fd.tile0 + fd.ntiles] - ex_t;
     uint32_t ex_p = 0, kp = 0;
@@ -340,12 +422,8 @@ __global__ void __launch_bounds__(256) finalize_kernel(const Plan* __restrict__ 
         ex_p = p.excl[p.T + fd.tile0];
         kp = p.excl[p.T + fd.tile0 + fd.ntiles] - ex_p;
     }
-    const uint32_t ex_c = p.excl[cbase + fd.chunk0];
-    const uint64_t csum = (uint32_t)(p.excl[cbase + fd.chunk0 + fd.nchunks] - ex_c);
-    const uint64_t rze_len = 8ull + 4ull * fd.nchunks + csum;
-    const uint64_t rze_bytes = (rze_len + 3) & ~3ull;
     const uint32_t ko = min(k, fd.max_out), kpo = min(kp, fd.max_patch);
-    uint64_t sz[7] = {rze_bytes, 4ull * ko, 4ull * ko, 4, 4ull * kpo, 4ull * kpo, 4};
+    uint64_t sz[7] = {bytes, 4ull * ko, 4ull * ko, 4, 4ull * kpo, 4ull * kpo, 4};
     uint64_t off[7];
     uint64_t o = p.hdr;
     for (uint32_t i = 0; i < p.nout; i++) {
@@ -356,7 +434,7 @@ __global__ void __launch_bounds__(256) finalize_kernel(const Plan* __restrict__ 
     res.bytes = o;
     res.k = k;
     res.kp = kp;
-    res.flags = (k > fd.max_out ? kOverflowOutliers : 0u) | (kp > fd.max_patch ? kOverflowPatches : 0u);
+    res.flags = flags | (k > fd.max_out ? kOverflowOutliers : 0u) | (kp > fd.max_patch ? kOverflowPatches : 0u);
     res.pad[0] = res.pad[1] = res.pad[2] = 0;
     Derived d;
     d.o_err = off[1];
@@ -380,13 +458,61 @@ __global__ void __launch_bounds__(256) finalize_kernel(const Plan* __restrict__ 
             b32[2 + 2 * i] = (uint32_t)(sz[i] >> 32);
         }
         zero_range(b, 4 + 8ull * p.nout, p.hdr);
-        zero_range(b, off[0] + rze_len, off[0] + pad16(rze_bytes));
+        zero_range(b, off[0] + len, off[0] + pad16(bytes));
         for (uint32_t i = 1; i < p.nout; i++) zero_range(b, off[i] + sz[i], off[i] + pad16(sz[i]));
         b32[off[3] / 4] = k;
         if (p.strict) b32[off[6] / 4] = kp;
     }
     p.derived[f] = d;
     p.results[f] = res;
+    return (res.flags & kOverflowCapacity) == 0;
+}
+
+__global__ void __launch_bounds__(256) finalize_kernel(const Plan* __restrict__ pp) {
+    const Plan& p = *pp;
+    const uint32_t f = blockIdx.x * 256 + threadIdx.x;
+    if (f >= p.F) return;
+    const Field& fd = p.fields[f];
+    const uint32_t cbase = p.T * (p.strict ? 2u : 1u);
+    const uint32_t ex_c = p.excl[cbase + fd.chunk0];
+    const uint64_t csum = (uint32_t)(p.excl[cbase + fd.chunk0 + fd.nchunks] - ex_c);
+    const uint64_t rze_len = 8ull + 4ull * fd.nchunks + csum;
+    (void)finalize_field(p, f, fd, rze_len, (rze_len + 3) & ~3ull, ex_c, 0u);
+}
+
+// The same for a Huffman stream, one wave per field: the lanes add up the
+// partitions' bit counts for phf_header (hf.h:38-44).
+__global__ void __launch_bounds__(256) finalize_huf_kernel(const Plan* __restrict__ pp) {
+    const Plan& p = *pp;
+    const uint32_t f = blockIdx.x * 4 + wave_in_wg();
+    if (f >= p.F) return;
+    const Field& fd = p.fields[f];
+    const uint32_t cbase = p.T * (p.strict ? 2u : 1u);
+    const uint32_t ex_c = p.excl[cbase + fd.chunk0];
+    const uint32_t ncell = p.excl[cbase + fd.chunk0 + fd.nchunks] - ex_c;
+    const uint32_t ent1 = HDR_BYTES, ent2 = ent1 + p.huf.rev_bytes, ent3 = ent2 + 4 * fd.nchunks,
+                   ent4 = ent3 + 4 * fd.nchunks, ent5 = ent4 + 4 * ncell;
+    uint8_t* st = p.out + fd.out_off + p.hdr;
+    uint64_t bits = 0;
+    for (uint32_t i = lane_id(); i < fd.nchunks; i += 64) bits += reinterpret_cast<const uint32_t*>(st + ent2)[i];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) bits += __shfl_xor(bits, off, 64);
+    if (lane_id() != 0) return;
+    if (!finalize_field(p, f, fd, ent5, ent5, ex_c, p.huf.status[f] ? kBadBook : 0u)) return;
+    uint32_t* h32 = reinterpret_cast<uint32_t*>(st);
+    h32[0] = p.huf.bklen & 0xFFFFu;
+    h32[1] = kHufPart;
+    h32[2] = fd.nchunks;
+    h32[3] = 0;
+    reinterpret_cast<uint64_t*>(st)[2] = fd.n;
+    reinterpret_cast<uint64_t*>(st)[3] = bits;
+    reinterpret_cast<uint64_t*>(st)[4] = ncell;
+    h32[10] = 0;
+    h32[11] = ent1;
+    h32[12] = ent2;
+    h32[13] = ent3;
+    h32[14] = ent4;
+    h32[15] = ent5;
 }
 
 // ---------------------------------------------------------------------------
@@ -413,6 +539,25 @@ __global__ void __launch_bounds__(256) pack_batch_kernel(const Plan* __restrict_
             copy_to_unaligned16(reinterpret_cast<const uint8_t*>(p.codes + fd.codes_off) + off, cb - off, dst, clean);
         else
             copy_to_unaligned16(p.chunk_scratch + (uint64_t)gc * kChunk, kChunk, dst, clean);
+    }
+}
+
+// Partitions' cells to their place in the field's Huffman stream.
+__global__ void __launch_bounds__(256) huf_pack_batch_kernel(const Plan* __restrict__ pp) {
+    const Plan& p = *pp;
+    const uint32_t waves = gridDim.x * 4;
+    const uint32_t cbase = p.T * (p.strict ? 2u : 1u);
+    for (uint32_t gc = blockIdx.x * 4 + wave_in_wg(); gc < p.NC; gc += waves) {
+        const uint32_t f = rfl(gp(p.cfield)[gc]);
+        if (p.results[f].flags & kOverflowCapacity) continue;
+        const Field& fd = p.fields[f];
+        const uint32_t e = p.excl[cbase + gc] - p.derived[f].ex_c, c = p.counts[cbase + gc];
+        const uint32_t ent3 = HDR_BYTES + p.huf.rev_bytes + 4 * fd.nchunks;
+        uint32_t* st = reinterpret_cast<uint32_t*>(p.out + fd.out_off + p.hdr + ent3);
+        if (lane_id() == 0) gp(st)[gc - fd.chunk0] = e;
+        uint32_t* dst = st + fd.nchunks + e;
+        const uint32_t* src = p.huf.cells + (uint64_t)gc * kHufCells;
+        for (uint32_t i = lane_id(); i < c; i += 64) gp(dst)[i] = gp(src)[i];
     }
 }
 
@@ -545,19 +690,36 @@ int launch_rze(hipStream_t s, const Plan& p, const Plan* dp) {
     return FZH_OK;
 }
 
+int launch_huffman(hipStream_t s, const Plan& p, const Plan* dp) {
+    const Huffman& h = p.huf;
+    if (int rc = zero_bytes(s, h.freq, 4 * (size_t)p.F * h.bklen)) return rc;
+    hist_batch_kernel<<<p.U, 256, 32 * (h.bklen + 1), s>>>(dp);
+    if (int rc = build_books_device(s, p.F, h.freq, h.bklen, h.n_of, h.bk4, h.rev, h.rev_stride, h.status)) return rc;
+    huf_enc_batch_kernel<<<h.NW, 256, 4 * (4 * kHufCells + h.bklen), s>>>(dp);
+    FZH_CHECK_LAUNCH("batch huffman");
+    return FZH_OK;
+}
+
 int launch_scan(hipStream_t s, const Plan& p) {
     return fzh::scan_u32<true>(s, p.counts, p.excl, p.n_counts, nullptr, p.excl + p.n_counts, p.scan_ws);
 }
 
 int launch_finalize(hipStream_t s, const Plan& p, const Plan* dp) {
-    finalize_kernel<<<(unsigned)cdiv(p.F, 256), 256, 0, s>>>(dp);
+    if (p.huf.bklen)
+        finalize_huf_kernel<<<(unsigned)cdiv(p.F, 4), 256, 0, s>>>(dp);
+    else
+        finalize_kernel<<<(unsigned)cdiv(p.F, 256), 256, 0, s>>>(dp);
     FZH_CHECK_LAUNCH("batch finalize");
     return FZH_OK;
 }
 
 int launch_pack(hipStream_t s, const Plan& p, const Plan* dp, uint32_t grid) {
     const unsigned g = std::max<uint32_t>(1, std::min<uint32_t>(grid, (uint32_t)cdiv(p.NC, 4)));
-    pack_batch_kernel<<<g, 256, 0, s>>>(dp);
+    if (p.huf.bklen)
+        huf_pack_batch_kernel<<<(unsigned)std::max<size_t>(1, std::min<size_t>(8 * (size_t)grid, cdiv(p.NC, 4))), 256, 0,
+                                s>>>(dp);
+    else
+        pack_batch_kernel<<<g, 256, 0, s>>>(dp);
     FZH_CHECK_LAUNCH("batch pack");
     return FZH_OK;
 }

@@ -4,7 +4,8 @@
 // A batch is flattened into three global index spaces, each with a per-field
 // start table (F + 1 entries, strictly increasing):
 //   tiles   Lorenzo tiles of every field (1024 / 32x32 / 8x8x8 elements)
-//   chunks  16 KiB chunks of every field's codes (Bitshuffle block = RZE chunk)
+//   chunks  16 KiB chunks of every field's codes (Bitshuffle block = RZE chunk),
+//           or 768-code partitions when the codes are Huffman coded
 //   units   VB_UNIT-element slices of every field (value-base reduction)
 // Each kernel walks one space -- with a fixed persistent grid, except the
 // RZE encoder, which takes one workgroup per chunk -- mapping a global index
@@ -54,7 +55,24 @@ struct Result {
     uint32_t flags;  // kOverflowOutliers | kOverflowPatches | kOverflowCapacity
     uint32_t pad[3];
 };
-constexpr uint32_t kOverflowOutliers = 1u, kOverflowPatches = 2u, kOverflowCapacity = 4u;
+constexpr uint32_t kOverflowOutliers = 1u, kOverflowPatches = 2u, kOverflowCapacity = 4u, kBadBook = 8u;
+
+// Huffman coder of a batch (bklen 0: Bitshuffle -> RZE).
+constexpr uint32_t kHufPart = 768;                       // codes per partition
+constexpr uint32_t kHufCells = (768 * 28 + 31) / 32 + 2; // cells of a partition's scratch slot
+constexpr uint32_t kHufUnit = 16;                        // partitions per encode workgroup
+struct Huffman {
+    uint32_t bklen, rev_bytes, rev_stride;
+    uint32_t NW;               // encode workgroups
+    const uint32_t* wg_field;  // NW: the field of each
+    const uint32_t* wg_part;   // NW: its first partition inside the field
+    const uint64_t* n_of;      // F: codes per field
+    uint32_t* freq;            // F * bklen
+    uint32_t* bk4;             // F * bklen
+    uint8_t* rev;              // F * rev_stride
+    int* status;               // F
+    uint32_t* cells;           // NC * kHufCells
+};
 
 struct Plan {
     const Field* fields;
@@ -102,6 +120,7 @@ struct Plan {
     Result* results;         // F
     uint8_t* out;
     void* scan_ws;
+    Huffman huf;
 };
 
 size_t scan_ws_bytes_for(size_t n_counts);
@@ -113,6 +132,8 @@ size_t scan_ws_bytes_for(size_t n_counts);
 int launch_value_base(hipStream_t s, const Plan& p, const Plan* dp, uint32_t grid);
 int launch_lorenzo(hipStream_t s, const Plan& p, const Plan* dp, uint32_t grid, uint32_t tiles_per_unit);
 int launch_rze(hipStream_t s, const Plan& p, const Plan* dp);
+// Histograms, codebooks and partitions' codewords of every field.
+int launch_huffman(hipStream_t s, const Plan& p, const Plan* dp);
 int launch_scan(hipStream_t s, const Plan& p);
 int launch_finalize(hipStream_t s, const Plan& p, const Plan* dp);
 int launch_pack(hipStream_t s, const Plan& p, const Plan* dp, uint32_t grid);

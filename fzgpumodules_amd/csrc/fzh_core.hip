@@ -140,6 +140,66 @@ __global__ void __launch_bounds__(256) gather_kernel(const fzh_copy_desc* __rest
     }
 }
 
+// CRC-32 (IEEE 802.3, reflected polynomial 0xEDB88320) of one segment per
+// workgroup.  The register is linear in its start and its data, so every
+// thread runs its own stretch of the segment from 0 (four table lookups per
+// word, tables in LDS) and the stretches are joined pairwise: left
+// x^(8 right bytes) + right modulo the polynomial.  All stretches have the
+// same length; zeros in front, which leave a register of 0 at 0, fill the
+// segment up.
+__device__ __forceinline__ uint32_t gf2_mul(uint32_t a, uint32_t b) {  // bit 31 is x^0
+    uint32_t p = 0;
+#pragma unroll
+    for (int i = 31; i >= 0; i--) {
+        p ^= ((a >> i) & 1u) ? b : 0u;
+        b = (b >> 1) ^ ((b & 1u) ? 0xEDB88320u : 0u);
+    }
+    return p;
+}
+
+__global__ void __launch_bounds__(256) crc32_kernel(const fzh_copy_desc* __restrict__ d, uint32_t* __restrict__ out) {
+    __shared__ uint32_t tab[4][256], part[256];
+    const uint32_t t = threadIdx.x;
+    uint32_t c = t;
+#pragma unroll
+    for (int i = 0; i < 8; i++) c = (c >> 1) ^ ((c & 1u) ? 0xEDB88320u : 0u);
+    tab[0][t] = c;
+    __syncthreads();
+#pragma unroll
+    for (int k = 1; k < 4; k++) {  // one more zero byte behind
+        c = (c >> 8) ^ tab[0][c & 0xFFu];
+        tab[k][t] = c;
+    }
+    __syncthreads();
+    const uint8_t* p = (const uint8_t*)d[blockIdx.x].dst;
+    const uint64_t units = d[blockIdx.x].bytes / 16, per = (units + 255) / 256, front = per * 256 - units;
+    uint32_t r = 0;
+    for (uint64_t u = t * per; u < (t + 1) * per; u++) {
+        if (u < front) continue;
+        const uint4 v = gld_u4(p + 16 * (u - front));
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            r ^= w[k];
+            r = tab[3][r & 0xFFu] ^ tab[2][(r >> 8) & 0xFFu] ^ tab[1][(r >> 16) & 0xFFu] ^ tab[0][r >> 24];
+        }
+    }
+    part[t] = r;
+    // x^(128 per), then its square for every level
+    uint32_t f = 0x80000000u, sq = 0x80000000u >> 1;  // 1, x
+    for (int i = 0; i < 7; i++) sq = gf2_mul(sq, sq);  // x^128
+    for (uint64_t n = per; n; n >>= 1) {
+        if (n & 1) f = gf2_mul(f, sq);
+        sq = gf2_mul(sq, sq);
+    }
+    for (uint32_t k = 1; k < 256; k <<= 1) {
+        __syncthreads();
+        if (t % (2 * k) == 0) part[t] = gf2_mul(part[t], f) ^ part[t + k];
+        f = gf2_mul(f, f);
+    }
+    if (t == 0) out[blockIdx.x] = part[0];
+}
+
 // Grid-stride device copy with 16-byte accesses (both ends 16-byte aligned).
 __global__ void __launch_bounds__(256) copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t nw) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -418,6 +478,13 @@ int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_
     launch_k("concat_readback_kernel", concat_readback_kernel, dim3(grid), dim3(256), 0, s, a, n, (uint8_t*)d_out,
              (uint8_t*)d_copy, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
     FZH_CHECK_LAUNCH("concat_readback_kernel");
+    return FZH_OK;
+}
+
+int crc32_segments(hipStream_t s, const fzh_copy_desc* d_descs, int n_segs, uint32_t* d_out) {
+    if (n_segs <= 0) return FZH_OK;
+    launch_k("crc32_kernel", crc32_kernel, dim3((unsigned)n_segs), dim3(256), 0, s, d_descs, d_out);
+    FZH_CHECK_LAUNCH("crc32_kernel");
     return FZH_OK;
 }
 

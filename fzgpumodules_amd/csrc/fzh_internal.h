@@ -49,6 +49,16 @@ int rze_pack_concat_readback(hipStream_t s, const RzePackDesc& d, const fzh_conc
                              void* d_copy, uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries,
                              int n_entries, void* d_mapped_dst);
 
+// out[i]: CRC-32 register, started at 0, over segment i's destination bytes
+// (16-byte aligned, a multiple of 16 bytes).
+int crc32_segments(hipStream_t s, const fzh_copy_desc* d_descs, int n_segs, uint32_t* d_out);
+
+// fzh_huffman_build_book_device for n_books histograms of 2-byte symbols in
+// one launch: bklen counts and bklen codes each, one after another, reverse
+// books every rev_stride bytes, d_n[i] = symbols of histogram i.
+int build_books_device(hipStream_t s, uint32_t n_books, const uint32_t* d_freq, uint32_t bklen, const uint64_t* d_n,
+                       uint32_t* d_bk4, uint8_t* d_revbook, size_t rev_stride, int* d_status);
+
 // fzh_concat_readback with a second destination of the whole result (both
 // launches: d_copy null, or 16-byte aligned and out_cap bytes).
 int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, uint64_t out_cap,

@@ -33,22 +33,51 @@ uint64_t align_to(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
 
+// A plan's device memory: one allocation, kept for the next plan if that one
+// fits it (a selector plans its chunks anew for every field; some twenty
+// allocations and table copies were 2 ms of each plan).  Tables come first
+// and are collected on the host, so they go up in one copy.
 struct BatchCompressor::Impl {
     fzh::batch::Plan plan{};
     fzh::batch::Plan* d_plan = nullptr;  // device copy read by the kernels
-    std::vector<void*> allocs;
+    uint8_t* arena = nullptr;
+    size_t cap = 0, used = 0;
+    std::vector<uint8_t> tables;         // host image of the arena's first bytes
     fzh::batch::Result* h_results = nullptr;  // host-mapped
+    size_t results_cap = 0;
     void* d_results_map = nullptr;
     hipEvent_t ev[9] = {};
 
+    static size_t piece(size_t bytes) { return align_to(std::max<size_t>(bytes, 256), 256); }
+    // Starts a plan of `bytes` (a sum of pieces).
+    void reserve(size_t bytes) {
+        used = 0;
+        tables.clear();
+        if (cap >= bytes) return;
+        if (arena) (void)hipFree(arena);
+        arena = nullptr;
+        cap = 0;
+        hipck(hipMalloc((void**)&arena, bytes), "hipMalloc (batch)");
+        cap = bytes;
+    }
     void* dev(size_t bytes) {
-        void* p = nullptr;
-        hipck(hipMalloc(&p, std::max<size_t>(bytes, 256)), "hipMalloc (batch)");
-        allocs.push_back(p);
+        if (used + piece(bytes) > cap) throw std::logic_error("BatchCompressor: plan exceeds its reservation");
+        void* p = arena + used;
+        used += piece(bytes);
         return p;
     }
+    template <typename T>
+    T* table(const T* src, size_t count) {
+        T* d = (T*)dev(count * sizeof(T));
+        tables.resize(used);
+        if (count) std::memcpy(tables.data() + ((uint8_t*)d - arena), src, count * sizeof(T));
+        return d;
+    }
+    template <typename T>
+    T* table(const std::vector<T>& v) { return table(v.data(), v.size()); }
+    void upload() { hipck(hipMemcpy(arena, tables.data(), tables.size(), hipMemcpyHostToDevice), "hipMemcpy (tables)"); }
     ~Impl() {
-        for (void* p : allocs) (void)hipFree(p);
+        if (arena) (void)hipFree(arena);
         if (h_results) (void)hipHostFree(h_results);
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
@@ -64,6 +93,8 @@ BatchCompressor::BatchCompressor(const BatchConfig& cfg) : cfg_(cfg) {
         throw std::invalid_argument("BatchCompressor: outlier_capacity must be in [0, 1]");
     if (!(cfg.patch_capacity >= 0.0f) || cfg.patch_capacity > 1.0f)
         throw std::invalid_argument("BatchCompressor: patch_capacity must be in [0, 1]");
+    if (cfg.huffman_bklen > 1024 || (cfg.huffman_bklen & 1))
+        throw std::invalid_argument("BatchCompressor: huffman_bklen must be 0 or an even number up to 1024");
     int dev = 0;
     hipck(hipGetDevice(&dev), "hipGetDevice");
     hipck(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
@@ -74,6 +105,12 @@ BatchCompressor::~BatchCompressor() {
     destroyGraph();
     if (graph_stream_) (void)hipStreamDestroy(graph_stream_);
     release();
+}
+
+void BatchCompressor::setErrorBound(float eb) {
+    if (!(eb > 0.0f) || !std::isfinite(eb))
+        throw std::invalid_argument("BatchCompressor: error_bound must be positive and finite");
+    cfg_.error_bound = eb;
 }
 
 void BatchCompressor::release() {
@@ -96,7 +133,11 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
     if (fields.empty()) throw std::invalid_argument("BatchCompressor: no fields");
     if (fields.size() > (1u << 24)) throw std::invalid_argument("BatchCompressor: more than 2^24 fields");
     destroyGraph();
-    release();
+    // a failed plan leaves none; a good one takes over the previous one's memory
+    std::unique_ptr<Impl> im(impl_ ? impl_ : new Impl());
+    impl_ = nullptr;
+    d_out_ = nullptr;
+    out_cap_ = 0;
     fields_ = fields;
     const size_t F = fields.size();
     std::vector<Field> tab(F);
@@ -104,7 +145,7 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
     uint64_t T = 0, NC = 0, U = 0, codes = 0, out = 0;
     in_bytes_ = 0;
     out_off_.assign(F, 0);
-    const bool strict = cfg_.strict;
+    const bool strict = cfg_.strict, huf = cfg_.huffman_bklen != 0;
     const uint32_t nout = strict ? 7 : 4;
     const uint32_t hdr = (uint32_t)align_to(4 + 8ull * nout, 16);
     for (size_t i = 0; i < F; i++) {
@@ -116,7 +157,8 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
             throw std::invalid_argument("BatchCompressor: field " + std::to_string(i) + " is empty");
         const uint64_t nv = (uint64_t)b.nx * b.ny * b.nz;
         const uint64_t bytes = 4 * nv;
-        const uint64_t n = align_to(bytes, kChunk) / 4;  // Pipeline pads the input to 16 KiB (Bitshuffle/RZE)
+        // Pipeline pads the input to 16 KiB for Bitshuffle/RZE
+        const uint64_t n = huf ? nv : align_to(bytes, kChunk) / 4;
         if (n > 0xFFFFFFFFull) throw std::invalid_argument("BatchCompressor: field larger than 2^32 elements");
         Field& f = tab[i];
         std::memset(&f, 0, sizeof(f));
@@ -129,7 +171,7 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
         f.ndim = b.nz > 1 ? 3 : (b.ny > 1 ? 2 : 1);
         uint64_t ntiles;
         if (f.ndim == 1) {
-            ntiles = n / 1024;
+            ntiles = fzh::cdiv(n, 1024);
         } else if (f.ndim == 2) {
             f.gx = (uint32_t)fzh::cdiv(b.nx, 32);
             ntiles = (uint64_t)f.gx * fzh::cdiv(b.ny, 32);
@@ -138,7 +180,7 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
             f.gy = (uint32_t)fzh::cdiv(b.ny, 8);
             ntiles = (uint64_t)f.gx * f.gy * fzh::cdiv(b.nz, 8);
         }
-        const uint64_t nch = fzh::cdiv(2 * n, kChunk);
+        const uint64_t nch = huf ? fzh::cdiv(n, kHufPart) : fzh::cdiv(2 * n, kChunk);
         const uint64_t nun = fzh::cdiv(nv, kVbUnit);
         // LorenzoQuantStage's capacities (maxOutliers / maxPatches)
         const uint64_t max_out = (uint64_t)std::ceil((double)n * cfg_.outlier_capacity);
@@ -152,7 +194,8 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
         f.max_out = (uint32_t)std::min<uint64_t>(max_out, 0xFFFFFFFFu);
         f.max_patch = strict ? (uint32_t)std::min<uint64_t>(max_patch, 0xFFFFFFFFu) : 0u;
         f.codes_off = codes;
-        uint64_t cap = hdr + align_to(fzh_rze_enc_bound(2 * n), 16) + 2 * align_to(4 * max_out, 16) + 16;
+        const uint64_t coder = huf ? fzh_huffman_enc_bound(n, cfg_.huffman_bklen, 2) : fzh_rze_enc_bound(2 * n);
+        uint64_t cap = hdr + align_to(coder, 16) + 2 * align_to(4 * max_out, 16) + 16;
         if (strict) cap += 2 * align_to(4 * max_patch, 16) + 16;
         f.out_off = out;
         f.out_cap = cap;
@@ -163,7 +206,7 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
         T += ntiles;
         NC += nch;
         U += nun;
-        codes += n;
+        codes += align_to(n, 8);  // 16-byte aligned
         out += align_to(cap, 256);
         in_bytes_ += bytes;
         if (T >= 0xFFFFFFF0ull || NC >= 0x0FFFFFFFull || U >= 0xFFFFFFF0ull)
@@ -175,8 +218,29 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
     const uint64_t n_counts = T * (strict ? 2 : 1) + NC;
     if (n_counts >= 0xFFFFFFF0ull) throw std::invalid_argument("BatchCompressor: batch too large (count table)");
 
-    impl_ = new Impl();
-    Plan& p = impl_->plan;
+    std::vector<uint32_t> hwf, hwp;  // encode workgroups
+    std::vector<uint64_t> hns;
+    const size_t rev_stride = huf ? align_to(fzh_huffman_revbook_bytes(cfg_.huffman_bklen, 2), 16) : 0;
+    if (huf)
+        for (uint32_t f = 0; f < F; f++) {
+            hns.push_back(tab[f].n);
+            for (uint32_t q = 0; q < tab[f].nchunks; q += kHufUnit) {
+                hwf.push_back(f);
+                hwp.push_back(q);
+            }
+        }
+    // pieces: the tables below (class tables sum to at most 3 F + 3 entries
+    // and a 64th of the tiles), then the buffers in the order they are taken
+    const size_t B = huf ? cfg_.huffman_bklen : 0;
+    const size_t lists = 4ull * kListSlots * T;
+    size_t need = sizeof(Field) * F + 4 * (10 * F + 16) + 4 * (T / 16 + 16) + 4 * (NC + U + 2) + sizeof(Plan) +
+                  8 * hns.size() + 8 * hwf.size() + 32 * 256;
+    need += 16 * F + 8 * (U + 1) + 2 * codes + (strict ? 4 : 2) * lists + 4 * n_counts + 4 * (n_counts + 1) +
+            (huf ? F * (8 * B + rev_stride + 4) + 4ull * kHufCells * NC : 4 * NC + (size_t)kChunk * NC) +
+            (sizeof(Derived) + sizeof(Result)) * F + scan_ws_bytes_for(n_counts) + out + 32 * 256;
+    im->reserve(Impl::piece(need));
+    im->plan = Plan{};
+    Plan& p = im->plan;
     p.F = (uint32_t)F;
     p.T = (uint32_t)T;
     p.NC = (uint32_t)NC;
@@ -188,14 +252,10 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
     p.strict = strict ? 1 : 0;
     p.hdr = hdr;
     p.nout = nout;
-    Field* d_tab = (Field*)impl_->dev(sizeof(Field) * F);
-    uint32_t* d_t0 = (uint32_t*)impl_->dev(4 * (F + 1));
-    uint32_t* d_c0 = (uint32_t*)impl_->dev(4 * (F + 1));
-    uint32_t* d_u0 = (uint32_t*)impl_->dev(4 * (F + 1));
-    hipck(hipMemcpy(d_tab, tab.data(), sizeof(Field) * F, hipMemcpyHostToDevice), "hipMemcpy (fields)");
-    hipck(hipMemcpy(d_t0, tile0.data(), 4 * (F + 1), hipMemcpyHostToDevice), "hipMemcpy (tiles)");
-    hipck(hipMemcpy(d_c0, chunk0.data(), 4 * (F + 1), hipMemcpyHostToDevice), "hipMemcpy (chunks)");
-    hipck(hipMemcpy(d_u0, unit0.data(), 4 * (F + 1), hipMemcpyHostToDevice), "hipMemcpy (units)");
+    p.fields = im->table(tab);
+    p.tile0 = im->table(tile0);
+    p.chunk0 = im->table(chunk0);
+    p.unit0 = im->table(unit0);
     // tiles by dimensionality: per class, its fields, their tile prefix and
     // the class field of every 64th class tile (the Lorenzo kernels start
     // their walk there instead of a binary search)
@@ -214,15 +274,9 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
             tf[k] = (uint32_t)j;
         }
         if (cf.empty()) cf.push_back(0);
-        uint32_t* d_cf = (uint32_t*)impl_->dev(4 * cf.size());
-        uint32_t* d_ct0 = (uint32_t*)impl_->dev(4 * ct0.size());
-        uint32_t* d_ctf = (uint32_t*)impl_->dev(4 * nb);
-        hipck(hipMemcpy(d_cf, cf.data(), 4 * cf.size(), hipMemcpyHostToDevice), "hipMemcpy (class fields)");
-        hipck(hipMemcpy(d_ct0, ct0.data(), 4 * ct0.size(), hipMemcpyHostToDevice), "hipMemcpy (class tiles)");
-        hipck(hipMemcpy(d_ctf, tf.data(), 4 * nb, hipMemcpyHostToDevice), "hipMemcpy (class tile fields)");
-        p.cls_field[d] = d_cf;
-        p.cls_tile0[d] = d_ct0;
-        p.cls_tfield[d] = d_ctf;
+        p.cls_field[d] = im->table(cf);
+        p.cls_tile0[d] = im->table(ct0);
+        p.cls_tfield[d] = im->table(tf);
         p.cls_F[d] = (uint32_t)(ct0.size() - 1);
         p.cls_T[d] = Td;
         if (d == 2) {  // 3D tiles in x-adjacent pairs of one field: ceil(gx / 2) gy gz per field
@@ -239,59 +293,75 @@ void BatchCompressor::setFields(const std::vector<BatchField>& fields) {
                 while (j + 2 < pr0.size() && pr0[j + 1] <= 64 * k) j++;
                 pf[k] = (uint32_t)j;
             }
-            uint32_t* d_pr0 = (uint32_t*)impl_->dev(4 * pr0.size());
-            uint32_t* d_pf = (uint32_t*)impl_->dev(4 * pb);
-            hipck(hipMemcpy(d_pr0, pr0.data(), 4 * pr0.size(), hipMemcpyHostToDevice), "hipMemcpy (tile pairs)");
-            hipck(hipMemcpy(d_pf, pf.data(), 4 * pb, hipMemcpyHostToDevice), "hipMemcpy (pair fields)");
-            p.pair0 = d_pr0;
-            p.pfield = d_pf;
+            p.pair0 = im->table(pr0);
+            p.pfield = im->table(pf);
             p.P = P;
         }
     }
     std::vector<uint32_t> cfield(std::max<uint64_t>(NC, 1), 0);
     for (uint32_t f = 0; f < F; f++)
         for (uint32_t c = chunk0[f]; c < chunk0[f + 1]; c++) cfield[c] = f;
-    uint32_t* d_cf = (uint32_t*)impl_->dev(4 * cfield.size());
-    hipck(hipMemcpy(d_cf, cfield.data(), 4 * cfield.size(), hipMemcpyHostToDevice), "hipMemcpy (chunk fields)");
-    p.cfield = d_cf;
+    p.cfield = im->table(cfield);
     std::vector<uint32_t> ufield(std::max<uint64_t>(U, 1), 0);
     for (uint32_t f = 0; f < F; f++)
         for (uint32_t u = unit0[f]; u < unit0[f + 1]; u++) ufield[u] = f;
-    uint32_t* d_uf = (uint32_t*)impl_->dev(4 * ufield.size());
-    hipck(hipMemcpy(d_uf, ufield.data(), 4 * ufield.size(), hipMemcpyHostToDevice), "hipMemcpy (unit fields)");
-    p.ufield = d_uf;
-    p.fields = d_tab;
-    p.tile0 = d_t0;
-    p.chunk0 = d_c0;
-    p.unit0 = d_u0;
-    p.params = (float*)impl_->dev(16 * F);
-    p.vb_part = (float2*)impl_->dev(8 * std::max<uint64_t>(U, 1));
-    p.codes = (uint16_t*)impl_->dev(2 * codes);
-    p.lerr = (float*)impl_->dev(4ull * kListSlots * T);
-    p.lidx = (uint32_t*)impl_->dev(4ull * kListSlots * T);
+    p.ufield = im->table(ufield);
+    if (huf) {
+        p.huf.wg_field = im->table(hwf);
+        p.huf.wg_part = im->table(hwp);
+        p.huf.n_of = im->table(hns);
+    }
+    Plan* hp = im->table(&p, 1);  // its contents follow once every pointer is known
+    p.params = (float*)im->dev(16 * F);
+    p.vb_part = (float2*)im->dev(8 * std::max<uint64_t>(U, 1));
+    p.codes = (uint16_t*)im->dev(2 * codes);
+    p.lerr = (float*)im->dev(lists);
+    p.lidx = (uint32_t*)im->dev(lists);
     if (strict) {
-        p.lpval = (float*)impl_->dev(4ull * kListSlots * T);
-        p.lpidx = (uint32_t*)impl_->dev(4ull * kListSlots * T);
+        p.lpval = (float*)im->dev(lists);
+        p.lpidx = (uint32_t*)im->dev(lists);
     }
     p.n_counts = (uint32_t)n_counts;
-    p.counts = (uint32_t*)impl_->dev(4 * n_counts);
-    p.excl = (uint32_t*)impl_->dev(4 * (n_counts + 1));
-    p.sizes = (uint32_t*)impl_->dev(4 * NC);
-    p.chunk_scratch = (uint8_t*)impl_->dev((size_t)kChunk * NC);
-    p.derived = (Derived*)impl_->dev(sizeof(Derived) * F);
-    p.results = (Result*)impl_->dev(sizeof(Result) * F);
-    p.scan_ws = impl_->dev(scan_ws_bytes_for(n_counts));
-    d_out_ = (uint8_t*)impl_->dev(out);
-    p.out = d_out_;
+    p.counts = (uint32_t*)im->dev(4 * n_counts);
+    p.excl = (uint32_t*)im->dev(4 * (n_counts + 1));
+    if (huf) {
+        Huffman& h = p.huf;
+        h.bklen = cfg_.huffman_bklen;
+        h.rev_bytes = (uint32_t)fzh_huffman_revbook_bytes(h.bklen, 2);
+        h.rev_stride = (uint32_t)rev_stride;
+        h.NW = (uint32_t)hwf.size();
+        h.freq = (uint32_t*)im->dev(4ull * F * h.bklen);
+        h.bk4 = (uint32_t*)im->dev(4ull * F * h.bklen);
+        h.rev = (uint8_t*)im->dev((size_t)F * h.rev_stride);
+        h.status = (int*)im->dev(4 * F);
+        h.cells = (uint32_t*)im->dev(4ull * kHufCells * NC);
+    } else {
+        p.sizes = (uint32_t*)im->dev(4 * NC);
+        p.chunk_scratch = (uint8_t*)im->dev((size_t)kChunk * NC);
+    }
+    p.derived = (Derived*)im->dev(sizeof(Derived) * F);
+    p.results = (Result*)im->dev(sizeof(Result) * F);
+    p.scan_ws = im->dev(scan_ws_bytes_for(n_counts));
+    p.out = (uint8_t*)im->dev(out);
+    if (im->results_cap < F) {
+        if (im->h_results) (void)hipHostFree(im->h_results);
+        im->h_results = nullptr;
+        im->results_cap = 0;
+        void* mapped = nullptr;
+        hipck(hipHostMalloc(&mapped, sizeof(Result) * F, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
+        im->h_results = (Result*)mapped;
+        im->results_cap = F;
+        hipck(hipHostGetDevicePointer(&im->d_results_map, mapped, 0), "hipHostGetDevicePointer");
+    }
+    std::memset(im->h_results, 0, sizeof(Result) * F);
+    std::memcpy(im->tables.data() + ((uint8_t*)hp - im->arena), &p, sizeof(Plan));
+    im->d_plan = hp;
+    im->upload();
+    for (auto& e : im->ev)
+        if (!e) hipck(hipEventCreate(&e), "hipEventCreate");
+    d_out_ = p.out;
     out_cap_ = out;
-    void* mapped = nullptr;
-    hipck(hipHostMalloc(&mapped, sizeof(Result) * F, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
-    impl_->h_results = (Result*)mapped;
-    std::memset(mapped, 0, sizeof(Result) * F);
-    hipck(hipHostGetDevicePointer(&impl_->d_results_map, mapped, 0), "hipHostGetDevicePointer");
-    impl_->d_plan = (Plan*)impl_->dev(sizeof(Plan));
-    hipck(hipMemcpy(impl_->d_plan, &p, sizeof(Plan), hipMemcpyHostToDevice), "hipMemcpy (plan)");
-    for (auto& e : impl_->ev) hipck(hipEventCreate(&e), "hipEventCreate");
+    impl_ = im.release();
 }
 
 void BatchCompressor::setLaunch(const BatchLaunch& l) {
@@ -322,7 +392,10 @@ void BatchCompressor::enqueue(hipStream_t s) {
     if (prof) hipck(hipEventRecord(ev[1], s), "hipEventRecord");
     fzck(launch_lorenzo(s, p, dp, cu * launch_.lz_wg_per_cu, launch_.lz_tiles_per_unit), "batch lorenzo");
     if (prof) hipck(hipEventRecord(ev[2], s), "hipEventRecord");
-    fzck(launch_rze(s, p, dp), "batch rze");
+    if (p.huf.bklen)
+        fzck(launch_huffman(s, p, dp), "batch huffman");
+    else
+        fzck(launch_rze(s, p, dp), "batch rze");
     if (prof) hipck(hipEventRecord(ev[3], s), "hipEventRecord");
     fzck(launch_scan(s, p), "batch scan");
     if (prof) hipck(hipEventRecord(ev[4], s), "hipEventRecord");
@@ -360,7 +433,7 @@ void BatchCompressor::compress(hipStream_t stream) {
     calls_since_plan_++;
     hipck(hipStreamSynchronize(stream), "hipStreamSynchronize (batch)");
     if (profiling_ && !use_graph) {
-        static const char* names[7] = {"value_base", "lorenzo", "bitshuffle_rze", "scan", "finalize", "pack", "scatter"};
+        const char* names[7] = {"value_base", "lorenzo", impl_->plan.huf.bklen ? "huffman" : "bitshuffle_rze", "scan", "finalize", "pack", "scatter"};
         stage_ms_.clear();
         for (int i = 0; i < 7; i++) {
             float ms = 0.0f;
@@ -373,6 +446,9 @@ void BatchCompressor::compress(hipStream_t stream) {
     size_t over = 0;
     for (size_t i = 0; i < fields_.size(); i++) {
         const uint32_t fl = r[i].flags;
+        if (fl & kBadBook)
+            throw std::runtime_error("BatchCompressor: field " + std::to_string(i) +
+                                     ": no Huffman codebook (codes outside the alphabet)");
         if (fl & kOverflowCapacity)
             throw std::runtime_error("BatchCompressor: field " + std::to_string(i) + " exceeds its output capacity");
         if (cfg_.strict && (fl & kOverflowPatches))

@@ -182,4 +182,23 @@ uint32_t crc32Feed(uint32_t crc, const void* data, size_t len) {
     return crc;
 }
 
+// Product of two polynomials modulo the CRC's (reflected: bit 31 is x^0).
+static uint32_t gf2Mul(uint32_t a, uint32_t b) {
+    uint32_t p = 0;
+    for (int i = 31; i >= 0; i--) {
+        if ((a >> i) & 1u) p ^= b;
+        b = (b >> 1) ^ ((b & 1u) ? 0xEDB88320u : 0u);
+    }
+    return p;
+}
+
+uint32_t crc32Append(uint32_t crc, uint32_t part, size_t len) {
+    uint32_t f = 0x80000000u, sq = 0x00800000u;  // 1, x^8
+    for (size_t n = len; n; n >>= 1) {
+        if (n & 1) f = gf2Mul(f, sq);
+        sq = gf2Mul(sq, sq);
+    }
+    return gf2Mul(crc, f) ^ part;
+}
+
 }  // namespace fz

@@ -213,48 +213,52 @@ class ChainSelectCompressor {
             }
         }
         const double t1 = now_ms();
-        // compress every chunk with its chain: kWorkers host threads, each
-        // with its own stream and its own pipeline per chain, take the chunks
-        // in turn (each fz::Pipeline::compress ends with a host wait, so one
-        // thread would leave the GPU idle between chunks)
+        // Chains 1 (LorenzoQuant -> Bitshuffle -> RZE) and 2 (LorenzoQuant ->
+        // Huffman): one launch per stage for all of a chain's chunks
+        // (fz::BatchCompressor, whose per-field bytes equal
+        // fz::Pipeline::compress of each chunk).  The other chunks, and the
+        // last chunk of each batched chain -- so the container's stage records
+        // come from a real run, and its bytes check the batch's -- run through
+        // pipelines on up to kWorkers host threads, each with its own stream
+        // and its own pipeline per chain (each fz::Pipeline::compress ends
+        // with a host wait, so one thread would leave the GPU idle between
+        // chunks).
         uint32_t mask = 0;
-        for (uint8_t k : choice_) mask |= 1u << k;
+        std::vector<uint64_t> list[FZS_NCHAINS], last(FZS_NCHAINS, 0);
+        for (uint64_t c = 0; c < n; c++) {
+            mask |= 1u << choice_[c];
+            list[choice_[c]].push_back(c);
+            last[choice_[c]] = c;
+        }
         hipck(hipStreamSynchronize(s), "hipStreamSynchronize");  // chunks_ and the choices are ready
-        const int W = (int)std::max<uint64_t>(1, std::min<uint64_t>(kWorkers, n));
+        const auto batched = [&](int k) { return (k == 1 || k == 2) && list[k].size() >= kBatchMin; };
+        std::vector<uint64_t> single;
+        for (uint64_t c = 0; c < n; c++)
+            if (!batched(choice_[c]) || c == last[choice_[c]]) single.push_back(c);
+        const int W = (int)std::min<size_t>(kWorkers, single.size());
         while ((int)workers_.size() < W) {
             workers_.push_back(std::make_unique<Worker>());
             hipck(hipStreamCreate(&workers_.back()->s), "hipStreamCreate");
         }
-        for (int w = 0; w < W; w++)
-            for (int k = 0; k < FZS_NCHAINS; k++)
-                if ((mask >> k) & 1u) {
-                    Worker& wk = *workers_[w];
-                    if (!wk.chain[k].p || wk.chain_eb[k] != abs_eb) {
-                        wk.chain[k] = make_chain(k, abs_eb, cx_, cy_, cz_);
-                        wk.chain_eb[k] = abs_eb;
-                    }
-                }
-        // the chunks on chain 1 (LorenzoQuant -> Bitshuffle -> RZE) go through
-        // fz::BatchCompressor, one launch per stage for all of them, whose
-        // per-field bytes equal fz::Pipeline::compress of each chunk; the
-        // last such chunk still runs through its pipeline on a worker, so the
-        // container's stage records come from a real run and its bytes check
-        // the batch's
-        std::vector<uint64_t> c1;
-        for (uint64_t c = 0; c < n; c++)
-            if (choice_[c] == 1) c1.push_back(c);
-        const bool batch1 = c1.size() >= kBatchMin;
-        const uint64_t c1_last = batch1 ? c1.back() : 0;
+        int rec_worker[FZS_NCHAINS] = {0, 0, 0, 0};  // the worker that ran each chain's last chunk
+        for (size_t i = 0; i < single.size(); i++) {
+            const int w = (int)(i % (size_t)W), k = choice_[single[i]];
+            if (single[i] == last[k]) rec_worker[k] = w;
+            Worker& wk = *workers_[w];
+            if (!wk.chain[k].p || wk.chain_eb[k] != abs_eb) {
+                wk.chain[k] = make_chain(k, abs_eb, cx_, cy_, cz_);
+                wk.chain_eb[k] = abs_eb;
+            }
+        }
         std::vector<std::vector<uint8_t>> blobs(n);
-        std::vector<uint8_t> batch_last;
         std::vector<std::exception_ptr> errs(W);
         std::vector<std::thread> th;
         for (int w = 0; w < W; w++)
             th.emplace_back([&, w] {
                 try {
                     Worker& wk = *workers_[w];
-                    for (uint64_t c = (uint64_t)w; c < n; c += (uint64_t)W) {
-                        if (batch1 && choice_[c] == 1 && c != c1_last) continue;
+                    for (size_t i = (size_t)w; i < single.size(); i += (size_t)W) {
+                        const uint64_t c = single[i];
                         void* d_out = nullptr;
                         size_t bytes = 0;
                         wk.chain[choice_[c]].p->compress((const float*)chunks_.p + c * E, 4 * E, &d_out, &bytes, wk.s);
@@ -268,40 +272,67 @@ class ChainSelectCompressor {
                 }
             });
         std::exception_ptr batch_err;
-        if (batch1) {
-            try {
-                run_batch1(s, abs_eb, c1, blobs, batch_last);
-            } catch (...) {
-                batch_err = std::current_exception();
-            }
+        try {
+            for (int k = 1; k <= 2; k++)
+                if (batched(k)) run_batch(s, k, abs_eb, list[k]);
+        } catch (...) {
+            batch_err = std::current_exception();
         }
         for (auto& t : th) t.join();
         for (auto& e : errs)
             if (e) std::rethrow_exception(e);
         if (batch_err) std::rethrow_exception(batch_err);
-        if (batch1 && batch_last != blobs[c1_last])
-            throw std::runtime_error("selector: batched chain-1 bytes differ from the pipeline's");
         const double t2 = now_ms();
         // container: chain k's stages are described by the pipeline that
-        // compressed the last chunk choosing k (chunk c went to worker c % W)
-        std::vector<uint64_t> last(FZS_NCHAINS, 0);
-        for (uint64_t c = 0; c < n; c++) last[choice_[c]] = c;
+        // compressed the last chunk choosing k
         std::vector<std::vector<FZMStageInfo>> recs(FZS_NCHAINS);
         size_t hdr = 64 + 4;
         for (int k = 0; k < FZS_NCHAINS; k++)
             if ((mask >> k) & 1u) {
-                recs[k] = workers_[last[k] % (uint64_t)W]->chain[k].p->buildHeader().stages;
+                recs[k] = workers_[rec_worker[k]]->chain[k].p->buildHeader().stages;
                 hdr += 4 + recs[k].size() * sizeof(FZMStageInfo);
             }
         const size_t o_choice = hdr;
         const size_t o_bytes = o_choice + ((n + 7) & ~7ull);
-        size_t total = o_bytes + 8 * n;
-        std::vector<size_t> o_blob(n);
+        const size_t o_first = o_bytes + 8 * n;
+        size_t total = o_first;
+        std::vector<size_t> o_blob(n), size(n);
+        std::vector<fzh_copy_desc> desc;
+        std::vector<uint64_t> desc_chunk;
+        size_t at[FZS_NCHAINS] = {0, 0, 0, 0};
         for (uint64_t c = 0; c < n; c++) {
+            const int k = choice_[c];
+            size[c] = blobs[c].size();
+            if (batched(k)) {
+                const size_t i = at[k]++;
+                size[c] = batch_[k].b->fieldBytes(i);
+                // the device copy of the container starts at its first result
+                desc.push_back({batch_[k].b->output() + batch_[k].b->fieldOffset(i), (void*)(total - o_first), size[c]});
+                desc_chunk.push_back(c);
+            }
             o_blob[c] = total;
-            total += (blobs[c].size() + 15) & ~15ull;
+            total += (size[c] + 15) & ~15ull;
         }
-        out_.assign(total, 0);
+        // the batched results go to their places in one device buffer, are
+        // checksummed there and reach the host in one copy (a copy per chunk
+        // and the checksum on one host thread were 6 ms of 15 MB)
+        std::vector<uint32_t> crcs(desc.size());
+        out_.resize(total);
+        if (!desc.empty()) {
+            pack_.ensure(total - o_first);
+            for (auto& d : desc) d.dst = (uint8_t*)pack_.p + (size_t)d.dst;
+            const size_t db = sizeof(fzh_copy_desc) * desc.size();
+            pack_desc_.ensure(db + 4 * desc.size());
+            uint32_t* d_crc = (uint32_t*)((uint8_t*)pack_desc_.p + db);
+            hipck(hipMemcpyAsync(pack_desc_.p, desc.data(), db, hipMemcpyHostToDevice, s), "hipMemcpyAsync (descriptors)");
+            fzck(fzh_gather(s, (const fzh_copy_desc*)pack_desc_.p, (int)desc.size()), "gather (container)");
+            fzck(fzh::crc32_segments(s, (const fzh_copy_desc*)pack_desc_.p, (int)desc.size(), d_crc), "checksums");
+            hipck(hipMemcpyAsync(crcs.data(), d_crc, 4 * crcs.size(), hipMemcpyDeviceToHost, s), "hipMemcpyAsync (checksums)");
+            hipck(hipMemcpyAsync(out_.data() + o_first, pack_.p, total - o_first, hipMemcpyDeviceToHost, s),
+                  "hipMemcpyAsync (container)");
+            hipck(hipStreamSynchronize(s), "hipStreamSynchronize (container)");
+        }
+        std::memset(out_.data(), 0, o_first);
         put<uint32_t>(out_, 0, kMagic);
         put<uint16_t>(out_, 4, kVersion);
         put<uint8_t>(out_, 6, (uint8_t)mode);
@@ -329,11 +360,27 @@ class ChainSelectCompressor {
                 }
             }
         std::memcpy(out_.data() + o_choice, choice_.data(), n);
-        for (uint64_t c = 0; c < n; c++) {
-            put<uint64_t>(out_, o_bytes + 8 * c, (uint64_t)blobs[c].size());
-            std::memcpy(out_.data() + o_blob[c], blobs[c].data(), blobs[c].size());
+        for (uint64_t c = 0; c < n; c++) put<uint64_t>(out_, o_bytes + 8 * c, (uint64_t)size[c]);
+        // checksum of [64, end) in file order: device sums of the batched
+        // results, the host's of the rest
+        uint32_t crc = crc32Feed(0xFFFFFFFFu, out_.data() + 64, o_first - 64);
+        for (uint64_t c = 0, j = 0; c < n; c++) {
+            uint8_t* b = out_.data() + o_blob[c];
+            const size_t padded = (size[c] + 15) & ~15ull;
+            if (j < desc_chunk.size() && desc_chunk[j] == c) {
+                if (c == last[choice_[c]] &&
+                    (blobs[c].size() != size[c] || std::memcmp(b, blobs[c].data(), size[c]) != 0))
+                    throw std::runtime_error("selector: batched chain-" + std::to_string((int)choice_[c]) +
+                                             " bytes differ from the pipeline's");
+                if (padded != size[c]) throw std::runtime_error("selector: a batched result is not 16-byte padded");
+                crc = crc32Append(crc, crcs[j++], size[c]);
+            } else {
+                std::memcpy(b, blobs[c].data(), size[c]);
+                std::memset(b + size[c], 0, padded - size[c]);
+                crc = crc32Feed(crc, b, padded);
+            }
         }
-        put<uint32_t>(out_, 60, crc32(out_.data() + 64, out_.size() - 64));
+        put<uint32_t>(out_, 60, crc ^ 0xFFFFFFFFu);
         const double t3 = now_ms();
         select_ms_ = (float)(t1 - t0);
         compress_ms_ = (float)(t2 - t1);
@@ -415,14 +462,13 @@ class ChainSelectCompressor {
     }
 
   private:
-    // Compresses the chunks `c1` (all on chain 1) in one batch on stream s:
-    // every result but the last into blobs, the last into `last`.  The batch
-    // plan is kept while the chunk list and the bound stay the same.
-    void run_batch1(hipStream_t s, float abs_eb, const std::vector<uint64_t>& c1,
-                    std::vector<std::vector<uint8_t>>& blobs, std::vector<uint8_t>& last) {
+    // Compresses the chunks `c` (all on chain k, 1 or 2) in one batch on
+    // stream s.  The plan is kept while the chunk list and the bound stay the
+    // same; a new one reuses the batch's memory.
+    void run_batch(hipStream_t s, int k, float abs_eb, const std::vector<uint64_t>& c) {
         const uint64_t E = (uint64_t)cx_ * cy_ * cz_;
-        if (!batch_ || batch_eb_ != abs_eb || batch_idx_ != c1 || batch_base_ != chunks_.p) {
-            batch_.reset();
+        Batch& B = batch_[k];
+        if (!B.b) {
             BatchConfig cfg;
             cfg.error_bound = abs_eb;
             cfg.eb_mode = ErrorBoundMode::ABS;
@@ -430,50 +476,30 @@ class ChainSelectCompressor {
             cfg.outlier_capacity = FZS_OUTLIER_CAP;
             cfg.zigzag = true;
             cfg.strict = false;
-            auto b = std::make_unique<BatchCompressor>(cfg);
-            std::vector<BatchField> f(c1.size());
-            for (size_t i = 0; i < c1.size(); i++) {
-                f[i].d_in = (const float*)chunks_.p + c1[i] * E;
+            cfg.huffman_bklen = k == 2 ? FZS_HUF_BKLEN : 0;
+            B.b = std::make_unique<BatchCompressor>(cfg);
+            B.b->enableGraphMode(false);  // the plan changes with the choices; no capture to amortise
+        }
+        if (B.eb != abs_eb || B.idx != c || B.base != chunks_.p) {
+            B.base = nullptr;  // no plan if this one fails
+            B.b->setErrorBound(abs_eb);
+            std::vector<BatchField> f(c.size());
+            for (size_t i = 0; i < c.size(); i++) {
+                f[i].d_in = (const float*)chunks_.p + c[i] * E;
                 f[i].nx = cx_;
                 f[i].ny = cy_;
                 f[i].nz = cz_;
             }
-            b->setFields(f);
-            b->enableGraphMode(false);  // the plan changes with the choices; no capture to amortise
-            batch_ = std::move(b);
-            batch_eb_ = abs_eb;
-            batch_idx_ = c1;
-            batch_base_ = chunks_.p;
+            B.b->setFields(f);
+            B.eb = abs_eb;
+            B.idx = c;
+            B.base = chunks_.p;
         }
-        batch_->compress(s);
-        // the results packed back to back (16-byte steps) by one gather
-        // launch, then one copy to the host
-        const uint8_t* d = batch_->output();
-        const size_t F = c1.size();
-        std::vector<fzh_copy_desc> desc(F);
-        std::vector<uint64_t> pos(F + 1, 0);
-        for (size_t i = 0; i < F; i++) {
-            const uint64_t b = batch_->fieldBytes(i);
-            pos[i + 1] = pos[i] + ((b + 15) & ~15ull);
-        }
-        pack_.ensure(pos[F]);
-        pack_desc_.ensure(sizeof(fzh_copy_desc) * F);
-        for (size_t i = 0; i < F; i++)
-            desc[i] = {d + batch_->fieldOffset(i), (uint8_t*)pack_.p + pos[i], batch_->fieldBytes(i)};
-        hipck(hipMemcpyAsync(pack_desc_.p, desc.data(), sizeof(fzh_copy_desc) * F, hipMemcpyHostToDevice, s),
-              "hipMemcpyAsync (batch descriptors)");
-        fzck(fzh_gather(s, (const fzh_copy_desc*)pack_desc_.p, (int)F), "gather (batch)");
-        pack_host_.resize(pos[F]);
-        hipck(hipMemcpyAsync(pack_host_.data(), pack_.p, pos[F], hipMemcpyDeviceToHost, s), "hipMemcpyAsync (batch)");
-        hipck(hipStreamSynchronize(s), "hipStreamSynchronize (batch)");
-        for (size_t i = 0; i < F; i++) {
-            std::vector<uint8_t>& dst = i + 1 < F ? blobs[c1[i]] : last;
-            dst.assign(pack_host_.data() + pos[i], pack_host_.data() + pos[i] + batch_->fieldBytes(i));
-        }
+        B.b->compress(s);
     }
 
     static constexpr int kWorkers = 8;
-    static constexpr size_t kBatchMin = 2;  // chain-1 chunks below this run per chunk
+    static constexpr size_t kBatchMin = 2;  // fewer chunks of a chain run per chunk
     struct Worker {
         hipStream_t s = nullptr;
         Chain chain[FZS_NCHAINS];
@@ -490,12 +516,14 @@ class ChainSelectCompressor {
     std::vector<uint8_t> choice_, out_;
     std::vector<uint64_t> sizes_;
     float select_ms_ = 0, compress_ms_ = 0, total_ms_ = 0;
-    std::unique_ptr<BatchCompressor> batch_;
+    struct Batch {
+        std::unique_ptr<BatchCompressor> b;
+        float eb = 0;
+        std::vector<uint64_t> idx;
+        const void* base = nullptr;
+    };
+    Batch batch_[FZS_NCHAINS];
     DevBuf pack_, pack_desc_;
-    std::vector<uint8_t> pack_host_;
-    float batch_eb_ = 0;
-    std::vector<uint64_t> batch_idx_;
-    const void* batch_base_ = nullptr;
 };
 
 }  // namespace fz

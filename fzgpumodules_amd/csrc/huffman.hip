@@ -30,14 +30,11 @@
 //     and leave in 16-byte stores.  Long streams: one lane per partition.
 #include <type_traits>
 
+#include "fzh_huffman_enc.h"
 #include "fzh_scan.h"
 
 namespace fzh {
 namespace {
-
-constexpr int SUBLEN = 768;       // coarse partitions
-constexpr int SUBLEN_FINE = 1024; // fine partitions
-constexpr int HDR_BYTES = 128;
 
 template <typename T>
 __device__ __forceinline__ uint32_t ld_sym(const T* p, uint64_t i) { return (uint32_t)p[i]; }
@@ -112,30 +109,18 @@ hist_global_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, uint32_
 // ---------------------------------------------------------------------------
 // Encode
 // ---------------------------------------------------------------------------
-// cells per partition slot (every codeword is at most 28 bits)
-constexpr int cells_of(int sl) { return (sl * 28 + 31) / 32 + 2; }
 constexpr unsigned ENC_BLOCKS = 4096;  // encode workgroups, at most
 
-// A lane takes SL / 64 consecutive symbols: their lengths add up in the lane,
-// so one wave scan places all of them, and their codes are shifted together
-// in a register that goes to LDS a whole cell at a time (about two OR
-// operations per lane and 12 symbols of 6.5 bits).  With symbols strided by
-// 64 over the lanes every symbol took a wave scan and one or two LDS ORs that
-// collide with its neighbours' in the same cell: 2^27 symbols 234 us, now 96.
-// Each workgroup stages the codebook once and takes several partitions; more
-// workgroups (one partition a wave: 117 us) stage it more often, fewer (2048:
-// 103) leave too few waves to cover the loads.
-// BOOK_LDS: the codebook is staged in LDS (bklen <= 8192), else read from
-// global memory.  (A template parameter, not a pointer chosen at run time:
-// a pointer that may be either LDS or global makes every lookup a FLAT
-// access.)
+// Each workgroup stages the codebook once (bklen <= 8192: BOOK_LDS) and takes
+// several partitions, one per wave at a time (huf_encode_partition); more
+// workgroups (one partition a wave: 117 us for 2^27 symbols, now 96) stage it
+// more often, fewer (2048: 103) leave too few waves to cover the loads.
 template <typename T, int SL, bool BOOK_LDS>
 __global__ void __launch_bounds__(256)
 huf_enc_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, const uint32_t* __restrict__ bk4,
                const uint8_t* __restrict__ revbook, uint32_t rev_bytes, uint8_t* __restrict__ out,
                uint32_t* __restrict__ scells, uint32_t* __restrict__ ncell_out, uint32_t pardeg) {
     constexpr int CELLS = cells_of(SL);
-    constexpr int K = SL / 64;  // symbols per lane
     extern __shared__ uint32_t smem[];
     const int wv = threadIdx.x >> 6;
     uint32_t* cells = smem + wv * CELLS;
@@ -146,60 +131,12 @@ huf_enc_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, const uint3
     }
     const uint32_t ent1 = HDR_BYTES, ent2 = ent1 + rev_bytes;
     const int l = lane_id();
-    constexpr int B = K * (int)sizeof(T);
-    constexpr int V = B % 16 == 0 ? 16 : (B % 8 == 0 ? 8 : 4);  // bytes per load
-    const bool wide = (uintptr_t)in % V == 0;
+    const bool wide = (uintptr_t)in % enc_load_bytes<T, SL>() == 0;
     for (uint32_t p = blockIdx.x * 4 + wv; p < pardeg; p += gridDim.x * 4) {
         const uint64_t s0 = (uint64_t)p * SL;
         const uint32_t cnt = (uint32_t)((n - s0) < (uint64_t)SL ? (n - s0) : SL);
-        // lane l: symbols K l .. K l + K - 1 of the partition
-        T sym[K];
-        if (cnt == SL && wide) {
-            const T* src = in + s0 + K * l;
-#pragma unroll
-            for (int i = 0; i < B / V; i++) {
-                if constexpr (V == 16)
-                    reinterpret_cast<uint4*>(sym)[i] = reinterpret_cast<const uint4*>(src)[i];
-                else if constexpr (V == 8)
-                    reinterpret_cast<uint2*>(sym)[i] = reinterpret_cast<const uint2*>(src)[i];
-                else
-                    reinterpret_cast<uint32_t*>(sym)[i] = reinterpret_cast<const uint32_t*>(src)[i];
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < K; k++) sym[k] = K * l + k < (int)cnt ? in[s0 + K * l + k] : (T)0;
-        }
-        uint32_t word[K], bits = 0;  // length << 27 | code
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const uint32_t x = (uint32_t)sym[k];
-            // a symbol past the partition's end or out of range (reported by the caller) gets no code
-            const bool ok = x < bklen && (cnt == SL || K * l + k < (int)cnt);
-            word[k] = ok ? (BOOK_LDS ? s_bk[x] : bk4[x]) : 0u;
-            bits += word[k] >> 27;
-        }
-        const uint32_t incl = wave_incl_scan(bits);
-        const uint32_t nbit = lane63(incl);
+        const uint32_t nbit = huf_encode_partition<T, SL, BOOK_LDS>(in + s0, cnt, wide, s_bk, bk4, bklen, cells);
         const uint32_t ncell = (nbit + 31) / 32;
-        for (uint32_t i = l; i <= ncell; i += 64) cells[i] = 0u;
-        wave_lds_sync();
-        // the lane's codes shifted into place; a cell leaves the register when it
-        // is full, and what lanes share of a cell is ORed together in LDS
-        uint32_t at = (incl - bits) >> 5, fill = (incl - bits) & 31u, hi = 0;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const uint32_t c = word[k] & 0x07FFFFFFu;
-            const uint32_t to = fill + (word[k] >> 27);  // 0 .. 62
-            const uint32_t x = __builtin_amdgcn_alignbit(c, 0u, to);  // c << (32 - to % 32), 0 if that is 32
-            if (to >= 32) {
-                atomicOr(&cells[at], hi | (c >> (to & 31u)));
-                at++;
-            }
-            hi = to >= 32 ? x : hi | x;
-            fill = to & 31u;
-        }
-        if (fill) atomicOr(&cells[at], hi);
-        wave_lds_sync();
         uint32_t* dst = scells + (uint64_t)p * CELLS;
         for (uint32_t i = l; i < ncell; i += 64) dst[i] = cells[i];
         if (l == 0) {

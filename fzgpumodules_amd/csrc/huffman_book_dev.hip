@@ -35,9 +35,18 @@ __device__ __forceinline__ uint64_t efreq(uint64_t e) { return e >> NODE_BITS; }
 // Status codes (0 = ok): 1 = the histogram does not sum to n (symbols out of
 // range), 2 = a code longer than 58 bits (the host builder's error; a tree
 // that deep needs a total count above fib(61), about 2.5e12).
+// One workgroup per book (histograms, books and status words one after
+// another, reverse books every rev_stride bytes): the replay is serial, so
+// many books at once cost hardly more than one.
 __global__ void __launch_bounds__(256)
-huf_book_kernel(const uint32_t* __restrict__ freq, uint32_t bklen, int eb, uint64_t n_expected,
-                uint32_t* __restrict__ bk4, uint8_t* __restrict__ revbook, int* __restrict__ status) {
+huf_book_kernel(const uint32_t* __restrict__ freq, uint32_t bklen, int eb, uint64_t n_one,
+                const uint64_t* __restrict__ n_of, uint32_t* __restrict__ bk4, uint8_t* __restrict__ revbook,
+                size_t rev_stride, int* __restrict__ status) {
+    freq += (size_t)blockIdx.x * bklen;
+    bk4 += (size_t)blockIdx.x * bklen;
+    revbook += (size_t)blockIdx.x * rev_stride;
+    status += blockIdx.x;
+    const uint64_t n_expected = n_of ? n_of[blockIdx.x] : n_one;
     __shared__ __align__(16) uint64_t q[2 * DBOOK_MAX + 2];  // the heap, 1-indexed
     __shared__ uint32_t fq[DBOOK_MAX];           // the histogram
     __shared__ uint32_t lfq[DBOOK_MAX];          // leaf node -> frequency (nonzero counts in symbol order)
@@ -236,9 +245,23 @@ int fzh_huffman_build_book_device(void* stream, const uint32_t* d_freq, uint32_t
         return fail(FZH_E_INVALID, "huffman device book: bklen above 256 with 1-byte symbols");
     if (!d_freq || !d_bk4 || !d_revbook || !d_status) return fail(FZH_E_INVALID, "huffman device book: null pointer");
     launch_k("huf_book_kernel", huf_book_kernel, dim3(1), dim3(256), 0, S(stream), d_freq, bklen, elem_bytes,
-             n_expected, d_bk4, d_revbook, d_status);
+             n_expected, (const uint64_t*)nullptr, d_bk4, d_revbook, (size_t)0, d_status);
     FZH_CHECK_LAUNCH("huf_book_kernel");
     return FZH_OK;
 }
 
 }  // extern "C"
+
+namespace fzh {
+
+int build_books_device(hipStream_t s, uint32_t n_books, const uint32_t* d_freq, uint32_t bklen, const uint64_t* d_n,
+                       uint32_t* d_bk4, uint8_t* d_revbook, size_t rev_stride, int* d_status) {
+    if (bklen == 0 || bklen > DBOOK_MAX) return fail(FZH_E_INVALID, "huffman device books: bklen must be in [1, 1024]");
+    if (n_books == 0) return FZH_OK;
+    launch_k("huf_book_kernel", huf_book_kernel, dim3(n_books), dim3(256), 0, s, d_freq, bklen, 2, (uint64_t)0, d_n,
+             d_bk4, d_revbook, rev_stride, d_status);
+    FZH_CHECK_LAUNCH("huf_book_kernel");
+    return FZH_OK;
+}
+
+}  // namespace fzh

@@ -32,6 +32,10 @@ struct BatchConfig {
     bool zigzag = true;
     bool strict = false;
     float patch_capacity = 0.01f;
+    // 0: codes go through Bitshuffle -> RZE; else HuffmanStage<uint16_t> with
+    // this alphabet (coarse partitions; at least 2 x quant_radius with zigzag
+    // codes, at most 1024)
+    uint32_t huffman_bklen = 0;
 };
 
 // Persistent-grid geometry (workgroups per CU per kernel; Lorenzo tiles per
@@ -54,8 +58,11 @@ class BatchCompressor {
     BatchCompressor(const BatchCompressor&) = delete;
     BatchCompressor& operator=(const BatchCompressor&) = delete;
 
-    // Plans the batch: device tables, codes/scratch/output buffers.
+    // Plans the batch: device tables, codes/scratch/output buffers (one
+    // allocation, kept for later plans that fit it).
     void setFields(const std::vector<BatchField>& fields);
+    // The bound of the plans made from now on.
+    void setErrorBound(float eb);
     size_t numFields() const { return fields_.size(); }
 
     // Compresses every field on `stream` and waits for it; throws

@@ -197,6 +197,9 @@ inline std::string stageTypeToString(StageType t) {
 // IEEE 802.3 CRC32 (reflected, poly 0xEDB88320); `crc` is the running
 // register: start with 0xFFFFFFFF, finish with ^ 0xFFFFFFFF.
 uint32_t crc32Feed(uint32_t crc, const void* data, size_t len);
+// The register after `len` more bytes whose own register, started at 0, is
+// `part`: crc x^(8 len) + part in GF(2)[x] modulo the polynomial.
+uint32_t crc32Append(uint32_t crc, uint32_t part, size_t len);
 inline uint32_t crc32(const void* data, size_t len) { return crc32Feed(0xFFFFFFFFu, data, len) ^ 0xFFFFFFFFu; }
 
 }  // namespace fz
