@@ -17,14 +17,16 @@
 //     input is read twice and the output written once, no position scratch.
 //     (The reference does 5 passes plus a CUB scan through ~15 B/element of
 //     scratch.)
-//   decode: a three-launch segmented scan of the run lengths gives the run
-//     starts and a map "output tile -> first run overlapping it" (every run
-//     marks the tile boundaries it covers; the lengths and starts pass
-//     through LDS so global accesses stay coalesced); then one wave per
-//     1024-element output tile stages that tile's runs in LDS (33 KiB per
-//     four-wave workgroup), each lane binary-searches its first run and
-//     fills 16 consecutive outputs.  No host round trip
-//     (the reference syncs twice and fills with one thread per run).
+//   decode: run lengths are summed per 4096 runs and the sums scanned.  Where
+//     no 4096 runs cover more than 32768 elements, each workgroup expands its
+//     own.  Otherwise the run starts go to memory with a map "output tile ->
+//     first run overlapping it" (every run marks the tile boundaries it
+//     covers; the lengths and starts pass through LDS so global accesses stay
+//     coalesced); then one wave per 1024-element output tile stages that
+//     tile's runs in LDS (33 KiB per four-wave workgroup), each lane
+//     binary-searches its first run and fills 16 consecutive outputs.  No
+//     host round trip (the reference syncs twice and fills with one thread
+//     per run).
 #include "fzh_scan.h"
 
 namespace fzh {
@@ -32,6 +34,7 @@ namespace {
 
 constexpr int STEPS = 8;
 constexpr uint32_t DTILE = 1024;  // decode output tile (elements), one wave each
+constexpr uint32_t SEG_OUT = 8 * SCAN_SEG;  // most elements of a segment that one workgroup expands
 
 // Run-start flags of one wave's tile: mask[j] bit k <=> element
 // base + 64 E j + E l + k starts a run (k < E, E elements per 16-byte load).
@@ -211,8 +214,10 @@ struct RleDecState {
 // Validated run count (0 and status = 1 if the header is inconsistent).
 template <typename T>
 __global__ void rle_dec_prep_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, uint64_t n,
-                                    uint32_t* __restrict__ Rv, int* __restrict__ d_status) {
+                                    uint32_t* __restrict__ Rv, uint32_t* __restrict__ d_long,
+                                    int* __restrict__ d_status) {
     if (threadIdx.x != 0) return;
+    *d_long = 0;
     uint32_t R = 0;
     bool ok = in_bytes >= 4;
     if (ok) R = *reinterpret_cast<const uint32_t*>(in);
@@ -229,7 +234,7 @@ __device__ __forceinline__ const uint32_t* rle_lengths(const uint8_t* in, uint32
 template <typename T>
 __global__ void __launch_bounds__(256)
 rle_dec_reduce_kernel(const uint8_t* __restrict__ in, const uint32_t* __restrict__ Rv,
-                      uint32_t* __restrict__ seg_sum) {
+                      uint32_t* __restrict__ seg_sum, uint32_t* __restrict__ d_long) {
     __shared__ uint64_t s_w[4];
     const uint32_t R = *Rv;
     const uint32_t* lens = rle_lengths(in, R, sizeof(T));
@@ -247,23 +252,118 @@ rle_dec_reduce_kernel(const uint8_t* __restrict__ in, const uint32_t* __restrict
     if (threadIdx.x == 0) {
         const uint64_t t = s_w[0] + s_w[1] + s_w[2] + s_w[3];
         seg_sum[blockIdx.x] = t > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)t;
+        if (t > SEG_OUT) *d_long = 1;
+    }
+}
+
+// Streams of short runs: a workgroup expands its segment of SCAN_SEG runs
+// itself.  Its lengths become starts in LDS, and each wave takes windows of
+// 16 bytes of output per lane: the runs that start in the window mark their
+// first element, a running maximum over the marks gives every element its
+// run.  Nothing but the stream is read and nothing but the output written (a
+// start per run and a tile's runs, written by one launch and read by the
+// next, were 70 us for 2^24 two-byte values in runs of one or two; this is
+// 50).  A segment covers at most SEG_OUT elements here, so no workgroup
+// works much longer than the others; if any covers more, the whole stream
+// goes by output tiles (rle_dec_starts and the expand launch).
+template <typename T>
+__device__ __forceinline__ void rle_dec_segment(const uint8_t* __restrict__ in, uint64_t n, uint32_t R,
+                                                const uint32_t* __restrict__ seg_base,
+                                                const uint32_t* __restrict__ total, T* __restrict__ out,
+                                                int* __restrict__ d_status, uint32_t* s_x, uint32_t* s_w) {
+    constexpr uint32_t E = 16 / sizeof(T), WIN = 64 * E;  // elements per lane and per window
+    constexpr uint32_t NWIN = SEG_OUT / WIN + 2;
+    __shared__ T s_val[SCAN_SEG];
+    __shared__ uint16_t s_first[NWIN];  // window -> the run at its first element
+    __shared__ __align__(16) uint16_t s_mark[4][WIN];
+    auto px = [](uint32_t i) { return i + (i >> 4); };
+    const uint64_t seg0 = (uint64_t)blockIdx.x * SCAN_SEG;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && R != 0 && *total != n) *d_status = 1;
+    if (seg0 >= R) return;
+    const uint32_t m = (uint32_t)min((uint64_t)SCAN_SEG, R - seg0);  // runs of this segment
+    const uint32_t* lens = rle_lengths(in, R, sizeof(T)) + seg0;
+    const T* vals = reinterpret_cast<const T*>(in + 4) + seg0;
+    const uint32_t tid = threadIdx.x, w = wave_in_wg(), l = (uint32_t)lane_id();
+#pragma unroll
+    for (uint32_t k = 0; k < 16; k++) {
+        const uint32_t i = 256 * k + tid;
+        s_x[px(i)] = i < m ? lens[i] : 0u;
+        if (i < m) s_val[i] = vals[i];
+    }
+    __syncthreads();
+    uint32_t v[16], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 16; k++) {
+        v[k] = s_x[px(16 * tid + k)];
+        sum += v[k];
+    }
+    const uint32_t incl = wave_incl_scan(sum);
+    if (l == 63) s_w[w] = incl;
+    __syncthreads();
+    // starts relative to the segment's first window
+    const uint64_t S0 = seg_base[blockIdx.x], W0 = S0 / WIN;
+    uint32_t run = (uint32_t)(S0 - W0 * WIN) + incl - sum;
+    for (uint32_t j = 0; j < w; j++) run += s_w[j];
+    const uint32_t end = (uint32_t)(S0 - W0 * WIN) + s_w[0] + s_w[1] + s_w[2] + s_w[3];
+#pragma unroll
+    for (uint32_t k = 0; k < 16; k++) {
+        s_x[px(16 * tid + k)] = run;  // after this thread's own reads
+        for (uint32_t t = (run + WIN - 1) / WIN; t * WIN < run + v[k]; t++) s_first[t] = (uint16_t)(16 * tid + k);
+        run += v[k];
+    }
+    if (tid == 0) s_x[px(SCAN_SEG)] = end;
+    const uint32_t off0 = (uint32_t)(S0 - W0 * WIN);
+    if (tid == 0 && off0) s_first[0] = 0;
+    __syncthreads();
+    uint16_t* mark = s_mark[w];
+    const uint32_t nwin = (end + WIN - 1) / WIN;
+    for (uint32_t t = w; t < nwin; t += 4) {
+        const uint32_t b = t * WIN;
+        const uint32_t r0 = s_first[t], r1 = t + 1 < nwin ? s_first[t + 1] : m - 1;  // runs r0 .. r1 reach into it
+#pragma unroll
+        for (uint32_t q = 0; q < E; q += 4) *reinterpret_cast<uint2*>(mark + E * l + q) = make_uint2(0, 0);
+        wave_lds_sync();
+        for (uint32_t i = r0 + 1 + l; i <= r1; i += 64) {
+            const uint32_t p = s_x[px(i)];
+            if (p - b < WIN && s_x[px(i + 1)] > p) mark[p - b] = (uint16_t)(i - r0);
+        }
+        wave_lds_sync();
+        uint16_t mk[E];
+#pragma unroll
+        for (uint32_t q = 0; q < E; q += 4)
+            *reinterpret_cast<uint2*>(mk + q) = *reinterpret_cast<const uint2*>(mark + E * l + q);
+        uint32_t last = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < E; q++) last = max(last, (uint32_t)mk[q]);
+        uint32_t cur = wave_shr1(wave_incl_max(last));
+        T buf[E];
+#pragma unroll
+        for (uint32_t q = 0; q < E; q++) {
+            cur = max(cur, (uint32_t)mk[q]);
+            buf[q] = s_val[r0 + cur];
+        }
+        wave_lds_sync();  // the marks are read before the next window clears them
+        const uint32_t e0 = b + E * l;
+        const uint64_t g0 = W0 * WIN + e0;
+        if (e0 >= off0 && e0 + E <= end && g0 + E <= n) {
+            *reinterpret_cast<uint4*>(out + g0) = *reinterpret_cast<const uint4*>(buf);
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < E; q++)
+                if (e0 + q >= off0 && e0 + q < end && g0 + q < n) out[g0 + q] = buf[q];
+        }
     }
 }
 
 // start[r] = exclusive prefix of the lengths (clamped to n), start[R] = the
 // total; each run marks the output tiles whose first element it covers.
 template <typename T>
-__global__ void __launch_bounds__(256)
-rle_dec_apply_kernel(const uint8_t* __restrict__ in, uint64_t n, const uint32_t* __restrict__ Rv,
-                     const uint32_t* __restrict__ seg_base, const uint32_t* __restrict__ total,
-                     uint32_t* __restrict__ start, uint32_t* __restrict__ tile_first, int* __restrict__ d_status) {
-    __shared__ uint32_t s_w[4];
-    // the segment's lengths, then its starts, in LDS: loaded and stored
-    // coalesced, read by thread t as its 16 consecutive runs (one padding
-    // word per 16 keeps those reads on distinct banks)
-    __shared__ uint32_t s_x[SCAN_SEG + SCAN_SEG / 16];
+__device__ __forceinline__ void rle_dec_starts(const uint8_t* __restrict__ in, uint64_t n, uint32_t R,
+                                               const uint32_t* __restrict__ seg_base,
+                                               const uint32_t* __restrict__ total, uint32_t* __restrict__ start,
+                                               uint32_t* __restrict__ tile_first, int* __restrict__ d_status,
+                                               uint32_t* s_x, uint32_t* s_w) {
     auto px = [](uint32_t i) { return i + (i >> 4); };
-    const uint32_t R = *Rv;
     const uint32_t* lens = rle_lengths(in, R, sizeof(T));
     const int tid = threadIdx.x, w = tid >> 6;
     const uint64_t seg0 = (uint64_t)blockIdx.x * SCAN_SEG;
@@ -309,11 +409,29 @@ rle_dec_apply_kernel(const uint8_t* __restrict__ in, uint64_t n, const uint32_t*
     }
 }
 
+// One segment of SCAN_SEG runs per workgroup.  s_x: the segment's lengths,
+// then its starts: loaded and stored coalesced, read by thread t as its 16
+// consecutive runs (one padding word per 16 keeps those reads on distinct
+// banks).
+template <typename T>
+__global__ void __launch_bounds__(256)
+rle_dec_apply_kernel(const uint8_t* __restrict__ in, uint64_t n, const uint32_t* __restrict__ Rv,
+                     const uint32_t* __restrict__ d_long, const uint32_t* __restrict__ seg_base,
+                     const uint32_t* __restrict__ total, uint32_t* __restrict__ start,
+                     uint32_t* __restrict__ tile_first, T* __restrict__ out, int* __restrict__ d_status) {
+    __shared__ uint32_t s_w[4], s_x[SCAN_SEG + SCAN_SEG / 16 + 1];
+    if (*d_long)
+        rle_dec_starts<T>(in, n, *Rv, seg_base, total, start, tile_first, d_status, s_x, s_w);
+    else
+        rle_dec_segment<T>(in, n, *Rv, seg_base, total, out, d_status, s_x, s_w);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256)
 rle_dec_expand_kernel(const uint8_t* __restrict__ in, uint64_t n, const uint32_t* __restrict__ start,
-                      const uint32_t* __restrict__ tile_first, const int* __restrict__ d_status, T* __restrict__ out,
-                      uint32_t ntiles) {
+                      const uint32_t* __restrict__ tile_first, const uint32_t* __restrict__ d_long,
+                      const int* __restrict__ d_status, T* __restrict__ out, uint32_t ntiles) {
+    if (*d_long == 0) return;
     __shared__ uint32_t s_start[4][DTILE + 2];
     __shared__ T s_val[4][DTILE + 2];
     const int wv = threadIdx.x >> 6;
@@ -453,17 +571,17 @@ int dec_impl(hipStream_t s, const void* in, size_t in_bytes, void* out, size_t n
     if (L.nseg > SCAN_MAX_SEGS) return fail(FZH_E_INVALID, "RLE dec: too many elements");
     uint8_t* w = (uint8_t*)ws;
     uint32_t* Rv = (uint32_t*)(w + L.o_R);
-    uint32_t* tot = Rv + 1;
+    uint32_t *tot = Rv + 1, *lng = Rv + 2;
     uint32_t* seg = (uint32_t*)(w + L.o_seg);
     uint32_t* start = (uint32_t*)(w + L.o_start);
     uint32_t* tf = (uint32_t*)(w + L.o_tf);
     const uint8_t* bin = (const uint8_t*)in;
-    launch_k("rle_dec_prep_kernel", rle_dec_prep_kernel<T>, dim3(1), dim3(64), 0, s, bin, in_bytes, n, Rv, d_status);
-    launch_k("rle_dec_reduce_kernel", rle_dec_reduce_kernel<T>, dim3((unsigned)L.nseg), dim3(256), 0, s, bin, Rv, seg);
+    launch_k("rle_dec_prep_kernel", rle_dec_prep_kernel<T>, dim3(1), dim3(64), 0, s, bin, in_bytes, n, Rv, lng, d_status);
+    launch_k("rle_dec_reduce_kernel", rle_dec_reduce_kernel<T>, dim3((unsigned)L.nseg), dim3(256), 0, s, bin, Rv, seg, lng);
     launch_k("scan_partials_kernel", scan_partials_kernel<false>, dim3(1), dim3(1024), 0, s, seg, (uint32_t)L.nseg, tot);
-    launch_k("rle_dec_apply_kernel", rle_dec_apply_kernel<T>, dim3((unsigned)L.nseg), dim3(256), 0, s, bin, n, Rv, seg, tot, start, tf, d_status);
+    launch_k("rle_dec_apply_kernel", rle_dec_apply_kernel<T>, dim3((unsigned)L.nseg), dim3(256), 0, s, bin, n, Rv, lng, seg, tot, start, tf, (T*)out, d_status);
     const unsigned eb = (unsigned)cdiv(L.ntiles, 4);
-    launch_k("rle_dec_expand_kernel", rle_dec_expand_kernel<T>, dim3(eb), dim3(256), 0, s, (const uint8_t*)in, n, start, tf, d_status, (T*)out, (uint32_t)L.ntiles);
+    launch_k("rle_dec_expand_kernel", rle_dec_expand_kernel<T>, dim3(eb), dim3(256), 0, s, (const uint8_t*)in, n, start, tf, lng, d_status, (T*)out, (uint32_t)L.ntiles);
     FZH_CHECK_LAUNCH("rle decode");
     return FZH_OK;
 }
