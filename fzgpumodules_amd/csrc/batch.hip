@@ -63,16 +63,26 @@ __global__ void __launch_bounds__(256) vb_partial_kernel(const Plan* __restrict_
             if (0.0f > mx) mx = 0.0f;
         }
         const uint64_t e4 = b + ((e - b) & ~3ull);
-        for (uint64_t i = b + 4 * (uint64_t)threadIdx.x; i < e4; i += 1024) {
-            const float4 v = gld_f4(in + i);
-            if (v.x < mn) mn = v.x;
-            if (v.x > mx) mx = v.x;
-            if (v.y < mn) mn = v.y;
-            if (v.y > mx) mx = v.y;
-            if (v.z < mn) mn = v.z;
-            if (v.z > mx) mx = v.z;
-            if (v.w < mn) mn = v.w;
-            if (v.w > mx) mx = v.w;
+        // eight 16-byte loads in flight per thread (one: 110 us for the 0.4 GB
+        // of 60 fields, now 97)
+        for (uint64_t i0 = b + 4 * (uint64_t)threadIdx.x; i0 < e4; i0 += 8192) {
+            float4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint64_t i = i0 + 1024 * u;
+                v[u] = gld_f4(in + (i < e4 ? i : b));
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                if (v[u].x < mn) mn = v[u].x;
+                if (v[u].x > mx) mx = v[u].x;
+                if (v[u].y < mn) mn = v[u].y;
+                if (v[u].y > mx) mx = v[u].y;
+                if (v[u].z < mn) mn = v[u].z;
+                if (v[u].z > mx) mx = v[u].z;
+                if (v[u].w < mn) mn = v[u].w;
+                if (v[u].w > mx) mx = v[u].w;
+            }
         }
         for (uint64_t i = e4 + threadIdx.x; i < e; i += 256) {
             const float v = gp(in)[i];
