@@ -5,7 +5,7 @@
 // plus a per-tile count.  launch_compact then places every tile's list at
 // its exclusive prefix with a place kernel in which a wave takes 32 tiles
 // of each list, finds the non-empty ones by ballot and copies them with all
-// 64 lanes.  Up to COMPACT_INLINE tiles each workgroup sums the counts
+// 64 lanes.  Up to COMPACT_INLINE counts each workgroup sums the counts
 // before its 128 tiles itself (one launch in all); beyond that a
 // device-wide scan of the counts (fzh_scan.h) runs first.  No workgroup
 // waits on another.
@@ -32,7 +32,11 @@ struct CompactListT {
 };
 using CompactList = CompactListT<float>;
 
-constexpr uint32_t COMPACT_INLINE = 16384;
+// Counts (of all lists) up to which the place kernel sums those before each
+// workgroup itself.  39 Ki counts (301 x 203 x 157 doubles): 4.4 us against
+// 12.8 + 4.5 us and a launch gap with a one-workgroup scan; past that the
+// longest sum outgrows the scan's launches.
+constexpr uint32_t COMPACT_INLINE = 65536;
 
 // excl: exclusive prefix (mod 2^32) of the NL*T counts, excl[NL*T] = sum
 // (INL: unused, the prefixes are summed in the kernel).
@@ -134,7 +138,7 @@ inline int launch_compact(hipStream_t s, void* state, size_t T, uint32_t E, Comp
     if (L1 && L1->cnt != L0.cnt + T) return fail(FZH_E_INVALID, "compact: second count list must follow the first");
     uint32_t* excl = (uint32_t*)state;
     void* ws = (uint8_t*)state + align_up(4 * (2 * T + 1), 256);
-    const bool inl = T <= COMPACT_INLINE;
+    const bool inl = nl * T <= COMPACT_INLINE;
     if (!inl)
         if (int rc = scan_u32<true>(s, L0.cnt, excl, nl * T, nullptr, excl + nl * T, ws)) return rc;
     const unsigned blocks = (unsigned)cdiv(cdiv(T, 32), 4);

