@@ -28,6 +28,7 @@ __device__ __forceinline__ uint64_t slot_size(const fzh_concat_slot& s) {
 // have stored it: size0 replaces slot 0's device size, and readback words
 // at ptr (a u64) read val.
 struct SizeOverride {
+    bool first_done;  // slot 0's producer writes the second destination too
     bool has_size0;
     uint64_t size0;
     uintptr_t ptr;
@@ -41,8 +42,8 @@ struct SizeOverride {
 // in the header or the total from the values it just computed (so the
 // readback never depends on another workgroup's stores).
 // With `copy` (16-byte aligned, as large as the concat can get) the whole
-// result goes there too, each word stored twice; slot 0 of a fused RZE
-// launch is copied by the workgroups that place its chunks.
+// result goes there too, each word stored twice; a slot 0 whose producer
+// stores its stream twice itself (first_done) needs the pad only.
 __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n, uint8_t* __restrict__ out,
                                                     uint8_t* __restrict__ copy, uint64_t* __restrict__ total,
                                                     const ReadbackArgs& r, int nr, uint8_t* __restrict__ mapped,
@@ -74,7 +75,7 @@ __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n,
         uint8_t* d8 = out + s_off[si];
         uint8_t* c8 = copy ? copy + s_off[si] : nullptr;
         const bool placed = reinterpret_cast<const void*>(d8) == reinterpret_cast<const void*>(src);
-        if (placed && (!c8 || ov.has_size0)) {  // produced in place: the pad only
+        if (placed && (!c8 || ov.first_done)) {  // produced in place: the pad only
             if (g < nw * 16 - sz) {
                 d8[sz + g] = 0;
                 if (c8) c8[sz + g] = 0;

@@ -277,8 +277,10 @@ concat_copy_kernel(ConcatArgs a, uint8_t* __restrict__ out, const uint64_t* __re
 // Concat and readback in one launch (body in fzh_concat.h).
 __global__ void __launch_bounds__(256)
 concat_readback_kernel(ConcatArgs a, int n, uint8_t* __restrict__ out, uint8_t* __restrict__ copy,
-                       uint64_t* __restrict__ total, ReadbackArgs r, int nr, uint8_t* __restrict__ mapped) {
-    concat_readback_body(a, n, out, copy, total, r, nr, mapped, blockIdx.x, gridDim.x, SizeOverride{});
+                       bool first_done, uint64_t* __restrict__ total, ReadbackArgs r, int nr,
+                       uint8_t* __restrict__ mapped) {
+    concat_readback_body(a, n, out, copy, total, r, nr, mapped, blockIdx.x, gridDim.x,
+                         SizeOverride{first_done, false, 0, 0, 0});
 }
 
 // out[z][y][x] = base[(z0 + z) % bz][(y0 + y) % by][(x0 + x) % bx]
@@ -460,23 +462,24 @@ int fzh_concat(void* stream, const fzh_concat_slot* slots, int n, void* d_out, u
 
 int fzh_concat_readback(void* stream, const fzh_concat_slot* slots, int n, void* d_out, uint64_t out_cap,
                         uint64_t* d_total, const fzh_readback_entry* entries, int n_entries, void* d_mapped_dst) {
-    return concat_readback(S(stream), slots, n, d_out, nullptr, out_cap, d_total, entries, n_entries, d_mapped_dst);
+    return concat_readback(S(stream), slots, n, d_out, nullptr, false, out_cap, d_total, entries, n_entries, d_mapped_dst);
 }
 
 }  // extern "C"
 
 namespace fzh {
 
-int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, uint64_t out_cap,
-                    uint64_t* d_total, const fzh_readback_entry* entries, int n_entries, void* d_mapped_dst) {
+int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, bool first_done,
+                    uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries, int n_entries,
+                    void* d_mapped_dst) {
     ConcatArgs a;
     ReadbackArgs r;
     unsigned grid = 1;
-    if (int rc = build_concat_args(slots, n, d_out, d_copy, true, out_cap, d_total, entries, n_entries, d_mapped_dst,
-                                   a, r, grid))
+    if (int rc = build_concat_args(slots, n, d_out, d_copy, !first_done, out_cap, d_total, entries, n_entries,
+                                   d_mapped_dst, a, r, grid))
         return rc;
     launch_k("concat_readback_kernel", concat_readback_kernel, dim3(grid), dim3(256), 0, s, a, n, (uint8_t*)d_out,
-             (uint8_t*)d_copy, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
+             (uint8_t*)d_copy, first_done, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
     FZH_CHECK_LAUNCH("concat_readback_kernel");
     return FZH_OK;
 }

@@ -60,9 +60,20 @@ int build_books_device(hipStream_t s, uint32_t n_books, const uint32_t* d_freq, 
                        uint32_t* d_bk4, uint8_t* d_revbook, size_t rev_stride, int* d_status);
 
 // fzh_concat_readback with a second destination of the whole result (both
-// launches: d_copy null, or 16-byte aligned and out_cap bytes).
-int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, uint64_t out_cap,
-                    uint64_t* d_total, const fzh_readback_entry* entries, int n_entries, void* d_mapped_dst);
+// launches: d_copy null, or 16-byte aligned and out_cap bytes).  first_done:
+// slot 0, produced in place, is in d_copy already.
+int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_out, void* d_copy, bool first_done,
+                    uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries, int n_entries,
+                    void* d_mapped_dst);
+
+// fzh_rle_enc and fzh_huffman_encode (fine: fzh_huffman_encode_fine) with a
+// second destination of the stream: d_copy null, or aligned and as large as
+// d_out.
+int rle_enc(hipStream_t s, const void* d_in, size_t n, int elem_bytes, void* d_out, size_t out_cap, void* d_copy,
+            uint64_t* d_out_size, void* d_ws, size_t ws_bytes);
+int huffman_encode(hipStream_t s, bool fine, const void* d_in, size_t n, int elem_bytes, uint32_t bklen,
+                   const uint32_t* d_bk4, const uint8_t* d_revbook, void* d_out, size_t out_cap, void* d_copy,
+                   uint64_t* d_out_size, void* d_ws, size_t ws_bytes);
 
 // Optional per-kernel device timing.  launch_k launches like
 // kernel<<<grid, block, shm, s>>>(args...); while timing is on

@@ -324,6 +324,7 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
     // an RZE stage writing the concat's first slot leaves its pack step to
     // the final concat + readback launch
     RZEStage* defer_rze = nullptr;
+    bool first_done = false;
     if (outputs_.size() > 1) {
         const Buffer& P = buffers_[outputs_[0]];
         if (P.aliased && P.producer >= 0 && !nodes_[P.producer].elided)
@@ -345,6 +346,15 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
             hipck(hipEventCreate(&e0), "hipEventCreate");
             hipck(hipEventCreate(&e1), "hipEventCreate");
             hipck(hipEventRecord(e0, stream), "hipEventRecord");
+        }
+        // the stage that writes the concat's first slot may store it in the
+        // caller's buffer too, unless a later stage could still read an input
+        // that lies in it
+        if (copy_to_ && outputs_.size() > 1 && n.out_buf[0] == outputs_[0] && buffers_[outputs_[0]].aliased) {
+            const uint8_t *c = (const uint8_t*)copy_to_, *i = (const uint8_t*)d_in;
+            if (i + padded <= c || c + concat_cap_ <= i)
+                first_done = n.stage->copyOutputTo((uint8_t*)copy_to_ +
+                                                   ((uint8_t*)buffers_[outputs_[0]].ptr - (uint8_t*)concat_buf_));
         }
         n.stage->execute(stream, pool_.get(), {in.ptr}, outs, {in.size});
         if (e1) hipck(hipEventRecord(e1, stream), "hipEventRecord");
@@ -393,9 +403,9 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
                                                      (int)rb.size(), rb_dev_),
                        "Pipeline concat");
         else
-            throwIfFzh(fzh::concat_readback(stream, slots.data(), (int)slots.size(), concat_buf_, copy_to_, concat_cap_,
-                                            (uint64_t*)((uint8_t*)concat_ws_ + 512), rb.data(), (int)rb.size(),
-                                            rb_dev_),
+            throwIfFzh(fzh::concat_readback(stream, slots.data(), (int)slots.size(), concat_buf_, copy_to_, first_done,
+                                            concat_cap_, (uint64_t*)((uint8_t*)concat_ws_ + 512), rb.data(),
+                                            (int)rb.size(), rb_dev_),
                        "Pipeline concat");
         return;
     }

@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 
 #include "fz/stages.h"
 #include "fzh_internal.h"
@@ -452,6 +453,7 @@ void RZEStage::postStreamSync(hipStream_t) {
 template <typename T>
 void RLEStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                           const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
+    void* copy = std::exchange(copy_out_, nullptr);
     if (inputs.empty() || outputs.empty() || sizes.empty()) throw std::runtime_error("RLEStage: Invalid inputs/outputs");
     small_.ensure(256, pool, stream);
     clearReadbacks();
@@ -460,8 +462,8 @@ void RLEStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vecto
         const size_t n = sizes[0] / sizeof(T);
         cached_num_elements_ = (uint32_t)n;
         ws_.ensure(fzh_rle_enc_ws_bytes(n), pool, stream);
-        throwIfFzh(fzh_rle_enc(stream, inputs[0], n, (int)sizeof(T), outputs[0], fzh_rle_enc_bound(n, sizeof(T)),
-                               (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes),
+        throwIfFzh(fzh::rle_enc(stream, inputs[0], n, (int)sizeof(T), outputs[0], fzh_rle_enc_bound(n, sizeof(T)), copy,
+                                (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes),
                    "RLEStage");
         actual_output_size_ = fzh_rle_enc_bound(n, sizeof(T));
         size_pending_ = true;
@@ -515,6 +517,7 @@ std::vector<size_t> HuffmanStage<T>::estimateOutputSizes(const std::vector<size_
 template <typename T>
 void HuffmanStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                               const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
+    void* copy = std::exchange(copy_out_, nullptr);
     if (inputs.empty() || outputs.empty() || sizes.empty())
         throw std::runtime_error("HuffmanStage: inputs, outputs, and sizes must be non-empty");
     clearReadbacks();
@@ -537,10 +540,10 @@ void HuffmanStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::v
                                                  (uint32_t*)book_.ptr, (uint8_t*)book_.ptr + 4 * (size_t)bklen_,
                                                  (int*)((uint8_t*)small_.ptr + 16)),
                    "HuffmanStage device codebook");
-        throwIfFzh(fzh_huffman_encode(stream, inputs[0], n, (int)sizeof(T), bklen_, (const uint32_t*)book_.ptr,
-                                      (const uint8_t*)book_.ptr + 4 * (size_t)bklen_, outputs[0],
-                                      fzh_huffman_enc_bound(n, bklen_, sizeof(T)), (uint64_t*)small_.ptr, ws_.ptr,
-                                      ws_.bytes),
+        throwIfFzh(fzh::huffman_encode(stream, false, inputs[0], n, (int)sizeof(T), bklen_, (const uint32_t*)book_.ptr,
+                                       (const uint8_t*)book_.ptr + 4 * (size_t)bklen_, outputs[0],
+                                       fzh_huffman_enc_bound(n, bklen_, sizeof(T)), copy, (uint64_t*)small_.ptr,
+                                       ws_.ptr, ws_.bytes),
                    "HuffmanStage encode");
         original_len_ = n;
         actual_output_size_ = fzh_huffman_enc_bound(n, bklen_, sizeof(T));
@@ -573,10 +576,10 @@ void HuffmanStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::v
         uint32_t max_cl = 0;
         for (uint32_t i = 0; i < bklen_; i++) max_cl = std::max(max_cl, ((const uint32_t*)book.data())[i] >> 27);
         const bool fine = encode_mode_ == HuffmanEncodeMode::Fine && max_cl <= 8;
-        throwIfFzh((fine ? fzh_huffman_encode_fine : fzh_huffman_encode)(
-                       stream, inputs[0], n, (int)sizeof(T), bklen_, (const uint32_t*)book_.ptr,
-                       (const uint8_t*)book_.ptr + 4 * (size_t)bklen_, outputs[0],
-                       fzh_huffman_enc_bound(n, bklen_, sizeof(T)), (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes),
+        throwIfFzh(fzh::huffman_encode(stream, fine, inputs[0], n, (int)sizeof(T), bklen_, (const uint32_t*)book_.ptr,
+                                       (const uint8_t*)book_.ptr + 4 * (size_t)bklen_, outputs[0],
+                                       fzh_huffman_enc_bound(n, bklen_, sizeof(T)), copy, (uint64_t*)small_.ptr,
+                                       ws_.ptr, ws_.bytes),
                    "HuffmanStage encode");
         // keep the host copy alive until the copy has been consumed
         FZ_HIP(hipStreamSynchronize(stream));

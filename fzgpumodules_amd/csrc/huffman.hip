@@ -153,12 +153,15 @@ huf_enc_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, const uint3
 
 // Cells of partition p -> stream cell par_entry[p] (one wave per partition);
 // each workgroup adds its partitions' bit counts to one of NBIT_SLOTS
-// accumulators (one atomic per workgroup) for the header.
+// accumulators (one atomic per workgroup) for the header.  With `copy` the
+// stream goes there as well, the cells and what earlier launches wrote before
+// them: for 2^27 symbols 57 -> 81 us here, but the concat of the caller's
+// buffer 63 -> 32 as it doesn't read the stream again.
 constexpr uint32_t NBIT_SLOTS = 256;
 
 __global__ void __launch_bounds__(256)
 huf_pack_kernel(const uint32_t* __restrict__ scells, const uint32_t* __restrict__ ncell,
-                uint8_t* __restrict__ out, uint32_t ent2, uint32_t ent3, uint32_t ent4, uint32_t pardeg,
+                uint8_t* __restrict__ out, uint8_t* __restrict__ copy, uint32_t ent1, uint32_t ent2, uint32_t ent3, uint32_t ent4, uint32_t pardeg,
                 uint32_t cells, unsigned long long* __restrict__ nbit_acc) {
     __shared__ uint32_t s_nb[4];
     const int w = (int)wave_in_wg();
@@ -170,6 +173,7 @@ huf_pack_kernel(const uint32_t* __restrict__ scells, const uint32_t* __restrict_
         const uint32_t c = ncell[p];
         const uint32_t* src = scells + (uint64_t)p * cells;
         uint32_t* dst = reinterpret_cast<uint32_t*>(out + ent4) + e;
+        uint32_t* cdst = copy ? reinterpret_cast<uint32_t*>(copy + ent4) + e : nullptr;
         // up to four loads in flight per lane before their stores
         for (uint32_t i = l; i < c; i += 256) {
             uint32_t v[4];
@@ -178,8 +182,19 @@ huf_pack_kernel(const uint32_t* __restrict__ scells, const uint32_t* __restrict_
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 if (i + 64 * k < c) dst[i + 64 * k] = v[k];
+            if (copy)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (i + 64 * k < c) cdst[i + 64 * k] = v[k];
         }
         nb = reinterpret_cast<const uint32_t*>(out + ent2)[p];
+    }
+    if (copy) {  // the reverse book, and the workgroup's bit counts and entries
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(out);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(copy);
+        for (uint32_t i = ent1 / 4 + blockIdx.x * 256 + threadIdx.x; i < ent2 / 4; i += gridDim.x * 256) dst[i] = src[i];
+        const uint32_t q = blockIdx.x * 4 + (threadIdx.x & 3), i = (threadIdx.x & 4 ? ent3 : ent2) / 4 + q;
+        if (threadIdx.x < 8 && q < pardeg) dst[i] = src[i];
     }
     if (l == 0) s_nb[w] = nb;
     __syncthreads();
@@ -190,7 +205,7 @@ huf_pack_kernel(const uint32_t* __restrict__ scells, const uint32_t* __restrict_
 // phf_header (hf.h:38-44) once every partition is placed; sums the bit
 // total from the NBIT_SLOTS accumulators and clears them for the next call.
 __global__ void __launch_bounds__(256)
-huf_header_kernel(uint8_t* __restrict__ out, uint64_t n, uint32_t bklen, uint32_t sublen, uint32_t ent1, uint32_t ent2,
+huf_header_kernel(uint8_t* __restrict__ out, uint8_t* __restrict__ copy, uint64_t n, uint32_t bklen, uint32_t sublen, uint32_t ent1, uint32_t ent2,
                   uint32_t ent3, uint32_t ent4, uint32_t pardeg, const uint32_t* __restrict__ total_ncell,
                   uint64_t* __restrict__ out_size, unsigned long long* __restrict__ nbit_acc) {
     __shared__ unsigned long long s_w[4];
@@ -203,24 +218,29 @@ huf_header_kernel(uint8_t* __restrict__ out, uint64_t n, uint32_t bklen, uint32_
     for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
     if (lane_id() == 0) s_w[threadIdx.x >> 6] = a;
     __syncthreads();
+    if (copy)
+        for (uint32_t i = 64 + threadIdx.x; i < HDR_BYTES; i += 256) copy[i] = 0;
     if (threadIdx.x == 0) {
         const unsigned long long tnb = s_w[0] + s_w[1] + s_w[2] + s_w[3];
         const uint32_t tc = *total_ncell;
         const uint32_t ent5 = ent4 + 4 * tc;
-        uint32_t* h32 = reinterpret_cast<uint32_t*>(out);
-        h32[0] = bklen & 0xFFFFu;
-        h32[1] = sublen;
-        h32[2] = pardeg;
-        h32[3] = 0;
-        reinterpret_cast<uint64_t*>(out)[2] = n;
-        reinterpret_cast<uint64_t*>(out)[3] = tnb;
-        reinterpret_cast<uint64_t*>(out)[4] = tc;
-        h32[10] = 0;
-        h32[11] = ent1;
-        h32[12] = ent2;
-        h32[13] = ent3;
-        h32[14] = ent4;
-        h32[15] = ent5;
+        for (uint8_t* o : {out, copy}) {
+            if (!o) continue;
+            uint32_t* h32 = reinterpret_cast<uint32_t*>(o);
+            h32[0] = bklen & 0xFFFFu;
+            h32[1] = sublen;
+            h32[2] = pardeg;
+            h32[3] = 0;
+            reinterpret_cast<uint64_t*>(o)[2] = n;
+            reinterpret_cast<uint64_t*>(o)[3] = tnb;
+            reinterpret_cast<uint64_t*>(o)[4] = tc;
+            h32[10] = 0;
+            h32[11] = ent1;
+            h32[12] = ent2;
+            h32[13] = ent3;
+            h32[14] = ent4;
+            h32[15] = ent5;
+        }
         *out_size = ent5;
     }
 }
@@ -906,7 +926,7 @@ EncWs enc_layout(size_t n, int sl) {
 
 template <typename T, int SL>
 int enc_impl(hipStream_t s, const void* in, size_t n, uint32_t bklen, const uint32_t* bk4, const uint8_t* rev,
-             void* out, size_t cap, uint64_t* out_size, void* ws, size_t ws_bytes) {
+             void* out, size_t cap, void* copy, uint64_t* out_size, void* ws, size_t ws_bytes) {
     constexpr int CELLS = cells_of(SL);
     const EncWs L = enc_layout(n, SL);
     if (ws_bytes < L.total) return fail(FZH_E_CAPACITY, "huffman enc: workspace too small");
@@ -915,7 +935,7 @@ int enc_impl(hipStream_t s, const void* in, size_t n, uint32_t bklen, const uint
     if (cap < fzh_huffman_enc_bound(n, bklen, sizeof(T))) return fail(FZH_E_CAPACITY, "huffman enc: output below bound");
     const uint32_t rev_bytes = (uint32_t)fzh_huffman_revbook_bytes(bklen, sizeof(T));
     if (rev_bytes % 4) return fail(FZH_E_INVALID, "huffman enc: bklen * sizeof(T) must be a multiple of 4");
-    if ((uintptr_t)out % 16) return fail(FZH_E_INVALID, "huffman enc: output must be 16-byte aligned");
+    if (((uintptr_t)out | (uintptr_t)copy) % 16) return fail(FZH_E_INVALID, "huffman enc: output must be 16-byte aligned");
     const uint32_t pardeg = (uint32_t)L.pardeg;
     const uint32_t ent1 = HDR_BYTES, ent2 = ent1 + rev_bytes, ent3 = ent2 + 4 * pardeg, ent4 = ent3 + 4 * pardeg;
     uint8_t* w = (uint8_t*)ws;
@@ -936,28 +956,35 @@ int enc_impl(hipStream_t s, const void* in, size_t n, uint32_t bklen, const uint
     if (int rc = scan_u32(s, ncell, reinterpret_cast<uint32_t*>(o8 + ent3), pardeg, nullptr, tot, w + L.o_scan))
         return rc;
     unsigned long long* nbit_acc = reinterpret_cast<unsigned long long*>(w + L.o_nbit);
-    launch_k("huf_pack_kernel", huf_pack_kernel, dim3(blocks), dim3(256), 0, s, scells, ncell, o8, ent2, ent3, ent4,
-             pardeg, (uint32_t)CELLS, nbit_acc);
-    launch_k("huf_header_kernel", huf_header_kernel, dim3(1), dim3(256), 0, s, o8, n, bklen, (uint32_t)SL, ent1, ent2,
-             ent3, ent4, pardeg, tot, out_size, nbit_acc);
+    launch_k("huf_pack_kernel", huf_pack_kernel, dim3(blocks), dim3(256), 0, s, scells, ncell, o8, (uint8_t*)copy, ent1,
+             ent2, ent3, ent4, pardeg, (uint32_t)CELLS, nbit_acc);
+    launch_k("huf_header_kernel", huf_header_kernel, dim3(1), dim3(256), 0, s, o8, (uint8_t*)copy, n, bklen, (uint32_t)SL,
+             ent1, ent2, ent3, ent4, pardeg, tot, out_size, nbit_acc);
     FZH_CHECK_LAUNCH("huffman encode");
     return FZH_OK;
 }
 
 template <int SL>
-int encode_sl(void* stream, const void* d_in, size_t n, int elem_bytes, uint32_t bklen, const uint32_t* d_bk4,
-                     const uint8_t* d_revbook, void* d_out, size_t out_cap, uint64_t* d_out_size, void* d_ws,
-                     size_t ws_bytes) {
+int encode_sl(hipStream_t s, const void* d_in, size_t n, int elem_bytes, uint32_t bklen, const uint32_t* d_bk4,
+              const uint8_t* d_revbook, void* d_out, size_t out_cap, void* d_copy, uint64_t* d_out_size, void* d_ws,
+              size_t ws_bytes) {
     if (ws_bytes < std::max(enc_layout(n, SUBLEN).total, enc_layout(n, SUBLEN_FINE).total)) return fail(FZH_E_CAPACITY, "huffman enc: workspace too small");
     switch (elem_bytes) {
-    case 1: return enc_impl<uint8_t, SL>(S(stream), d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_out_size, d_ws, ws_bytes);
-    case 2: return enc_impl<uint16_t, SL>(S(stream), d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_out_size, d_ws, ws_bytes);
-    case 4: return enc_impl<uint32_t, SL>(S(stream), d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_out_size, d_ws, ws_bytes);
+    case 1: return enc_impl<uint8_t, SL>(s, d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_copy, d_out_size, d_ws, ws_bytes);
+    case 2: return enc_impl<uint16_t, SL>(s, d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_copy, d_out_size, d_ws, ws_bytes);
+    case 4: return enc_impl<uint32_t, SL>(s, d_in, n, bklen, d_bk4, d_revbook, d_out, out_cap, d_copy, d_out_size, d_ws, ws_bytes);
     default: return fail(FZH_E_INVALID, "huffman enc: elem_bytes must be 1, 2 or 4");
     }
 }
 
 }  // namespace
+
+int huffman_encode(hipStream_t s, bool fine, const void* d_in, size_t n, int elem_bytes, uint32_t bklen,
+                   const uint32_t* d_bk4, const uint8_t* d_revbook, void* d_out, size_t out_cap, void* d_copy,
+                   uint64_t* d_out_size, void* d_ws, size_t ws_bytes) {
+    return (fine ? encode_sl<SUBLEN_FINE> : encode_sl<SUBLEN>)(s, d_in, n, elem_bytes, bklen, d_bk4, d_revbook, d_out,
+                                                               out_cap, d_copy, d_out_size, d_ws, ws_bytes);
+}
 }  // namespace fzh
 
 using namespace fzh;
@@ -1002,15 +1029,15 @@ size_t fzh_huffman_enc_ws_bytes(size_t n) {
 int fzh_huffman_encode(void* stream, const void* d_in, size_t n, int elem_bytes, uint32_t bklen,
                        const uint32_t* d_bk4, const uint8_t* d_revbook, void* d_out, size_t out_cap,
                        uint64_t* d_out_size, void* d_ws, size_t ws_bytes) {
-    return encode_sl<SUBLEN>(stream, d_in, n, elem_bytes, bklen, d_bk4, d_revbook, d_out, out_cap, d_out_size, d_ws,
-                             ws_bytes);
+    return huffman_encode(S(stream), false, d_in, n, elem_bytes, bklen, d_bk4, d_revbook, d_out, out_cap, nullptr,
+                          d_out_size, d_ws, ws_bytes);
 }
 
 int fzh_huffman_encode_fine(void* stream, const void* d_in, size_t n, int elem_bytes, uint32_t bklen,
                             const uint32_t* d_bk4, const uint8_t* d_revbook, void* d_out, size_t out_cap,
                             uint64_t* d_out_size, void* d_ws, size_t ws_bytes) {
-    return encode_sl<SUBLEN_FINE>(stream, d_in, n, elem_bytes, bklen, d_bk4, d_revbook, d_out, out_cap, d_out_size,
-                                  d_ws, ws_bytes);
+    return huffman_encode(S(stream), true, d_in, n, elem_bytes, bklen, d_bk4, d_revbook, d_out, out_cap, nullptr,
+                          d_out_size, d_ws, ws_bytes);
 }
 
 int fzh_huffman_decode(void* stream, const void* d_in, size_t in_bytes, int elem_bytes, void* d_out, size_t n,

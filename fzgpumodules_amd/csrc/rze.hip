@@ -158,7 +158,7 @@ rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__
     const uint64_t end = 8ull + 4ull * d.nc + sum;
     const uint64_t size0 = (end + 3) & ~3ull;
     concat_readback_body(a, n, out, copy, total, r, nr, mapped, b - d.nc, gridDim.x - d.nc,
-                         SizeOverride{true, size0, reinterpret_cast<uintptr_t>(d.out_size), size0});
+                         SizeOverride{true, true, size0, reinterpret_cast<uintptr_t>(d.out_size), size0});
 }
 
 // ---------------------------------------------------------------------------

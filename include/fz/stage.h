@@ -127,6 +127,10 @@ class Stage {
     // stage cannot: it then stores all of it.
     virtual bool limitInverseOutput(size_t bytes) { (void)bytes; return false; }
 
+    // Asks the next forward execute() to store its output 0 at d_copy as well
+    // (aligned and as large as outputs[0]).  False if the stage cannot.
+    virtual bool copyOutputTo(void* d_copy) { (void)d_copy; return false; }
+
     virtual DeviceSize getDeviceOutputSize(int index) const { (void)index; return {}; }
 
     // Device values postStreamSync() needs, registered by execute().  A

@@ -370,6 +370,7 @@ class RLEStage : public Stage {
   public:
     void setInverse(bool inv) override { is_inverse_ = inv; }
     bool isInverse() const override { return is_inverse_; }
+    bool copyOutputTo(void* d_copy) override { copy_out_ = d_copy; return true; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -403,6 +404,7 @@ class RLEStage : public Stage {
     void restoreState() override { cached_num_elements_ = saved_n_; actual_output_size_ = saved_out_; }
 
   private:
+    void* copy_out_ = nullptr;  // second destination of the next forward execute()
     bool is_inverse_ = false;
     uint32_t cached_num_elements_ = 0, saved_n_ = 0;
     size_t actual_output_size_ = 0, saved_out_ = 0;
@@ -448,6 +450,7 @@ class HuffmanStage : public Stage {
     // With the host codebook the histogram has to reach the host builder.
     bool isGraphCompatible() const override { return is_inverse_ || device_book_; }
 
+    bool copyOutputTo(void* d_copy) override { copy_out_ = d_copy; return true; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -488,6 +491,7 @@ class HuffmanStage : public Stage {
     }
 
   private:
+    void* copy_out_ = nullptr;  // second destination of the next forward execute()
     bool is_inverse_ = false;
     uint32_t bklen_ = std::is_same_v<T, uint8_t> ? 256 : 1024;
     HuffmanEncodeMode encode_mode_ = HuffmanEncodeMode::Coarse;
