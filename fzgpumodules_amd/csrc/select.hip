@@ -73,6 +73,17 @@ __device__ __forceinline__ float wmax_f(float v) {
     return v;
 }
 
+// One workgroup per chunk; thread t takes elements t, t + 256, ... in order
+// (the double sums depend on it).  Bound by vector instructions, most of them
+// the double sums, so the loop spends none on divisions (coordinates step by
+// 256 elements with a carry; they were 64-bit divisions), the histogram is one
+// shifted add into byte counters (a compare and an add per bin before), and
+// four elements' neighbours are loaded ahead of their sums, each from an
+// address that is valid for every element: 512 chunks of 256 x 256 250 -> 145 us,
+// 1024 of 32 x 32 x 32 284 -> 171.
+constexpr uint32_t FEAT_FLUSH = 248;  // elements per thread between histogram flushes (< 256)
+
+template <bool ZN>
 __global__ void __launch_bounds__(256)
 features_kernel(const float* __restrict__ chunks, uint32_t nx, uint32_t ny, uint32_t nz,
                 const float* __restrict__ d_eb, float* __restrict__ feat) {
@@ -94,54 +105,90 @@ features_kernel(const float* __restrict__ chunks, uint32_t nx, uint32_t ny, uint
     for (int k = 0; k < 7; k++) a.c[k] = 0;
 #pragma unroll
     for (int k = 0; k < 15; k++) a.h[k] = 0;
-    for (uint64_t i = threadIdx.x; i < E; i += 256) {
-        const uint32_t ix = (uint32_t)(i % nx);
-        const uint32_t iy = (uint32_t)((i / nx) % ny);
-        const uint32_t iz = (uint32_t)(i / sxy);
-        const float v = x[i];
-        const float w = ix ? x[i - 1] : 0.0f;
-        const float nn = iy ? x[i - nx] : 0.0f;
-        const float wn = (ix && iy) ? x[i - 1 - nx] : 0.0f;
-        float res;
-        if (nz > 1) {
-            const float b = iz ? x[i - sxy] : 0.0f;
-            const float wb = (ix && iz) ? x[i - 1 - sxy] : 0.0f;
-            const float nb = (iy && iz) ? x[i - nx - sxy] : 0.0f;
-            const float wnb = (ix && iy && iz) ? x[i - 1 - nx - sxy] : 0.0f;
-            res = v - w - nn - b + wn + wb + nb - wnb;
-            if (iz) a.sdz += fabs((double)v - (double)b);
-        } else {
-            res = v - w - nn + wn;
-        }
-        a.sx += v;
-        a.sx2 += (double)v * v;
-        a.mn = fminf(a.mn, v);
-        a.mx = fmaxf(a.mx, v);
-        a.mxabs = fmaxf(a.mxabs, fabsf(v));
-        a.sabs += fabsf(v);
-        a.c[0] += v == 0.0f;
-        a.c[1] += v == rintf(v);
-        a.c[6] += v > 0.0f;
-        if (ix) {
-            a.c[2] += v == w;
-            const double d = fabs((double)v - (double)w);
-            a.sdx += d;
-            a.c[3] += d * inv2eb < 0.5;
-        }
-        if (iy) a.sdy += fabs((double)v - (double)nn);
-        const float l = fabsf(res) * inv2eb;
-        a.sl += l;
-        const float lp = l + 0.5f;
-        int bin;
-        if (!(lp >= 1.0f)) bin = 0;
-        else if (lp >= 16384.0f) bin = 14;
-        else bin = 32 - __clz((uint32_t)lp);
-        bin = bin > 14 ? 14 : bin;
+    // coordinates of this thread's next element, and the step to the one after
+    uint32_t ix = threadIdx.x % nx, iy = threadIdx.x / nx % ny, iz = threadIdx.x / nx / ny;
+    const uint32_t dx = 256 % nx, dy = 256 / nx % ny, dz = 256 / nx / ny;
+    constexpr int U = 4;
+    uint64_t h0 = 0, h1 = 0;  // byte b of h0: bin b, of h1: bin 8 + b
+    uint32_t since = 0;
+    const auto flush = [&]() {
 #pragma unroll
-        for (int k = 0; k < 15; k++) a.h[k] += bin == k;  // no dynamic register indexing
-        a.c[4] += l >= 511.5f;
-        a.c[5] += fabsf(v) * inv2eb >= 32767.5f;
+        for (int k = 0; k < 15; k++) a.h[k] += (uint32_t)((k < 8 ? h0 : h1) >> (8 * (k & 7))) & 0xFFu;
+        h0 = h1 = 0;
+        since = 0;
+    };
+    for (uint64_t i0 = threadIdx.x; i0 < E; i0 += 256 * U) {
+        float v[U], w[U], nn[U], wn[U], bb[U], wb[U], nb[U], wnb[U];
+        bool hx[U], hy[U], hz[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint64_t i = i0 + 256 * u;
+            hx[u] = ix != 0;
+            hy[u] = iy != 0;
+            hz[u] = iz != 0;
+            const float* q = x + (i < E ? i : 0);
+            const uint64_t ox = i < E && hx[u] ? 1 : 0, oy = i < E && hy[u] ? nx : 0, oz = i < E && hz[u] ? sxy : 0;
+            v[u] = q[0];
+            w[u] = *(q - ox);
+            nn[u] = *(q - oy);
+            wn[u] = *(q - ox - oy);
+            if constexpr (ZN) {
+                bb[u] = *(q - oz);
+                wb[u] = *(q - ox - oz);
+                nb[u] = *(q - oy - oz);
+                wnb[u] = *(q - ox - oy - oz);
+            }
+            ix += dx;
+            const uint32_t cx = ix >= nx;
+            ix -= cx ? nx : 0;
+            iy += dy + cx;
+            const uint32_t cy = iy >= ny;
+            iy -= cy ? ny : 0;
+            iz += dz + cy;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (i0 + 256 * u >= E) break;
+            const float w_ = hx[u] ? w[u] : 0.0f, nn_ = hy[u] ? nn[u] : 0.0f, wn_ = hx[u] && hy[u] ? wn[u] : 0.0f;
+            float res;
+            if constexpr (ZN) {
+                const float b_ = hz[u] ? bb[u] : 0.0f, wb_ = hx[u] && hz[u] ? wb[u] : 0.0f;
+                const float nb_ = hy[u] && hz[u] ? nb[u] : 0.0f, wnb_ = hx[u] && hy[u] && hz[u] ? wnb[u] : 0.0f;
+                res = v[u] - w_ - nn_ - b_ + wn_ + wb_ + nb_ - wnb_;
+                a.sdz += hz[u] ? fabs((double)v[u] - (double)b_) : 0.0;
+            } else {
+                res = v[u] - w_ - nn_ + wn_;
+            }
+            a.sx += v[u];
+            a.sx2 += (double)v[u] * v[u];
+            a.mn = fminf(a.mn, v[u]);
+            a.mx = fmaxf(a.mx, v[u]);
+            a.mxabs = fmaxf(a.mxabs, fabsf(v[u]));
+            a.sabs += fabsf(v[u]);
+            a.c[0] += v[u] == 0.0f;
+            a.c[1] += v[u] == rintf(v[u]);
+            a.c[6] += v[u] > 0.0f;
+            const double d = fabs((double)v[u] - (double)w_);
+            a.c[2] += hx[u] && v[u] == w_;
+            a.sdx += hx[u] ? d : 0.0;
+            a.c[3] += hx[u] && d * inv2eb < 0.5;
+            a.sdy += hy[u] ? fabs((double)v[u] - (double)nn_) : 0.0;
+            const float l = fabsf(res) * inv2eb;
+            a.sl += l;
+            const float lp = l + 0.5f;
+            // bin: 0 below 1 (and NaN), else the exponent + 1, at most 14
+            const uint32_t e1 = 32 - __clz((uint32_t)fminf(lp, 16384.0f));
+            const uint32_t bin = !(lp >= 1.0f) ? 0 : e1 > 14 ? 14 : e1;
+            const uint64_t one = 1ull << (8 * (bin & 7));
+            if (bin < 8) h0 += one;
+            else h1 += one;
+            a.c[4] += l >= 511.5f;
+            a.c[5] += fabsf(v[u]) * inv2eb >= 32767.5f;
+        }
+        since += U;
+        if (since >= FEAT_FLUSH) flush();
     }
+    flush();
     const int wv = threadIdx.x >> 6, l = lane_id();
     double d[7] = {a.sx, a.sx2, a.sdx, a.sdy, a.sdz, a.sl, a.sabs};
 #pragma unroll
@@ -257,18 +304,44 @@ __device__ __forceinline__ void forward_one(const Lds& s, const float* __restric
     }
 }
 
+// Forward of a batch, one sample per wave: lane o sums output o of each layer
+// in forward_one's order, the activations pass through LDS.  (One thread per
+// sample, as in training, is a chain of 6.5 Ki dependent multiply-adds on two
+// workgroups for 512 samples: 54 us, now 18.)
 __global__ void __launch_bounds__(256)
 mlp_forward_kernel(const float* __restrict__ p, const float* __restrict__ norm, const float* __restrict__ feat,
                    uint64_t n, float* __restrict__ logits) {
+    static_assert(NF <= 64 && H1 <= 64 && H2 <= 64 && NC <= 64, "one lane per output");
     __shared__ Lds s;
+    __shared__ float act[4][3][64];
     load_params(s, p, norm);
     __syncthreads();
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const int l = lane_id();
+    float(&t)[3][64] = act[threadIdx.x >> 6];
+    const uint64_t i = (uint64_t)blockIdx.x * 4 + wave_in_wg();
     if (i >= n) return;
-    float xb[NF], h1b[H1], h2b[H2], z[NC];
-    forward_one(s, feat + i * NF, xb, h1b, h2b, z);
+    if (l < NF) t[0][l] = bf16r((feat[i * NF + l] - s.shift[l]) * s.scale[l]);
+    wave_lds_sync();
+    if (l < H1) {
+        float acc = s.b1[l];
 #pragma unroll
-    for (int o = 0; o < NC; o++) logits[i * NC + o] = z[o];
+        for (int k = 0; k < NF; k++) acc = acc + s.w1[l * NF + k] * t[0][k];
+        t[1][l] = bf16r(acc > 0.0f ? acc : 0.0f);
+    }
+    wave_lds_sync();
+    if (l < H2) {
+        float acc = s.b2[l];
+#pragma unroll
+        for (int k = 0; k < H1; k++) acc = acc + s.w2[l * H1 + k] * t[1][k];
+        t[2][l] = bf16r(acc > 0.0f ? acc : 0.0f);
+    }
+    wave_lds_sync();
+    if (l < NC) {
+        float acc = s.b3[l];
+#pragma unroll
+        for (int k = 0; k < H2; k++) acc = acc + s.w3[l * H2 + k] * t[2][k];
+        logits[i * NC + l] = acc;
+    }
 }
 
 // Per-sample record kept for the gradient kernel (BF16 values stored as float).
@@ -429,20 +502,47 @@ adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restric
 
 // Chunk-major copy of a field: chunk c = (bz, by, bx) in row-major order of
 // the chunk grid, element (z, y, x) of the chunk at field (bz cz + z, by cy +
-// y, bx cx + x).  TO_CHUNKS = false scatters back.  One thread per element.
-template <bool TO_CHUNKS>
+// y, bx cx + x).  TO_CHUNKS = false scatters back.  One thread per V elements
+// of a chunk row (V = 4 where rows and pointers are 16-byte multiples); cx,
+// nx in units of V.  I: the index type, 32 bits where it holds the total:
+// the decomposition's divisions were 64-bit ones, which bound it (128 MiB
+// gathered in 149 us, now 38).
+template <bool TO_CHUNKS, typename V, typename I>
 __global__ void __launch_bounds__(256)
-chunk_copy_kernel(const float* __restrict__ src, float* __restrict__ dst, uint64_t total, uint32_t nx, uint32_t ny,
+chunk_copy_kernel(const V* __restrict__ src, V* __restrict__ dst, uint64_t total, uint32_t nx, uint32_t ny,
                   uint32_t cx, uint32_t cy, uint32_t cz, uint32_t gx, uint32_t gy) {
-    const uint64_t E = (uint64_t)cx * cy * cz;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (uint64_t)gridDim.x * 256) {
-        const uint64_t c = i / E, e = i % E;
-        const uint32_t x = (uint32_t)(e % cx), y = (uint32_t)((e / cx) % cy), z = (uint32_t)(e / ((uint64_t)cx * cy));
-        const uint32_t bx = (uint32_t)(c % gx), by = (uint32_t)((c / gx) % gy), bz = (uint32_t)(c / ((uint64_t)gx * gy));
+        I r = (I)i;
+        const uint32_t x = (uint32_t)(r % cx);
+        r /= cx;
+        const uint32_t y = (uint32_t)(r % cy);
+        r /= cy;
+        const uint32_t z = (uint32_t)(r % cz);
+        r /= cz;
+        const uint32_t bx = (uint32_t)(r % gx);
+        r /= gx;
+        const uint32_t by = (uint32_t)(r % gy), bz = (uint32_t)(r / gy);
         const uint64_t f = ((uint64_t)(bz * cz + z) * ny + (by * cy + y)) * nx + (bx * cx + x);
         if constexpr (TO_CHUNKS) dst[i] = src[f];
         else dst[f] = src[i];
     }
+}
+
+template <bool TO_CHUNKS, typename V>
+void launch_chunk_copy(hipStream_t s, const float* src, float* dst, uint64_t nx, uint64_t ny, uint64_t nz, uint32_t cx,
+                       uint32_t cy, uint32_t cz) {
+    constexpr uint32_t VE = sizeof(V) / sizeof(float);
+    const uint64_t total = nx * ny * nz / VE;
+    const unsigned blocks = (unsigned)std::min<uint64_t>(cdiv(total, 256), 65536);
+    const uint32_t gx = (uint32_t)(nx / cx), gy = (uint32_t)(ny / cy);
+    const auto* in = reinterpret_cast<const V*>(src);
+    auto* out = reinterpret_cast<V*>(dst);
+    if (total <= 0xFFFFFFFFull)
+        chunk_copy_kernel<TO_CHUNKS, V, uint32_t><<<blocks, 256, 0, s>>>(in, out, total, (uint32_t)(nx / VE),
+                                                                         (uint32_t)ny, cx / VE, cy, cz, gx, gy);
+    else
+        chunk_copy_kernel<TO_CHUNKS, V, uint64_t><<<blocks, 256, 0, s>>>(in, out, total, (uint32_t)(nx / VE),
+                                                                         (uint32_t)ny, cx / VE, cy, cz, gx, gy);
 }
 
 __global__ void __launch_bounds__(256) select_kernel(const float* __restrict__ logits, uint64_t n,
@@ -612,7 +712,10 @@ int fzs_features_f32(void* stream, const float* d_chunks, size_t n_chunks, uint3
     if (!d_chunks || !d_abs_eb || !d_feat) return fail(FZH_E_INVALID, "features: null pointer");
     if (nx == 0 || ny == 0 || nz == 0) return fail(FZH_E_INVALID, "features: empty chunk shape");
     if (n_chunks > 0x7FFFFFFFull) return fail(FZH_E_INVALID, "features: too many chunks");
-    features_kernel<<<(unsigned)n_chunks, 256, 0, S(stream)>>>(d_chunks, nx, ny, nz, d_abs_eb, d_feat);
+    if (nz > 1)
+        features_kernel<true><<<(unsigned)n_chunks, 256, 0, S(stream)>>>(d_chunks, nx, ny, nz, d_abs_eb, d_feat);
+    else
+        features_kernel<false><<<(unsigned)n_chunks, 256, 0, S(stream)>>>(d_chunks, nx, ny, nz, d_abs_eb, d_feat);
     FZH_CHECK_LAUNCH("features_kernel");
     return FZH_OK;
 }
@@ -623,7 +726,7 @@ int fzs_mlp_forward(void* stream, const float* d_params, const float* d_norm, co
                     float* d_logits) {
     if (n == 0) return FZH_OK;
     if (!d_params || !d_norm || !d_feat || !d_logits) return fail(FZH_E_INVALID, "mlp forward: null pointer");
-    mlp_forward_kernel<<<(unsigned)cdiv(n, 256), 256, 0, S(stream)>>>(d_params, d_norm, d_feat, n, d_logits);
+    mlp_forward_kernel<<<(unsigned)cdiv(n, 4), 256, 0, S(stream)>>>(d_params, d_norm, d_feat, n, d_logits);
     FZH_CHECK_LAUNCH("mlp_forward_kernel");
     return FZH_OK;
 }
@@ -666,16 +769,13 @@ static int chunk_copy(void* stream, const float* src, float* dst, uint64_t nx, u
     if (!src || !dst) return fail(FZH_E_INVALID, "chunk copy: null pointer");
     if (!cx || !cy || !cz || nx % cx || ny % cy || nz % cz)
         return fail(FZH_E_INVALID, "chunk copy: the field must be a whole number of chunks");
-    const uint64_t total = nx * ny * nz;
-    if (total == 0) return FZH_OK;
-    const unsigned blocks = (unsigned)std::min<uint64_t>(cdiv(total, 256), 65536);
-    const uint32_t gx = (uint32_t)(nx / cx), gy = (uint32_t)(ny / cy);
-    if (to_chunks)
-        chunk_copy_kernel<true><<<blocks, 256, 0, S(stream)>>>(src, dst, total, (uint32_t)nx, (uint32_t)ny, cx, cy, cz,
-                                                               gx, gy);
-    else
-        chunk_copy_kernel<false><<<blocks, 256, 0, S(stream)>>>(src, dst, total, (uint32_t)nx, (uint32_t)ny, cx, cy,
-                                                                cz, gx, gy);
+    if (nx * ny * nz == 0) return FZH_OK;
+    const bool wide = cx % 4 == 0 && ((uintptr_t)src | (uintptr_t)dst) % 16 == 0;  // (nx is a multiple of cx)
+    hipStream_t s = S(stream);
+    if (to_chunks && wide) launch_chunk_copy<true, float4>(s, src, dst, nx, ny, nz, cx, cy, cz);
+    else if (to_chunks) launch_chunk_copy<true, float>(s, src, dst, nx, ny, nz, cx, cy, cz);
+    else if (wide) launch_chunk_copy<false, float4>(s, src, dst, nx, ny, nz, cx, cy, cz);
+    else launch_chunk_copy<false, float>(s, src, dst, nx, ny, nz, cx, cy, cz);
     FZH_CHECK_LAUNCH("chunk_copy_kernel");
     return FZH_OK;
 }
