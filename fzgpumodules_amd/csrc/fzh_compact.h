@@ -32,19 +32,25 @@ struct CompactListT {
 };
 using CompactList = CompactListT<float>;
 
+template <typename V>
+inline CompactListT<V> compact_list(const PlaceDesc::List& l) {
+    return {static_cast<const V*>(l.s_val), l.s_idx, l.cnt, static_cast<V*>(l.val), l.idx, l.total, l.cap};
+}
+
 // Counts (of all lists) up to which the place kernel sums those before each
 // workgroup itself.  39 Ki counts (301 x 203 x 157 doubles): 4.4 us against
 // 12.8 + 4.5 us and a launch gap with a one-workgroup scan; past that the
 // longest sum outgrows the scan's launches.
 constexpr uint32_t COMPACT_INLINE = 65536;
 
-// excl: exclusive prefix (mod 2^32) of the NL*T counts, excl[NL*T] = sum
-// (INL: unused, the prefixes are summed in the kernel).
+// Workgroup `blk` of `nblk` of the placement.  excl: exclusive prefix (mod
+// 2^32) of the NL*T counts, excl[NL*T] = sum (INL: unused, the prefixes are
+// summed here).
 template <int NL, bool INL, typename V>
-__global__ void __launch_bounds__(256)
-place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, const uint32_t* __restrict__ excl) {
+__device__ __forceinline__ void place_tiles(const CompactListT<V>& L0, const CompactListT<V>& L1, uint32_t T, uint32_t E,
+                                            const uint32_t* __restrict__ excl, uint32_t blk, uint32_t nblk) {
     const int w = (int)wave_in_wg();
-    const uint32_t wave = blockIdx.x * 4 + (uint32_t)w;
+    const uint32_t wave = blk * 4 + (uint32_t)w;
     const int l = lane_id();
     const uint32_t tb = wave * 32;
     const uint32_t li = (uint32_t)l >> 5;
@@ -60,7 +66,7 @@ place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, con
         const uint32_t* lists[NL];
 #pragma unroll
         for (int k = 0; k < NL; k++) lists[k] = L0.cnt + (uint64_t)k * T;
-        wg256_sums_before_u32<NL>(lists, min(blockIdx.x * 128u, T), s_sum, before);
+        wg256_sums_before_u32<NL>(lists, min(blk * 128u, T), s_sum, before);
         const uint32_t h0 = (uint32_t)__builtin_amdgcn_readlane((int)inc, 31);  // list 0 part of the wave
         const uint32_t h1 = lane63(inc) - h0;                                    // list 1 part
         if (l == 0) {
@@ -74,7 +80,7 @@ place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, con
             p1 += s_wave[k][1];
         }
         ex = inc - c - (li ? h0 : 0u) + (li ? p1 : p0);
-        if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {  // the last workgroup ends at or past T
+        if (blk == nblk - 1 && threadIdx.x == 0) {  // the last workgroup ends at or past T
             uint32_t q0 = before[0], q1 = NL == 2 ? before[NL - 1] : 0u;
             for (int k = 0; k < 4; k++) {
                 q0 += s_wave[k][0];
@@ -126,13 +132,24 @@ place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, con
     }
 }
 
+template <int NL, bool INL, typename V>
+__global__ void __launch_bounds__(256)
+place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, const uint32_t* __restrict__ excl) {
+    place_tiles<NL, INL, V>(L0, L1, T, E, excl, blockIdx.x, gridDim.x);
+}
+
 // Compaction state: exclusive prefixes (2T + 1 u32) and the scan workspace.
 inline size_t compact_state_bytes(size_t T) {
     return align_up(4 * (2 * T + 1), 256) + scan_ws_bytes(2 * std::max<size_t>(T, 1));
 }
 
+// With `defer`, a placement that needs no scan is described there for a later
+// launch instead (defer->blocks workgroups of place_tiles<lists, true, V>);
+// otherwise it is launched and defer->blocks is 0.
 template <typename V>
-inline int launch_compact(hipStream_t s, void* state, size_t T, uint32_t E, CompactListT<V> L0, CompactListT<V>* L1) {
+inline int launch_compact(hipStream_t s, void* state, size_t T, uint32_t E, CompactListT<V> L0, CompactListT<V>* L1,
+                          PlaceDesc* defer = nullptr) {
+    if (defer) defer->blocks = 0;
     if (T == 0) return FZH_OK;
     const int nl = L1 ? 2 : 1;
     if (L1 && L1->cnt != L0.cnt + T) return fail(FZH_E_INVALID, "compact: second count list must follow the first");
@@ -142,6 +159,18 @@ inline int launch_compact(hipStream_t s, void* state, size_t T, uint32_t E, Comp
     if (!inl)
         if (int rc = scan_u32<true>(s, L0.cnt, excl, nl * T, nullptr, excl + nl * T, ws)) return rc;
     const unsigned blocks = (unsigned)cdiv(cdiv(T, 32), 4);
+    if (defer && inl) {
+        const CompactListT<V>* lists[2] = {&L0, L1};
+        for (int i = 0; i < nl; i++)
+            defer->list[i] = {lists[i]->s_val, lists[i]->s_idx, lists[i]->cnt, lists[i]->val,
+                              lists[i]->idx,   lists[i]->total, lists[i]->cap};
+        defer->T = (uint32_t)T;
+        defer->E = E;
+        defer->lists = (uint32_t)nl;
+        defer->value_bytes = sizeof(V);
+        defer->blocks = blocks;
+        return FZH_OK;
+    }
     auto* k = inl ? (L1 ? place_kernel<2, true, V> : place_kernel<1, true, V>)
                   : (L1 ? place_kernel<2, false, V> : place_kernel<1, false, V>);
     launch_k("place_kernel", k, dim3(blocks), dim3(256), 0, s, L0, L1 ? *L1 : CompactListT<V>{}, (uint32_t)T, E,

@@ -27,10 +27,44 @@ int zero_bytes(hipStream_t s, void* p, size_t n);
 // copy); others fall back to hipMemcpyAsync.
 int read_small(hipStream_t s, const void* d_src, size_t bytes, void* h_dst);
 
+// The placement of a forward predictor's outlier (and patch) lists, left to
+// the launch that encodes its codes: the encoder doesn't read the lists, so
+// the two run side by side.  blocks = 0: nothing was left.
+struct PlaceDesc {
+    struct List {
+        const void* s_val;
+        const uint32_t* s_idx;
+        const uint32_t* cnt;
+        void* val;
+        uint32_t* idx;
+        uint32_t* total;
+        uint64_t cap;
+    } list[2];
+    uint32_t T, E, lists, value_bytes, blocks;
+};
+// fzh_lorenzo_quant_fwd_f32, _strict_f32 and _f64 with such a description
+// (null: they place the lists themselves).
+int lorenzo_quant_fwd_f32(hipStream_t s, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz, float ebx2_r,
+                          const float* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes,
+                          float* d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count,
+                          size_t max_outliers, void* d_ws, size_t ws_bytes, PlaceDesc* defer);
+int lorenzo_quant_fwd_strict_f32(hipStream_t s, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz,
+                                 float ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes,
+                                 void* d_codes, float* d_outlier_err, uint32_t* d_outlier_idx,
+                                 uint32_t* d_outlier_count, size_t max_outliers, float eb, float ebx2,
+                                 const float* d_eb_params, float* d_patch_val, uint32_t* d_patch_idx,
+                                 uint32_t* d_patch_count, size_t max_patches, void* d_ws, size_t ws_bytes,
+                                 PlaceDesc* defer);
+int lorenzo_quant_fwd_f64(hipStream_t s, const double* d_in, size_t n, size_t nx, size_t ny, size_t nz, double ebx2_r,
+                          const double* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes,
+                          double* d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count,
+                          size_t max_outliers, void* d_ws, size_t ws_bytes, PlaceDesc* defer);
+
 // RZE encode without its pack launch: the encoder (and, past 4096 chunks,
 // the offset scan) run, and the pack step is described for a later launch
 // that also does the pipeline's concat and readback
-// (rze_pack_concat_readback), saving one launch per compress.
+// (rze_pack_concat_readback), saving one launch per compress.  place: a
+// predictor's placement to run in the encoder's launch, or null.
 struct RzePackDesc {
     const uint8_t* in;
     uint64_t nbytes;
@@ -44,7 +78,7 @@ struct RzePackDesc {
     uint64_t nshuf;
 };
 int rze_enc_prepare(hipStream_t s, const void* d_in, size_t nbytes, int sew, void* d_out, size_t out_cap,
-                    uint64_t* d_out_size, void* d_ws, size_t ws_bytes, RzePackDesc* desc);
+                    uint64_t* d_out_size, void* d_ws, size_t ws_bytes, const PlaceDesc* place, RzePackDesc* desc);
 int rze_pack_concat_readback(hipStream_t s, const RzePackDesc& d, const fzh_concat_slot* slots, int n, void* d_out,
                              void* d_copy, uint64_t out_cap, uint64_t* d_total, const fzh_readback_entry* entries,
                              int n_entries, void* d_mapped_dst);

@@ -93,6 +93,14 @@ std::unordered_map<std::string, size_t> LorenzoQuantStage<TI, TC>::getActualOutp
 template <typename TI, typename TC>
 void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                                         const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
+    const bool defer = std::exchange(defer_place_, false);
+    fzh::PlaceDesc* place = nullptr;
+    if (defer) {
+        static_assert(sizeof(fzh::PlaceDesc) <= sizeof(place_desc_), "placement description storage");
+        place = reinterpret_cast<fzh::PlaceDesc*>(place_desc_);
+        place->blocks = 0;
+    }
+    place_left_ = defer;
     if (is_inverse_) {
         if (inputs.size() < numPorts() || outputs.empty() || sizes.size() < numPorts())
             throw std::runtime_error("LorenzoQuantStage (inverse): Requires " + std::to_string(numPorts()) +
@@ -155,7 +163,7 @@ void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, co
     else if (nx * ny * nz > valid)
         throw std::runtime_error("LorenzoQuantStage: dims exceed the unpadded input");
     if constexpr (std::is_same_v<TI, double>) {
-        executeF64(stream, pool, inputs, outputs, n, valid, nx, ny, nz, max_out);
+        executeF64(stream, pool, inputs, outputs, n, valid, nx, ny, nz, max_out, place);
     } else {
         // Resolve the absolute bound (lorenzo_quant.cu:612-644).
         const float* d_r = nullptr;
@@ -185,20 +193,20 @@ void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, co
                                               : fzh_lorenzo_quant_fwd_ws_bytes(n, nx, ny, nz),
                    pool, stream);
         if (!config_.strict_error_bound) {
-            throwIfFzh(fzh_lorenzo_quant_fwd_f32(stream, (const float*)inputs[0], n, nx, ny, nz, r, d_r,
+            throwIfFzh(fzh::lorenzo_quant_fwd_f32(stream, (const float*)inputs[0], n, nx, ny, nz, r, d_r,
                                                  (uint32_t)config_.quant_radius, config_.zigzag_codes ? 1 : 0,
                                                  (int)sizeof(TC), outputs[0], (float*)outputs[1], (uint32_t*)outputs[2],
-                                                 (uint32_t*)outputs[3], max_out, ws_.ptr, ws_.bytes),
+                                                 (uint32_t*)outputs[3], max_out, ws_.ptr, ws_.bytes, place),
                        "LorenzoQuantStage");
         } else {
             const size_t pm = maxPatches(n);
             const float eb = computed_abs_eb_;
-            throwIfFzh(fzh_lorenzo_quant_fwd_strict_f32(
+            throwIfFzh(fzh::lorenzo_quant_fwd_strict_f32(
                            stream, (const float*)inputs[0], n, nx, ny, nz, r, d_r, (uint32_t)config_.quant_radius,
                            config_.zigzag_codes ? 1 : 0, (int)sizeof(TC), outputs[0], (float*)outputs[1],
                            (uint32_t*)outputs[2], (uint32_t*)outputs[3], max_out, eb, 2.0f * eb,
                            params_pending_ ? (const float*)params_.ptr : nullptr, (float*)outputs[4],
-                           (uint32_t*)outputs[5], (uint32_t*)outputs[6], pm, ws_.ptr, ws_.bytes),
+                           (uint32_t*)outputs[5], (uint32_t*)outputs[6], pm, ws_.ptr, ws_.bytes, place),
                        "LorenzoQuantStage (strict)");
             d_pcount_ptr_ = outputs[6];
             addReadback(d_pcount_ptr_, &h_pcount_, 4);
@@ -219,7 +227,7 @@ void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, co
 template <typename TI, typename TC>
 void LorenzoQuantStage<TI, TC>::executeF64(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                                            const std::vector<void*>& outputs, size_t n, size_t valid, size_t nx,
-                                           size_t ny, size_t nz, size_t max_out) {
+                                           size_t ny, size_t nz, size_t max_out, fzh::PlaceDesc* place) {
     if constexpr (std::is_same_v<TI, double>) {
         if (config_.strict_error_bound)
             throw std::runtime_error("LorenzoQuantStage: the strict error bound is available for float input only");
@@ -246,10 +254,10 @@ void LorenzoQuantStage<TI, TC>::executeF64(hipStream_t stream, MemoryPool* pool,
             addReadback(d_params, h_params_, sizeof(h_params_));
         }
         ws_.ensure(fzh_lorenzo_quant_fwd_f64_ws_bytes(n, nx, ny, nz), pool, stream);
-        throwIfFzh(fzh_lorenzo_quant_fwd_f64(stream, (const double*)inputs[0], n, nx, ny, nz, r, d_r,
+        throwIfFzh(fzh::lorenzo_quant_fwd_f64(stream, (const double*)inputs[0], n, nx, ny, nz, r, d_r,
                                              (uint32_t)config_.quant_radius, config_.zigzag_codes ? 1 : 0, (int)sizeof(TC),
                                              outputs[0], (double*)outputs[1], (uint32_t*)outputs[2], (uint32_t*)outputs[3],
-                                             max_out, ws_.ptr, ws_.bytes),
+                                             max_out, ws_.ptr, ws_.bytes, place),
                    "LorenzoQuantStage");
         d_count_ptr_ = outputs[3];
         addReadback(d_count_ptr_, &h_count_, 4);
@@ -385,6 +393,7 @@ void RZEStage::execute(hipStream_t stream, MemoryPool* pool, const std::vector<v
         throw std::runtime_error("RZEStage: only chunk_size == 16384 is currently supported; got " + std::to_string(chunk_size_));
     if (levels_ != 4)
         throw std::runtime_error("RZEStage: only levels == 4 is currently supported; got " + std::to_string((int)levels_));
+    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
     small_.ensure(256, pool, stream);
     clearReadbacks();
     size_pending_ = status_pending_ = false;
@@ -398,7 +407,7 @@ void RZEStage::execute(hipStream_t stream, MemoryPool* pool, const std::vector<v
         if (defer_pack_) {
             throwIfFzh(fzh::rze_enc_prepare(stream, inputs[0], in_bytes, pre_shuffle_, outputs[0],
                                             fzh_rze_enc_bound(in_bytes), (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes,
-                                            reinterpret_cast<fzh::RzePackDesc*>(pack_desc_)),
+                                            place, reinterpret_cast<fzh::RzePackDesc*>(pack_desc_)),
                        "RZEStage");
             pack_deferred_ = true;
         } else if (pre_shuffle_)

@@ -709,7 +709,7 @@ struct PatchOut {
 template <typename TCode, bool STRICT>
 int launch_fwd(hipStream_t s, const float* in, size_t n, size_t nx, size_t ny, size_t nz, float r,
                const float* d_r, uint32_t radius, int zz, void* codes, float* oerr, uint32_t* oidx,
-               uint32_t* ocount, size_t max_out, void* ws, size_t ws_bytes, const PatchOut& po) {
+               uint32_t* ocount, size_t max_out, void* ws, size_t ws_bytes, const PatchOut& po, PlaceDesc* defer) {
     const FwdWs L = fwd_layout(n, nx, ny, nz, STRICT);
     if (ws_bytes < L.total) return fail(FZH_E_CAPACITY, "lorenzo fwd: workspace too small");
     const size_t T = L.T;
@@ -752,8 +752,7 @@ int launch_fwd(hipStream_t s, const float* in, size_t n, size_t nx, size_t ny, s
     FZH_CHECK_LAUNCH("lorenzo fwd");
     CompactList L0{tl.err, tl.idx, tl.cnt, oerr, oidx, ocount, max_out};
     CompactList L1{tl.pval, tl.pidx, tl.pcnt, po.val, po.idx, po.count, po.cap};
-    if (int rc = launch_compact<float>(s, w + L.o_ctx, T, (uint32_t)L.E, L0, STRICT ? &L1 : nullptr)) return rc;
-    return FZH_OK;
+    return launch_compact<float>(s, w + L.o_ctx, T, (uint32_t)L.E, L0, STRICT ? &L1 : nullptr, defer);
 }
 
 // Inverse, part 2: the tiles, with the binned outliers of part 1.
@@ -872,22 +871,12 @@ int vb_scratch_address(hipStream_t s, float2** out) {
 }  // namespace
 }  // namespace fzh
 
-using namespace fzh;
+namespace fzh {
 
-extern "C" {
-
-size_t fzh_lorenzo_quant_fwd_ws_bytes(size_t n, size_t nx, size_t ny, size_t nz) {
-    return fwd_layout(n, nx, ny, nz, false).total;
-}
-
-size_t fzh_lorenzo_quant_fwd_strict_ws_bytes(size_t n, size_t nx, size_t ny, size_t nz) {
-    return fwd_layout(n, nx, ny, nz, true).total;
-}
-
-int fzh_lorenzo_quant_fwd_f32(void* stream, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz,
-                              float ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag,
-                              int code_bytes, void* d_codes, float* d_outlier_err, uint32_t* d_outlier_idx,
-                              uint32_t* d_outlier_count, size_t max_outliers, void* d_ws, size_t ws_bytes) {
+int lorenzo_quant_fwd_f32(hipStream_t s, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz, float ebx2_r,
+                          const float* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes, float*
+                          d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count, size_t max_outliers,
+                          void* d_ws, size_t ws_bytes, PlaceDesc* defer) {
     if (int rc = check_dims(n, nx, ny, nz, "lorenzo fwd")) return rc;
     if (n == 0) return FZH_OK;
     if (!d_in || !d_codes || !d_outlier_count) return fail(FZH_E_INVALID, "lorenzo fwd: null pointer");
@@ -898,24 +887,24 @@ int fzh_lorenzo_quant_fwd_f32(void* stream, const float* d_in, size_t n, size_t 
     const PatchOut none{};
     switch (code_bytes) {
     case 1:
-        return launch_fwd<uint8_t, false>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
+        return launch_fwd<uint8_t, false>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
                                           d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws,
-                                          ws_bytes, none);
+                                          ws_bytes, none, defer);
     case 2:
-        return launch_fwd<uint16_t, false>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag,
+        return launch_fwd<uint16_t, false>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag,
                                            d_codes, d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers,
-                                           d_ws, ws_bytes, none);
+                                           d_ws, ws_bytes, none, defer);
     default:
         return fail(FZH_E_INVALID, "lorenzo fwd: code_bytes must be 1 or 2");
     }
 }
 
-int fzh_lorenzo_quant_fwd_strict_f32(void* stream, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz,
-                                     float ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag,
-                                     int code_bytes, void* d_codes, float* d_outlier_err, uint32_t* d_outlier_idx,
-                                     uint32_t* d_outlier_count, size_t max_outliers, float eb, float ebx2,
-                                     const float* d_eb_params, float* d_patch_val, uint32_t* d_patch_idx,
-                                     uint32_t* d_patch_count, size_t max_patches, void* d_ws, size_t ws_bytes) {
+int lorenzo_quant_fwd_strict_f32(hipStream_t s, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz, float
+                                 ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void*
+                                 d_codes, float* d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count,
+                                 size_t max_outliers, float eb, float ebx2, const float* d_eb_params, float*
+                                 d_patch_val, uint32_t* d_patch_idx, uint32_t* d_patch_count, size_t max_patches,
+                                 void* d_ws, size_t ws_bytes, PlaceDesc* defer) {
     if (int rc = check_dims(n, nx, ny, nz, "lorenzo fwd (strict)")) return rc;
     if (n == 0) return FZH_OK;
     if (!d_in || !d_codes || !d_outlier_count || !d_patch_count) return fail(FZH_E_INVALID, "lorenzo fwd (strict): null pointer");
@@ -935,16 +924,51 @@ int fzh_lorenzo_quant_fwd_strict_f32(void* stream, const float* d_in, size_t n, 
     po.cap = max_patches;
     switch (code_bytes) {
     case 1:
-        return launch_fwd<uint8_t, true>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
+        return launch_fwd<uint8_t, true>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
                                          d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws,
-                                         ws_bytes, po);
+                                         ws_bytes, po, defer);
     case 2:
-        return launch_fwd<uint16_t, true>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag,
+        return launch_fwd<uint16_t, true>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag,
                                           d_codes, d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers,
-                                          d_ws, ws_bytes, po);
+                                          d_ws, ws_bytes, po, defer);
     default:
         return fail(FZH_E_INVALID, "lorenzo fwd (strict): code_bytes must be 1 or 2");
     }
+}
+
+}  // namespace fzh
+
+using namespace fzh;
+
+extern "C" {
+
+size_t fzh_lorenzo_quant_fwd_ws_bytes(size_t n, size_t nx, size_t ny, size_t nz) {
+    return fwd_layout(n, nx, ny, nz, false).total;
+}
+
+size_t fzh_lorenzo_quant_fwd_strict_ws_bytes(size_t n, size_t nx, size_t ny, size_t nz) {
+    return fwd_layout(n, nx, ny, nz, true).total;
+}
+
+int fzh_lorenzo_quant_fwd_f32(void* stream, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz,
+                              float ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag,
+                              int code_bytes, void* d_codes, float* d_outlier_err, uint32_t* d_outlier_idx,
+                              uint32_t* d_outlier_count, size_t max_outliers, void* d_ws, size_t ws_bytes) {
+    return lorenzo_quant_fwd_f32(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, code_bytes,
+                                 d_codes, d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws, ws_bytes,
+                                 nullptr);
+}
+
+int fzh_lorenzo_quant_fwd_strict_f32(void* stream, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz,
+                                     float ebx2_r, const float* d_ebx2_r, uint32_t radius, int zigzag,
+                                     int code_bytes, void* d_codes, float* d_outlier_err, uint32_t* d_outlier_idx,
+                                     uint32_t* d_outlier_count, size_t max_outliers, float eb, float ebx2,
+                                     const float* d_eb_params, float* d_patch_val, uint32_t* d_patch_idx,
+                                     uint32_t* d_patch_count, size_t max_patches, void* d_ws, size_t ws_bytes) {
+    return lorenzo_quant_fwd_strict_f32(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, code_bytes,
+                                        d_codes, d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, eb,
+                                        ebx2, d_eb_params, d_patch_val, d_patch_idx, d_patch_count, max_patches, d_ws,
+                                        ws_bytes, nullptr);
 }
 
 int fzh_lorenzo_apply_patches(void* stream, float* d_out, const float* d_patch_val, const uint32_t* d_patch_idx,

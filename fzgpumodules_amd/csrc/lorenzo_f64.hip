@@ -640,7 +640,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 template <typename TCode>
 int launch_fwd64(hipStream_t s, const double* in, size_t n, size_t nx, size_t ny, size_t nz, double r,
                  const double* d_r, uint32_t radius, int zz, void* codes, double* oerr, uint32_t* oidx,
-                 uint32_t* ocount, size_t max_out, void* ws, size_t ws_bytes) {
+                 uint32_t* ocount, size_t max_out, void* ws, size_t ws_bytes, PlaceDesc* defer) {
     const FwdWs L = fwd_layout(n, nx, ny, nz, false, sizeof(double));
     if (ws_bytes < L.total) return fail(FZH_E_CAPACITY, "lorenzo fwd (f64): workspace too small");
     const size_t T = L.T;
@@ -670,7 +670,7 @@ int launch_fwd64(hipStream_t s, const double* in, size_t n, size_t nx, size_t ny
 #undef FZH_LZ64_FWD
     FZH_CHECK_LAUNCH("lorenzo fwd (f64)");
     CompactListT<double> L0{tl.err, tl.idx, tl.cnt, oerr, oidx, ocount, max_out};
-    return launch_compact<double>(s, w + L.o_ctx, T, (uint32_t)L.E, L0, nullptr);
+    return launch_compact<double>(s, w + L.o_ctx, T, (uint32_t)L.E, L0, nullptr, defer);
 }
 
 template <typename TCode>
@@ -718,6 +718,33 @@ int launch_inv64(hipStream_t s, const void* codes, size_t n, size_t nx, size_t n
 }  // namespace
 }  // namespace fzh
 
+namespace fzh {
+
+int lorenzo_quant_fwd_f64(hipStream_t s, const double* d_in, size_t n, size_t nx, size_t ny, size_t nz, double ebx2_r,
+                          const double* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes, double*
+                          d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count, size_t max_outliers,
+                          void* d_ws, size_t ws_bytes, PlaceDesc* defer) {
+    if (code_bytes != 2 && code_bytes != 4) return fail(FZH_E_INVALID, "lorenzo fwd (f64): code_bytes must be 2 or 4");
+    if (int rc = check_dims(n, nx, ny, nz, "lorenzo fwd (f64)")) return rc;
+    if (n == 0) {
+        if (d_outlier_count) return zero_bytes(s, d_outlier_count, 4);
+        return FZH_OK;
+    }
+    if (!d_in || !d_codes || !d_outlier_count || !d_ws || (max_outliers > 0 && (!d_outlier_err || !d_outlier_idx)))
+        return fail(FZH_E_INVALID, "lorenzo fwd (f64): null pointer");
+    if (!aligned16(d_in) || !aligned16(d_codes))
+        return fail(FZH_E_INVALID, "lorenzo fwd (f64): input and codes must be 16-byte aligned");
+    return code_bytes == 2
+               ? launch_fwd64<uint16_t>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
+                                        d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws,
+                                        ws_bytes, defer)
+               : launch_fwd64<uint32_t>(s, d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
+                                        d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws,
+                                        ws_bytes, defer);
+}
+
+}  // namespace fzh
+
 using namespace fzh;
 
 extern "C" {
@@ -730,21 +757,9 @@ int fzh_lorenzo_quant_fwd_f64(void* stream, const double* d_in, size_t n, size_t
                               double ebx2_r, const double* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes,
                               void* d_codes, double* d_outlier_err, uint32_t* d_outlier_idx,
                               uint32_t* d_outlier_count, size_t max_outliers, void* d_ws, size_t ws_bytes) {
-    if (code_bytes != 2 && code_bytes != 4) return fail(FZH_E_INVALID, "lorenzo fwd (f64): code_bytes must be 2 or 4");
-    if (int rc = check_dims(n, nx, ny, nz, "lorenzo fwd (f64)")) return rc;
-    if (n == 0) {
-        if (d_outlier_count) return zero_bytes(S(stream), d_outlier_count, 4);
-        return FZH_OK;
-    }
-    if (!d_in || !d_codes || !d_outlier_count || !d_ws || (max_outliers > 0 && (!d_outlier_err || !d_outlier_idx)))
-        return fail(FZH_E_INVALID, "lorenzo fwd (f64): null pointer");
-    if (!aligned16(d_in) || !aligned16(d_codes))
-        return fail(FZH_E_INVALID, "lorenzo fwd (f64): input and codes must be 16-byte aligned");
-    return code_bytes == 2
-               ? launch_fwd64<uint16_t>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
-                                        d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws, ws_bytes)
-               : launch_fwd64<uint32_t>(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, d_codes,
-                                        d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws, ws_bytes);
+    return lorenzo_quant_fwd_f64(S(stream), d_in, n, nx, ny, nz, ebx2_r, d_ebx2_r, radius, zigzag, code_bytes,
+                                 d_codes, d_outlier_err, d_outlier_idx, d_outlier_count, max_outliers, d_ws, ws_bytes,
+                                 nullptr);
 }
 
 size_t fzh_lorenzo_quant_inv_f64_ws_bytes(size_t n, size_t nx, size_t ny, size_t nz, size_t max_outliers) {

@@ -131,6 +131,12 @@ class Stage {
     // (aligned and as large as outputs[0]).  False if the stage cannot.
     virtual bool copyOutputTo(void* d_copy) { (void)d_copy; return false; }
 
+    // Lets the next forward execute() leave the placement of its small outputs
+    // (not output 0) to the launch that encodes output 0, which gets
+    // deferredPlacement() (an fzh::PlaceDesc; null: nothing was left).
+    virtual void deferPlacement(bool on) { (void)on; }
+    virtual const void* deferredPlacement() const { return nullptr; }
+
     virtual DeviceSize getDeviceOutputSize(int index) const { (void)index; return {}; }
 
     // Device values postStreamSync() needs, registered by execute().  A

@@ -27,6 +27,10 @@
 #include "fz/mempool.h"
 #include "fz/stage.h"
 
+namespace fzh {
+struct PlaceDesc;
+}
+
 namespace fz {
 
 enum class ErrorBoundMode : uint8_t { ABS = 0, REL = 1, NOA = 2 };
@@ -115,6 +119,8 @@ class LorenzoQuantStage : public Stage {
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
+    void deferPlacement(bool on) override { defer_place_ = on; }
+    const void* deferredPlacement() const override { return place_left_ ? place_desc_ : nullptr; }
 
     std::string getName() const override { return "LorenzoQuant"; }
     size_t getNumInputs() const override { return is_inverse_ ? numPorts() : 1; }
@@ -209,9 +215,11 @@ class LorenzoQuantStage : public Stage {
     void resolveDims(size_t n, size_t& nx, size_t& ny, size_t& nz) const;
     void executeF64(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                     const std::vector<void*>& outputs, size_t n, size_t valid, size_t nx, size_t ny, size_t nz,
-                    size_t max_out);
+                    size_t max_out, fzh::PlaceDesc* place);
 
     Config config_;
+    bool defer_place_ = false, place_left_ = false;
+    alignas(8) unsigned char place_desc_[136] = {};
     bool is_inverse_ = false;
     size_t inv_limit_ = 0;  // elements of the next inverse execute() (0: all)
     std::vector<size_t> actual_output_sizes_ = std::vector<size_t>(4, 0), saved_output_sizes_;
@@ -303,6 +311,7 @@ class RZEStage : public Stage {
     // concat + readback launch, and deferredPack() describes it (until the
     // next execute).
     void setDeferPack(bool on) { defer_pack_ = on; }
+    void setPlacement(const void* desc) { place_desc_ = desc; }  // for the next forward execute()
     const void* deferredPack() const { return pack_deferred_ ? pack_desc_ : nullptr; }
 
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
@@ -343,6 +352,7 @@ class RZEStage : public Stage {
     bool is_inverse_ = false;
     int pre_shuffle_ = 0;
     bool defer_pack_ = false, pack_deferred_ = false;
+    const void* place_desc_ = nullptr;
     alignas(8) unsigned char pack_desc_[96] = {};
     uint32_t chunk_size_ = 16384;
     uint8_t levels_ = 4;
