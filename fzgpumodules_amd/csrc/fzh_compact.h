@@ -11,6 +11,8 @@
 // waits on another.
 #pragma once
 
+#include <type_traits>
+
 #include "fzh_scan.h"
 
 namespace fzh {
@@ -136,6 +138,17 @@ template <int NL, bool INL, typename V>
 __global__ void __launch_bounds__(256)
 place_kernel(CompactListT<V> L0, CompactListT<V> L1, uint32_t T, uint32_t E, const uint32_t* __restrict__ excl) {
     place_tiles<NL, INL, V>(L0, L1, T, E, excl, blockIdx.x, gridDim.x);
+}
+
+// f(NL as an integral constant, L0, L1) for the lists left in p.
+template <typename F>
+inline void with_placement(const PlaceDesc& p, F f) {
+    if (p.value_bytes == 8)  // doubles have no patches
+        f(std::integral_constant<int, 1>{}, compact_list<double>(p.list[0]), CompactListT<double>{});
+    else if (p.lists == 1)
+        f(std::integral_constant<int, 1>{}, compact_list<float>(p.list[0]), CompactList{});
+    else
+        f(std::integral_constant<int, 2>{}, compact_list<float>(p.list[0]), compact_list<float>(p.list[1]));
 }
 
 // Compaction state: exclusive prefixes (2T + 1 u32) and the scan workspace.

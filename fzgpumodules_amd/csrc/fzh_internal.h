@@ -42,7 +42,8 @@ struct PlaceDesc {
     } list[2];
     uint32_t T, E, lists, value_bytes, blocks;
 };
-// fzh_lorenzo_quant_fwd_f32, _strict_f32 and _f64 with such a description
+// fzh_lorenzo_quant_fwd_f32, _strict_f32 and _f64 and fzh_quant_abs_fwd_f32 with
+// such a description
 // (null: they place the lists themselves).
 int lorenzo_quant_fwd_f32(hipStream_t s, const float* d_in, size_t n, size_t nx, size_t ny, size_t nz, float ebx2_r,
                           const float* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes,
@@ -59,6 +60,10 @@ int lorenzo_quant_fwd_f64(hipStream_t s, const double* d_in, size_t n, size_t nx
                           const double* d_ebx2_r, uint32_t radius, int zigzag, int code_bytes, void* d_codes,
                           double* d_outlier_err, uint32_t* d_outlier_idx, uint32_t* d_outlier_count,
                           size_t max_outliers, void* d_ws, size_t ws_bytes, PlaceDesc* defer);
+
+int quant_abs_fwd_f32(hipStream_t s, const float* d_in, size_t n, float ebx2_r, float threshold, uint32_t radius,
+                      int zigzag, int code_bytes, void* d_codes, float* d_oval, uint32_t* d_oidx, uint32_t* d_ocount,
+                      size_t max_outliers, void* d_ws, size_t ws_bytes, PlaceDesc* defer);
 
 // RZE encode without its pack launch: the encoder (and, past 4096 chunks,
 // the offset scan) run, and the pack step is described for a later launch
@@ -102,9 +107,11 @@ int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_
 
 // fzh_rle_enc and fzh_huffman_encode (fine: fzh_huffman_encode_fine) with a
 // second destination of the stream: d_copy null, or aligned and as large as
-// d_out.
+// d_out.  place: a predictor's placement to run in the first launch, or null.
 int rle_enc(hipStream_t s, const void* d_in, size_t n, int elem_bytes, void* d_out, size_t out_cap, void* d_copy,
-            uint64_t* d_out_size, void* d_ws, size_t ws_bytes);
+            uint64_t* d_out_size, void* d_ws, size_t ws_bytes, const PlaceDesc* place);
+int max_u32(hipStream_t s, const void* d_in, size_t n, int elem_bytes, uint32_t* d_max, void* d_ws, size_t ws_bytes,
+            const PlaceDesc* place);
 int huffman_encode(hipStream_t s, bool fine, const void* d_in, size_t n, int elem_bytes, uint32_t bklen,
                    const uint32_t* d_bk4, const uint8_t* d_revbook, void* d_out, size_t out_cap, void* d_copy,
                    uint64_t* d_out_size, void* d_ws, size_t ws_bytes);

@@ -348,19 +348,16 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
             hipck(hipEventRecord(e0, stream), "hipEventRecord");
         }
         // a predictor's outlier lists, unless a stage reads them, are placed in
-        // the launch of the encoder with the deferred pack that reads its codes
-        const auto left_to = [&](const Node& pred) {
-            const Node& enc = nodes_[buffers_[outputs_[0]].producer];
-            if (pred.out_buf[0] != (enc.fused_from >= 0 ? nodes_[enc.fused_from].in_buf : enc.in_buf)) return false;
-            for (size_t i = 1; i < pred.out_buf.size(); i++)
-                if (buffers_[pred.out_buf[i]].consumer >= 0) return false;
-            return true;
-        };
-        n.stage->deferPlacement(defer_rze && left_to(n));
-        if (defer_rze && n.stage == defer_rze) {
-            const int p = buffers_[n.fused_from >= 0 ? nodes_[n.fused_from].in_buf : n.in_buf].producer;
-            defer_rze->setPlacement(p >= 0 ? nodes_[p].stage->deferredPlacement() : nullptr);
-        }
+        // a launch of the encoder that reads its codes, where that takes them
+        n.stage->deferPlacement([&] {
+            int c = buffers_[n.out_buf[0]].consumer;
+            for (size_t i = 1; i < n.out_buf.size(); i++)
+                if (buffers_[n.out_buf[i]].consumer >= 0) return false;
+            if (c >= 0 && nodes_[c].elided) c = buffers_[nodes_[c].out_buf[0]].consumer;
+            return c >= 0 && nodes_[c].stage->takesPlacement();
+        }());
+        const int pred = buffers_[n.fused_from >= 0 ? nodes_[n.fused_from].in_buf : n.in_buf].producer;
+        n.stage->setPlacement(pred >= 0 ? nodes_[pred].stage->deferredPlacement() : nullptr);
         // the stage that writes the concat's first slot may store it in the
         // caller's buffer too, unless a later stage could still read an input
         // that lies in it

@@ -93,14 +93,13 @@ std::unordered_map<std::string, size_t> LorenzoQuantStage<TI, TC>::getActualOutp
 template <typename TI, typename TC>
 void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                                         const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
-    const bool defer = std::exchange(defer_place_, false);
     fzh::PlaceDesc* place = nullptr;
-    if (defer) {
+    place_left_ = std::exchange(defer_place_, false);
+    if (place_left_) {
         static_assert(sizeof(fzh::PlaceDesc) <= sizeof(place_desc_), "placement description storage");
         place = reinterpret_cast<fzh::PlaceDesc*>(place_desc_);
         place->blocks = 0;
     }
-    place_left_ = defer;
     if (is_inverse_) {
         if (inputs.size() < numPorts() || outputs.empty() || sizes.size() < numPorts())
             throw std::runtime_error("LorenzoQuantStage (inverse): Requires " + std::to_string(numPorts()) +
@@ -463,6 +462,7 @@ template <typename T>
 void RLEStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                           const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
     void* copy = std::exchange(copy_out_, nullptr);
+    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
     if (inputs.empty() || outputs.empty() || sizes.empty()) throw std::runtime_error("RLEStage: Invalid inputs/outputs");
     small_.ensure(256, pool, stream);
     clearReadbacks();
@@ -472,7 +472,7 @@ void RLEStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vecto
         cached_num_elements_ = (uint32_t)n;
         ws_.ensure(fzh_rle_enc_ws_bytes(n), pool, stream);
         throwIfFzh(fzh::rle_enc(stream, inputs[0], n, (int)sizeof(T), outputs[0], fzh_rle_enc_bound(n, sizeof(T)), copy,
-                                (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes),
+                                (uint64_t*)small_.ptr, ws_.ptr, ws_.bytes, place),
                    "RLEStage");
         actual_output_size_ = fzh_rle_enc_bound(n, sizeof(T));
         size_pending_ = true;
@@ -661,6 +661,13 @@ std::unordered_map<std::string, size_t> QuantizerStage<TI, TC>::getActualOutputS
 template <typename TI, typename TC>
 void QuantizerStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                                      const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
+    fzh::PlaceDesc* place = nullptr;
+    place_left_ = std::exchange(defer_place_, false);
+    if (place_left_) {
+        static_assert(sizeof(fzh::PlaceDesc) <= sizeof(place_desc_), "placement description storage");
+        place = reinterpret_cast<fzh::PlaceDesc*>(place_desc_);
+        place->blocks = 0;
+    }
     if (isInplaceMode()) {  // quantizer.cu:396-452 / 492-615, one port each way
         if (!config_.zigzag_codes)
             throw std::runtime_error("QuantizerStage: setInplaceOutliers(true) requires setZigzagCodes(true)");
@@ -746,10 +753,10 @@ void QuantizerStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, const
         return;
     }
     ws_.ensure(256 + fzh_quant_abs_fwd_ws_bytes(n), pool, stream);
-    throwIfFzh(fzh_quant_abs_fwd_f32(stream, (const float*)inputs[0], n, r, config_.outlier_threshold,
-                                     (uint32_t)config_.quant_radius, config_.zigzag_codes ? 1 : 0, (int)sizeof(TC),
-                                     outputs[0], (float*)outputs[1], (uint32_t*)outputs[2], (uint32_t*)outputs[3], m,
-                                     (uint8_t*)ws_.ptr + 256, ws_.bytes - 256),
+    throwIfFzh(fzh::quant_abs_fwd_f32(stream, (const float*)inputs[0], n, r, config_.outlier_threshold,
+                                      (uint32_t)config_.quant_radius, config_.zigzag_codes ? 1 : 0, (int)sizeof(TC),
+                                      outputs[0], (float*)outputs[1], (uint32_t*)outputs[2], (uint32_t*)outputs[3], m,
+                                      (uint8_t*)ws_.ptr + 256, ws_.bytes - 256, place),
                "QuantizerStage");
     d_count_ptr_ = outputs[3];
     addReadback(d_count_ptr_, &h_count_, 4);
@@ -820,6 +827,7 @@ template class QuantizerStage<float, uint32_t>;
 template <typename T>
 void BitpackStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                               const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
+    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
     if (inputs.empty() || outputs.empty() || sizes.empty())
         throw std::runtime_error("BitpackStage: inputs, outputs, and sizes must be non-empty");
     if (!is_inverse_) {
@@ -828,8 +836,8 @@ void BitpackStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::v
         if (n == 0) { actual_output_size_ = 0; return; }
         if (auto_detect_) {
             ws_.ensure(256 + fzh_max_u32_ws_bytes(), pool, stream);
-            throwIfFzh(fzh_max_u32(stream, inputs[0], n, (int)sizeof(T), (uint32_t*)ws_.ptr, (uint8_t*)ws_.ptr + 256,
-                                   ws_.bytes - 256),
+            throwIfFzh(fzh::max_u32(stream, inputs[0], n, (int)sizeof(T), (uint32_t*)ws_.ptr, (uint8_t*)ws_.ptr + 256,
+                                    ws_.bytes - 256, place),
                        "BitpackStage max");
             uint32_t mx = 0;
             throwIfFzh(fzh::read_small(stream, ws_.ptr, 4, &mx), "BitpackStage max readback");

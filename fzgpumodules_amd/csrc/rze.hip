@@ -104,16 +104,11 @@ void launch_rze_enc(hipStream_t s, const RzeEncArgs& a, const PlaceDesc* p) {
         launch_k("rze_enc_kernel", rze_enc_kernel<SEW>, dim3(a.nc), dim3(256), 0, s, a);
         return;
     }
-    const dim3 grid(p->blocks + a.nc);
-    if (p->value_bytes == 8)
-        launch_k("rze_enc_place_kernel", rze_enc_place_kernel<SEW, 1, double>, grid, dim3(256), 0, s, a,
-                 compact_list<double>(p->list[0]), CompactListT<double>{}, p->T, p->E, p->blocks);
-    else if (p->lists == 1)
-        launch_k("rze_enc_place_kernel", rze_enc_place_kernel<SEW, 1, float>, grid, dim3(256), 0, s, a,
-                 compact_list<float>(p->list[0]), CompactList{}, p->T, p->E, p->blocks);
-    else
-        launch_k("rze_enc_place_kernel", rze_enc_place_kernel<SEW, 2, float>, grid, dim3(256), 0, s, a,
-                 compact_list<float>(p->list[0]), compact_list<float>(p->list[1]), p->T, p->E, p->blocks);
+    with_placement(*p, [&](auto nl, auto L0, auto L1) {
+        using V = std::remove_pointer_t<decltype(L0.val)>;
+        launch_k("rze_enc_place_kernel", rze_enc_place_kernel<SEW, decltype(nl)::value, V>, dim3(p->blocks + a.nc),
+                 dim3(256), 0, s, a, L0, L1, p->T, p->E, p->blocks);
+    });
 }
 
 // Places chunk c at [8 + 4 nc + offs[c]) of the stream, one workgroup per

@@ -136,6 +136,10 @@ class Stage {
     // deferredPlacement() (an fzh::PlaceDesc; null: nothing was left).
     virtual void deferPlacement(bool on) { (void)on; }
     virtual const void* deferredPlacement() const { return nullptr; }
+    // The encoder's side: whether its next forward execute() would run such a
+    // placement in one of its launches, and the placement (null: none).
+    virtual bool takesPlacement() const { return false; }
+    virtual void setPlacement(const void* desc) { (void)desc; }
 
     virtual DeviceSize getDeviceOutputSize(int index) const { (void)index; return {}; }
 

@@ -311,7 +311,8 @@ class RZEStage : public Stage {
     // concat + readback launch, and deferredPack() describes it (until the
     // next execute).
     void setDeferPack(bool on) { defer_pack_ = on; }
-    void setPlacement(const void* desc) { place_desc_ = desc; }  // for the next forward execute()
+    bool takesPlacement() const override { return defer_pack_; }
+    void setPlacement(const void* desc) override { place_desc_ = desc; }
     const void* deferredPack() const { return pack_deferred_ ? pack_desc_ : nullptr; }
 
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
@@ -381,6 +382,8 @@ class RLEStage : public Stage {
     void setInverse(bool inv) override { is_inverse_ = inv; }
     bool isInverse() const override { return is_inverse_; }
     bool copyOutputTo(void* d_copy) override { copy_out_ = d_copy; return true; }
+    bool takesPlacement() const override { return !is_inverse_; }
+    void setPlacement(const void* desc) override { place_desc_ = desc; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -414,6 +417,7 @@ class RLEStage : public Stage {
     void restoreState() override { cached_num_elements_ = saved_n_; actual_output_size_ = saved_out_; }
 
   private:
+    const void* place_desc_ = nullptr;
     void* copy_out_ = nullptr;  // second destination of the next forward execute()
     bool is_inverse_ = false;
     uint32_t cached_num_elements_ = 0, saved_n_ = 0;
@@ -566,6 +570,8 @@ class QuantizerStage : public Stage {
     };
     explicit QuantizerStage(const Config& c = Config()) : config_(c) {}
 
+    void deferPlacement(bool on) override { defer_place_ = on; }
+    const void* deferredPlacement() const override { return place_left_ ? place_desc_ : nullptr; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -619,6 +625,8 @@ class QuantizerStage : public Stage {
     size_t getMaxHeaderSize(size_t) const override { return sizeof(QuantizerConfig); }
 
   private:
+    bool defer_place_ = false, place_left_ = false;
+    alignas(8) unsigned char place_desc_[136] = {};
     bool isInplaceMode() const { return config_.inplace_outliers && config_.eb_mode != ErrorBoundMode::REL; }
     size_t maxOutliers(size_t n) const { return (size_t)std::ceil((double)n * config_.outlier_capacity); }
     Config config_;
@@ -656,6 +664,8 @@ class BitpackStage : public Stage {
     bool isAutoDetect() const { return auto_detect_; }
     bool isGraphCompatible() const override { return !auto_detect_ || is_inverse_; }
 
+    bool takesPlacement() const override { return !is_inverse_ && auto_detect_; }
+    void setPlacement(const void* desc) override { place_desc_ = desc; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     std::string getName() const override { return "Bitpack"; }
@@ -698,6 +708,7 @@ class BitpackStage : public Stage {
     }
 
   private:
+    const void* place_desc_ = nullptr;
     bool is_inverse_ = false, auto_detect_ = false;
     uint8_t nbits_ = 8 * sizeof(T);
     size_t num_elements_ = 0, actual_output_size_ = 0;

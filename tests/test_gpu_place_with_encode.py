@@ -1,9 +1,9 @@
-"""Outlier and patch lists that the RZE encoder's launch places: whole
-containers against the same chain with its stages unfused (which places them in
-a launch of their own), and the lists against another coder's chain, for each
-code width, both value types, tile counts around a workgroup's 128 and past the
-limit of the kernel's own sums, graph replays, and a chain whose indices feed
-another stage."""
+"""Outlier and patch lists that an encoder's launch places: RZE containers
+against the same chain with its stages unfused and bit packing of a detected
+width against a given one (which place the lists in a launch of their own), the
+RLE chain's lists against those, for each code width, both value types, tile
+counts around a workgroup's 128 and past the limit of the kernel's own sums,
+graph replays, and a chain whose indices feed another stage."""
 import numpy as np
 import pytest
 
@@ -13,8 +13,12 @@ pytestmark = pytest.mark.gpu
 def _pipe(dims, coder, cb=2, dtype="f32", strict=False, fused=True, index_stage=False):
     from fzgpumodules_amd.pipeline import Pipeline
     p = Pipeline(int(np.prod(dims)) * (8 if dtype == "f64" else 4))
-    a = p.add_lorenzo(1e-3, mode="ABS", quant_radius=100 if cb == 1 else 512, outlier_capacity=0.5, zigzag=True,
-                      code_bytes=cb, dtype=dtype)
+    if dtype == "quantizer":
+        a = p.add_quantizer(1e-3, mode="ABS", quant_radius=100 if cb == 1 else 512, outlier_capacity=0.5, zigzag=True,
+                            code_bytes=cb)
+    else:
+        a = p.add_lorenzo(1e-3, mode="ABS", quant_radius=100 if cb == 1 else 512, outlier_capacity=0.5, zigzag=True,
+                          code_bytes=cb, dtype=dtype)
     if strict:
         p.set_strict(a, True, 0.2)
     if coder == "bitshuffle":
@@ -23,8 +27,10 @@ def _pipe(dims, coder, cb=2, dtype="f32", strict=False, fused=True, index_stage=
         p.connect(p.add_rze(16384, 4), b)
     elif coder == "rze":
         p.connect(p.add_rze(16384, 4), a, "codes")
-    else:
+    elif coder == "rle":
         p.connect(p.add_rle(cb), a, "codes")
+    else:
+        p.connect(p.add_bitpack(cb, 0 if coder == "pack" else 8 * cb), a, "codes")
     if index_stage:
         p.connect(p.add_rle(4), a, "outlier_indices")
     p.set_dims(*dims)
@@ -70,6 +76,22 @@ def test_lists_with_the_encoder(dims, kind):
     assert np.array_equal(blobs[0], blobs[1])
     with _pipe(dims, "rle", cb, dtype, strict) as p:
         assert _slots(p.compress_array(x))[1:] == _slots(blobs[0])[1:]
+
+
+@pytest.mark.parametrize("dims", SHAPES)
+@pytest.mark.parametrize("cb,dtype,strict", [(1, "quantizer", False), (2, "quantizer", False), (4, "quantizer", False),
+                                             (1, "f32", False), (2, "f32", True), (4, "f64", False)])
+def test_lists_with_the_code_maximum(dims, cb, dtype, strict):
+    x = _field(dims, dtype)
+    x[:] = np.where(np.abs(x) > 1, x, 0.06 * x)  # codes below 2^8
+    lists = []
+    for coder in ("pack", "fixed"):
+        with _pipe(dims, coder, cb, dtype, strict) as p:
+            blob = p.compress_array(x)
+            lists.append(_slots(blob)[1:])
+            y = p.decompress_array(blob, x.dtype)[:x.size]
+            assert np.abs(y.astype(np.float64) - x).max() <= 1.01e-3
+    assert lists[0] == lists[1]
 
 
 @pytest.mark.parametrize("strict", [False, True])
