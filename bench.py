@@ -872,19 +872,20 @@ def chain_workload(kind, args):
         # charged to the kernel that reads the codes and writes the stream
         main["rle_enc_write_kernel"] = 2 * n + 4 + (2 * R + 3) // 4 * 4 + 4 * R
         helpers = ["place_kernel", "scan_small_kernel", "scan_reduce_kernel", "scan_partials_kernel",
-                   "scan_apply_kernel", "rle_enc_count_kernel", "rle_enc_fix_kernel", "rle_dec_prep_kernel",
+                   "scan_apply_kernel", "rle_enc_count_kernel", "rle_enc_count_place_kernel", "rle_enc_fix_kernel",
+                   "rle_dec_prep_kernel",
                    "rle_dec_reduce_kernel",
                    "rle_dec_apply_kernel", "rle_dec_expand_kernel", "concat_readback_kernel",
-                   "readback_kernel", "apply_patches_kernel", "bin_count_kernel", "bin_place_kernel"]
+                   "readback_kernel", "apply_patches_kernel", "bin_check_kernel", "bin_count_kernel", "bin_place_kernel"]
     else:
         R = None
         main["hist_kernel"] = 2 * n
         main["huf_enc_kernel"] = 2 * n + Cc
-        main["huf_dec_kernel"] = Cc + 2 * n
+        main["huf_dec_lane_kernel"] = main["huf_dec_kernel"] = Cc + 2 * n
         helpers = ["minmax_final_kernel", "place_kernel", "scan_small_kernel", "scan_reduce_kernel",
                    "scan_partials_kernel", "scan_apply_kernel", "huf_pack_kernel", "huf_header_kernel",
-                   "concat_readback_kernel", "readback_kernel", "apply_patches_kernel", "bin_count_kernel",
-                   "bin_place_kernel"]
+                   "concat_readback_kernel", "readback_kernel", "apply_patches_kernel", "bin_check_kernel",
+                   "bin_count_kernel", "bin_place_kernel"]
     kern = {}
     tot, cnt_ = C.c_double(), C.c_uint64()
     for kname in list(main) + helpers:

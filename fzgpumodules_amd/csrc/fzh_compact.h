@@ -6,9 +6,9 @@
 // its exclusive prefix with a place kernel in which a wave takes 32 tiles
 // of each list, finds the non-empty ones by ballot and copies them with all
 // 64 lanes.  Up to COMPACT_INLINE counts each workgroup sums the counts
-// before its 128 tiles itself (one launch in all); beyond that a
-// device-wide scan of the counts (fzh_scan.h) runs first.  No workgroup
-// waits on another.
+// before its 128 tiles itself (one launch in all, or the first workgroups
+// of an encoder's launch: PlaceDesc); beyond that a device-wide scan of the
+// counts (fzh_scan.h) runs first.  No workgroup waits on another.
 #pragma once
 
 #include <type_traits>

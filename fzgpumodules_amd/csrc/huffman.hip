@@ -18,10 +18,11 @@
 //   encode: one wave per partition packs its codewords in parallel (a run of
 //     symbols per lane, bit offsets from one wave prefix sum, whole cells
 //     ORed into LDS) and writes them to the partition's scratch slot plus
-//     par_nbit; a segmented device scan of
-//     the cell counts writes par_entry into the stream; a pack kernel moves
-//     the cells and a one-workgroup kernel writes the header: no host prefix
-//     sum, no host sync (reference phases 1-4 + two syncs).
+//     par_nbit; a segmented device scan of the cell counts writes par_entry
+//     into the stream; a pack kernel moves the cells (to a second destination
+//     as well where there is one) and a one-workgroup kernel writes the
+//     header: no host prefix sum, no host sync (reference phases 1-4 + two
+//     syncs).
 //   decode: a 2048-entry prefix table in LDS yields the symbol of any code
 //     of up to 11 bits in one probe, chained tables those of longer ones.
 //     Short streams: one wave per partition, 64 lanes decode equal spans of

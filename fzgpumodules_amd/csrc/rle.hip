@@ -117,7 +117,7 @@ __device__ __forceinline__ uint64_t rle_values_bytes(uint32_t R, int eb) { retur
 // lengths[r] for every run that ends inside it; the tile's last run gets its
 // start position in its length slot and first[tile] the tile's first start,
 // for rle_enc_fix_kernel.  With `copy` the stream goes there as well (24 -> 38
-// us for 49 MB, where a copy of the finished stream is 27 us).
+// us for 98 MB, where a copy of the finished stream is 27 us).
 template <typename T>
 __global__ void __launch_bounds__(256)
 rle_enc_write_kernel(const T* __restrict__ in, uint64_t n, const uint32_t* __restrict__ pre,
