@@ -7,8 +7,9 @@
 //
 // MI355X design
 //   encode: one wave per tile of 8 x 64 x (16/sizeof T) elements.  K1
-//     counts the tile's run starts (boundary flags from 16-byte loads); a
-//     scan of the counts gives each tile's first run index and R; K2 finds
+//     counts the tile's run starts (boundary flags from 16-byte loads); the
+//     counts summed by K2's workgroups (a scan launch where there are many)
+//     give each tile's first run index and R; K2 finds
 //     the starts again and writes every run's value and every length whose
 //     run ends inside the tile straight to the output (the previous start
 //     from a running maximum across lanes), leaving the start of the tile's
@@ -33,6 +34,11 @@ namespace fzh {
 namespace {
 
 constexpr int STEPS = 8;
+// Tiles up to which the encoder's write kernel sums the counts itself, against
+// a scan launch: 16 tiles (2-byte values) 18.3 against 23.4 us, 4096 tiles 33.7
+// against 39.5, 16384 tiles 130.2 against 132.5, 32768 tiles 301 against 275
+// (every workgroup reads all counts).
+constexpr uint32_t RLE_SUM = 16384;
 constexpr uint32_t DTILE = 1024;  // decode output tile (elements), one wave each
 constexpr uint32_t SEG_OUT = 8 * SCAN_SEG;  // most elements of a segment that one workgroup expands
 
@@ -113,16 +119,17 @@ rle_enc_count_place_kernel(const T* __restrict__ in, uint64_t n, uint32_t* __res
 __device__ __forceinline__ uint64_t rle_values_bytes(uint32_t R, int eb) { return ((uint64_t)R * eb + 3) & ~3ull; }
 
 // pre[tile] = index of the tile's first run (exclusive scan of the counts),
-// *d_R = the run count.  Writes values[r] for every run of the tile and
+// *d_R = the run count; with SUM every workgroup sums the counts itself and
+// stores both for rle_enc_fix_kernel.  Writes values[r] for every run of the tile and
 // lengths[r] for every run that ends inside it; the tile's last run gets its
 // start position in its length slot and first[tile] the tile's first start,
 // for rle_enc_fix_kernel.  With `copy` the stream goes there as well (24 -> 38
 // us for 98 MB, where a copy of the finished stream is 27 us).
-template <typename T>
+template <typename T, bool SUM>
 __global__ void __launch_bounds__(256)
-rle_enc_write_kernel(const T* __restrict__ in, uint64_t n, const uint32_t* __restrict__ pre,
-                     const uint32_t* __restrict__ d_R, uint32_t* __restrict__ first, uint8_t* __restrict__ out,
-                     uint8_t* __restrict__ copy, uint32_t ntiles) {
+rle_enc_write_kernel(const T* __restrict__ in, uint64_t n, const uint32_t* __restrict__ cnt,
+                     uint32_t* __restrict__ pre, uint32_t* __restrict__ d_R, uint32_t* __restrict__ first,
+                     uint8_t* __restrict__ out, uint8_t* __restrict__ copy, uint32_t ntiles) {
     constexpr int E = 16 / sizeof(T);
     constexpr uint32_t TILE = 64 * E * STEPS;
     constexpr uint32_t SR = 64 * E;  // most run starts of one step
@@ -131,19 +138,49 @@ rle_enc_write_kernel(const T* __restrict__ in, uint64_t n, const uint32_t* __res
     __shared__ T s_v[4][SR];
     __shared__ uint32_t s_l[4][SR];
     const uint32_t tile = blockIdx.x * 4 + wave_in_wg();
-    if (tile >= ntiles) return;
     const int l = lane_id();
     const int wv = (int)wave_in_wg();
+    uint32_t R, r;  // r, wave-uniform: index of the next run start in tile order
+    if constexpr (SUM) {
+        __shared__ uint32_t s_sum[4][2];
+        // a quad of counts lies wholly before this workgroup's tiles or not
+        const uint4* quads = reinterpret_cast<const uint4*>(cnt);
+        const uint32_t nq = ntiles / 4;
+        uint32_t before = 0, all = 0;
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < nq; i += 256) {
+            const uint4 q = quads[i];
+            const uint32_t c = (q.x + q.y) + (q.z + q.w);
+            all += c;
+            before += i < blockIdx.x ? c : 0u;
+        }
+        if (threadIdx.x < ntiles - 4 * nq) all += cnt[4 * nq + threadIdx.x];
+        before = wave_sum(before);
+        all = wave_sum(all);
+        if (l == 0) {
+            s_sum[wv][0] = before;
+            s_sum[wv][1] = all;
+        }
+        __syncthreads();
+        R = s_sum[0][1] + s_sum[1][1] + s_sum[2][1] + s_sum[3][1];
+        r = s_sum[0][0] + s_sum[1][0] + s_sum[2][0] + s_sum[3][0];
+        if (tile >= ntiles) return;
+        for (uint32_t k = blockIdx.x * 4; k < tile; k++) r += cnt[k];
+        if (l == 0) pre[tile] = r;
+        if (tile == 0 && l == 0) *d_R = R;
+    } else {
+        if (tile >= ntiles) return;
+        R = *d_R;
+        r = pre[tile];
+    }
     const uint64_t base = (uint64_t)tile * TILE;
     T v[STEPS][E];
     uint32_t mask[STEPS];
     rle_tile_starts<T>(in, n, base, v, mask);
-    const uint32_t R = *d_R;
     T* vals = reinterpret_cast<T*>(out + 4);
     uint32_t* lens = reinterpret_cast<uint32_t*>(out + 4 + rle_values_bytes(R, sizeof(T)));
     T* cvals = copy ? reinterpret_cast<T*>(copy + 4) : nullptr;
     uint32_t* clens = copy ? reinterpret_cast<uint32_t*>(copy + 4 + rle_values_bytes(R, sizeof(T))) : nullptr;
-    uint32_t r = pre[tile];     // wave-uniform: index of the next run start in tile order
     uint32_t last1 = 0;         // wave-uniform: (last start so far in this tile) + 1, 0 if none
     uint32_t first1 = 0;        // wave-uniform: (first start of the tile) + 1
 #pragma unroll
@@ -581,9 +618,12 @@ int enc_impl(hipStream_t s, const void* in, size_t n, void* out, size_t cap, voi
     else
         launch_k("rle_enc_count_kernel", rle_enc_count_kernel<T>, dim3(blocks), dim3(256), 0, s, (const T*)in, n, cnt,
                  ntiles);
-    if (int rc = scan_u32(s, cnt, pre, ntiles, nullptr, dR, w + L.o_scan)) return rc;
-    launch_k("rle_enc_write_kernel", rle_enc_write_kernel<T>, dim3(blocks), dim3(256), 0, s, (const T*)in, n,
-             (const uint32_t*)pre, (const uint32_t*)dR, first, (uint8_t*)out, (uint8_t*)copy, ntiles);
+    const bool sum = ntiles <= RLE_SUM;
+    if (!sum)
+        if (int rc = scan_u32(s, cnt, pre, ntiles, nullptr, dR, w + L.o_scan)) return rc;
+    launch_k("rle_enc_write_kernel", sum ? rle_enc_write_kernel<T, true> : rle_enc_write_kernel<T, false>, dim3(blocks),
+             dim3(256), 0, s, (const T*)in, (uint64_t)n, (const uint32_t*)cnt, pre, dR, first, (uint8_t*)out,
+             (uint8_t*)copy, ntiles);
     launch_k("rle_enc_fix_kernel", rle_enc_fix_kernel<T>, dim3((unsigned)cdiv(ntiles, 256)), dim3(256), 0, s,
              (const uint32_t*)cnt, (const uint32_t*)pre, (const uint32_t*)first, (const uint32_t*)dR, (uint64_t)n,
              (uint8_t*)out, (uint8_t*)copy, out_size, ntiles);
