@@ -37,6 +37,12 @@ bool isDeviceMemory(const void* p) {
     return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
 }
 
+// [a, a + na) and [b, b + nb) share a byte (no sum that could wrap).
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x <= y ? y - x < na : x - y < nb;
+}
+
 struct Timer {
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
     float ms() const {
@@ -828,12 +834,17 @@ void Pipeline::decompress(const void* d_input, size_t input_size, void* d_output
     const auto slots = parseConcat(d_input, input_size, stream);
     void* res = nullptr;
     size_t rs = 0;
-    const bool direct = reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0;
+    // The inverse stores while it still reads the lists, and a single-output
+    // stream, where they lie in d_input: a result that would meet the input
+    // goes to a buffer of the pipeline's and is copied at the end.
+    const size_t room = std::min(output_buf_capacity, std::max(input_size_, want));
+    const bool direct = reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0 &&
+                        !overlap(d_output_buf, room, d_input, input_size);
     // a buffer of the original size: the source stage leaves out the padding
     // (a padded result of its own, a copy and a second wait were 20 of 75 us
     // for 1800 x 3600 values)
     const size_t limit = direct && want < input_size_ && isDeviceMemory(d_output_buf) ? want : 0;
-    runInverse(slots, stream, direct ? d_output_buf : nullptr, direct ? output_buf_capacity : 0, limit, &res, &rs);
+    runInverse(slots, stream, direct ? d_output_buf : nullptr, direct ? room : 0, limit, &res, &rs);
     const size_t n = std::min(rs, want);
     if (res != d_output_buf) {
         hipck(hipMemcpyAsync(d_output_buf, res, n, hipMemcpyDeviceToDevice, stream), "hipMemcpyAsync");

@@ -97,6 +97,7 @@ class Pipeline {
     // hipMalloc'd buffer the caller frees with hipFree.
     void decompress(const void* d_input, size_t input_size, void** d_output, size_t* output_size,
                     hipStream_t stream = nullptr);
+    // Caller-owned output buffer; it may share memory with d_input.
     void decompress(const void* d_input, size_t input_size, void* d_output_buf, size_t output_buf_capacity,
                     size_t* actual_output_size, hipStream_t stream = nullptr);
     void reset(hipStream_t stream = nullptr);
