@@ -365,14 +365,10 @@ void Pipeline::launchForward(const void* d_in, size_t padded, bool zero_view, hi
         const int pred = buffers_[n.fused_from >= 0 ? nodes_[n.fused_from].in_buf : n.in_buf].producer;
         n.stage->setPlacement(pred >= 0 ? nodes_[pred].stage->deferredPlacement() : nullptr);
         // the stage that writes the concat's first slot may store it in the
-        // caller's buffer too, unless a later stage could still read an input
-        // that lies in it
-        if (copy_to_ && outputs_.size() > 1 && n.out_buf[0] == outputs_[0] && buffers_[outputs_[0]].aliased) {
-            const uint8_t *c = (const uint8_t*)copy_to_, *i = (const uint8_t*)d_in;
-            if (i + padded <= c || c + concat_cap_ <= i)
-                first_done = n.stage->copyOutputTo((uint8_t*)copy_to_ +
-                                                   ((uint8_t*)buffers_[outputs_[0]].ptr - (uint8_t*)concat_buf_));
-        }
+        // caller's buffer too (which is apart from the input)
+        if (copy_to_ && outputs_.size() > 1 && n.out_buf[0] == outputs_[0] && buffers_[outputs_[0]].aliased)
+            first_done = n.stage->copyOutputTo((uint8_t*)copy_to_ +
+                                               ((uint8_t*)buffers_[outputs_[0]].ptr - (uint8_t*)concat_buf_));
         n.stage->execute(stream, pool_.get(), {in.ptr}, outs, {in.size});
         if (e1) hipck(hipEventRecord(e1, stream), "hipEventRecord");
         stage_events_.push_back({e0, e1});
@@ -575,17 +571,16 @@ void Pipeline::compress(const void* d_input, size_t input_size, void* d_output_b
     size_t sz = 0;
     // The concat launch writes the caller's buffer along with the pool's (which
     // writeToFile reads) where that is safe: a result of any size fits, the
-    // buffer is this GPU's memory, aligned, and not part of the pool's.  A copy
-    // of its own behind the host's wait for the size took a launch and a second
-    // wait (10 us of a 73 us compress of 1800 x 3600 values).
-    const uint8_t* lo = (const uint8_t*)d_output_buf;
-    const bool direct = finalized_ && outputs_.size() > 1 && !graph_mode_ &&
-                        reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0 &&
-                        output_buf_capacity >= getMaxCompressedSize(input_size) && isDeviceMemory(d_output_buf);
-    if (direct) {
+    // buffer is this GPU's memory, aligned, not part of the pool's and apart
+    // from the input, which a call that fails behind that launch (a strict
+    // bound that the lists cannot hold) must leave as it was.  A copy of its
+    // own behind the host's wait for the size took a launch and a second wait
+    // (10 us of a 73 us compress of 1800 x 3600 values).
+    const size_t most = finalized_ && outputs_.size() > 1 && !graph_mode_ ? getMaxCompressedSize(input_size) : 0;
+    if (most > 0 && output_buf_capacity >= most && reinterpret_cast<uintptr_t>(d_output_buf) % 16 == 0 &&
+        !overlap(d_output_buf, most, d_input, input_size) && isDeviceMemory(d_output_buf)) {
         ensureBuffers(round_up(input_size, input_alignment_));
-        const uint8_t* c = (const uint8_t*)concat_buf_;
-        if (lo + output_buf_capacity <= c || c + concat_cap_ <= lo) copy_to_ = d_output_buf;
+        if (!overlap(d_output_buf, most, concat_buf_, concat_cap_)) copy_to_ = d_output_buf;
     }
     const bool copied = copy_to_ != nullptr;
     try {

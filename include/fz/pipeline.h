@@ -89,7 +89,9 @@ class Pipeline {
     // Pool-owned output, valid until the next compress().
     void compress(const void* d_input, size_t input_size, void** d_output, size_t* output_size,
                   hipStream_t stream = nullptr);
-    // Caller-owned output buffer.
+    // Caller-owned output buffer.  A call that throws leaves d_input as it was
+    // (also where the two share memory) and may have written the rest of the
+    // buffer.
     void compress(const void* d_input, size_t input_size, void* d_output_buf, size_t output_buf_capacity,
                   size_t* actual_output_size, hipStream_t stream = nullptr);
     // d_input is what compress() returned.  The result is pool-owned (valid

@@ -108,7 +108,8 @@ int fzp_compress(fzp_pipeline* p, void* stream, const void* d_in, size_t in_byte
  * caller-owned (release with fzh_device_free). */
 int fzp_decompress(fzp_pipeline* p, void* stream, const void* d_in, size_t in_bytes,
                    void** d_out, size_t* out_bytes);
-/* Caller-owned output buffers. */
+/* Caller-owned output buffers; d_out may share memory with d_in.  A call that
+ * fails may have written d_out, but not what it shares with d_in. */
 int fzp_compress_into(fzp_pipeline* p, void* stream, const void* d_in, size_t in_bytes,
                       void* d_out, size_t out_cap, size_t* out_bytes);
 int fzp_decompress_into(fzp_pipeline* p, void* stream, const void* d_in, size_t in_bytes,

@@ -3,7 +3,8 @@ the compressed bytes at the start, in the middle and at the end of the output
 buffer, byte for byte the result of separate buffers.  Sizes that a chain pads
 and that it doesn't, outlier and patch lists short enough for the inverse
 kernel to read itself (256) and longer ones, a chain with one output, buffers
-of exactly the original size and with room for the padding."""
+of exactly the original size and with room for the padding.  Compress with the
+input inside the output buffer, where a call that fails leaves the input."""
 import numpy as np
 import pytest
 
@@ -85,3 +86,34 @@ def test_decompress_over_its_input(fzh, chain, dims, dtype, strict, lists):
                 assert (got[max(base + cap, at + blob.size):] == 0xA5).all()
                 d.free()
         assert d_b.ptr
+
+
+@pytest.mark.parametrize("chain", ["rze", "huffman", "rle"])
+@pytest.mark.parametrize("at", [0, 4096, -1])
+def test_failed_compress_leaves_its_input(fzh, chain, at):
+    from fzgpumodules_amd.pipeline import Pipeline
+    dims = (403, 97, 1)
+    x = _field(dims, "f32", "long")
+    with Pipeline(x.nbytes) as p:
+        a = p.add_lorenzo(1e-3, mode="ABS", quant_radius=512, outlier_capacity=0.3, zigzag=True)
+        p.set_strict(a, True, 1e-4)  # room for 4 patches
+        if chain == "rze":
+            b = p.add_bitshuffle(16384, 2)
+            p.connect(b, a, "codes")
+            p.connect(p.add_rze(16384, 4), b)
+        else:
+            p.connect(p.add_huffman(2, 1024) if chain == "huffman" else p.add_rle(2), a, "codes")
+        p.set_dims(*dims)
+        p.finalize()
+        cap = (p.max_compressed_size(x.nbytes) + x.nbytes + 15) // 16 * 16
+        if at < 0:
+            at = (cap - x.nbytes) // 16 * 16
+        start = np.full(cap + 64, 0xA5, np.uint8)
+        start[at:at + x.nbytes] = x.view(np.uint8)
+        d = fzh.DeviceBuffer.from_array(start)
+        for _ in range(2):  # the second call runs on the first one's buffers
+            with pytest.raises(fzh.FzhError, match="patch"):
+                p.compress_into(d.ptr + at, x.nbytes, d, cap)
+            got = d.download(np.uint8, start.size)
+            assert np.array_equal(got[at:at + x.nbytes], x.view(np.uint8))
+            assert (got[cap:] == 0xA5).all()
