@@ -544,7 +544,12 @@ template <typename T, int BLOCK, int PER, typename F>
 __device__ __forceinline__ void dec_level(uint32_t* tab, uint32_t count, uint32_t l0, uint32_t b, uint32_t fv,
                                           const int32_t* diff, const T* __restrict__ keys, uint32_t nkeys, F&& longer) {
     constexpr bool FOLD = sizeof(T) <= 2;
-    for (uint32_t i0 = threadIdx.x; i0 < count; i0 += BLOCK * PER) {
+    // The trip count is the wave's (its first entry < count), so readlane never
+    // names a lane that has left the loop, whose copy of fv no instruction need
+    // keep; lanes past `count` compute an entry that they don't store.
+    const uint32_t lane = (uint32_t)lane_id();
+    for (uint32_t w0 = wave_in_wg() * 64; w0 < count; w0 += BLOCK * PER) {
+        const uint32_t i0 = w0 + lane;
         uint32_t W[PER], lv[PER], k[PER], key[PER];
 #pragma unroll
         for (int i = 0; i < PER; i++) {
