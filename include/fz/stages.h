@@ -189,7 +189,10 @@ class LorenzoQuantStage : public Stage {
         if (index == 5 && d_pcount_ptr_) return {d_pcount_ptr_, 2, 4};
         return {};
     }
-    void setInverse(bool inv) override { is_inverse_ = inv; }
+    void setInverse(bool inv) override {
+        is_inverse_ = inv;
+        inv_limit_ = 0;  // also one that an inverse which threw left behind
+    }
     bool isInverse() const override { return is_inverse_; }
 
     uint16_t getStageTypeId() const override { return (uint16_t)StageType::LORENZO_QUANT; }

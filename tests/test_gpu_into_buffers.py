@@ -119,3 +119,23 @@ def test_file_after_the_buffer_is_reused(fzh, tmp_path, chain):
         p.write_file(tmp_path / "a.fzm")
         from fzgpumodules_amd.pipeline import Pipeline
         assert np.array_equal(Pipeline.decompress_file(tmp_path / "a.fzm")[:x.size], want)
+
+
+def test_decompress_after_one_that_failed(fzh):
+    """A decompress that throws before its inverse ran leaves nothing to the next one."""
+    from fzgpumodules_amd.pipeline import Pipeline
+    small, large = _field((5_001, 1, 1), "f32"), _field((70_001, 1, 1), "f32")
+    with Pipeline(large.nbytes) as p:
+        a = p.add_lorenzo(1e-3, mode="ABS", quant_radius=512, outlier_capacity=0.3, zigzag=True)
+        b = p.add_bitshuffle(16384, 2)
+        p.connect(b, a, "codes")
+        p.connect(p.add_rze(16384, 4), b)
+        p.finalize()
+        blob = p.compress_array(small)
+        d_b, d_y = fzh.DeviceBuffer.from_array(blob), fzh.DeviceBuffer(small.nbytes)
+        p.set_strict(a, True)  # the stage now expects patch lists that this pipeline doesn't have
+        with pytest.raises(fzh.FzhError):
+            p.decompress_into(d_b, blob.size, d_y, small.nbytes)
+        p.set_strict(a, False)
+        y = p.decompress_array(p.compress_array(large))
+        assert y.size == large.size and np.abs(y - large).max() <= 1.001e-3
