@@ -96,8 +96,8 @@ void LorenzoQuantStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, co
     fzh::PlaceDesc* place = nullptr;
     place_left_ = std::exchange(defer_place_, false);
     if (place_left_) {
-        static_assert(sizeof(fzh::PlaceDesc) <= sizeof(place_desc_), "placement description storage");
-        place = reinterpret_cast<fzh::PlaceDesc*>(place_desc_);
+        if (place_desc_.use_count() != 1) place_desc_ = std::make_shared<fzh::PlaceDesc>();
+        place = place_desc_.get();
         place->blocks = 0;
     }
     if (is_inverse_) {
@@ -392,7 +392,7 @@ void RZEStage::execute(hipStream_t stream, MemoryPool* pool, const std::vector<v
         throw std::runtime_error("RZEStage: only chunk_size == 16384 is currently supported; got " + std::to_string(chunk_size_));
     if (levels_ != 4)
         throw std::runtime_error("RZEStage: only levels == 4 is currently supported; got " + std::to_string((int)levels_));
-    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
+    const auto* place = std::exchange(place_desc_, nullptr);
     small_.ensure(256, pool, stream);
     clearReadbacks();
     size_pending_ = status_pending_ = false;
@@ -462,7 +462,7 @@ template <typename T>
 void RLEStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                           const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
     void* copy = std::exchange(copy_out_, nullptr);
-    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
+    const auto* place = std::exchange(place_desc_, nullptr);
     if (inputs.empty() || outputs.empty() || sizes.empty()) throw std::runtime_error("RLEStage: Invalid inputs/outputs");
     small_.ensure(256, pool, stream);
     clearReadbacks();
@@ -664,8 +664,8 @@ void QuantizerStage<TI, TC>::execute(hipStream_t stream, MemoryPool* pool, const
     fzh::PlaceDesc* place = nullptr;
     place_left_ = std::exchange(defer_place_, false);
     if (place_left_) {
-        static_assert(sizeof(fzh::PlaceDesc) <= sizeof(place_desc_), "placement description storage");
-        place = reinterpret_cast<fzh::PlaceDesc*>(place_desc_);
+        if (place_desc_.use_count() != 1) place_desc_ = std::make_shared<fzh::PlaceDesc>();
+        place = place_desc_.get();
         place->blocks = 0;
     }
     if (isInplaceMode()) {  // quantizer.cu:396-452 / 492-615, one port each way
@@ -827,7 +827,7 @@ template class QuantizerStage<float, uint32_t>;
 template <typename T>
 void BitpackStage<T>::execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                               const std::vector<void*>& outputs, const std::vector<size_t>& sizes) {
-    const auto* place = static_cast<const fzh::PlaceDesc*>(std::exchange(place_desc_, nullptr));
+    const auto* place = std::exchange(place_desc_, nullptr);
     if (inputs.empty() || outputs.empty() || sizes.empty())
         throw std::runtime_error("BitpackStage: inputs, outputs, and sizes must be non-empty");
     if (!is_inverse_) {

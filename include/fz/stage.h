@@ -17,6 +17,10 @@
 
 #include "fz/fzm_format.h"
 
+namespace fzh {
+struct PlaceDesc;  // a placement left to an encoder (csrc/fzh_internal.h)
+}
+
 namespace fz {
 
 class MemoryPool;
@@ -114,7 +118,7 @@ class Stage {
 
     virtual size_t estimateScratchBytes(const std::vector<size_t>& /*input_sizes*/) const { return 0; }
 
-    // ---- Extensions of this build (no counterpart in the reference) ----
+    // ---- Extensions (no counterpart in the reference) ----
 
     // The pipeline input is zero-padded to a multiple of the stages'
     // alignment.  A source stage that returns true here reads only the first
@@ -133,13 +137,13 @@ class Stage {
 
     // Lets the next forward execute() leave the placement of its small outputs
     // (not output 0) to the launch that encodes output 0, which gets
-    // deferredPlacement() (an fzh::PlaceDesc; null: nothing was left).
+    // deferredPlacement() (null: nothing was left).
     virtual void deferPlacement(bool on) { (void)on; }
-    virtual const void* deferredPlacement() const { return nullptr; }
+    virtual const fzh::PlaceDesc* deferredPlacement() const { return nullptr; }
     // The encoder's side: whether its next forward execute() would run such a
     // placement in one of its launches, and the placement (null: none).
     virtual bool takesPlacement() const { return false; }
-    virtual void setPlacement(const void* desc) { (void)desc; }
+    virtual void setPlacement(const fzh::PlaceDesc* desc) { (void)desc; }
 
     virtual DeviceSize getDeviceOutputSize(int index) const { (void)index; return {}; }
 

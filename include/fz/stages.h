@@ -27,10 +27,6 @@
 #include "fz/mempool.h"
 #include "fz/stage.h"
 
-namespace fzh {
-struct PlaceDesc;
-}
-
 namespace fz {
 
 enum class ErrorBoundMode : uint8_t { ABS = 0, REL = 1, NOA = 2 };
@@ -120,7 +116,7 @@ class LorenzoQuantStage : public Stage {
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
     void deferPlacement(bool on) override { defer_place_ = on; }
-    const void* deferredPlacement() const override { return place_left_ ? place_desc_ : nullptr; }
+    const fzh::PlaceDesc* deferredPlacement() const override { return place_left_ ? place_desc_.get() : nullptr; }
 
     std::string getName() const override { return "LorenzoQuant"; }
     size_t getNumInputs() const override { return is_inverse_ ? numPorts() : 1; }
@@ -222,7 +218,7 @@ class LorenzoQuantStage : public Stage {
 
     Config config_;
     bool defer_place_ = false, place_left_ = false;
-    alignas(8) unsigned char place_desc_[136] = {};
+    std::shared_ptr<fzh::PlaceDesc> place_desc_;  // this object's own (a copy makes another)
     bool is_inverse_ = false;
     size_t inv_limit_ = 0;  // elements of the next inverse execute() (0: all)
     std::vector<size_t> actual_output_sizes_ = std::vector<size_t>(4, 0), saved_output_sizes_;
@@ -315,7 +311,7 @@ class RZEStage : public Stage {
     // next execute).
     void setDeferPack(bool on) { defer_pack_ = on; }
     bool takesPlacement() const override { return defer_pack_; }
-    void setPlacement(const void* desc) override { place_desc_ = desc; }
+    void setPlacement(const fzh::PlaceDesc* desc) override { place_desc_ = desc; }
     const void* deferredPack() const { return pack_deferred_ ? pack_desc_ : nullptr; }
 
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
@@ -356,7 +352,7 @@ class RZEStage : public Stage {
     bool is_inverse_ = false;
     int pre_shuffle_ = 0;
     bool defer_pack_ = false, pack_deferred_ = false;
-    const void* place_desc_ = nullptr;
+    const fzh::PlaceDesc* place_desc_ = nullptr;
     alignas(8) unsigned char pack_desc_[96] = {};
     uint32_t chunk_size_ = 16384;
     uint8_t levels_ = 4;
@@ -386,7 +382,7 @@ class RLEStage : public Stage {
     bool isInverse() const override { return is_inverse_; }
     bool copyOutputTo(void* d_copy) override { copy_out_ = d_copy; return true; }
     bool takesPlacement() const override { return !is_inverse_; }
-    void setPlacement(const void* desc) override { place_desc_ = desc; }
+    void setPlacement(const fzh::PlaceDesc* desc) override { place_desc_ = desc; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -420,7 +416,7 @@ class RLEStage : public Stage {
     void restoreState() override { cached_num_elements_ = saved_n_; actual_output_size_ = saved_out_; }
 
   private:
-    const void* place_desc_ = nullptr;
+    const fzh::PlaceDesc* place_desc_ = nullptr;
     void* copy_out_ = nullptr;  // second destination of the next forward execute()
     bool is_inverse_ = false;
     uint32_t cached_num_elements_ = 0, saved_n_ = 0;
@@ -574,7 +570,7 @@ class QuantizerStage : public Stage {
     explicit QuantizerStage(const Config& c = Config()) : config_(c) {}
 
     void deferPlacement(bool on) override { defer_place_ = on; }
-    const void* deferredPlacement() const override { return place_left_ ? place_desc_ : nullptr; }
+    const fzh::PlaceDesc* deferredPlacement() const override { return place_left_ ? place_desc_.get() : nullptr; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     void postStreamSync(hipStream_t stream) override;
@@ -629,7 +625,7 @@ class QuantizerStage : public Stage {
 
   private:
     bool defer_place_ = false, place_left_ = false;
-    alignas(8) unsigned char place_desc_[136] = {};
+    std::shared_ptr<fzh::PlaceDesc> place_desc_;  // this object's own (a copy makes another)
     bool isInplaceMode() const { return config_.inplace_outliers && config_.eb_mode != ErrorBoundMode::REL; }
     size_t maxOutliers(size_t n) const { return (size_t)std::ceil((double)n * config_.outlier_capacity); }
     Config config_;
@@ -668,7 +664,7 @@ class BitpackStage : public Stage {
     bool isGraphCompatible() const override { return !auto_detect_ || is_inverse_; }
 
     bool takesPlacement() const override { return !is_inverse_ && auto_detect_; }
-    void setPlacement(const void* desc) override { place_desc_ = desc; }
+    void setPlacement(const fzh::PlaceDesc* desc) override { place_desc_ = desc; }
     void execute(hipStream_t stream, MemoryPool* pool, const std::vector<void*>& inputs,
                  const std::vector<void*>& outputs, const std::vector<size_t>& sizes) override;
     std::string getName() const override { return "Bitpack"; }
@@ -711,7 +707,7 @@ class BitpackStage : public Stage {
     }
 
   private:
-    const void* place_desc_ = nullptr;
+    const fzh::PlaceDesc* place_desc_ = nullptr;
     bool is_inverse_ = false, auto_detect_ = false;
     uint8_t nbits_ = 8 * sizeof(T);
     size_t num_elements_ = 0, actual_output_size_ = 0;
