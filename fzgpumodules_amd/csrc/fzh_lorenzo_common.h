@@ -119,9 +119,20 @@ __device__ __forceinline__ bool tile_of(const TileMap& m, uint32_t idx, uint32_t
     return true;
 }
 
+// Tile T for an index outside the tiles' region: such an entry is dropped, so
+// at the list's end it is in order.  (A padded 1D field's last value has an
+// outlier behind it, the step down to the zeros of the padding, which an
+// inverse of the unpadded field does not cover.)
+__device__ __forceinline__ uint32_t bin_tile(const TileMap& m, uint32_t T, uint32_t idx, uint32_t& local) {
+    uint32_t t = T;
+    local = 0;
+    if (!tile_of(m, idx, t, local)) t = T;
+    return t;
+}
+
 // Outlier binning.  A list in tile order (what the forward writes) is
 // binned without atomics: bin_check_kernel finds out whether the list is in
-// tile order with valid indices; if it is, the counting kernels return at
+// tile order (bin_tile); if it is, the counting kernels return at
 // once, the scan sees a count of zero, and bin_place_kernel takes each
 // tile's range from the tile changes along the list.  Otherwise (the
 // reference's atomic order) a counting sort runs: per-tile counts with
@@ -148,9 +159,8 @@ bin_check_kernel(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ 
         for (int u = 0; u < 4; u++) {
             const uint64_t i = i0 + u * stride;
             if (i >= k) continue;
-            uint32_t t, loc, tp, lp;
-            if (!tile_of(m, q[u], t, loc)) unordered = true;
-            else if (i > 0 && (!tile_of(m, qp[u], tp, lp) || tp > t)) unordered = true;
+            uint32_t loc;
+            if (i > 0 && bin_tile(m, T, qp[u], loc) > bin_tile(m, T, q[u], loc)) unordered = true;
         }
     }
     if (__ballot(unordered) && lane_id() == 0) {
@@ -209,11 +219,10 @@ bin_place_kernel(const V* __restrict__ err, const uint32_t* __restrict__ idx,
         for (int u = 0; u < 4; u++) {
             const uint64_t i = i0 + u * stride;
             if (i > k) continue;
-            uint32_t t = T, loc = 0, tp = 0, lp;
-            if (i < k) (void)tile_of(m, q[u], t, loc);
-            const bool head = i == 0 || (tile_of(m, qp[u], tp, lp), tp != t);
-            if (head)
-                for (uint32_t w = i == 0 ? 0u : tp + 1; w <= t; w++) off[w] = (uint32_t)i;
+            uint32_t loc = 0, lp;
+            const uint32_t t = i < k ? bin_tile(m, T, q[u], loc) : T;
+            const uint32_t from = i == 0 ? 0u : bin_tile(m, T, qp[u], lp) + 1;  // past the predecessor's tile
+            for (uint32_t w = from; w <= t; w++) off[w] = (uint32_t)i;
             if (i < k) {
                 serr[i] = e[u];
                 sloc[i] = loc;
