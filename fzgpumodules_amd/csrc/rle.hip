@@ -335,21 +335,36 @@ rle_dec_reduce_kernel(const uint8_t* __restrict__ in, const uint32_t* __restrict
 // 16 bytes of output per lane: the runs that start in the window mark their
 // first element, a running maximum over the marks gives every element its
 // run.  Nothing but the stream is read and nothing but the output written (a
-// start per run and a tile's runs, written by one launch and read by the
-// next, were 70 us for 2^24 two-byte values in runs of one or two; this is
-// 50).  A segment covers at most SEG_OUT elements here, so no workgroup
-// works much longer than the others; if any covers more, the whole stream
-// goes by output tiles (rle_dec_starts and the expand launch).
+// start per run and a tile's runs go from one launch to the next otherwise).
+// Decode of 2^24 two-byte values in runs of 1.5, 3, 5 and 7.5 on average: 51,
+// 39, 35 and 36 us, by output tiles 77, 57, 53 and 50.  A segment covers at
+// most SEG_OUT elements here (runs of 8 on average), so no workgroup works
+// much longer than the others; if any covers more, the whole stream goes by
+// output tiles (rle_dec_starts and the expand launch: 44 us for runs of 32).
+constexpr uint32_t START_SLOTS = SCAN_SEG + SCAN_SEG / 16 + 1;  // one of padding per 16
+
+// Four-byte values with starts in 16 bits (a segment and its first window's
+// offset are below 2^16) leave the kernel the five workgroups per CU that its
+// registers allow; smaller ones have room for 32 bits, which are 2% faster.
+template <typename T>
+struct RleSegLds {
+    static constexpr uint32_t E = 16 / sizeof(T), WIN = 64 * E;  // elements per lane and per window
+    static constexpr uint32_t NWIN = SEG_OUT / WIN + 2;
+    static_assert(SEG_OUT + WIN <= 65536, "16-bit starts");
+    using Start = std::conditional_t<sizeof(T) == 4, uint16_t, uint32_t>;
+    uint16_t mark[4][WIN];
+    Start x[START_SLOTS];
+    uint16_t first[NWIN];  // window -> the run at its first element
+    T val[SCAN_SEG];
+};
+
 template <typename T>
 __device__ __forceinline__ void rle_dec_segment(const uint8_t* __restrict__ in, uint64_t n, uint32_t R,
                                                 const uint32_t* __restrict__ seg_base,
                                                 const uint32_t* __restrict__ total, T* __restrict__ out,
-                                                int* __restrict__ d_status, uint32_t* s_x, uint32_t* s_w) {
-    constexpr uint32_t E = 16 / sizeof(T), WIN = 64 * E;  // elements per lane and per window
-    constexpr uint32_t NWIN = SEG_OUT / WIN + 2;
-    __shared__ T s_val[SCAN_SEG];
-    __shared__ uint16_t s_first[NWIN];  // window -> the run at its first element
-    __shared__ __align__(16) uint16_t s_mark[4][WIN];
+                                                int* __restrict__ d_status, RleSegLds<T>& L, uint32_t* s_w) {
+    using Start = typename RleSegLds<T>::Start;
+    constexpr uint32_t E = RleSegLds<T>::E, WIN = RleSegLds<T>::WIN;
     auto px = [](uint32_t i) { return i + (i >> 4); };
     const uint64_t seg0 = (uint64_t)blockIdx.x * SCAN_SEG;
     if (blockIdx.x == 0 && threadIdx.x == 0 && R != 0 && *total != n) *d_status = 1;
@@ -358,17 +373,24 @@ __device__ __forceinline__ void rle_dec_segment(const uint8_t* __restrict__ in, 
     const uint32_t* lens = rle_lengths(in, R, sizeof(T)) + seg0;
     const T* vals = reinterpret_cast<const T*>(in + 4) + seg0;
     const uint32_t tid = threadIdx.x, w = wave_in_wg(), l = (uint32_t)lane_id();
+    uint32_t v[16], sum = 0;
+    T u[16];
+#pragma unroll
+    for (uint32_t k = 0; k < 16; k++) {  // all loads in flight: none behind a branch
+        const uint32_t i = min(256 * k + tid, m - 1);
+        v[k] = lens[i];
+        u[k] = vals[i];
+    }
 #pragma unroll
     for (uint32_t k = 0; k < 16; k++) {
         const uint32_t i = 256 * k + tid;
-        s_x[px(i)] = i < m ? lens[i] : 0u;
-        if (i < m) s_val[i] = vals[i];
+        L.x[px(i)] = i < m ? (Start)v[k] : (Start)0;
+        L.val[i] = u[k];
     }
     __syncthreads();
-    uint32_t v[16], sum = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 16; k++) {
-        v[k] = s_x[px(16 * tid + k)];
+        v[k] = L.x[px(16 * tid + k)];
         sum += v[k];
     }
     const uint32_t incl = wave_incl_scan(sum);
@@ -381,25 +403,25 @@ __device__ __forceinline__ void rle_dec_segment(const uint8_t* __restrict__ in, 
     const uint32_t end = (uint32_t)(S0 - W0 * WIN) + s_w[0] + s_w[1] + s_w[2] + s_w[3];
 #pragma unroll
     for (uint32_t k = 0; k < 16; k++) {
-        s_x[px(16 * tid + k)] = run;  // after this thread's own reads
-        for (uint32_t t = (run + WIN - 1) / WIN; t * WIN < run + v[k]; t++) s_first[t] = (uint16_t)(16 * tid + k);
+        L.x[px(16 * tid + k)] = (Start)run;  // after this thread's own reads
+        for (uint32_t t = (run + WIN - 1) / WIN; t * WIN < run + v[k]; t++) L.first[t] = (uint16_t)(16 * tid + k);
         run += v[k];
     }
-    if (tid == 0) s_x[px(SCAN_SEG)] = end;
+    if (tid == 0) L.x[px(SCAN_SEG)] = (Start)end;
     const uint32_t off0 = (uint32_t)(S0 - W0 * WIN);
-    if (tid == 0 && off0) s_first[0] = 0;
+    if (tid == 0 && off0) L.first[0] = 0;
     __syncthreads();
-    uint16_t* mark = s_mark[w];
+    uint16_t* mark = L.mark[w];
     const uint32_t nwin = (end + WIN - 1) / WIN;
     for (uint32_t t = w; t < nwin; t += 4) {
         const uint32_t b = t * WIN;
-        const uint32_t r0 = s_first[t], r1 = t + 1 < nwin ? s_first[t + 1] : m - 1;  // runs r0 .. r1 reach into it
+        const uint32_t r0 = L.first[t], r1 = t + 1 < nwin ? L.first[t + 1] : m - 1;  // runs r0 .. r1 reach into it
 #pragma unroll
         for (uint32_t q = 0; q < E; q += 4) *reinterpret_cast<uint2*>(mark + E * l + q) = make_uint2(0, 0);
         wave_lds_sync();
         for (uint32_t i = r0 + 1 + l; i <= r1; i += 64) {
-            const uint32_t p = s_x[px(i)];
-            if (p - b < WIN && s_x[px(i + 1)] > p) mark[p - b] = (uint16_t)(i - r0);
+            const uint32_t p = L.x[px(i)];
+            if (p - b < WIN && L.x[px(i + 1)] > p) mark[p - b] = (uint16_t)(i - r0);
         }
         wave_lds_sync();
         uint16_t mk[E];
@@ -414,7 +436,7 @@ __device__ __forceinline__ void rle_dec_segment(const uint8_t* __restrict__ in, 
 #pragma unroll
         for (uint32_t q = 0; q < E; q++) {
             cur = max(cur, (uint32_t)mk[q]);
-            buf[q] = s_val[r0 + cur];
+            buf[q] = L.val[r0 + cur];
         }
         wave_lds_sync();  // the marks are read before the next window clears them
         const uint32_t e0 = b + E * l;
@@ -442,13 +464,17 @@ __device__ __forceinline__ void rle_dec_starts(const uint8_t* __restrict__ in, u
     const int tid = threadIdx.x, w = tid >> 6;
     const uint64_t seg0 = (uint64_t)blockIdx.x * SCAN_SEG;
     const uint64_t b = seg0 + 16ull * tid;
+    uint32_t v[16] = {}, sum = 0;
+    if (seg0 < R) {  // all loads in flight: none behind a branch of its lane
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[k] = lens[min(seg0 + 256 * k + tid, (uint64_t)R - 1)];
+    }
 #pragma unroll
     for (int k = 0; k < 16; k++) {
         const uint32_t i = (uint32_t)(256 * k + tid);
-        s_x[px(i)] = (seg0 + i < R) ? lens[seg0 + i] : 0u;
+        s_x[px(i)] = (seg0 + i < R) ? v[k] : 0u;
     }
     __syncthreads();
-    uint32_t v[16], sum = 0;
 #pragma unroll
     for (int k = 0; k < 16; k++) {
         v[k] = s_x[px(16 * tid + k)];
@@ -483,9 +509,9 @@ __device__ __forceinline__ void rle_dec_starts(const uint8_t* __restrict__ in, u
     }
 }
 
-// One segment of SCAN_SEG runs per workgroup.  s_x: the segment's lengths,
+// One segment of SCAN_SEG runs per workgroup.  x: the segment's lengths,
 // then its starts: loaded and stored coalesced, read by thread t as its 16
-// consecutive runs (one padding word per 16 keeps those reads on distinct
+// consecutive runs (one padding entry per 16 keeps those reads on distinct
 // banks).
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -493,11 +519,15 @@ rle_dec_apply_kernel(const uint8_t* __restrict__ in, uint64_t n, const uint32_t*
                      const uint32_t* __restrict__ d_long, const uint32_t* __restrict__ seg_base,
                      const uint32_t* __restrict__ total, uint32_t* __restrict__ start,
                      uint32_t* __restrict__ tile_first, T* __restrict__ out, int* __restrict__ d_status) {
-    __shared__ uint32_t s_w[4], s_x[SCAN_SEG + SCAN_SEG / 16 + 1];
+    __shared__ uint32_t s_w[4];
+    __shared__ __align__(16) union {
+        uint32_t x[START_SLOTS];
+        RleSegLds<T> seg;
+    } L;
     if (*d_long)
-        rle_dec_starts<T>(in, n, *Rv, seg_base, total, start, tile_first, d_status, s_x, s_w);
+        rle_dec_starts<T>(in, n, *Rv, seg_base, total, start, tile_first, d_status, L.x, s_w);
     else
-        rle_dec_segment<T>(in, n, *Rv, seg_base, total, out, d_status, s_x, s_w);
+        rle_dec_segment<T>(in, n, *Rv, seg_base, total, out, d_status, L.seg, s_w);
 }
 
 template <typename T>

@@ -62,3 +62,19 @@ def test_wrong_total(gpu, kind, by):
     vals = np.arange(lens.size).astype(np.uint16)
     with pytest.raises(ValueError):
         gpu.rle_dec(_stream(vals, lens), np.uint16, int(lens.sum()) + by)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.uint32])
+@pytest.mark.parametrize("offset", [0, 1, -1])
+@pytest.mark.parametrize("kind", ["even", "one_run"])
+def test_largest_starts(gpu, dtype, offset, kind):
+    """A segment at the limit that begins anywhere in its first window: the largest 16-bit starts."""
+    win = 64 * 16 // np.dtype(dtype).itemsize
+    first = np.ones(4096, np.int64)
+    first[7] += offset % win
+    last = np.full(4096, 8) if kind == "even" else np.r_[np.ones(4000), 32768 - 4095, np.ones(95)]
+    lens = np.r_[first, last].astype(np.int64)
+    assert first.sum() <= 32768 and last.sum() == 32768
+    vals = np.random.default_rng(offset + 5).integers(0, 251, lens.size).astype(dtype)
+    want = np.repeat(vals, lens)
+    assert np.array_equal(gpu.rle_dec(_stream(vals, lens), dtype, want.size), want)
