@@ -881,7 +881,7 @@ def chain_workload(kind, args):
         R = None
         main["hist_kernel"] = 2 * n
         main["huf_enc_kernel"] = 2 * n + Cc
-        main["huf_dec_lane_kernel"] = main["huf_dec_kernel"] = Cc + 2 * n
+        main["huf_dec_long_kernel"] = main["huf_dec_kernel"] = Cc + 2 * n
         helpers = ["minmax_final_kernel", "place_kernel", "scan_small_kernel", "scan_reduce_kernel",
                    "scan_partials_kernel", "scan_apply_kernel", "huf_pack_kernel", "huf_header_kernel",
                    "concat_readback_kernel", "readback_kernel", "apply_patches_kernel", "bin_check_kernel",

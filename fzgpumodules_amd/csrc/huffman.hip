@@ -28,7 +28,8 @@
 //     Short streams: one wave per partition, 64 lanes decode equal spans of
 //     its bits speculatively and settle the span starts in rounds (a prefix
 //     code resynchronises within a few codewords); symbols are staged in LDS
-//     and leave in 16-byte stores.  Long streams: one lane per partition.
+//     and leave in 16-byte stores.  Long streams: one lane per partition
+//     where their partitions, bits and runs make that the faster.
 #include <type_traits>
 
 #include "fzh_huffman_enc.h"
@@ -501,6 +502,7 @@ constexpr int cdiv_c(int a, int b) { return (a + b - 1) / b; }
 
 struct DecHead {
     uint32_t sublen, pardeg, e1, nkeys, ncells;
+    bool zero_len;  // a book of one symbol, whose code may have no bits
     const uint32_t* par_nbit;
     const uint32_t* par_entry;
     const uint32_t* cells;
@@ -525,6 +527,7 @@ __device__ __forceinline__ bool dec_head(const uint8_t* __restrict__ in, uint64_
     h.par_nbit = reinterpret_cast<const uint32_t*>(in + e2);
     h.par_entry = reinterpret_cast<const uint32_t*>(in + e3);
     h.cells = reinterpret_cast<const uint32_t*>(in + e4);
+    h.zero_len = reinterpret_cast<const uint32_t*>(in + e1)[33] == 1;  // entry[1]
     return true;
 }
 
@@ -578,8 +581,7 @@ __device__ __forceinline__ void dec_level(uint32_t* tab, uint32_t count, uint32_
 // Builds the tables of the stream's book (all BLOCK threads; ends with a
 // barrier).
 template <typename T, int BLOCK>
-__device__ __forceinline__ DecTables dec_build(const uint8_t* __restrict__ in, const DecHead& h, DecLds& t,
-                                               bool& zero_len) {
+__device__ __forceinline__ DecTables dec_build(const uint8_t* __restrict__ in, const DecHead& h, DecLds& t) {
     const uint32_t* fb = reinterpret_cast<const uint32_t*>(in + h.e1);
     const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
     const uint32_t nkeys = h.nkeys;
@@ -592,7 +594,6 @@ __device__ __forceinline__ DecTables dec_build(const uint8_t* __restrict__ in, c
     const uint32_t all = (uint32_t)__ballot(l32 > 0 && fv == 0);
     uint32_t maxl = used ? 31u - (uint32_t)__builtin_clz(used) : 1u;
     if (all) maxl = min(maxl, (uint32_t)__builtin_ctz(all));
-    zero_len = (uint32_t)__builtin_amdgcn_readlane((int)en, 1) == 1;
     if (threadIdx.x < 32) {
         t.lim[threadIdx.x] = threadIdx.x ? (uint64_t)fv << (32 - threadIdx.x) : ~0ull;
         t.diff[threadIdx.x] = (int32_t)(en - fv);
@@ -639,6 +640,51 @@ __device__ __forceinline__ void dec_constant(T* __restrict__ dst, uint32_t cnt, 
     for (uint32_t j = (uint32_t)lane_id(); j < cnt; j += 64) dst[j] = v;
 }
 
+// Partition p, decoded by one wave; cst and ost: the wave's DEC_CELLS + 4 words
+// and DEC_SUBLEN_MAX symbols of LDS.
+template <typename T>
+__device__ __forceinline__ void dec_wave(const DecHead& h, const DecTables& tb, const T* __restrict__ keys,
+                                         uint32_t p, uint64_t n, T* __restrict__ out, uint32_t* cst, uint4* ost,
+                                         int* __restrict__ d_status) {
+    const uint32_t l = (uint32_t)lane_id();
+    const uint32_t nbit = h.par_nbit[p];
+    const uint32_t pe = h.par_entry[p];
+    const uint32_t ncell = (uint32_t)(((uint64_t)nbit + 31) / 32);
+    const uint64_t o0 = (uint64_t)p * h.sublen;
+    const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
+    T* dst = out + o0;
+    if ((uint64_t)pe + ncell > h.ncells) {
+        if (l == 0) *d_status = 1;
+        return;
+    }
+    if (h.zero_len && nbit == 0) {
+        dec_constant(dst, cnt, h.nkeys ? keys[0] : (T)0);
+        return;
+    }
+    bool ok;
+    if (ncell <= DEC_CELLS && h.sublen <= DEC_SUBLEN_MAX) {
+        wave_lds_sync();  // the previous partition's staging reads are done
+        for (uint32_t i = l; i < ncell + 4; i += 64) cst[i] = i < ncell ? h.cells[pe + i] : 0u;
+        wave_lds_sync();
+        T* st = reinterpret_cast<T*>(ost);
+        ok = dec_partition<T, true>(cst, ncell, tb, nbit, cnt, keys, st, dst);
+        wave_lds_sync();
+        if (ok) {
+            const uint32_t bytes = cnt * (uint32_t)sizeof(T);
+            uint32_t done = 0;
+            if (((uintptr_t)dst & 15u) == 0) {
+                const uint32_t nv = bytes / 16;
+                for (uint32_t i = l; i < nv; i += 64) reinterpret_cast<uint4*>(dst)[i] = ost[i];
+                done = nv * 16 / (uint32_t)sizeof(T);
+            }
+            for (uint32_t i = done + l; i < cnt; i += 64) dst[i] = st[i];
+        }
+    } else {
+        ok = dec_partition<T, false>(h.cells + pe, ncell, tb, nbit, cnt, keys, nullptr, dst);
+    }
+    if (!ok && l == 0) *d_status = 1;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(64 * dec_waves<T>())
 huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
@@ -653,49 +699,10 @@ huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict_
         return;
     }
     const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
-    bool zero_len;
-    const DecTables tb = dec_build<T, 64 * DEC_WAVES>(in, h, s_tab, zero_len);
+    const DecTables tb = dec_build<T, 64 * DEC_WAVES>(in, h, s_tab);
     const uint32_t w = wave_in_wg();
-    const uint32_t l = (uint32_t)lane_id();
-    uint32_t* cst = s_cells[w];
-    T* ost = reinterpret_cast<T*>(s_out[w]);
-    for (uint32_t p = blockIdx.x * DEC_WAVES + w; p < h.pardeg; p += gridDim.x * DEC_WAVES) {
-        const uint32_t nbit = h.par_nbit[p];
-        const uint32_t pe = h.par_entry[p];
-        const uint32_t ncell = (uint32_t)(((uint64_t)nbit + 31) / 32);
-        const uint64_t o0 = (uint64_t)p * h.sublen;
-        const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
-        T* dst = out + o0;
-        if ((uint64_t)pe + ncell > h.ncells) {
-            if (l == 0) *d_status = 1;
-            continue;
-        }
-        if (zero_len && nbit == 0) {
-            dec_constant(dst, cnt, h.nkeys ? keys[0] : (T)0);
-            continue;
-        }
-        bool ok;
-        if (ncell <= DEC_CELLS && h.sublen <= DEC_SUBLEN_MAX) {
-            wave_lds_sync();  // the previous partition's staging reads are done
-            for (uint32_t i = l; i < ncell + 4; i += 64) cst[i] = i < ncell ? h.cells[pe + i] : 0u;
-            wave_lds_sync();
-            ok = dec_partition<T, true>(cst, ncell, tb, nbit, cnt, keys, ost, dst);
-            wave_lds_sync();
-            if (ok) {
-                const uint32_t bytes = cnt * (uint32_t)sizeof(T);
-                uint32_t done = 0;
-                if (((uintptr_t)dst & 15u) == 0) {
-                    const uint32_t nv = bytes / 16;
-                    for (uint32_t i = l; i < nv; i += 64) reinterpret_cast<uint4*>(dst)[i] = s_out[w][i];
-                    done = nv * 16 / (uint32_t)sizeof(T);
-                }
-                for (uint32_t i = done + l; i < cnt; i += 64) dst[i] = ost[i];
-            }
-        } else {
-            ok = dec_partition<T, false>(h.cells + pe, ncell, tb, nbit, cnt, keys, ost, dst);
-        }
-        if (!ok && l == 0) *d_status = 1;
-    }
+    for (uint32_t p = blockIdx.x * DEC_WAVES + w; p < h.pardeg; p += gridDim.x * DEC_WAVES)
+        dec_wave<T>(h, tb, keys, p, n, out, s_cells[w], s_out[w], d_status);
 }
 
 // ---------------------------------------------------------------------------
@@ -721,13 +728,9 @@ huf_dec_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict_
 //     its 64 partitions (2-byte symbols).
 // Serial over a partition (about 113 us for 768 symbols on any stream), and
 // bound by VALU issue (33 instructions a step) beside the LDS probe latency
-// once three waves share a SIMD.  One wave per partition against one lane
-// per partition, 768 symbols each, spiky / smooth field: 2^24 symbols 95 /
-// 70 against 121 / 127 us, 20 Mi 115 / 95 against 120 / 131, 2^25 185 / 141
-// against 121 / 128, 2^26 340 / 257 against 161 / 171, 2^27 595 / 490
-// against 244 / 246.
-constexpr size_t DECL_MIN_PARTS = 32768;
-constexpr int DECL_WAVES = 4;  // with 52.6 KiB of LDS three workgroups fit a CU: three waves per SIMD
+// once three waves share a SIMD: 2^27 symbols 244 us, one wave per partition
+// 595 / 490 (spiky / smooth field).  dec_by_lanes says which streams.
+constexpr int DECL_WAVES = 4;  // with 52.4 KiB of LDS three workgroups fit a CU: three waves per SIMD
 
 typedef uint32_t huf_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -742,19 +745,29 @@ struct LaneDec {
     uint4 q0, q1;
     uint32_t w0, w1, s;  // window = {w0, w1} >> s, s < 32; w1 = cell rp - 1
 
+    // Both arms write whole tuples: with the tail's words loaded behind a branch
+    // each, the compiler lost one word of a tuple (its store's address was
+    // computed into the tuple's own second register).
     __device__ __forceinline__ void fetch(const DecHead& h) {
         // the stream is below 4 GiB: 32-bit byte offsets
         const char* c = reinterpret_cast<const char*>(h.cells);
-        const uint32_t o = 4 * (base + F);
         if (F + 8 <= left) {
+            const uint32_t o = 4 * (base + F);
             const huf_u32x4_a4 x = *reinterpret_cast<const huf_u32x4_a4*>(c + o);
             const huf_u32x4_a4 y = *reinterpret_cast<const huf_u32x4_a4*>(c + o + 16);
             q0 = make_uint4(x.x, x.y, x.z, x.w);
             q1 = make_uint4(y.x, y.y, y.z, y.w);
-        } else {
-            auto at = [&](uint32_t i) { return F + i < left ? *reinterpret_cast<const uint32_t*>(c + o + 4 * i) : 0u; };
-            q0 = make_uint4(at(0), at(1), at(2), at(3));
-            q1 = make_uint4(at(4), at(5), at(6), at(7));
+        } else {  // the stream's last cells (it has one: dec_by_lanes), zeros past them
+            uint32_t v[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) {
+                const uint32_t k = min(base + min(F + i, left), h.ncells - 1);
+                v[i] = *reinterpret_cast<const uint32_t*>(c + 4 * k);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) v[i] = F + i < left ? v[i] : 0u;
+            q0 = make_uint4(v[0], v[1], v[2], v[3]);
+            q1 = make_uint4(v[4], v[5], v[6], v[7]);
         }
     }
     __device__ __forceinline__ void commit() {
@@ -866,51 +879,98 @@ __device__ __forceinline__ void dec_lanes(const DecHead& h, const DecTables& t, 
     if (on && ((acc & (1u << 30)) || d.bitpos() != nbit)) *d_status = 1;
 }
 
+// Streams of at least this many coarse partitions are decoded by lanes or by
+// waves as dec_by_lanes says; shorter ones by waves.
+constexpr size_t DECL_MIN_PARTS = 32768;
+constexpr unsigned DEC_MAX_BLOCKS = 768;  // of the decode by waves: three per CU
+
+// What the two take, from 24 Mi to 48 Mi symbols of 1.1 to 7.7 bits:
+//   lanes  0.168 us (2-byte keys; 1-byte 0.156) a symbol of a partition, for
+//          any number of partitions up to a wave per SIMD (65536)
+//   waves  a partition: 1.35 ns, 0.4 (0.35) a bit of its average code, 0.06 for
+//          each codeword that a lane's span of at least 32 bits holds beyond
+//          a 64th of the partition; 10 more where it repeats one code of two
+//          or more bits, as spans then never fall into step and settle one lane
+//          a round
+// Waves / lanes in us, partitions of 768 symbols, 2-byte keys, bits a symbol in
+// brackets: 24 Mi symbols [7.3] 145 / 126, [2.8] 82 / 128, [1.1] 87 / 109; 36 Mi
+// 214 / 128, 118 / 130, 131 / 111; 48 Mi 264 / 130, 141 / 131, 165 / 112; 32 Mi in
+// runs 560 / 107.  1024 symbols [7.3]: 24 Mi 117 / 173, 36 Mi 169 / 175, 48 Mi
+// 215 / 176.  Partitions of more than DEC_SUBLEN_MAX symbols (the encoder writes 768
+// and 1024), or whose segments of 16 are not 16-byte aligned, go by waves.
 template <typename T>
-__global__ void __launch_bounds__(64 * DECL_WAVES)
-huf_dec_lane_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
+__device__ __forceinline__ bool dec_by_lanes(const DecHead& h, uint64_t n) {
+    if (h.sublen % 16 != 0 || h.sublen > DEC_SUBLEN_MAX || h.zero_len || h.ncells == 0) return false;
+    constexpr float LANE = sizeof(T) == 1 ? 156.0f : 168.0f, BIT = sizeof(T) == 1 ? 0.35f : 0.4f;  // ns
+    const float lanes = LANE * (float)h.sublen;
+    const float bits = 32.0f * (float)h.ncells / (float)n;
+    const float steps = 32.0f / bits - (float)h.sublen / 64.0f;
+    const float wave = 1.35f + BIT * bits + (steps > 0.0f ? 0.06f * steps : 0.0f);
+    if (wave * (float)h.pardeg > lanes) return true;
+    // two cells in the middle of 64 partitions across the stream: do they
+    // repeat with a period of up to 12 bits?
+    const uint32_t p = (uint32_t)((uint64_t)lane_id() * (h.pardeg - 1) / 64);
+    const uint32_t nbit = h.par_nbit[p], at = h.par_entry[p] + nbit / 64;
+    bool repeats = false;
+    if (nbit >= h.sublen + h.sublen / 2 && (uint64_t)at + 2 <= h.ncells) {
+        const uint64_t w = ((uint64_t)h.cells[at] << 32) | h.cells[at + 1];
+#pragma unroll
+        for (int l = 1; l <= 12; l++) repeats |= ((w ^ (w << l)) >> l) == 0;
+    }
+    const float runs = (float)__popcll(__ballot(repeats)) / 64.0f;
+    return (wave + 10.0f * runs) * (float)h.pardeg > lanes;
+}
+
+template <typename T>
+union DecLongLds {
+    struct {
+        uint32_t cells[dec_waves<T>()][DEC_CELLS + 4];
+        uint4 out[dec_waves<T>()][DEC_SUBLEN_MAX * sizeof(T) / 16];
+    } wave;
+    struct {
+        uint4 ring[DECL_WAVES][64 * 4];
+        uint32_t strip[DECL_WAVES][64 * 8 * sizeof(T)];
+    } lane;
+};
+
+// Long streams: huf_dec_kernel's waves, or the first DECL_WAVES of them with a
+// partition per lane; one launch for both, as only the stream says which (the
+// LDS and the 78 registers of either leave room for three workgroups per CU; a
+// table build in each branch, as one before both spilled scalars).
+template <typename T>
+__global__ void __launch_bounds__(64 * dec_waves<T>())
+huf_dec_long_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes, T* __restrict__ out, uint64_t n,
                     int* __restrict__ d_status) {
     static_assert(sizeof(T) <= 2, "the tables hold the symbols of 1- and 2-byte keys");
+    constexpr uint32_t WAVES = dec_waves<T>();
     __shared__ DecLds s_tab;
-    __shared__ uint4 s_ring[DECL_WAVES][64 * 4];
-    __shared__ uint32_t s_strip[DECL_WAVES][64 * 8 * sizeof(T)];
+    __shared__ DecLongLds<T> s;
     DecHead h;
     if (!dec_head<T>(in, in_bytes, n, h)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) *d_status = 1;
         return;
     }
     const T* keys = reinterpret_cast<const T*>(in + h.e1 + 256);
-    bool zero_len;
-    const DecTables tb = dec_build<T, 64 * DECL_WAVES>(in, h, s_tab, zero_len);
     const uint32_t w = wave_in_wg();
-    const uint32_t l = (uint32_t)lane_id();
-    const bool whole = h.sublen % 16 == 0;  // segments of 16 symbols, 16-byte aligned
+    if (!dec_by_lanes<T>(h, n)) {
+        if (blockIdx.x >= DEC_MAX_BLOCKS) return;
+        const DecTables tb = dec_build<T, 64 * WAVES>(in, h, s_tab);
+        const uint32_t stride = min(gridDim.x, DEC_MAX_BLOCKS) * WAVES;
+        for (uint32_t p = blockIdx.x * WAVES + w; p < h.pardeg; p += stride)
+            dec_wave<T>(h, tb, keys, p, n, out, s.wave.cells[w], s.wave.out[w], d_status);
+        return;
+    }
+    if (blockIdx.x * DECL_WAVES * 64 >= h.pardeg) return;
+    const DecTables tb = dec_build<T, 64 * WAVES>(in, h, s_tab);
+    if (w >= DECL_WAVES) return;
     for (uint32_t p0 = (blockIdx.x * DECL_WAVES + w) * 64; p0 < h.pardeg; p0 += gridDim.x * DECL_WAVES * 64) {
-        const uint32_t p = p0 + l;
-        bool odd = false;
-        if (p < h.pardeg) {
-            const uint32_t nbit = h.par_nbit[p];
-            odd = (uint64_t)h.par_entry[p] + ((uint64_t)nbit + 31) / 32 > h.ncells || (zero_len && nbit == 0);
-        }
-        if (whole && !__ballot(odd)) {
-            dec_lanes<T>(h, tb, keys, p0, n, out, reinterpret_cast<uint32_t*>(s_ring[w]), s_strip[w], d_status);
+        const uint32_t p = p0 + (uint32_t)lane_id();
+        const bool bad = p < h.pardeg && (uint64_t)h.par_entry[p] + ((uint64_t)h.par_nbit[p] + 31) / 32 > h.ncells;
+        if (__ballot(bad)) {  // cells past the end: the stream is refused
+            if (lane_id() == 0) *d_status = 1;
             continue;
         }
-        // other layouts, constant and malformed partitions: the wave takes them in turn
-        for (uint32_t r = 0; r < 64 && p0 + r < h.pardeg; r++) {
-            const uint32_t nbit = h.par_nbit[p0 + r], pe = h.par_entry[p0 + r];
-            const uint32_t ncell = (uint32_t)(((uint64_t)nbit + 31) / 32);
-            const uint64_t o0 = (uint64_t)(p0 + r) * h.sublen;
-            const uint32_t cnt = (uint32_t)((n - o0) < (uint64_t)h.sublen ? (n - o0) : (uint64_t)h.sublen);
-            bool ok = (uint64_t)pe + ncell <= h.ncells;
-            if (ok) {
-                if (zero_len && nbit == 0)
-                    dec_constant(out + o0, cnt, h.nkeys ? keys[0] : (T)0);
-                else
-                    ok = dec_partition<T, false>(h.cells + pe, ncell, tb, nbit, cnt, keys, nullptr, out + o0);
-            }
-            if (!ok && l == 0) *d_status = 1;
-        }
+        dec_lanes<T>(h, tb, keys, p0, n, out, reinterpret_cast<uint32_t*>(s.lane.ring[w]), s.lane.strip[w], d_status);
     }
 }
 
@@ -1056,13 +1116,14 @@ int fzh_huffman_decode(void* stream, const void* d_in, size_t in_bytes, int elem
     const size_t pardeg = cdiv(n, SUBLEN);
     hipStream_t s = S(stream);
 #define FZH_HUF_DEC(T)                                                                                         \
-    if (sizeof(T) <= 2 && pardeg >= DECL_MIN_PARTS) {                                                        \
+    if (sizeof(T) <= 2 && pardeg >= DECL_MIN_PARTS) {                                                          \
         using U = std::conditional_t<sizeof(T) <= 2, T, uint16_t>;                                             \
-        const unsigned blocks = (unsigned)std::min<size_t>(cdiv(pardeg, 64 * DECL_WAVES), 65536);              \
-        launch_k("huf_dec_lane_kernel", huf_dec_lane_kernel<U>, dim3(blocks), dim3(64 * DECL_WAVES), 0, s,     \
+        const unsigned blocks = (unsigned)std::min<size_t>(                                                    \
+            std::max<size_t>(cdiv(pardeg, 64 * DECL_WAVES), DEC_MAX_BLOCKS), 65536);                           \
+        launch_k("huf_dec_long_kernel", huf_dec_long_kernel<U>, dim3(blocks), dim3(64 * dec_waves<U>()), 0, s, \
                  (const uint8_t*)d_in, in_bytes, (U*)d_out, n, d_status);                                      \
     } else {                                                                                                   \
-        const unsigned blocks = (unsigned)std::min<size_t>(cdiv(pardeg, dec_waves<T>()), 768);                \
+        const unsigned blocks = (unsigned)std::min<size_t>(cdiv(pardeg, dec_waves<T>()), DEC_MAX_BLOCKS);     \
         launch_k("huf_dec_kernel", huf_dec_kernel<T>, dim3(blocks), dim3(64 * dec_waves<T>()), 0, s,          \
                  (const uint8_t*)d_in, in_bytes, (T*)d_out, n, d_status);                                      \
     }
