@@ -637,7 +637,14 @@ __device__ __forceinline__ DecTables dec_build(const uint8_t* __restrict__ in, c
 // A partition whose book has one symbol with a zero-length code.
 template <typename T>
 __device__ __forceinline__ void dec_constant(T* __restrict__ dst, uint32_t cnt, T v) {
-    for (uint32_t j = (uint32_t)lane_id(); j < cnt; j += 64) dst[j] = v;
+    constexpr uint32_t E = 16 / sizeof(T);
+    uint32_t done = 0;
+    if (((uintptr_t)dst & 15u) == 0) {
+        const uint32_t w = sizeof(T) == 4 ? (uint32_t)v : (uint32_t)v * (sizeof(T) == 1 ? 0x01010101u : 0x00010001u);
+        for (uint32_t j = (uint32_t)lane_id(); j < cnt / E; j += 64) reinterpret_cast<uint4*>(dst)[j] = make_uint4(w, w, w, w);
+        done = cnt / E * E;
+    }
+    for (uint32_t j = done + (uint32_t)lane_id(); j < cnt; j += 64) dst[j] = v;
 }
 
 // Partition p, decoded by one wave; cst and ost: the wave's DEC_CELLS + 4 words

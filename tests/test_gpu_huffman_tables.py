@@ -54,3 +54,17 @@ def test_long_streams(gpu, orc, c, d, deep):
     reps = -(-LONG // block.size)
     s, n = _repeat(block, block[:100], bk4, rev, 1024, 768, reps)
     assert np.array_equal(gpu.huffman_decode(s, np.uint16, n), np.concatenate([np.tile(block, reps), block[:100]]))
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.uint32])
+@pytest.mark.parametrize("sublen", [768, 333, 5])
+@pytest.mark.parametrize("n", [1, 15, 767, 769, 100_003])
+def test_constant(gpu, orc, dtype, sublen, n):
+    """One symbol, whose code has no bits: partitions on and off 16-byte alignment."""
+    from test_cpu_oracle import huffman_stream_def
+    bklen = 256 if dtype == np.uint8 else 1024
+    f = np.zeros(bklen, np.uint32)
+    f[201] = n
+    bk4, rev = orc.huffman_book(f, np.dtype(dtype).itemsize)
+    v = np.full(n, 201, dtype)
+    assert np.array_equal(gpu.huffman_decode(huffman_stream_def(v, bk4, rev, bklen, sublen), dtype, n), v)
