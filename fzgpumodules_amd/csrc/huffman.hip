@@ -116,7 +116,9 @@ constexpr unsigned ENC_BLOCKS = 4096;  // encode workgroups, at most
 // Each workgroup stages the codebook once (bklen <= 8192: BOOK_LDS) and takes
 // several partitions, one per wave at a time (huf_encode_partition); more
 // workgroups (one partition a wave: 117 us for 2^27 symbols, now 96) stage it
-// more often, fewer (2048: 103) leave too few waves to cover the loads.
+// more often, fewer (2048: 103) leave too few waves to cover the loads.  A
+// larger book stays in memory, and every wave takes one partition (2^25
+// symbols of 16384: 93 us, 97 with ENC_BLOCKS).
 template <typename T, int SL, bool BOOK_LDS>
 __global__ void __launch_bounds__(256)
 huf_enc_kernel(const T* __restrict__ in, uint64_t n, uint32_t bklen, const uint32_t* __restrict__ bk4,
@@ -1019,7 +1021,7 @@ int enc_impl(hipStream_t s, const void* in, size_t n, uint32_t bklen, const uint
     const bool book_in_lds = bklen <= 8192;
     const size_t lds = (size_t)4 * CELLS * 4 + (book_in_lds ? 4 * (size_t)bklen : 0);
     const unsigned blocks = (unsigned)cdiv(pardeg, 4);
-    const unsigned eb = std::min(blocks, ENC_BLOCKS);
+    const unsigned eb = book_in_lds ? std::min(blocks, ENC_BLOCKS) : blocks;
     if (book_in_lds)
         launch_k("huf_enc_kernel", huf_enc_kernel<T, SL, true>, dim3(eb), dim3(256), (uint32_t)lds, s, (const T*)in, n,
                  bklen, bk4, rev, rev_bytes, o8, scells, ncell, pardeg);
