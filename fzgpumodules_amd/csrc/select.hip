@@ -304,13 +304,32 @@ __device__ __forceinline__ void forward_one(const Lds& s, const float* __restric
     }
 }
 
-// Forward of a batch, one sample per wave: lane o sums output o of each layer
-// in forward_one's order, the activations pass through LDS.  (One thread per
-// sample, as in training, is a chain of 6.5 Ki dependent multiply-adds on two
-// workgroups for 512 samples: 54 us, now 18.)
+// Forward of a batch, one sample per thread as in training: a chain of 6.5 Ki
+// dependent multiply-adds (54 us for any count that leaves a CU one
+// workgroup) whose weights, read from LDS, serve 64 samples at a time.
 __global__ void __launch_bounds__(256)
 mlp_forward_kernel(const float* __restrict__ p, const float* __restrict__ norm, const float* __restrict__ feat,
                    uint64_t n, float* __restrict__ logits) {
+    __shared__ Lds s;
+    load_params(s, p, norm);
+    __syncthreads();
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float xb[NF], h1b[H1], h2b[H2], z[NC];
+    forward_one(s, feat + i * NF, xb, h1b, h2b, z);
+#pragma unroll
+    for (int o = 0; o < NC; o++) logits[i * NC + o] = z[o];
+}
+
+// The same for fewer samples, one per wave: lane o sums output o of each layer
+// in forward_one's order, the activations pass through LDS.  512 samples 18 us
+// (54 by threads), 2048 29 (55), 4096 51 (55), but 8192 98 (55) and 2^20 11.5 ms
+// (0.39).
+constexpr uint64_t MLP_WAVES_MAX = 4096;  // samples that go by waves, at most
+
+__global__ void __launch_bounds__(256)
+mlp_forward_wave_kernel(const float* __restrict__ p, const float* __restrict__ norm, const float* __restrict__ feat,
+                        uint64_t n, float* __restrict__ logits) {
     static_assert(NF <= 64 && H1 <= 64 && H2 <= 64 && NC <= 64, "one lane per output");
     __shared__ Lds s;
     __shared__ float act[4][3][64];
@@ -726,7 +745,10 @@ int fzs_mlp_forward(void* stream, const float* d_params, const float* d_norm, co
                     float* d_logits) {
     if (n == 0) return FZH_OK;
     if (!d_params || !d_norm || !d_feat || !d_logits) return fail(FZH_E_INVALID, "mlp forward: null pointer");
-    mlp_forward_kernel<<<(unsigned)cdiv(n, 4), 256, 0, S(stream)>>>(d_params, d_norm, d_feat, n, d_logits);
+    if (n <= MLP_WAVES_MAX)
+        mlp_forward_wave_kernel<<<(unsigned)cdiv(n, 4), 256, 0, S(stream)>>>(d_params, d_norm, d_feat, n, d_logits);
+    else
+        mlp_forward_kernel<<<(unsigned)cdiv(n, 256), 256, 0, S(stream)>>>(d_params, d_norm, d_feat, n, d_logits);
     FZH_CHECK_LAUNCH("mlp_forward_kernel");
     return FZH_OK;
 }

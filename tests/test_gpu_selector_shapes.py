@@ -56,3 +56,29 @@ def test_forward_batch_sizes(n):
         np.testing.assert_array_equal(sel.forward(d_f.ptr, n), R.forward(p, norm, feat, "exact32")[0])
     finally:
         sel.close()
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 8449])  # by waves up to 4096, then by threads
+def test_forward_around_the_choice(n):
+    test_forward_batch_sizes(n)
+
+
+def test_forward_time_of_many_samples():
+    """65536 samples take about as long as 4096 (60 and 51 us; 730 by waves)."""
+    from fzgpumodules_amd._fzh import Event, synchronize
+    sel = S.Selector()
+    d_f, d_z = DeviceBuffer.zeros(65536 * 128), DeviceBuffer(65536 * 16)
+    try:
+        best = {}
+        for n in (4096, 65536):
+            best[n] = 1e9
+            for _ in range(8):
+                a, b = Event(), Event()
+                a.record()
+                call("fzs_mlp_forward", None, sel.params.ptr, sel.norm.ptr, d_f.ptr, n, d_z.ptr)
+                b.record()
+                synchronize()
+                best[n] = min(best[n], a.elapsed_ms(b))
+    finally:
+        sel.close()
+    assert best[65536] < 4 * best[4096]
