@@ -62,8 +62,12 @@ def _parse(blob, n):
     return out, blob[oc:oc + n]
 
 
-@pytest.mark.parametrize("shape,n", SHAPES)
-@pytest.mark.parametrize("chain", [1, 2])
+# chunks from which the Huffman chain is batched, and one fewer
+HUFFMAN = [((4096,), 67), ((64, 64), 67), ((64, 64), 66), ((8, 24, 64), 62), ((256, 256), 41), ((256, 256), 40),
+           ((16, 64, 64), 41), ((3, 20, 4096), 19), ((3, 20, 4096), 18)]
+
+
+@pytest.mark.parametrize("chain,shape,n", [(c, *x) for c in (1, 2) for x in SHAPES] + [(2, *x) for x in HUFFMAN])
 def test_chunks_equal_the_pipeline(shape, n, chain):
     sc = S.SelectingCompressor(shape)
     try:
@@ -106,3 +110,23 @@ def test_all_chains_in_one_container():
             assert np.array_equal(got[i], p.compress_array(np.ascontiguousarray(ch))), (i, choice[i])
     sc.close()
     d.free()
+
+
+def test_time_of_a_few_huffman_chunks():
+    """Two noisy chunks through pipelines (0.5 ms, as the quantizer's chain; 3.1 in a batch)."""
+    import time
+    from fzgpumodules_amd._fzh import synchronize
+    x = np.random.default_rng(2).standard_normal((512, 256)).astype(np.float32)
+    d = DeviceBuffer.from_array(x)
+    sc = S.SelectingCompressor((256, 256))
+    best = {}
+    for chain in (2, 3):
+        best[chain] = 1e9
+        for _ in range(12):
+            synchronize()
+            t = time.perf_counter()
+            sc.compress(d.ptr, x.shape, 1e-3, mode=S.FIXED, chain=chain)
+            best[chain] = min(best[chain], time.perf_counter() - t)
+    sc.close()
+    d.free()
+    assert best[2] < 3 * best[3]
