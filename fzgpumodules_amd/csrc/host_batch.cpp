@@ -57,7 +57,11 @@ struct BatchCompressor::Impl {
         if (arena) (void)hipFree(arena);
         arena = nullptr;
         cap = 0;
-        hipck(hipMalloc((void**)&arena, bytes), "hipMalloc (batch)");
+        if (const hipError_t e = hipMalloc((void**)&arena, bytes); e != hipSuccess) {
+            arena = nullptr;
+            (void)hipGetLastError();
+            throw OutOfDeviceMemory(std::string("hipMalloc (batch): ") + hipGetErrorString(e));
+        }
         cap = bytes;
     }
     void* dev(size_t bytes) {
@@ -106,6 +110,8 @@ BatchCompressor::~BatchCompressor() {
     if (graph_stream_) (void)hipStreamDestroy(graph_stream_);
     release();
 }
+
+size_t BatchCompressor::memoryBytes() const { return impl_ ? impl_->cap : 0; }
 
 void BatchCompressor::setErrorBound(float eb) {
     if (!(eb > 0.0f) || !std::isfinite(eb))

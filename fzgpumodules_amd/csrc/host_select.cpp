@@ -231,59 +231,74 @@ class ChainSelectCompressor {
             last[choice_[c]] = c;
         }
         hipck(hipStreamSynchronize(s), "hipStreamSynchronize");  // chunks_ and the choices are ready
-        const auto batched = [&](int k) {
-            return (k == 1 && list[k].size() >= kBatchMin) || (k == 2 && list[k].size() >= huffmanBatchMin(E));
-        };
+        bool in_batch[FZS_NCHAINS] = {false, list[1].size() >= kBatchMin, list[2].size() >= huffmanBatchMin(E), false};
+        const auto batched = [&](int k) { return in_batch[k]; };
         std::vector<uint64_t> single;
         for (uint64_t c = 0; c < n; c++)
             if (!batched(choice_[c]) || c == last[choice_[c]]) single.push_back(c);
-        const int W = (int)std::min<size_t>(kWorkers, single.size());
-        while ((int)workers_.size() < W) {
-            workers_.push_back(std::make_unique<Worker>());
-            hipck(hipStreamCreate(&workers_.back()->s), "hipStreamCreate");
-        }
-        int rec_worker[FZS_NCHAINS] = {0, 0, 0, 0};  // the worker that ran each chain's last chunk
-        for (size_t i = 0; i < single.size(); i++) {
-            const int w = (int)(i % (size_t)W), k = choice_[single[i]];
-            if (single[i] == last[k]) rec_worker[k] = w;
-            Worker& wk = *workers_[w];
-            if (!wk.chain[k].p || wk.chain_eb[k] != abs_eb) {
-                wk.chain[k] = make_chain(k, abs_eb, cx_, cy_, cz_);
-                wk.chain_eb[k] = abs_eb;
-            }
-        }
         std::vector<std::vector<uint8_t>> blobs(n);
-        std::vector<std::exception_ptr> errs(W);
-        std::vector<std::thread> th;
-        for (int w = 0; w < W; w++)
-            th.emplace_back([&, w] {
-                try {
-                    Worker& wk = *workers_[w];
-                    for (size_t i = (size_t)w; i < single.size(); i += (size_t)W) {
-                        const uint64_t c = single[i];
-                        void* d_out = nullptr;
-                        size_t bytes = 0;
-                        wk.chain[choice_[c]].p->compress((const float*)chunks_.p + c * E, 4 * E, &d_out, &bytes, wk.s);
-                        blobs[c].resize(bytes);
-                        hipck(hipMemcpyAsync(blobs[c].data(), d_out, bytes, hipMemcpyDeviceToHost, wk.s),
-                              "hipMemcpyAsync");
-                        hipck(hipStreamSynchronize(wk.s), "hipStreamSynchronize");
-                    }
-                } catch (...) {
-                    errs[w] = std::current_exception();
+        int rec_worker[FZS_NCHAINS] = {0, 0, 0, 0};  // the worker that ran each chain's last chunk
+        // the chunks of `single` through the workers' pipelines, `meanwhile` on this thread
+        const auto run_single = [&](auto meanwhile) {
+            const int W = (int)std::min<size_t>(kWorkers, single.size());
+            while ((int)workers_.size() < W) {
+                workers_.push_back(std::make_unique<Worker>());
+                hipck(hipStreamCreate(&workers_.back()->s), "hipStreamCreate");
+            }
+            for (size_t i = 0; i < single.size(); i++) {
+                const int w = (int)(i % (size_t)W), k = choice_[single[i]];
+                if (single[i] == last[k]) rec_worker[k] = w;
+                Worker& wk = *workers_[w];
+                if (!wk.chain[k].p || wk.chain_eb[k] != abs_eb) {
+                    wk.chain[k] = make_chain(k, abs_eb, cx_, cy_, cz_);
+                    wk.chain_eb[k] = abs_eb;
                 }
-            });
-        std::exception_ptr batch_err;
-        try {
+            }
+            std::vector<std::exception_ptr> errs(W);
+            std::vector<std::thread> th;
+            for (int w = 0; w < W; w++)
+                th.emplace_back([&, w] {
+                    try {
+                        Worker& wk = *workers_[w];
+                        for (size_t i = (size_t)w; i < single.size(); i += (size_t)W) {
+                            const uint64_t c = single[i];
+                            void* d_out = nullptr;
+                            size_t bytes = 0;
+                            wk.chain[choice_[c]].p->compress((const float*)chunks_.p + c * E, 4 * E, &d_out, &bytes,
+                                                             wk.s);
+                            blobs[c].resize(bytes);
+                            hipck(hipMemcpyAsync(blobs[c].data(), d_out, bytes, hipMemcpyDeviceToHost, wk.s),
+                                  "hipMemcpyAsync");
+                            hipck(hipStreamSynchronize(wk.s), "hipStreamSynchronize");
+                        }
+                    } catch (...) {
+                        errs[w] = std::current_exception();
+                    }
+                });
+            std::exception_ptr err;
+            try {
+                meanwhile();
+            } catch (...) {
+                err = std::current_exception();
+            }
+            for (auto& t : th) t.join();
+            for (auto& e : errs)
+                if (e) std::rethrow_exception(e);
+            if (err) std::rethrow_exception(err);
+        };
+        run_single([&] {
             for (int k = 1; k <= 2; k++)
-                if (batched(k)) run_batch(s, k, abs_eb, list[k]);
-        } catch (...) {
-            batch_err = std::current_exception();
+                if (batched(k)) in_batch[k] = run_batch(s, k, abs_eb, list[k]);
+        });
+        // chains whose batch found no memory (its scratch is several times the
+        // chunks, a pipeline's that of one): their other chunks, too
+        std::vector<uint64_t> left;
+        for (uint64_t c = 0; c < n; c++)
+            if (!batched(choice_[c]) && blobs[c].empty()) left.push_back(c);
+        if (!left.empty()) {
+            single = std::move(left);
+            run_single([] {});
         }
-        for (auto& t : th) t.join();
-        for (auto& e : errs)
-            if (e) std::rethrow_exception(e);
-        if (batch_err) std::rethrow_exception(batch_err);
         const double t2 = now_ms();
         // container: chain k's stages are described by the pipeline that
         // compressed the last chunk choosing k
@@ -466,8 +481,9 @@ class ChainSelectCompressor {
   private:
     // Compresses the chunks `c` (all on chain k, 1 or 2) in one batch on
     // stream s.  The plan is kept while the chunk list and the bound stay the
-    // same; a new one reuses the batch's memory.
-    void run_batch(hipStream_t s, int k, float abs_eb, const std::vector<uint64_t>& c) {
+    // same; a new one reuses the batch's memory.  False if the device has no
+    // memory for it.
+    bool run_batch(hipStream_t s, int k, float abs_eb, const std::vector<uint64_t>& c) {
         const uint64_t E = (uint64_t)cx_ * cy_ * cz_;
         Batch& B = batch_[k];
         if (!B.b) {
@@ -492,12 +508,25 @@ class ChainSelectCompressor {
                 f[i].ny = cy_;
                 f[i].nz = cz_;
             }
-            B.b->setFields(f);
+            try {
+                B.b->setFields(f);
+            } catch (const OutOfDeviceMemory&) {
+                B.b.reset();
+                return false;
+            }
+            // a large batch has to leave something to the pipelines and the container
+            size_t free = 0, total = 0;
+            if (const size_t held = B.b->memoryBytes();
+                held > (1ull << 30) && hipMemGetInfo(&free, &total) == hipSuccess && free < held / 8) {
+                B.b.reset();
+                return false;
+            }
             B.eb = abs_eb;
             B.idx = c;
             B.base = chunks_.p;
         }
         B.b->compress(s);
+        return true;
     }
 
     static constexpr int kWorkers = 8;

@@ -12,6 +12,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <stdexcept>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,11 @@ struct BatchLaunch {
     uint32_t scatter_wg_per_cu = 2;
 };
 
+// A plan found no device memory.
+struct OutOfDeviceMemory : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
 class BatchCompressor {
   public:
     explicit BatchCompressor(const BatchConfig& cfg);
@@ -59,8 +65,9 @@ class BatchCompressor {
     BatchCompressor& operator=(const BatchCompressor&) = delete;
 
     // Plans the batch: device tables, codes/scratch/output buffers (one
-    // allocation, kept for later plans that fit it).
+    // allocation of memoryBytes(), kept for later plans that fit it).
     void setFields(const std::vector<BatchField>& fields);
+    size_t memoryBytes() const;
     // The bound of the plans made from now on.
     void setErrorBound(float eb);
     size_t numFields() const { return fields_.size(); }

@@ -130,3 +130,28 @@ def test_time_of_a_few_huffman_chunks():
     sc.close()
     d.free()
     assert best[2] < 3 * best[3]
+
+
+def test_batch_without_memory():
+    """A field whose batch does not fit the memory that is left: the same container
+    through pipelines, whose scratch is that of a chunk."""
+    import ctypes as C
+    from fzgpumodules_amd._fzh import lib
+    x = np.cumsum(np.random.default_rng(1).standard_normal((256 * 256, 256)) * 0.01, axis=1).astype(np.float32)
+    d = DeviceBuffer.from_array(x)  # 64 MiB; the batch takes 170
+    blobs = []
+    for leave in (None, 110 << 20):
+        sc = S.SelectingCompressor((256, 256))
+        if leave is not None:
+            sc.compress(d.ptr, (256 * 3, 256), 1e-3, mode=S.FIXED, chain=2)  # the handle's streams and pipelines
+            full = []
+            for _ in range(4):  # (the free size that is reported is coarse next to a large buffer)
+                free, total = C.c_size_t(), C.c_size_t()
+                assert lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+                if free.value > leave + x.nbytes + (8 << 20):
+                    full.append(DeviceBuffer(free.value - leave - x.nbytes))
+        blobs.append(sc.compress(d.ptr, x.shape, 1e-3, mode=S.FIXED, chain=2))
+        sc.close()
+    for b in [*full, d]:
+        b.free()
+    assert np.array_equal(*blobs)
