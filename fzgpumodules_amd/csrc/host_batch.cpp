@@ -34,9 +34,11 @@ uint64_t align_to(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 }  // namespace
 
 // A plan's device memory: one allocation, kept for the next plan if that one
-// fits it (a selector plans its chunks anew for every field; some twenty
-// allocations and table copies were 2 ms of each plan).  Tables come first
-// and are collected on the host, so they go up in one copy.
+// fits it and needs at least half of it (or it is below kKeep), so that a small
+// batch does not hold a large one's memory (a selector plans its chunks anew
+// for every field; some twenty allocations and table copies were 2 ms of each
+// plan).  Tables come first and are collected on the host, so they go up in
+// one copy.
 struct BatchCompressor::Impl {
     fzh::batch::Plan plan{};
     fzh::batch::Plan* d_plan = nullptr;  // device copy read by the kernels
@@ -49,11 +51,12 @@ struct BatchCompressor::Impl {
     hipEvent_t ev[9] = {};
 
     static size_t piece(size_t bytes) { return align_to(std::max<size_t>(bytes, 256), 256); }
+    static constexpr size_t kKeep = 64 << 20;
     // Starts a plan of `bytes` (a sum of pieces).
     void reserve(size_t bytes) {
         used = 0;
         tables.clear();
-        if (cap >= bytes) return;
+        if (cap >= bytes && cap <= std::max(2 * bytes, kKeep)) return;
         if (arena) (void)hipFree(arena);
         arena = nullptr;
         cap = 0;

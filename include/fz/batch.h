@@ -65,7 +65,8 @@ class BatchCompressor {
     BatchCompressor& operator=(const BatchCompressor&) = delete;
 
     // Plans the batch: device tables, codes/scratch/output buffers (one
-    // allocation of memoryBytes(), kept for later plans that fit it).
+    // allocation of memoryBytes(), kept for later plans that fit it and need
+    // half of it or more).
     void setFields(const std::vector<BatchField>& fields);
     size_t memoryBytes() const;
     // The bound of the plans made from now on.

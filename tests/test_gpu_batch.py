@@ -230,3 +230,45 @@ def test_batch_rejects_bad_fields():
         d.free()
     finally:
         b.close()
+
+
+def test_batch_memory_of_a_smaller_plan():
+    """A small batch after a large one gives its memory back; one of about the same size
+    keeps it, and the results are those of a new handle."""
+    import ctypes as C
+    import time
+
+    from fzgpumodules_amd._fzh import lib, synchronize
+
+    def free():
+        synchronize()  # freed memory is seen behind a synchronisation
+        time.sleep(0.05)
+        f, t = C.c_size_t(), C.c_size_t()
+        assert lib().hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    rng = np.random.default_rng(3)
+    n = 1 << 26
+    d = DeviceBuffer.zeros(4 * n)
+    x = np.cumsum(rng.standard_normal(3 << 20) * 0.01).astype(np.float32)
+    d.upload(x)
+    b = Batch(error_bound=1e-3, mode="REL")
+    small = [(d.ptr, (1 << 20, 1, 1)), (d.ptr + (4 << 20), (1024, 1024, 1))]
+    b.set_fields(small)
+    before = free()
+    b.compress()
+    want = [b.field_bytes(i) for i in range(2)]
+    b.set_fields([(d.ptr, (n, 1, 1))])  # 0.5 GiB of codes, scratch and output
+    assert before - free() > 400 << 20
+    b.compress()
+    large = b.output()[0]
+    b.set_fields([(d.ptr, (n - 4096 * 100, 1, 1))])
+    assert b.output()[0] - large < 256 << 20  # in the same allocation
+    b.compress()
+    b.set_fields(small)
+    assert before - free() < 96 << 20
+    b.compress()
+    for i in range(2):
+        assert np.array_equal(b.field_bytes(i), want[i])
+    b.close()
+    d.free()
