@@ -264,9 +264,6 @@ scatter_assign_kernel(const float* __restrict__ val, const uint32_t* __restrict_
 // ---------------------------------------------------------------------------
 // Bitpack
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ uint32_t ldv(const T* p, uint64_t i) { return (uint32_t)p[i]; }
-
 // Bound by memory: a thread takes 16 elements, which are whole 16-byte words
 // of the elements and 2 * NB bytes of the packed array, so both sides move in
 // wide accesses and the packing is constant shifts (6 Mi 16-bit codes at 16
@@ -348,22 +345,35 @@ bitpack_dec_vec_kernel(const uint8_t* __restrict__ in, uint64_t n, T* __restrict
     }
 }
 
-// Arrays that are not 16-byte aligned: one thread per packed byte (packing)
-// or element (unpacking).
+// One thread per packed byte (packing to less than 8 bits) or per element:
+// arrays that are not 16-byte aligned (a thread per packed byte of wider
+// elements loads each several times: 16 Mi 32-bit elements 67 us, 35), and
+// unpacking of up to 8 bits to four-byte elements, where a group's 64 bytes per
+// thread leave a wave's stores uncoalesced (16 Mi of 8 bits 24 us, 18; 16 bits 25
+// against 26 by elements, 32 bits 26 against 42).
 template <typename T>
 __global__ void __launch_bounds__(256)
 bitpack_enc_kernel(const T* __restrict__ in, uint64_t n, int nbits, uint8_t* __restrict__ out) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t nout = (n * nbits + 7) / 8;
-    const auto element = [&](uint64_t e) { return (uint32_t)in[e]; };
-    for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < nout; b += stride) {
-        switch (nbits) {
-        case 1: pack_tail<1>(n, out, b, nout, 0, element); break;
-        case 2: pack_tail<2>(n, out, b, nout, 0, element); break;
-        case 4: pack_tail<4>(n, out, b, nout, 0, element); break;
-        case 8: pack_tail<8>(n, out, b, nout, 0, element); break;
-        case 16: pack_tail<16>(n, out, b, nout, 0, element); break;
-        default: pack_tail<32>(n, out, b, nout, 0, element); break;
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (nbits < 8) {
+        const uint64_t nout = (n * nbits + 7) / 8;
+        const auto element = [&](uint64_t e) { return (uint32_t)in[e]; };
+        for (uint64_t b = first; b < nout; b += stride) {
+            switch (nbits) {
+            case 1: pack_tail<1>(n, out, b, nout, 0, element); break;
+            case 2: pack_tail<2>(n, out, b, nout, 0, element); break;
+            default: pack_tail<4>(n, out, b, nout, 0, element); break;
+            }
+        }
+    } else {
+        const int bytes = nbits / 8;
+        for (uint64_t i = first; i < n; i += stride) {
+            uint32_t v = (uint32_t)in[i];
+            for (int b = 0; b < bytes; b++) {
+                out[i * bytes + b] = (uint8_t)v;
+                v >>= 8;
+            }
         }
     }
 }
@@ -392,14 +402,15 @@ void launch_bitpack_vec(hipStream_t s, bool enc, const void* in, size_t n, void*
         const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(n / 16, 256), 8192));
         if (enc)
             bitpack_enc_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const T*)in, n, (uint8_t*)out);
-        else
+        else if constexpr (sizeof(T) < 4 || NB >= 16)
             bitpack_dec_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const uint8_t*)in, n, (T*)out);
     }
 }
 
 template <typename T>
 void launch_bitpack(hipStream_t s, bool enc, const void* in, size_t n, int nbits, void* out) {
-    if (((uintptr_t)in | (uintptr_t)out) % 16 == 0) {
+    const bool groups = enc || sizeof(T) < 4 || nbits >= 16;
+    if (groups && ((uintptr_t)in | (uintptr_t)out) % 16 == 0) {
         switch (nbits) {
         case 1: return launch_bitpack_vec<T, 1>(s, enc, in, n, out);
         case 2: return launch_bitpack_vec<T, 2>(s, enc, in, n, out);
@@ -409,7 +420,7 @@ void launch_bitpack(hipStream_t s, bool enc, const void* in, size_t n, int nbits
         default: return launch_bitpack_vec<T, 32>(s, enc, in, n, out);
         }
     }
-    const size_t work = enc ? (n * nbits + 7) / 8 : n;
+    const size_t work = enc && nbits < 8 ? (n * nbits + 7) / 8 : n;
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(work, 256), 4096));
     if (enc)
         bitpack_enc_kernel<T><<<blocks, 256, 0, s>>>((const T*)in, n, nbits, (uint8_t*)out);
