@@ -122,6 +122,10 @@ __global__ void __launch_bounds__(256) gather_kernel(const fzh_copy_desc* __rest
     uint8_t* dst = (uint8_t*)d[seg].dst;
     const size_t bytes = d[seg].bytes;
     if (!src || !dst || !bytes) return;
+    if (bytes <= 256) {  // a byte a thread, no loop to set up (200000 segments of 64 bytes 58 us, 68 through the loops)
+        if (blockIdx.y == 0 && threadIdx.x < (uint32_t)bytes) gp(dst)[threadIdx.x] = gp(src)[threadIdx.x];
+        return;
+    }
     const size_t G = (size_t)gridDim.y * 256, g = (size_t)blockIdx.y * 256 + threadIdx.x;
     if (((uintptr_t)src | (uintptr_t)dst) % 16 == 0) {
         const size_t nw = bytes / 16;
