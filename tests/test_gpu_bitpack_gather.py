@@ -80,3 +80,33 @@ def test_gather_segments(fzh, n_segs):
     d_desc = fzh.DeviceBuffer.from_array(desc)
     fzh.call("fzh_gather", None, d_desc.ptr, n_segs)
     assert np.array_equal(d_dst.download(np.uint8, want.size), want)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.uint32])
+@pytest.mark.parametrize("n", [65_535, 65_536, 65_537])  # one workgroup, then partial maxima
+@pytest.mark.parametrize("at", [0, 40_000, -1])
+def test_max_around_one_workgroup(fzh, dtype, n, at):
+    v = np.full(n, 3, dtype)
+    v[at] = 201
+    ws = fzh.workspace(fzh.lib().fzh_max_u32_ws_bytes())
+    m = fzh.DeviceBuffer(16)
+    d = fzh.DeviceBuffer.from_array(v)
+    fzh.call("fzh_max_u32", None, d.ptr, n, v.itemsize, m.ptr, ws.ptr, ws.nbytes)
+    assert int(m.download(np.uint32, 1)[0]) == 201
+
+
+@pytest.mark.parametrize("nbytes", [1, 15, 16, 255, 256, 257, 272])  # a byte a thread up to 256
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n_segs", [2, 5000])
+def test_gather_of_small_segments(fzh, nbytes, shift, n_segs):
+    step = 288
+    data = np.random.default_rng(nbytes).integers(0, 256, n_segs * step + 16).astype(np.uint8)
+    d_src, d_dst = fzh.DeviceBuffer.from_array(data), fzh.DeviceBuffer.from_array(np.full(n_segs * step, 7, np.uint8))
+    desc = np.zeros(n_segs, np.dtype([("s", np.uint64), ("d", np.uint64), ("n", np.uint64)]))
+    at = np.arange(n_segs, dtype=np.uint64) * step
+    desc["s"], desc["d"], desc["n"] = d_src.ptr + shift + at, d_dst.ptr + at, nbytes
+    d_desc = fzh.DeviceBuffer.from_array(desc)
+    fzh.call("fzh_gather", None, d_desc.ptr, n_segs)
+    got = d_dst.download(np.uint8, n_segs * step).reshape(n_segs, step)
+    assert np.array_equal(got[:, :nbytes], data[shift:shift + n_segs * step].reshape(n_segs, step)[:, :nbytes])
+    assert (got[:, nbytes:] == 7).all()
