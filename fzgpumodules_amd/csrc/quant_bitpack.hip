@@ -348,9 +348,10 @@ bitpack_dec_vec_kernel(const uint8_t* __restrict__ in, uint64_t n, T* __restrict
 // One thread per packed byte (packing to less than 8 bits) or per element:
 // arrays that are not 16-byte aligned (a thread per packed byte of wider
 // elements loads each several times: 16 Mi 32-bit elements 67 us, 35), and
-// unpacking of up to 8 bits to four-byte elements, where a group's 64 bytes per
-// thread leave a wave's stores uncoalesced (16 Mi of 8 bits 24 us, 18; 16 bits 25
-// against 26 by elements, 32 bits 26 against 42).
+// unpacking of up to 16 bits to four-byte elements, where a group's 64 bytes per
+// thread leave a wave's stores uncoalesced (16 Mi of 8 bits 24 us, 18 by elements;
+// of 16 bits 25 and 26, but with the inverse that reads them 51 and 48 us for 6
+// Mi; 32 bits 26 against 42).
 template <typename T>
 __global__ void __launch_bounds__(256)
 bitpack_enc_kernel(const T* __restrict__ in, uint64_t n, int nbits, uint8_t* __restrict__ out) {
@@ -402,14 +403,14 @@ void launch_bitpack_vec(hipStream_t s, bool enc, const void* in, size_t n, void*
         const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(cdiv(n / 16, 256), 8192));
         if (enc)
             bitpack_enc_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const T*)in, n, (uint8_t*)out);
-        else if constexpr (sizeof(T) < 4 || NB >= 16)
+        else if constexpr (sizeof(T) < 4 || NB > 16)
             bitpack_dec_vec_kernel<T, NB><<<blocks, 256, 0, s>>>((const uint8_t*)in, n, (T*)out);
     }
 }
 
 template <typename T>
 void launch_bitpack(hipStream_t s, bool enc, const void* in, size_t n, int nbits, void* out) {
-    const bool groups = enc || sizeof(T) < 4 || nbits >= 16;
+    const bool groups = enc || sizeof(T) < 4 || nbits > 16;
     if (groups && ((uintptr_t)in | (uintptr_t)out) % 16 == 0) {
         switch (nbits) {
         case 1: return launch_bitpack_vec<T, 1>(s, enc, in, n, out);
@@ -433,9 +434,10 @@ void launch_bitpack(hipStream_t s, bool enc, const void* in, size_t n, int nbits
 // launch whose last workgroup finishes the reduction needs a device fence in
 // every workgroup, which writes back the codes its XCD's L2 still holds: 26
 // us for 6 Mi 2-byte codes, 131 with a single thread reading the partials;
-// 5.9 us for the two launches.)  Up to MAX_ONE elements one workgroup does it in
-// 3.4 to 5.7 us, two launches taking 5.8.
-constexpr size_t MAX_ONE = 65536;
+// 5.9 us for the two launches.)  Up to MAX_ONE bytes one workgroup does it in one
+// launch (3.4 us; 256 KiB that another launch has just written take it 9, though,
+// where the two launches share their loads over many CUs).
+constexpr size_t MAX_ONE = 32768;
 
 template <typename T>
 __device__ __forceinline__ void max_block(const T* __restrict__ in, uint64_t n, uint32_t* __restrict__ partial,
@@ -531,7 +533,7 @@ int max_u32(hipStream_t s, const void* d_in, size_t n, int elem_bytes, uint32_t*
             const PlaceDesc* place) {
     if (ws_bytes < fzh_max_u32_ws_bytes()) return fail(FZH_E_CAPACITY, "max: workspace too small");
     uint32_t* partial = (uint32_t*)((uint8_t*)d_ws + 256);
-    const unsigned blocks = n <= MAX_ONE ? 1u : (unsigned)std::min<size_t>(cdiv(n, 256 * 32), 1024);
+    const unsigned blocks = n * elem_bytes <= MAX_ONE ? 1u : (unsigned)std::min<size_t>(cdiv(n, 256 * 32), 1024);
     if (blocks == 1) partial = d_max;
     const auto launch = [&](auto tag) {
         using T = decltype(tag);
