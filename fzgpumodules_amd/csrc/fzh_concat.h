@@ -41,13 +41,15 @@ struct SizeOverride {
 // the total and then serves the readback entries, taking any word that lies
 // in the header or the total from the values it just computed (so the
 // readback never depends on another workgroup's stores).
-// With `copy` (16-byte aligned, as large as the concat can get) the whole
-// result goes there too, each word stored twice; a slot 0 whose producer
+// With COPY the whole result goes to `copy_out` (16-byte aligned, as large as
+// the concat can get) too, each word stored twice; a slot 0 whose producer
 // stores its stream twice itself (first_done) needs the pad only.
+template <bool COPY>
 __device__ __forceinline__ void concat_readback_body(const ConcatArgs& a, int n, uint8_t* __restrict__ out,
-                                                    uint8_t* __restrict__ copy, uint64_t* __restrict__ total,
+                                                    uint8_t* __restrict__ copy_out, uint64_t* __restrict__ total,
                                                     const ReadbackArgs& r, int nr, uint8_t* __restrict__ mapped,
                                                     uint32_t blk, uint32_t nblk, const SizeOverride& ov) {
+    uint8_t* const copy = COPY ? copy_out : nullptr;
     __shared__ uint64_t s_off[FZH_CONCAT_MAX_SLOTS], s_sz[FZH_CONCAT_MAX_SLOTS];
     __shared__ uint64_t s_total;
     const int t = threadIdx.x;

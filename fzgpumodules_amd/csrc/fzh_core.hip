@@ -279,11 +279,12 @@ concat_copy_kernel(ConcatArgs a, uint8_t* __restrict__ out, const uint64_t* __re
 }
 
 // Concat and readback in one launch (body in fzh_concat.h).
+template <bool COPY>
 __global__ void __launch_bounds__(256)
 concat_readback_kernel(ConcatArgs a, int n, uint8_t* __restrict__ out, uint8_t* __restrict__ copy,
                        bool first_done, uint64_t* __restrict__ total, ReadbackArgs r, int nr,
                        uint8_t* __restrict__ mapped) {
-    concat_readback_body(a, n, out, copy, total, r, nr, mapped, blockIdx.x, gridDim.x,
+    concat_readback_body<COPY>(a, n, out, copy, total, r, nr, mapped, blockIdx.x, gridDim.x,
                          SizeOverride{first_done, false, 0, 0, 0});
 }
 
@@ -482,8 +483,9 @@ int concat_readback(hipStream_t s, const fzh_concat_slot* slots, int n, void* d_
     if (int rc = build_concat_args(slots, n, d_out, d_copy, !first_done, out_cap, d_total, entries, n_entries,
                                    d_mapped_dst, a, r, grid))
         return rc;
-    launch_k("concat_readback_kernel", concat_readback_kernel, dim3(grid), dim3(256), 0, s, a, n, (uint8_t*)d_out,
-             (uint8_t*)d_copy, first_done, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
+    auto* k = d_copy ? concat_readback_kernel<true> : concat_readback_kernel<false>;
+    launch_k("concat_readback_kernel", k, dim3(grid), dim3(256), 0, s, a, n, (uint8_t*)d_out, (uint8_t*)d_copy,
+             first_done, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
     FZH_CHECK_LAUNCH("concat_readback_kernel");
     return FZH_OK;
 }

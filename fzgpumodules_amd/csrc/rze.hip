@@ -117,6 +117,7 @@ void launch_rze_enc(hipStream_t s, const RzeEncArgs& a, const PlaceDesc* p) {
 // sizes before its chunk itself).  Raw chunks below `nshuf` (bit-shuffled
 // blocks) come from the scratch slot, other raw chunks straight from the
 // input.
+template <bool COPY>
 __device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c, uint32_t* s_sum,
                                                uint8_t* __restrict__ copy) {
     const uint8_t* __restrict__ in = d.in;
@@ -148,7 +149,7 @@ __device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c,
         limit = nbytes - (uint64_t)c * CS;
     }
     copy_to_unaligned16<256>(from, limit, out + dst, clean);
-    if (copy) {  // the stream's second place: what the encoder wrote of the header, too
+    if constexpr (COPY) {  // the stream's second place: what the encoder wrote of the header, too
         copy_to_unaligned16<256>(from, limit, copy + dst, clean);
         if (threadIdx.x == 0) {
             reinterpret_cast<uint32_t*>(copy + 8)[c] = size;
@@ -163,7 +164,7 @@ __device__ __forceinline__ void rze_pack_chunk(const RzePackDesc& d, uint32_t c,
         const uint64_t padded = (end + 3) & ~3ull;
         if ((uint64_t)threadIdx.x < padded - end) {
             out[end + threadIdx.x] = 0;
-            if (copy) copy[end + threadIdx.x] = 0;
+            if constexpr (COPY) copy[end + threadIdx.x] = 0;
         }
         if (threadIdx.x == 0) *d.out_size = padded;
     }
@@ -173,7 +174,7 @@ __global__ void __launch_bounds__(256) rze_pack_kernel(RzePackDesc d) {
     __shared__ uint32_t s_sum[4];
     const uint32_t c = xcd_swizzle(blockIdx.x, gridDim.x);
     if (c >= d.nc) return;  // uniform over the workgroup
-    rze_pack_chunk(d, c, s_sum, nullptr);
+    rze_pack_chunk<false>(d, c, s_sum, nullptr);
 }
 
 // The pack step and the pipeline's concat + readback in one launch:
@@ -181,13 +182,14 @@ __global__ void __launch_bounds__(256) rze_pack_kernel(RzePackDesc d) {
 // place), the rest lay out the other slots and serve the readback, with the
 // RZE stream's size summed from the clean sizes rather than read from the
 // size word the pack workgroups are still writing.
+template <bool COPY>
 __global__ void __launch_bounds__(256)
 rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__ out, uint8_t* __restrict__ copy,
                        uint64_t* __restrict__ total, ReadbackArgs r, int nr, uint8_t* __restrict__ mapped) {
     __shared__ uint32_t s_sum[4];
     const uint32_t b = blockIdx.x;
     if (b < d.nc) {
-        rze_pack_chunk(d, b, s_sum, copy ? copy + (d.out - out) : nullptr);
+        rze_pack_chunk<COPY>(d, b, s_sum, COPY ? copy + (d.out - out) : nullptr);
         return;
     }
     uint32_t sum;
@@ -200,7 +202,7 @@ rze_pack_concat_kernel(RzePackDesc d, ConcatArgs a, int n, uint8_t* __restrict__
     }
     const uint64_t end = 8ull + 4ull * d.nc + sum;
     const uint64_t size0 = (end + 3) & ~3ull;
-    concat_readback_body(a, n, out, copy, total, r, nr, mapped, b - d.nc, gridDim.x - d.nc,
+    concat_readback_body<COPY>(a, n, out, copy, total, r, nr, mapped, b - d.nc, gridDim.x - d.nc,
                          SizeOverride{true, true, size0, reinterpret_cast<uintptr_t>(d.out_size), size0});
 }
 
@@ -565,7 +567,8 @@ int rze_pack_concat_readback(hipStream_t s, const RzePackDesc& d, const fzh_conc
         return rc;
     if (n < 1 || slots[0].src != d.out)
         return fail(FZH_E_INVALID, "RZE pack + concat: slot 0 must be the RZE stream");
-    launch_k("rze_pack_concat_kernel", rze_pack_concat_kernel, dim3(d.nc + grid), dim3(256), 0, s, d, a, n,
+    auto* k = d_copy ? rze_pack_concat_kernel<true> : rze_pack_concat_kernel<false>;
+    launch_k("rze_pack_concat_kernel", k, dim3(d.nc + grid), dim3(256), 0, s, d, a, n,
              (uint8_t*)d_out, (uint8_t*)d_copy, d_total, r, n_entries, (uint8_t*)d_mapped_dst);
     FZH_CHECK_LAUNCH("rze_pack_concat_kernel");
     return FZH_OK;
