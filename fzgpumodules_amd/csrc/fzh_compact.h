@@ -40,9 +40,12 @@ inline CompactListT<V> compact_list(const PlaceDesc::List& l) {
 }
 
 // Counts (of all lists) up to which the place kernel sums those before each
-// workgroup itself.  39 Ki counts (301 x 203 x 157 doubles): 4.4 us against
-// 12.8 + 4.5 us and a launch gap with a one-workgroup scan; past that the
-// longest sum outgrows the scan's launches.
+// workgroup itself, beyond them a scan runs first.  One list, 1D floats of few
+// outliers, predictor and placement: 17000 counts 21.7 us (scan 31.9), 65000 83.8
+// (109.7); beyond the limit 70000 86.5 (scan 96.8), 131072 155 (161), 200000 235
+// (232), 262144 323 (304).  Doubles and lists of 1% cross at the same place.  The
+// last workgroups sum all counts, so the limit is below where the two meet: the
+// scan costs 4 to 11% more from there to 131072.
 constexpr uint32_t COMPACT_INLINE = 65536;
 
 // Workgroup `blk` of `nblk` of the placement.  excl: exclusive prefix (mod

@@ -113,7 +113,7 @@ int zero_bytes(hipStream_t s, void* p, size_t n) {
 // gridDim.y workgroups share each segment, 16-byte copies when both ends are
 // aligned (src/pipeline/concat_kernel.cu:27-61 semantics).  Bound by memory,
 // so a segment needs many workgroups and several loads in flight per thread:
-// 60 segments of 90 MiB in all took 651 us with one workgroup each, 33
+// 60 segments of 44 MiB in all took 651 us with one workgroup each, 33
 // us shared.
 __global__ void __launch_bounds__(256) gather_kernel(const fzh_copy_desc* __restrict__ d, int n) {
     const int seg = blockIdx.x;

@@ -395,13 +395,24 @@ int fzh_synth_power_law_f32(void* stream, float* d_out, uint64_t nx, uint64_t ny
  * benchmarks time whole stages).  While enabled, each launch of the chain's
  * main kernels outside stream capture is bracketed by a HIP event pair on
  * its own stream; fzh_kernel_timing_get waits for the recorded pairs and
- * returns the summed milliseconds and launch count under `name`:
+ * returns the summed milliseconds and launch count under `name`, the kernel's
+ * own without template arguments:
  * "minmax_partial_kernel", "lz1d_fwd_kernel" / "lz2d_fwd_kernel" /
- * "lz3d_fwd_kernel", "place_kernel", "scan_small_kernel", "rze_enc_kernel",
- * "rze_pack_kernel", "rze_offsets_kernel", "rze_dec_kernel",
- * "bin_count_kernel", "bin_place_kernel", "lz1d_inv_kernel" /
- * "lz2d_inv_kernel" / "lz3d_inv_kernel", "apply_patches_kernel",
- * "bitshuffle_kernel", "copy_kernel".  Enabling or disabling clears the
+ * "lz3d_fwd_kernel" ("lz1d_fwd64_kernel" and so on for doubles),
+ * "place_kernel", "scan_small_kernel" or "scan_reduce_kernel" /
+ * "scan_partials_kernel" / "scan_apply_kernel", "rze_enc_kernel",
+ * "rze_pack_kernel", "rze_offsets_kernel", "rze_dec_kernel", "hist_kernel",
+ * "huf_enc_kernel", "huf_pack_kernel", "huf_header_kernel", "huf_dec_kernel",
+ * "huf_dec_long_kernel" (32768 partitions and more of 1- and 2-byte symbols),
+ * "rle_enc_count_kernel", "rle_enc_write_kernel", "rle_enc_fix_kernel",
+ * "rle_dec_prep_kernel" / "rle_dec_reduce_kernel" / "rle_dec_apply_kernel" /
+ * "rle_dec_expand_kernel", "bin_check_kernel", "bin_count_kernel",
+ * "bin_place_kernel", "lz1d_inv_kernel" / "lz2d_inv_kernel" /
+ * "lz3d_inv_kernel", "apply_patches_kernel", "bitshuffle_kernel",
+ * "concat_readback_kernel", "copy_kernel".  In a pipeline a placement may run
+ * inside the next stage's launch ("rze_enc_place_kernel",
+ * "rle_enc_count_place_kernel") and the RZE pack inside the concat's
+ * ("rze_pack_concat_kernel").  Enabling or disabling clears the
  * totals.  The event records add a small gap between launches.            */
 int fzh_kernel_timing_enable(int on);
 int fzh_kernel_timing_get(const char* name, double* total_ms, uint64_t* count);
