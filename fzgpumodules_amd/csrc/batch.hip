@@ -700,11 +700,21 @@ int launch_rze(hipStream_t s, const Plan& p, const Plan* dp) {
     return FZH_OK;
 }
 
-int launch_huffman(hipStream_t s, const Plan& p, const Plan* dp) {
+int launch_histograms(hipStream_t s, const Plan& p, const Plan* dp) {
     const Huffman& h = p.huf;
     if (int rc = zero_bytes(s, h.freq, 4 * (size_t)p.F * h.bklen)) return rc;
     hist_batch_kernel<<<p.U, 256, 32 * (h.bklen + 1), s>>>(dp);
-    if (int rc = build_books_device(s, p.F, h.freq, h.bklen, h.n_of, h.bk4, h.rev, h.rev_stride, h.status)) return rc;
+    FZH_CHECK_LAUNCH("batch histograms");
+    return FZH_OK;
+}
+
+int launch_books(hipStream_t s, const Plan& p) {
+    const Huffman& h = p.huf;
+    return build_books_device(s, p.F, h.freq, h.bklen, h.n_of, h.bk4, h.rev, h.rev_stride, h.status);
+}
+
+int launch_huffman(hipStream_t s, const Plan& p, const Plan* dp) {
+    const Huffman& h = p.huf;
     huf_enc_batch_kernel<<<h.NW, 256, 4 * (4 * kHufCells + h.bklen), s>>>(dp);
     FZH_CHECK_LAUNCH("batch huffman");
     return FZH_OK;

@@ -133,6 +133,8 @@ int launch_value_base(hipStream_t s, const Plan& p, const Plan* dp, uint32_t gri
 int launch_lorenzo(hipStream_t s, const Plan& p, const Plan* dp, uint32_t grid, uint32_t tiles_per_unit);
 int launch_rze(hipStream_t s, const Plan& p, const Plan* dp);
 // Histograms, codebooks and partitions' codewords of every field.
+int launch_histograms(hipStream_t s, const Plan& p, const Plan* dp);
+int launch_books(hipStream_t s, const Plan& p);
 int launch_huffman(hipStream_t s, const Plan& p, const Plan* dp);
 int launch_scan(hipStream_t s, const Plan& p);
 int launch_finalize(hipStream_t s, const Plan& p, const Plan* dp);

@@ -231,7 +231,7 @@ class ChainSelectCompressor {
             last[choice_[c]] = c;
         }
         hipck(hipStreamSynchronize(s), "hipStreamSynchronize");  // chunks_ and the choices are ready
-        bool in_batch[FZS_NCHAINS] = {false, list[1].size() >= kBatchMin, list[2].size() >= huffmanBatchMin(E), false};
+        bool in_batch[FZS_NCHAINS] = {false, list[1].size() >= kBatchMin, list[2].size() >= kHuffmanMin, false};
         const auto batched = [&](int k) { return in_batch[k]; };
         std::vector<uint64_t> single;
         for (uint64_t c = 0; c < n; c++)
@@ -530,17 +530,11 @@ class ChainSelectCompressor {
     }
 
     static constexpr int kWorkers = 8;
-    static constexpr size_t kBatchMin = 2;  // fewer chunks of a chain run per chunk
-    // The same for chain 2.  Its batch builds the codebooks on the device, all
-    // at once but each by one lane: 0.4 ms for smooth chunks, 2.5 where every
-    // code of the alphabet occurs.  A pipeline builds on the host, 36 us a chunk
-    // and 0.4 ns a value with eight threads.  Batch / pipelines in ms: 64 chunks
-    // of 64 x 64 values of noise 2.5 / 2.7 (smooth 0.5 / 2.2), 32 2.7 / 1.7; of
-    // 256 x 256 48 3.5 / 3.9, 32 3.4 / 2.9, 2 3.1 / 0.5 (smooth 1.0 / 0.35); 16 of
-    // 1024 x 1024 smooth 3.3 / 3.2, 8 3.1 / 2.1.
-    static size_t huffmanBatchMin(uint64_t chunk_values) {
-        return std::max<size_t>(16, (size_t)std::ceil(2500.0 / (36.0 + 0.0004 * (double)chunk_values)));
-    }
+    static constexpr size_t kBatchMin = 2;  // fewer chunks of chain 1 run per chunk
+    // Of chain 2: its batch waits for the histograms, ms of pipelines / batch for 256
+    // x 256 noise: 2 0.56 / 0.67, 4 0.80 / 0.76, 8 1.3 / 0.79; smooth 2 0.36 / 0.44,
+    // 4 0.47 / 0.44, 8 0.91 / 0.43.
+    static constexpr size_t kHuffmanMin = 4;
     struct Worker {
         hipStream_t s = nullptr;
         Chain chain[FZS_NCHAINS];

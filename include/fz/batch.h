@@ -35,7 +35,8 @@ struct BatchConfig {
     float patch_capacity = 0.01f;
     // 0: codes go through Bitshuffle -> RZE; else HuffmanStage<uint16_t> with
     // this alphabet (coarse partitions; at least 2 x quant_radius with zigzag
-    // codes, at most 1024)
+    // codes, at most 1024).  Without graph mode the codebooks of a few fields
+    // are built on the host, which waits for the histograms.
     uint32_t huffman_bklen = 0;
 };
 
