@@ -62,9 +62,10 @@ struct BatchCompressor::Impl {
     // to every code of the alphabet); the host takes 11 to 120 us a book, here on up
     // to eight threads, and a wait.  Device / host, ms of a selector's call, fields of
     // 256 x 256 values of noise: 4 3.1 / 0.76, 64 3.7 / 1.8, 128 4.2 / 3.1, 256 5.2 / 5.7;
-    // smooth 128 1.29 / 1.08, 256 1.59 / 1.92; 64 x 64 smooth 64 0.47 / 0.49, 128 0.55 /
-    // 0.55, 256 0.59 / 0.83.
-    static constexpr uint32_t kHostBooks = 128;
+    // smooth 64 1.15 / 0.71, 128 1.29 / 1.08, 256 1.59 / 1.92; 64 x 64 smooth 64 0.47 /
+    // 0.49, 128 0.55 / 0.55, 256 0.59 / 0.83.  A handle's first call pays for new host
+    // memory: 24 smooth chunks 1.45 / 1.40, 114 2.05 / 2.30.
+    static constexpr uint32_t kHostBooks = 64;
     static size_t piece(size_t bytes) { return align_to(std::max<size_t>(bytes, 256), 256); }
     static constexpr size_t kKeep = 64 << 20;
     // Starts a plan of `bytes` (a sum of pieces).

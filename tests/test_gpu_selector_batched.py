@@ -62,8 +62,8 @@ def _parse(blob, n):
     return out, blob[oc:oc + n]
 
 
-# the Huffman chain is batched from 4 chunks on, with codebooks of the host up to 128
-HUFFMAN = [((4096,), 4), ((64, 64), 3), ((64, 64), 5), ((4096,), 128), ((64, 64), 129), ((8, 24, 64), 131),
+# the Huffman chain is batched from 4 chunks on, with codebooks of the host up to 64
+HUFFMAN = [((4096,), 4), ((64, 64), 3), ((64, 64), 5), ((4096,), 64), ((64, 64), 65), ((8, 24, 64), 67),
            ((256, 256), 41), ((16, 64, 64), 4), ((3, 20, 4096), 18)]
 
 
