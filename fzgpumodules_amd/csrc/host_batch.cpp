@@ -12,7 +12,6 @@
 #include <new>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -130,7 +129,7 @@ struct BatchCompressor::Impl {
         th.reserve(W);
         try {
             for (size_t w = 1; w < W; w++) th.emplace_back(build, w, W);
-        } catch (const std::system_error&) {  // no more threads: this one does their share
+        } catch (const std::exception&) {  // no more threads: this one does their share
         }
         build(0, W);
         for (size_t w = th.size() + 1; w < W; w++) build(w, W);
